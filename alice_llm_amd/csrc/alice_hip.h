@@ -359,6 +359,6 @@ int alice_sample(const float* logits, int* out, const float* uniform, void* work
 
 // internal
 int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype,
-                         int M, int N, int K, int epi, float epi_param, int full_precision,
+                         int M, int N, int K, int epi, float epi_param, int split_k, int full_precision,
                          hipStream_t stream);
 #endif

@@ -3,12 +3,13 @@
 #include "alice_hip.h"
 
 int alice_linear_split_hint_frag(int M, int N, int K);
+int alice_linear_split_hint_generic(int M, int N, int K);
 int alice_linear_frag(const void* x, int x_dtype, const void* w, void* y, int y_dtype, int M, int N, int K,
                       int epi, float epi_param, int split_k, int variant, int x_layout, int y_layout,
                       hipStream_t stream);
 
 extern "C" int alice_linear_split_hint(int M, int N, int K, int w_layout) {
-  return w_layout == ALICE_LAYOUT_FRAG16 ? alice_linear_split_hint_frag(M, N, K) : 1;
+  return w_layout == ALICE_LAYOUT_FRAG16 ? alice_linear_split_hint_frag(M, N, K) : alice_linear_split_hint_generic(M, N, K);
 }
 
 extern "C" int alice_linear(const void* x, int x_dtype, const void* w, int w_dtype, int w_layout, void* y,
@@ -19,10 +20,9 @@ extern "C" int alice_linear(const void* x, int x_dtype, const void* w, int w_dty
   if (w_layout == ALICE_LAYOUT_ROW) {
     ALICE_CHECK(variant == ALICE_LINEAR_AUTO || variant == ALICE_LINEAR_GENERIC,
                 "linear: row-major weights run on the generic kernel only");
-    ALICE_CHECK(split_k == 1, "linear: the generic kernel produces no partial sums");
     ALICE_CHECK(x_layout == ALICE_LAYOUT_ROW && y_layout == ALICE_LAYOUT_ROW, "linear: the generic kernel reads and writes rows");
     return alice_linear_generic(x, x_dtype, w, w_dtype, y, y_dtype, M, N, K, epilogue, epi_param,
-                                full_precision, stream);
+                                split_k, full_precision, stream);
   }
   if (w_layout == ALICE_LAYOUT_FRAG16) {
     ALICE_CHECK(w_dtype == DT_BF16, "linear: the fragment layout holds bfloat16 only");

@@ -1,6 +1,6 @@
 // Matrix product y[M, N] = x[M, K] . W[N, K]^T for every combination of 32-bit and bfloat16
-// operands, with plain 32-bit fused multiply-adds and 32-bit accumulation: the kernel of the
-// true 32-bit path, and the fallback of the bfloat16 path for shapes its MFMA kernels refuse.
+// operands, with 32-bit products and 32-bit accumulation: the kernels of the true 32-bit path, and
+// the fallback of the bfloat16 path for matrices that stay in 32-bit.
 //
 // Weight layout and orientation as in the reference: row-major [out, in], y[r] = sum_c W[r,c] x[c]
 // (gguf.rs:4063-4074, f32_matvec).  Epilogues: none; GeGLU gelu_tanh(gate) * up with W = [gate; up]
@@ -10,175 +10,334 @@
 
 namespace {
 
-constexpr int BM = 64, BN = 64, BK = 16;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// A block computes a 64 x 64 tile.  Its 64 columns are two runs of 32: columns [n0, n0+32) and
-// [n1, n1+32).  Without an epilogue n1 = n0 + 32; with GeGLU the first run are gate rows j0.. and
-// the second the up rows N + j0.. of the stacked weight, so that a thread holds gate and up of the
-// same output column.  The k loop runs in order, so a result does not depend on M or on the tile.
-template <typename TA, typename TW, typename TO, int EPI, bool FULL>
-__global__ __launch_bounds__(256) void linear_tiled_kernel(const TA* __restrict__ A, const TW* __restrict__ W,
-                                                           TO* __restrict__ Y, int M, int N, int K, float epi) {
-  __shared__ float As[BK][BM + 4];
-  __shared__ float Bs[BK][BN + 4];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int m0 = blockIdx.y * BM;
-  const int wrows = EPI == ALICE_EPI_GEGLU ? 2 * N : N;      // rows of W
-  int n0, n1;
-  if (EPI == ALICE_EPI_GEGLU) { n0 = blockIdx.x * 32; n1 = N + n0; }
-  else { n0 = blockIdx.x * 64; n1 = n0 + 32; }
-  const int lim0 = EPI == ALICE_EPI_GEGLU ? N : wrows;       // first run must stay below this row
+constexpr int BK = 32;       // inner elements a stage
+constexpr int LROW = BK + 4; // row length of a stage in LDS: 16-byte pieces of 16 neighbouring rows lie in different banks
 
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+// Four neighbouring elements of a row as float32.  VEC: in one load (rows start at multiples of four elements on memory
+// aligned for them, K is a multiple of four); else one by one, none beyond the row's end.  Loads are unconditional: one
+// behind a condition would be waited for where the ways join.
+template <typename T> __device__ __forceinline__ f32x4 load4(const T* __restrict__ p);
+template <> __device__ __forceinline__ f32x4 load4<float>(const float* __restrict__ p) { return *reinterpret_cast<const f32x4*>(p); }
+template <> __device__ __forceinline__ f32x4 load4<bf16_t>(const bf16_t* __restrict__ p) {
+  const uint2 w = *reinterpret_cast<const uint2*>(p);
+  return f32x4{bf16_bits_to_f32(w.x & 0xffffu), bf16_bits_to_f32(w.x >> 16), bf16_bits_to_f32(w.y & 0xffffu), bf16_bits_to_f32(w.y >> 16)};
+}
+template <typename T, bool VEC>
+__device__ __forceinline__ f32x4 load_row4(const T* __restrict__ row, int k, int K) {
+  if constexpr (VEC) return load4<T>(row + min(k, K - 4));
+  return f32x4{load_f32(row, min(k, K - 1)), load_f32(row, min(k + 1, K - 1)), load_f32(row, min(k + 2, K - 1)), load_f32(row, min(k + 3, K - 1))};
+}
 
-  const int lr = tid >> 2, lk = (tid & 3) * 4;               // loader: row 0..63, k offset 0,4,8,12
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    {
-      const int m = m0 + lr;
+// More than 16 tokens: the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: 32-bit products and sums, the rate of the
+// vector unit's FMA at a quarter of its register reads).  A block of 2 x 2 waves takes 32 TM tokens by 32 TN rows of W, a
+// wave 16 TM by 16 TN; both operands go through LDS 32 inner elements at a time in two buffers (one barrier a stage), the
+// next stage on its way from memory meanwhile.  A lane reads 16-byte pieces: lane group g of a 16-element chunk holds the
+// elements 4 g .. 4 g + 3 of its row, and product i of the chunk takes element i of every group, the same permutation of
+// the inner dimension on both sides.  W is the first operand, so that a lane ends up with four neighbouring outputs of a
+// token.  With GeGLU the first half of a wave's rows are gate rows, the second half the up rows of the same outputs.
+// blockIdx: the tiles of one set of W rows are neighbours on one XCD, whose L2 then serves W's rows to all of them.
+// split: slices of the inner dimension, slice z to Y + z M N (float32 sums that the residual add adds up).
+//
+// What bounds it: the matrix instruction (157 TFLOP/s at 256 CUs).  A product of 500 tokens with 18,432 x 2,304 rows
+// and GeGLU takes 438 us (97 TFLOP/s), the down product of 2,304 x 9,216 188 us (113) in slices, against 1,576 and
+// 1,444 us with a 64 x 64 tile of scalar FMAs, which read an LDS operand for every two of them.
+template <typename TA, typename TW, typename TO, int TM, int TN, bool VEC>
+__global__ __launch_bounds__(256) void linear_mfma32_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y,
+                                                            int M, int N, int K, int kslice, int mt, int nt, int epi, float param,
+                                                            int full, int wide) {
+  constexpr int BM = 32 * TM, BN = 32 * TN;
+  constexpr int YROW = BN + 4;
+  static_assert(BM * YROW <= 2 * (BM + BN) * LROW, "the outputs do not fit where the operands were");
+  __shared__ __align__(16) float lds[2 * (BM + BN) * LROW];
+  auto As = reinterpret_cast<float (*)[BM][LROW]>(lds);
+  auto Bs = reinterpret_cast<float (*)[BN][LROW]>(lds + 2 * BM * LROW);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+  const int wm = wave & 1, wn = wave >> 1;
+
+  // tile of this block: neighbours in m first, a run of tiles an XCD (blocks go to the 8 XCDs in turn)
+  const int total = mt * nt, per = (total + 7) >> 3;
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (tile >= total) return;                                  // the whole block: no barrier is missed
+  const int m0 = (tile % mt) * BM, nb = tile / mt;
+  const bool geglu = epi == ALICE_EPI_GEGLU;
+  const int n0 = nb * (geglu ? BN / 2 : BN);
+  const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);
+
+  // loaders: 16-byte piece `id` of a stage is row id / 8, elements (id % 8) * 4
+  const int lk = (tid & 7) * 4;
+  const TA* arow[TM];                                         // rows beyond the last are read as the last and not written
+  const TW* wrow[TN];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int k = k0 + lk + i;
-        As[lk + i][lr] = (m < M && k < K) ? load_f32(A, (size_t)m * K + k) : 0.f;
-      }
-      const int run = lr >> 5, c = lr & 31;
-      const int n = (run ? n1 : n0) + c;
-      const bool ok = run ? (n < wrows) : (n < lim0);
+  for (int j = 0; j < TM; ++j) arow[j] = A + (size_t)min(m0 + (tid >> 3) + 32 * j, M - 1) * K;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int k = k0 + lk + i;
-        Bs[lk + i][lr] = (ok && k < K) ? load_f32(W, (size_t)n * K + k) : 0.f;
+  for (int j = 0; j < TN; ++j) {
+    const int r = (tid >> 3) + 32 * j;
+    int row = min(n0 + r, N - 1);
+    if (geglu) {                                              // a wave's 16 TN rows: gate rows, then up rows of the same outputs
+      const int w = r / (16 * TN), rr = r % (16 * TN), half = rr / (8 * TN);
+      row = half * N + min(n0 + w * 8 * TN + rr % (8 * TN), N - 1);
+    }
+    wrow[j] = W + (size_t)row * K;
+  }
+  f32x4 pa[TM], pb[TN];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int j = 0; j < TM; ++j) pa[j] = load_row4<TA, VEC>(arow[j], k0 + lk, K);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) pb[j] = load_row4<TW, VEC>(wrow[j], k0 + lk, K);
+  };
+  auto stage = [&](int buf, int k0) {
+    if (k0 + BK > k_end) {                                    // the last stage of a slice: nothing beyond its end
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool in = k0 + lk + e < k_end;
+#pragma unroll
+        for (int j = 0; j < TM; ++j) pa[j][e] = in ? pa[j][e] : 0.f;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) pb[j][e] = in ? pb[j][e] : 0.f;
       }
     }
-    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < BK; ++k) {
-      float a[4], b[4];
+    for (int j = 0; j < TM; ++j) *reinterpret_cast<f32x4*>(&As[buf][(tid >> 3) + 32 * j][lk]) = pa[j];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[k][ty * 4 + i];
-      b[0] = Bs[k][tx * 2];
-      b[1] = Bs[k][tx * 2 + 1];
-      b[2] = Bs[k][32 + tx * 2];
-      b[3] = Bs[k][33 + tx * 2];
+    for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4*>(&Bs[buf][(tid >> 3) + 32 * j][lk]) = pb[j];
+  };
+
+  f32x4 acc[TN][TM];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < TN; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  fetch(k_begin);
+  stage(0, k_begin);
+  __syncthreads();
+  int cur = 0;
+  for (int k0 = k_begin; k0 < k_end; k0 += BK) {
+    const bool more = k0 + BK < k_end;
+    if (more) fetch(k0 + BK);
+#pragma unroll
+    for (int ch = 0; ch < BK; ch += 16) {
+      f32x4 wf[TN], xf[TM];
+#pragma unroll
+      for (int i = 0; i < TN; ++i) wf[i] = *reinterpret_cast<const f32x4*>(&Bs[cur][(wn * TN + i) * 16 + c][ch + g * 4]);
+#pragma unroll
+      for (int j = 0; j < TM; ++j) xf[j] = *reinterpret_cast<const f32x4*>(&As[cur][(wm * TM + j) * 16 + c][ch + g * 4]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], xf[j][e], acc[i][j], 0, 0, 0);
     }
+    if (more) stage(cur ^ 1, k0 + BK);                                 // read two stages ago, by waves that have passed a barrier since
     __syncthreads();
+    cur ^= 1;
   }
 
+  // The outputs go through LDS (the last barrier has passed): 16-byte pieces of a token's row, and the epilogue's functions stand
+  // in the code for four elements and not for a lane's 16 TM TN / 4 (which took 16,000 instructions).
+  auto Ys = reinterpret_cast<float (*)[YROW]>(lds);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
-    if (EPI == ALICE_EPI_GEGLU) {
+  for (int j = 0; j < TM; ++j)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int n = n0 + tx * 2 + j;
-        if (n < N) {
-          float g = acc[i][j], u = acc[i][j + 2];
-          store_f32(Y, (size_t)m * N + n, gated_act(g, u, epi, FULL));
-        }
-      }
+    for (int i = 0; i < TN; ++i) *reinterpret_cast<f32x4*>(&Ys[(wm * TM + j) * 16 + c][(wn * TN + i) * 16 + g * 4]) = acc[i][j];
+  __syncthreads();
+  TO* __restrict__ y = Y + (size_t)blockIdx.y * M * N;
+  const int pieces = geglu ? BN / 8 : BN / 4;                 // of a row
+#pragma unroll 1
+  for (int id = tid; id < BM * pieces; id += 256) {
+    const int r = id / pieces, q = (id % pieces) * 4, m = m0 + r, n = n0 + q;
+    if (m >= M || n >= N) continue;
+    f32x4 v;
+    if (geglu) {
+      const float* p = &Ys[r][q / (8 * TN) * 16 * TN + q % (8 * TN)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = gated_act(p[e], p[8 * TN + e], param, full);
     } else {
+      v = *reinterpret_cast<const f32x4*>(&Ys[r][q]);
+      if (epi == ALICE_EPI_SOFTCAP) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = (j < 2 ? n0 : n1) + tx * 2 + (j & 1);
-        if (n < N) {
-          float v = acc[i][j];
-          if (EPI == ALICE_EPI_SOFTCAP) v = unary_act(v, epi, FULL);
-          store_f32(Y, (size_t)m * N + n, v);
-        }
+        for (int e = 0; e < 4; ++e) v[e] = unary_act(v[e], param, full);
       }
     }
+    TO* dst = y + (size_t)m * N + n;
+    if constexpr (sizeof(TO) == 4) {
+      if (wide) {                                             // rows of whole, aligned pieces
+        *reinterpret_cast<f32x4*>(dst) = v;
+        continue;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) store_f32(dst, e, v[e]);
   }
 }
 
-// Up to 8 tokens: one wave per output feature streams that feature's weight row once (coalesced, four
-// elements a lane a step) against all the tokens' activations; the lanes' partial sums meet in a fixed
-// shuffle tree, so a token's result does not depend on the others.  For GeGLU the wave takes the gate
-// row and the up row of its feature.
-template <typename TA, typename TW, typename TO, int EPI, bool FULL, int MB>
-__global__ __launch_bounds__(256) void linear_rows_kernel(const TA* __restrict__ A, const TW* __restrict__ W,
-                                                          TO* __restrict__ Y, int M, int N, int K, float epi) {
-  const int lane = threadIdx.x & 63, n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  constexpr int NR = EPI == ALICE_EPI_GEGLU ? 2 : 1;
-  float acc[NR][MB];
+// Tile and number of slices for a product.  Estimated microseconds: rounds of blocks over the CUs times a block's products at
+// a CU's 0.61 TFLOP/s (less for small tiles, which read LDS more often, and for a CU with a single block, which waits for
+// its own barriers), not less than reading W takes; slices cost writing and reading their sums.
+struct Plan {
+  int tm, tn, split;
+};
+Plan plan_mfma32(int M, int N, int K, bool geglu, int max_split) {
+  static const struct { int tm, tn; float eff; } tiles[] = {{4, 4, 0.85f}, {2, 4, 0.80f}, {2, 2, 0.70f}, {1, 2, 0.50f}};
+  Plan best{2, 2, 1};
+  float best_us = 1e30f;
+  for (const auto& t : tiles) {
+    const int mt = ceil_div(M, 32 * t.tm), nt = ceil_div(N, geglu ? 16 * t.tn : 32 * t.tn);
+    for (int s = 1; s <= max_split; ++s) {
+      const int ks = ceil_div(ceil_div(K, s), BK) * BK;
+      if (s > 1 && (ks < 256 || (long)ks * (s - 1) >= K)) continue;      // no slice without elements
+      const float rounds = (float)ceil_div((long)mt * nt * s, 256);
+      const float block_us = 2.f * (32 * t.tm) * (32 * t.tn) * (float)ks / (0.614e6f * t.eff) + 2.f;
+      float us = rounds * block_us * (rounds < 2.f ? 1.25f : 1.f);
+      us = fmaxf(us, (geglu ? 2.f : 1.f) * N * (float)K * 4.f / 4.5e6f);
+      if (s > 1) us += 2.f * s * (float)M * N * 4.f / 4.0e6f;
+      if (us < best_us) { best_us = us; best = Plan{t.tm, t.tn, s}; }
+    }
+  }
+  return best;
+}
+constexpr int MAX_SPLIT = 8;
+
+// Up to 16 tokens: the tokens are the columns of the same matrix instruction, the rows of W its rows.  A block takes 16 R rows
+// (with GeGLU 16 gate rows and the up rows of the same outputs), its four waves every fourth chunk of 32 inner elements of
+// its slice; their sums meet in LDS.  W goes straight from memory into the instruction's operand, 128 bytes of a row a
+// chunk, the next two chunks on their way while two are multiplied; the tokens' elements come through the L1.  A token's
+// result depends on no other token.
+//
+// What bounds it: reading W.  At 4 tokens (2B shape): gate and up (170 MB) 42 us, 4.1 TB/s, the output head (2.36 GB)
+// 405 us, 5.8; a wave a row on FMAs, which read every token's elements again for every row, 49 and 652 us.
+template <typename T>
+__device__ __forceinline__ void load8(const T* __restrict__ p, f32x4* v);
+template <> __device__ __forceinline__ void load8<float>(const float* __restrict__ p, f32x4* v) {
+  v[0] = *reinterpret_cast<const f32x4*>(p);
+  v[1] = *reinterpret_cast<const f32x4*>(p + 4);
+}
+template <> __device__ __forceinline__ void load8<bf16_t>(const bf16_t* __restrict__ p, f32x4* v) {
+  const uint4 w = *reinterpret_cast<const uint4*>(p);
+  v[0] = f32x4{bf16_bits_to_f32(w.x & 0xffffu), bf16_bits_to_f32(w.x >> 16), bf16_bits_to_f32(w.y & 0xffffu), bf16_bits_to_f32(w.y >> 16)};
+  v[1] = f32x4{bf16_bits_to_f32(w.z & 0xffffu), bf16_bits_to_f32(w.z >> 16), bf16_bits_to_f32(w.w & 0xffffu), bf16_bits_to_f32(w.w >> 16)};
+}
+
+template <typename TA, typename TW, typename TO, int R>
+__global__ __launch_bounds__(256) void linear_rows_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y, int M,
+                                                          int N, int K, int kslice, int epi, float param, int full) {
+  constexpr int U = 2;                                        // chunks a step
+  __shared__ __align__(16) f32x4 red[4][R][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+  const bool geglu = R == 2 && epi == ALICE_EPI_GEGLU;
+  const int n0 = blockIdx.x * (geglu ? 16 : 16 * R);
+  const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);
+  const TW* wrow[R];                                          // rows and tokens beyond the last are read as the last and not written
 #pragma unroll
-  for (int r = 0; r < NR; ++r)
+  for (int r = 0; r < R; ++r) wrow[r] = W + (size_t)(geglu ? r * N + min(n0 + c, N - 1) : min(n0 + r * 16 + c, N - 1)) * K + g * 8;
+  const TA* arow = A + (size_t)min(c, M - 1) * K + g * 8;
+
+  f32x4 acc[R][2];
 #pragma unroll
-    for (int m = 0; m < MB; ++m) acc[r][m] = 0.f;
-  const int K4 = K & ~3;
-  for (int k = lane * 4; k < K4; k += 256) {
-    float w[NR][4];
+  for (int r = 0; r < R; ++r) acc[r][0] = acc[r][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 w[U][R][2], x[U][2], wn[U][R][2], xn[U][2];
+  const int k_last = K - 32;                                  // (K is a multiple of 8 and at least 32)
+  auto fetch = [&](int k0) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r)
+    for (int u = 0; u < U; ++u) {
+      const int k = min(k0 + u * 128, k_last + 24 - g * 8);   // stays inside the row: lane group g reads k + 8 g .. + 7
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[r][e] = load_f32(W, (size_t)(n + r * N) * K + k + e);
+      for (int r = 0; r < R; ++r) load8<TW>(wrow[r] + k, wn[u][r]);
+      load8<TA>(arow + k, xn[u]);
+    }
+  };
+  int k0 = k_begin + wave * 32;
+  if (k0 < k_end) fetch(k0);
+  for (; k0 < k_end; k0 += U * 128) {
 #pragma unroll
-    for (int m = 0; m < MB; ++m) {
-      if (m < M) {
+    for (int u = 0; u < U; ++u) {
+      // beyond the slice's end: zeros on both sides
+      const bool in = k0 + u * 128 + g * 8 < k_end;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float xv = load_f32(A, (size_t)m * K + k + e);
 #pragma unroll
-          for (int r = 0; r < NR; ++r) acc[r][m] = fmaf(w[r][e], xv, acc[r][m]);
+          for (int r = 0; r < R; ++r) w[u][r][i][e] = in ? wn[u][r][i][e] : 0.f;
+          x[u][i][e] = in ? xn[u][i][e] : 0.f;
         }
       }
     }
+    if (k0 + U * 128 < k_end) fetch(k0 + U * 128);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int r = 0; r < R; ++r) acc[r][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u][r][i][e], x[u][i][e], acc[r][e & 1], 0, 0, 0);
   }
-  if (lane < K - K4) {                                       // up to three columns beyond the last whole group of four
-    const int k = K4 + lane;
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
-      if (m < M) {
-        const float xv = load_f32(A, (size_t)m * K + k);
+  for (int r = 0; r < R; ++r) red[wave][r][lane] = acc[r][0] + acc[r][1];
+  __syncthreads();
+  if (wave >= (geglu ? 1 : R) || c >= M) return;
+  f32x4 v[R];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) acc[r][m] = fmaf(load_f32(W, (size_t)(n + r * N) * K + k), xv, acc[r][m]);
-      }
-  }
+  for (int r = 0; r < R; ++r) v[r] = (red[0][r][lane] + red[1][r][lane]) + (red[2][r][lane] + red[3][r][lane]);
+  if (R == 2 && !geglu && wave == 1) v[0] = v[R - 1];
+  const int n = n0 + (geglu ? 0 : wave * 16) + g * 4;
+  TO* y = Y + (size_t)blockIdx.y * M * N + (size_t)c * N;
 #pragma unroll
-  for (int m = 0; m < MB; ++m) {
-    if (m >= M) continue;
-    float v[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) v[r] = wave_sum(acc[r][m]);
-    if (lane == 0) {
-      float o = v[0];
-      if (EPI == ALICE_EPI_GEGLU) o = gated_act(v[0], v[NR - 1], epi, FULL);
-      if (EPI == ALICE_EPI_SOFTCAP) o = unary_act(o, epi, FULL);
-      store_f32(Y, (size_t)m * N + n, o);
-    }
+  for (int e = 0; e < 4; ++e) {
+    if (n + e >= N) continue;
+    float o = v[0][e];
+    if (geglu) o = gated_act(o, v[R - 1][e], param, full);
+    if (epi == ALICE_EPI_SOFTCAP) o = unary_act(o, param, full);
+    store_f32(y, n + e, o);
   }
 }
 
-template <typename TA, typename TW, typename TO, bool FULL>
-int launch_rows(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, hipStream_t stream) {
-  const int grid = ceil_div(N, 4);
-#define GO(E, MB) linear_rows_kernel<TA, TW, TO, E, FULL, MB><<<grid, 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, epi_param)
-#define BY_M(E) do { if (M <= 1) GO(E, 1); else if (M <= 2) GO(E, 2); else if (M <= 4) GO(E, 4); else GO(E, 8); } while (0)
-  if (epi == ALICE_EPI_NONE) BY_M(ALICE_EPI_NONE);
-  else if (epi == ALICE_EPI_GEGLU) BY_M(ALICE_EPI_GEGLU);
-  else BY_M(ALICE_EPI_SOFTCAP);
-#undef BY_M
+// Slices of the inner dimension for up to 16 tokens: two blocks a CU where the rows alone do not give them, slices of at
+// least 512 elements (2,304 rows by 9,216 and by 2,048 at 4 tokens: 16 us on average in four, 30 in one with a wave a row).
+int rows_split(int N, int K) { return max(1, min(min(ceil_div(512, ceil_div(N, 16)), K / 512), 8)); }
+bool rows_cover(int M, int K) { return M <= 16 && K % 8 == 0 && K >= 32; }
+
+template <typename TA, typename TW, typename TO>
+int launch_rows(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split,
+                hipStream_t stream) {
+  const int kslice = ceil_div(ceil_div(K, split), 128) * 128;
+#define GO(R, BLOCKS) linear_rows_kernel<TA, TW, TO, R><<<dim3(BLOCKS, split), 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, kslice, epi, epi_param, full)
+  if (epi == ALICE_EPI_GEGLU) GO(2, ceil_div(N, 16));
+  else if (N >= 16384) GO(2, ceil_div(N, 32));                // enough blocks: a token's elements serve 32 rows
+  else GO(1, ceil_div(N, 16));
 #undef GO
   ALICE_LAUNCH_CHECK();
   return 0;
 }
 
-template <typename TA, typename TW, typename TO, bool FULL>
-int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param,
+template <typename TA, typename TW, typename TO>
+int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split,
                  hipStream_t stream) {
-  dim3 grid(epi == ALICE_EPI_GEGLU ? ceil_div(N, 32) : ceil_div(N, 64), ceil_div(M, BM));
-#define GO(E) linear_tiled_kernel<TA, TW, TO, E, FULL><<<grid, 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, epi_param)
-  if (epi == ALICE_EPI_NONE) GO(ALICE_EPI_NONE);
-  else if (epi == ALICE_EPI_GEGLU) GO(ALICE_EPI_GEGLU);
-  else GO(ALICE_EPI_SOFTCAP);
+  Plan p = plan_mfma32(M, N, K, epi == ALICE_EPI_GEGLU, 1);
+  if (split > 1) {                                            // the tile that goes best with this many slices
+    const Plan q = plan_mfma32(M, N, K, false, MAX_SPLIT);
+    if (q.split == split) p = q;
+  }
+  const int vec = K % 4 == 0 && ((uintptr_t)x & (4 * sizeof(TA) - 1)) == 0 && ((uintptr_t)w & (4 * sizeof(TW) - 1)) == 0;
+  if (!vec) p.tm = p.tn = 2;                                  // one tile for rows that are no multiples of four elements
+  const int kslice = ceil_div(ceil_div(K, split), BK) * BK;
+  const int BM = 32 * p.tm, cols = epi == ALICE_EPI_GEGLU ? 16 * p.tn : 32 * p.tn;
+  const int mt = ceil_div(M, BM), nt = ceil_div(N, cols);
+  ALICE_CHECK((long)mt * nt < (1l << 30), "linear: too many tiles for one launch");
+  const int wide = N % 4 == 0 && ((uintptr_t)y & 15) == 0;
+  dim3 grid(8 * ceil_div((long)mt * nt, 8), split);
+#define GO(TM, TN, VEC) linear_mfma32_kernel<TA, TW, TO, TM, TN, VEC><<<grid, 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, kslice, mt, nt, epi, epi_param, full, wide)
+  if (!vec) GO(2, 2, false);
+  else if (p.tm == 4) GO(4, 4, true);
+  else if (p.tm == 2 && p.tn == 4) GO(2, 4, true);
+  else if (p.tm == 2) GO(2, 2, true);
+  else GO(1, 2, true);
 #undef GO
   ALICE_LAUNCH_CHECK();
   return 0;
@@ -186,25 +345,27 @@ int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int
 
 }  // namespace
 
+// Into how many slices of the inner dimension a product without an epilogue is best cut.
+int alice_linear_split_hint_generic(int M, int N, int K) {
+  return rows_cover(M, K) ? rows_split(N, K) : plan_mfma32(M, N, K, false, MAX_SPLIT).split;
+}
+
 int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype,
-                         int M, int N, int K, int epi, float epi_param, int full_precision,
+                         int M, int N, int K, int epi, float epi_param, int split_k, int full_precision,
                          hipStream_t stream) {
   ALICE_CHECK(dtype_ok(x_dtype) && dtype_ok(w_dtype) && dtype_ok(y_dtype), "linear: unknown dtype");
   ALICE_CHECK(M >= 0 && N > 0 && K > 0, "linear: bad sizes M=%d N=%d K=%d", M, N, K);
   ALICE_CHECK(epi == ALICE_EPI_NONE || epi == ALICE_EPI_GEGLU || epi == ALICE_EPI_SOFTCAP,
               "linear: unknown epilogue %d", epi);
   ALICE_CHECK(epi != ALICE_EPI_SOFTCAP || epi_param > 0.f || epi_param == ALICE_UNARY_RELU2 || epi_param == ALICE_UNARY_SILU, "linear: softcap must be positive");
-  ALICE_CHECK(ceil_div(M, BM) <= 65535, "linear: M=%d has too many row tiles for one launch", M);
+  ALICE_CHECK(split_k == 1 || (epi == ALICE_EPI_NONE && y_dtype == DT_F32), "linear: partial sums are float32 and take no epilogue");
+  ALICE_CHECK(split_k >= 1 && split_k <= MAX_SPLIT, "linear: %d slices of the inner dimension are outside 1..%d", split_k, MAX_SPLIT);
   if (M == 0) return 0;
   int rc = 0;
-  const bool rows = M <= 8 && N >= 64;                       // few tokens: stream each weight row once
+  const bool rows = rows_cover(M, K) && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
   DISPATCH_DTYPE(x_dtype, TA, DISPATCH_DTYPE(w_dtype, TW, DISPATCH_DTYPE(y_dtype, TO, {
-    if (rows)
-      rc = full_precision ? launch_rows<TA, TW, TO, true>(x, w, y, M, N, K, epi, epi_param, stream)
-                          : launch_rows<TA, TW, TO, false>(x, w, y, M, N, K, epi, epi_param, stream);
-    else
-      rc = full_precision ? launch_tiled<TA, TW, TO, true>(x, w, y, M, N, K, epi, epi_param, stream)
-                          : launch_tiled<TA, TW, TO, false>(x, w, y, M, N, K, epi, epi_param, stream);
+    rc = rows ? launch_rows<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream)
+              : launch_tiled<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
   })));
   return rc;
 }
