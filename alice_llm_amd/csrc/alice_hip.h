@@ -145,6 +145,15 @@ int alice_attention_tiled(const void* q, const void* k_pool, const void* v_pool,
                           int chunk, int keep_first, const float* bias_slopes, const float* sink,
                           const float* vrot_cos, const float* vrot_sin, const float* gate, int gate_stride,
                           int gate_mode, float out_scale, int heads_per_wave, hipStream_t stream);
+// Causal attention of the 32-bit path over a row-major cache on the 32-bit matrix instruction, with a window and a softcap
+// (attention_f32.hip): head sizes 64, 128 and 256, groups of at most 16 heads, pages of whole tiles of 16 positions.
+// splits > 1 spreads a tile's keys over that many blocks; work then holds T * nH * splits * (d + 2) floats.
+int alice_attention_f32_supported(int nH, int nKV, int d, int page_size);
+int alice_attention_f32_splits(int tiles, int nKV, int max_keys);
+int alice_attention_f32(const float* q, const float* k_pool, const float* v_pool, float* out, const int* positions,
+                        const int* cu_seqlens, const int* block_table, int bt_stride, int T, int n_seqs, int single_tokens,
+                        int nH, int nKV, int d, int page_size, float scale, float softcap, int window, int splits, float* work,
+                        hipStream_t stream);
 // alice_attention_masked's result for single tokens with the keys split over blocks (attention_split.hip), either
 // dtype, 32-bit arithmetic; max_keys: the most keys any token of the step sees; work: alice_attention_split_workspace
 // floats (runs = alice_attention_split_runs(max_keys)).

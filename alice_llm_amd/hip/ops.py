@@ -60,6 +60,9 @@ def _declare(lib) -> None:
         "alice_attention_prefill": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, F, I, I, I, P, P],
         "alice_attention_decode": [P, P, P, P, P, P, P, I, I, I, I, I, I, F, F, I, I, I, P, I, P, P],
         "alice_attention_generic": [P, I, P, P, P, P, P, P, I, I, I, I, I, I, F, F, I, P, I, I, P, I, P],
+        "alice_attention_f32_supported": [I, I, I, I],
+        "alice_attention_f32_splits": [I, I, I],
+        "alice_attention_f32": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, I, I, P, P],
         "alice_head_gate": [P, I, P, I, I, I, I, P],
         "alice_attention_masked": [P, I, P, P, P, P, P, P, I, I, I, I, I, I, F, F, I, P, I, I, P, I, I, F, I, I, P, P, P, P, P],
         "alice_attention_tiled": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, I, I, I, P, P, P, P, P, I, I, F, I, P],
@@ -543,6 +546,41 @@ def attention_generic(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tenso
           block_table.shape[1], T, num_heads, nKV, d, page_size, float(scale),
           float(softcap or 0.0), int(window or 0), None if bias_slopes is None else bias_slopes.data_ptr(),
           int(full_precision), int(dv), gate_ptr, int(gate_stride), _stream())
+
+
+def attention_f32(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, out: torch.Tensor, ctx,
+                  block_table: torch.Tensor, *, num_heads: int, scale: float, softcap: Optional[float],
+                  window: Optional[int], splits: Optional[int] = None) -> None:
+    """Causal attention in 32-bit over a row-major cache on the 32-bit matrix instruction (attention_f32.hip), for
+    prompts, pieces and single tokens; q: float32 [T, heads * d].  splits: blocks that a tile's keys are spread over
+    (None: from the step's sizes as captured steps round them, so that captured and eager steps add in one order)."""
+    T = q.shape[0]
+    if k_pool.dim() != 4:
+        raise HipLibraryError("k_pool must be [pages, nKV, page, d]")
+    n_pages, nKV, page_size, d = k_pool.shape
+    _dev(q, "q", torch.float32, (T, num_heads * d))
+    _dev(out, "out", torch.float32, (T, num_heads * d))
+    _dev(k_pool, "k_pool", torch.float32)
+    _dev(v_pool, "v_pool", torch.float32, tuple(k_pool.shape))
+    _dev(ctx.positions, "positions", torch.int32, (T,))
+    _dev(ctx.cu_seqlens, "cu_seqlens", torch.int32, (ctx.n_seqs + 1,))
+    _dev(block_table, "block_table", torch.int32)
+    if block_table.dim() != 2 or block_table.shape[0] < ctx.n_seqs or ctx.max_position // page_size >= block_table.shape[1]:
+        raise HipLibraryError(f"position {ctx.max_position} is beyond the block table {tuple(block_table.shape)}")
+    lib = library()
+    if not lib.alice_attention_f32_supported(num_heads, nKV, d, page_size):
+        raise HipLibraryError(f"attention: {num_heads} / {nKV} heads of size {d} on pages of {page_size} are outside this kernel's range")
+    if splits is None:
+        reach = ctx.rounded_context or ctx.max_context
+        if window:
+            reach = min(reach, window + 16)
+        per_tile = 16 // (num_heads // nKV)
+        tiles = (ctx.rounded_seqs or T) if ctx.is_decode else -(-frag_rows(T) // per_tile)
+        splits = lib.alice_attention_f32_splits(tiles, nKV, reach)
+    work = torch.empty((T * num_heads * splits * (d + 2),), dtype=torch.float32, device=q.device) if splits > 1 else None
+    _call("alice_attention_f32", q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), out.data_ptr(), ctx.positions.data_ptr(),
+          ctx.cu_seqlens.data_ptr(), block_table.data_ptr(), block_table.shape[1], T, ctx.n_seqs, int(ctx.is_decode), num_heads, nKV, d,
+          page_size, float(scale), float(softcap or 0.0), int(window or 0), splits, _opt(work, "work"), _stream())
 
 
 def attention_masked(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, out: Optional[torch.Tensor],
@@ -1533,6 +1571,11 @@ def attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, out: 
         return
     if out_layout != LAYOUT_ROW or sink is not None:
         raise HipLibraryError("only the matrix-core attention kernels write fragment order, and here only they take a sink")
+    # the 32-bit path at the matrix-core head sizes, without the terms that the generic kernel alone has
+    if (q.dtype == torch.float32 and full_precision and bias_slopes is None and gate is None and k_pool.shape[3] == v_pool.shape[3]
+            and library().alice_attention_f32_supported(num_heads, k_pool.shape[1], k_pool.shape[3], k_pool.shape[2])):
+        attention_f32(q, k_pool, v_pool, out, ctx, block_table, num_heads=num_heads, scale=scale, softcap=softcap, window=window)
+        return
     attention_generic(q, k_pool, v_pool, out, ctx.positions, ctx.seq_of_token, block_table,
                       num_heads=num_heads, scale=scale, softcap=softcap, window=window,
                       max_position=ctx.max_position, full_precision=full_precision, bias_slopes=bias_slopes, gate=gate)

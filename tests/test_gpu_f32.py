@@ -1,0 +1,98 @@
+"""The kernels of the true 32-bit path against 64-bit references: products and attention on the 32-bit matrix instruction, at
+the edges of their tiles, slices and splits."""
+import math
+from types import SimpleNamespace
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from alice_llm_amd.hip import ops
+from plain import gemma2_plain as P
+from test_gpu_kernels import DT, attention_case, close, rnd
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# ------------------------------------------------------------------ products
+@pytest.mark.parametrize("M,N,K", [(1, 64, 9216), (4, 16400, 72), (9, 64, 32), (13, 46, 1032), (16, 100, 2048), (17, 64, 40), (31, 33, 36), (33, 65, 68), (64, 128, 31), (129, 257, 96), (250, 2304, 2048), (500, 1000, 2308)])
+@pytest.mark.parametrize("xdt,wdt", [("float32", "float32"), ("float32", "bfloat16"), ("bfloat16", "float32")])
+def test_products_at_the_edges_of_tiles_and_slices(M, N, K, xdt, wdt):
+    x, w = rnd(M, K, seed=M, dtype=DT[xdt]), rnd(N, K, seed=N, scale=0.1, dtype=DT[wdt])
+    # K roundings of at most 2^-24 of a partial sum of size 0.1 sqrt(K) add up to 0.1 K 2^-24; eight times that over all elements
+    ref, tol = x.double() @ w.double().T, 8 * 0.1 * K * 2 ** -24
+    full = xdt == "float32"
+    y = torch.empty(M, N, device=DEV)
+    ops.linear(x, w, y, n_out=N, k_in=K, full_precision=full)
+    close(y, ref, tol)
+    for split in {2, 3, 8, ops.linear_split_hint(M, N, K, ops.LAYOUT_ROW)}:
+        parts = torch.full((split, M, N), float("nan"), device=DEV) if split > 1 else torch.empty(M, N, device=DEV)
+        ops.linear(x, w, parts, n_out=N, k_in=K, split_k=split, full_precision=full)
+        close(parts.sum(0) if split > 1 else parts, ref, tol)
+    if N % 2 == 0:
+        out = torch.empty(M, N // 2, device=DEV)
+        ops.linear(x, w, out, n_out=N // 2, k_in=K, epilogue=ops.EPI_GEGLU, full_precision=True)
+        g, u = ref[:, :N // 2], ref[:, N // 2:]
+        close(out, F.gelu(g, approximate="tanh") * u, 4 * tol, 1e-5)
+
+
+def test_products_of_rows_that_are_not_aligned():
+    big = rnd(40 * 64 + 1, seed=3)
+    x, w = big[1:].view(40, 64), rnd(48 * 64 + 2, seed=4)[2:].view(48, 64)
+    y = torch.empty(40, 48, device=DEV)
+    ops.linear(x, w, y, n_out=48, k_in=64, full_precision=True)
+    close(y, x.double() @ w.double().T, 8 * 64 * 2 ** -24)
+
+
+def test_products_refuse_slices_with_an_epilogue_and_too_many():
+    x, w = rnd(16, 64), rnd(64, 64)
+    with pytest.raises(ops.HipLibraryError, match="partial sums"):
+        ops.linear(x, w, torch.empty(2, 16, 64, device=DEV), n_out=64, k_in=64, epilogue=ops.EPI_SOFTCAP, epi_param=1.0, split_k=2, full_precision=True)
+    with pytest.raises(ops.HipLibraryError, match="slices"):
+        ops.linear(x, w, torch.empty(9, 16, 64, device=DEV), n_out=64, k_in=64, split_k=9, full_precision=True)
+
+
+# ------------------------------------------------------------------ attention
+def ctx_of(lens, new, pos, seq):
+    cu = [0]
+    for n in new:
+        cu.append(cu[-1] + n)
+    return SimpleNamespace(positions=pos, seq_of_token=seq, cu_seqlens=torch.tensor(cu, dtype=torch.int32, device=DEV), n_seqs=len(new),
+                           is_decode=max(new) == 1, max_context=max(lens), max_position=max(lens) - 1, rounded_seqs=len(new),
+                           rounded_context=max(lens))
+
+
+@pytest.mark.parametrize("nH,nKV,d", [(4, 1, 64), (6, 2, 128), (8, 4, 256), (5, 5, 64), (16, 1, 128)])
+@pytest.mark.parametrize("cap,window", [(None, None), (5.0, 50), (50.0, 7), (None, 16)])
+def test_attention_prompts_pieces_and_single_tokens(nH, nKV, d, cap, window):
+    for lens, new in (((5, 130, 66), (5, 130, 66)), ((200, 1, 77, 16), (1, 1, 1, 1)), ((150, 64, 33), (20, 3, 1))):
+        q, kp, vp, bt, pos, seq, ref, scale = attention_case("float32", nH, nKV, d, lens, new, cap, window, seed=3)
+        for splits in (None, 1, 2, 5):
+            out = torch.full_like(q, float("nan"))
+            ops.attention_f32(q, kp, vp, out, ctx_of(lens, new, pos, seq), bt, num_heads=nH, scale=scale, softcap=cap, window=window, splits=splits)
+            close(out, ref, 1e-5)
+
+
+def test_attention_keeps_values_that_are_no_numbers_to_the_queries_that_see_them():
+    """The value at position 37 is infinite and the one at 70 not a number: rows before see neither, rows behind the window
+    of 20 neither again, whatever tile of 16 keys or queries they share."""
+    nH, nKV, d, L, window = 4, 2, 64, 96, 20
+    q, kp, vp, bt, pos, seq, _, scale = attention_case("float32", nH, nKV, d, (L,), (L,), None, window, seed=8)
+    for at, what in ((37, math.inf), (70, math.nan)):
+        vp[int(bt[0, at // 64]), :, at % 64, 3] = what
+    rows = lambda pool: torch.cat([pool[int(bt[0, i])] for i in range(2)], dim=1)[:, :L].transpose(0, 1).double().cpu()   # noqa: E731
+    ref = P.attention_core(q.view(L, nH, d).double().cpu(), rows(kp), rows(vp), scale, None, window)
+    for splits in (1, 2):
+        out = torch.empty_like(q)
+        ops.attention_f32(q, kp, vp, out, ctx_of((L,), (L,), pos, seq), bt, num_heads=nH, scale=scale, softcap=None, window=window, splits=splits)
+        got = out.view(L, nH, d).double().cpu()
+        fine = torch.isfinite(ref)
+        assert not fine[37:57, :, 3].any() and fine[:37].all() and torch.equal(fine, torch.isfinite(got))
+        assert (got - ref)[fine].abs().max() < 1e-5
+
+
+def test_attention_refuses_what_is_outside_its_range():
+    q, kp, vp, bt, pos, seq, _, scale = attention_case("float32", 4, 2, 32, (20,), (20,), None, None, seed=8)
+    with pytest.raises(ops.HipLibraryError, match="outside"):
+        ops.attention_f32(q, kp, vp, torch.empty_like(q), ctx_of((20,), (20,), pos, seq), bt, num_heads=4, scale=scale, softcap=None, window=None)
