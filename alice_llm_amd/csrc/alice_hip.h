@@ -192,20 +192,28 @@ int alice_gla(const float* rows, int row_w, int q_col, int k_col, int v_col, int
 int alice_short_conv(const float* rows, int row_w, int col0, int channels, int taps, const float* w, const float* bias,
                      float* state, float* out, int act, const int* cu_seqlens, const int* seq_of_token, const int* slots,
                      int T, int n_seqs, hipStream_t stream);
-// step = softplus(rows[:, dt_col + h] + dt_bias[h]), decay = exp(-exp(a_log[h]) step), both [T, H]
+// step = softplus(rows[:, dt_col + h] + dt_bias[h]), decay = exp(-exp(a_log[h]) step) (as_log: its logarithm), both [T, H]
 int alice_ssm_prepare(const float* rows, int row_w, int dt_col, const float* dt_bias, const float* a_log, float* step,
-                      float* decay, int T, int H, hipStream_t stream);
+                      float* decay, int T, int H, int as_log, hipStream_t stream);
 // unit vectors of the q and k heads of qk [T, q (G d) | ... k at k_col (G d)] in place (q times q_scale); z [T, H d] turned
-// into decays exp(-exp(a_log[h]) softplus(z + dt_bias)) in place; beta[t, h] = sigmoid(rows[t, b_col + h])
+// into decays exp(-exp(a_log[h]) softplus(z + dt_bias)) (as_log: their logarithms) in place; beta[t, h] = sigmoid(rows[t, b_col + h])
 int alice_delta_prepare(float* qk, int qk_w, int k_col, int G, int d, float unit_eps, float q_scale, float* z,
                         const float* dt_bias, const float* a_log, const float* rows, int row_w, int b_col, float* beta,
-                        int T, int H, hipStream_t stream);
+                        int T, int H, int as_log, hipStream_t stream);
 // The matrix-state recurrence over a step's tokens (delta 0: S = diag(a) S + k (b v)^T; 1: the delta rule), o to out
 // [T, H dv] float32; q and k are shared by groups of H / qk_heads heads; decay [T, H d] (decay_per_row) or [T, H].
 int alice_matrix_recurrence(const float* q, int q_w, int q_col, const float* k, int k_w, int k_col, const float* v, int v_w,
                             int v_col, const float* decay, int decay_per_row, const float* b, const float* skip, float* out,
                             const int* cu_seqlens, const int* slots, float* S, int n_seqs, int n_slots, int H, int qk_heads,
                             int d, int dv, int delta, int columns, hipStream_t stream);
+// The same over pieces of many tokens, 16 at a time on the 32-bit matrix instruction (recurrent_chunks.hip); log_decay: the
+// decays' logarithms, [T, H d] with delta, else [T, H]; work: alice_recurrence_chunks_workspace floats (0: sizes outside
+// its range).
+long alice_recurrence_chunks_workspace(int T, int n_seqs, int H, int qk_heads, int d, int dv, int delta);
+int alice_recurrence_chunks(const float* q, int q_w, int q_col, const float* k, int k_w, int k_col, const float* v, int v_w,
+                            int v_col, const float* log_decay, const float* b, const float* skip, float* out, float* work,
+                            const int* cu_seqlens, const int* slots, float* S, int T, int n_seqs, int H, int qk_heads, int d,
+                            int dv, int delta, hipStream_t stream);
 // (columns: value columns a wave, 4, 8 or 16; 0: by the step's size, the rule of alice_matrix_recurrence_columns)
 int alice_matrix_recurrence_columns(int n_seqs, int H, int d, int dv);
 // Rows of `width` in `parts` equal parts, each RMS-normed and multiplied by a weight (w_shared: of a part's length);

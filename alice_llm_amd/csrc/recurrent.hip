@@ -80,25 +80,27 @@ __global__ __launch_bounds__(256) void short_conv_state_kernel(const float* __re
 
 // ------------------------------------------------------------------------------------------ what enters the recurrences
 
-// State space: step[t, h] = softplus(rows[t, dt_col + h] + dt_bias[h]); decay[t, h] = exp(-exp(a_log[h]) step[t, h]).
+// State space: step[t, h] = softplus(rows[t, dt_col + h] + dt_bias[h]); decay[t, h] = exp(-exp(a_log[h]) step[t, h]), or
+// with as_log its logarithm, which the chunk kernels take.
 __global__ void ssm_prepare_kernel(const float* __restrict__ rows, int row_w, int dt_col, const float* __restrict__ dt_bias,
-                                   const float* __restrict__ a_log, float* __restrict__ step, float* __restrict__ decay, long n, int H) {
+                                   const float* __restrict__ a_log, float* __restrict__ step, float* __restrict__ decay, long n, int H, int as_log) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int h = (int)(i % H);
   const long t = i / H;
   const float dt = softplus_full(rows[(size_t)t * row_w + dt_col + h] + dt_bias[h]);
   step[i] = dt;
-  decay[i] = expf(-expf(a_log[h]) * dt);
+  const float l = -expf(a_log[h]) * dt;
+  decay[i] = as_log ? l : expf(l);
 }
 
 // Delta rule: blocks y < 2 G make the q (y < G) and k heads of `qk` [T, q | k] unit vectors in place,
 // x / sqrt(sum x^2 + unit_eps), q also times q_scale; blocks beyond turn z [T, H d] into the decays
-// exp(-exp(a_log[h]) softplus(z + dt_bias)) in place and write beta[t, h] = sigmoid(rows[t, b_col + h]).
+// exp(-exp(a_log[h]) softplus(z + dt_bias)) (as_log: their logarithms) in place and write beta[t, h] = sigmoid(rows[t, b_col + h]).
 __global__ __launch_bounds__(64) void delta_prepare_kernel(float* __restrict__ qk, int qk_w, int k_col, int G, int d, float unit_eps,
                                                            float q_scale, float* __restrict__ z, const float* __restrict__ dt_bias,
                                                            const float* __restrict__ a_log, const float* __restrict__ rows, int row_w,
-                                                           int b_col, float* __restrict__ beta, int H) {
+                                                           int b_col, float* __restrict__ beta, int H, int as_log) {
   const int t = blockIdx.x, y = blockIdx.y, lane = threadIdx.x;
   if (y < 2 * G) {
     float* x = qk + (size_t)t * qk_w + (y < G ? y * d : k_col + (y - G) * d);
@@ -111,7 +113,10 @@ __global__ __launch_bounds__(64) void delta_prepare_kernel(float* __restrict__ q
     const int h = y - 2 * G;
     const float rate = expf(a_log[h]);
     float* zz = z + ((size_t)t * H + h) * d;
-    for (int e = lane; e < d; e += 64) zz[e] = expf(-rate * softplus_full(zz[e] + dt_bias[h * d + e]));
+    for (int e = lane; e < d; e += 64) {
+      const float l = -rate * softplus_full(zz[e] + dt_bias[h * d + e]);
+      zz[e] = as_log ? l : expf(l);
+    }
     if (lane == 0) beta[(size_t)t * H + h] = sigmoid_full(rows[(size_t)t * row_w + b_col + h]);
   }
 }
@@ -330,26 +335,26 @@ extern "C" int alice_short_conv(const float* rows, int row_w, int col0, int chan
 }
 
 extern "C" int alice_ssm_prepare(const float* rows, int row_w, int dt_col, const float* dt_bias, const float* a_log, float* step,
-                                 float* decay, int T, int H, hipStream_t stream) {
+                                 float* decay, int T, int H, int as_log, hipStream_t stream) {
   ALICE_CHECK(rows && dt_bias && a_log && step && decay, "ssm_prepare: a pointer is missing");
   ALICE_CHECK(T >= 0 && H >= 1 && dt_col >= 0 && dt_col + H <= row_w, "ssm_prepare: bad sizes");
   const long n = (long)T * H;
   if (n == 0) return 0;
-  ssm_prepare_kernel<<<ceil_div(n, 256), 256, 0, stream>>>(rows, row_w, dt_col, dt_bias, a_log, step, decay, n, H);
+  ssm_prepare_kernel<<<ceil_div(n, 256), 256, 0, stream>>>(rows, row_w, dt_col, dt_bias, a_log, step, decay, n, H, as_log);
   ALICE_LAUNCH_CHECK();
   return 0;
 }
 
 extern "C" int alice_delta_prepare(float* qk, int qk_w, int k_col, int G, int d, float unit_eps, float q_scale, float* z,
                                    const float* dt_bias, const float* a_log, const float* rows, int row_w, int b_col, float* beta,
-                                   int T, int H, hipStream_t stream) {
+                                   int T, int H, int as_log, hipStream_t stream) {
   ALICE_CHECK(qk && z && dt_bias && a_log && rows && beta, "delta_prepare: a pointer is missing");
   ALICE_CHECK(T >= 0 && H >= 1 && G >= 1 && d >= 1 && unit_eps >= 0.f, "delta_prepare: bad sizes");
   ALICE_CHECK(G * d <= k_col && k_col + G * d <= qk_w && b_col >= 0 && b_col + H <= row_w, "delta_prepare: the rows are too short for the heads");
   ALICE_CHECK(2 * G + H <= 65535, "delta_prepare: too many heads for one launch");
   if (T == 0) return 0;
   dim3 grid(T, 2 * G + H);
-  delta_prepare_kernel<<<grid, 64, 0, stream>>>(qk, qk_w, k_col, G, d, unit_eps, q_scale, z, dt_bias, a_log, rows, row_w, b_col, beta, H);
+  delta_prepare_kernel<<<grid, 64, 0, stream>>>(qk, qk_w, k_col, G, d, unit_eps, q_scale, z, dt_bias, a_log, rows, row_w, b_col, beta, H, as_log);
   ALICE_LAUNCH_CHECK();
   return 0;
 }

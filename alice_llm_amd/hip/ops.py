@@ -73,8 +73,9 @@ def _declare(lib) -> None:
         "alice_mix_heads": [P, P, P, I, F, P, I, I, I, I, I, I, P],
         "alice_qkv_prepare": [P, I, I, P, P, P, P, I, P, P, I, I, P, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, P],
         "alice_short_conv": [P, I, I, I, I, P, P, P, P, I, P, P, P, I, I, P],
-        "alice_ssm_prepare": [P, I, I, P, P, P, P, I, I, P],
-        "alice_delta_prepare": [P, I, I, I, I, F, F, P, P, P, P, I, I, P, I, I, P],
+        "alice_ssm_prepare": [P, I, I, P, P, P, P, I, I, I, P],
+        "alice_delta_prepare": [P, I, I, I, I, F, F, P, P, P, P, I, I, P, I, I, I, P],
+        "alice_recurrence_chunks": [P, I, I, P, I, I, P, I, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P],
         "alice_matrix_recurrence": [P, I, I, P, I, I, P, I, I, P, I, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
         "alice_matrix_recurrence_columns": [I, I, I, I],
         "alice_norm_gate": [P, I, I, P, I, I, I, I, P, I, F, P, I, I, P],
@@ -117,6 +118,8 @@ def _declare(lib) -> None:
     lib.alice_attention_split_workspace.restype = L
     lib.alice_mlstm_chunks_workspace.argtypes = [I, I, I, I, I, I]
     lib.alice_mlstm_chunks_workspace.restype = L
+    lib.alice_recurrence_chunks_workspace.argtypes = [I, I, I, I, I, I, I]
+    lib.alice_recurrence_chunks_workspace.restype = L
     lib.alice_lightning_chunks.argtypes = [I, I]
     lib.alice_lightning_chunks.restype = L
     lib.alice_expert_rows.argtypes = [I, I, I]
@@ -1161,8 +1164,9 @@ def short_conv(rows: torch.Tensor, col0: int, weight: torch.Tensor, bias: Option
 
 
 def ssm_prepare(rows: torch.Tensor, dt_col: int, dt_bias: torch.Tensor, a_log: torch.Tensor, step: torch.Tensor,
-                decay: torch.Tensor) -> None:
-    """step = softplus(rows[:, dt_col + h] + dt_bias[h]); decay = exp(-exp(a_log[h]) * step); float32 [T, heads] each."""
+                decay: torch.Tensor, *, as_log: bool = False) -> None:
+    """step = softplus(rows[:, dt_col + h] + dt_bias[h]); decay = exp(-exp(a_log[h]) * step), as_log: its logarithm;
+    float32 [T, heads] each."""
     T, H = step.shape
     _dev(rows, "rows", torch.float32)
     _dev(dt_bias, "dt_bias", torch.float32, (H,))
@@ -1172,13 +1176,14 @@ def ssm_prepare(rows: torch.Tensor, dt_col: int, dt_bias: torch.Tensor, a_log: t
     if rows.shape[0] != T or dt_col + H > rows.shape[1]:
         raise HipLibraryError("rows do not hold the step sizes")
     _call("alice_ssm_prepare", rows.data_ptr(), rows.shape[1], int(dt_col), dt_bias.data_ptr(), a_log.data_ptr(), step.data_ptr(),
-          decay.data_ptr(), T, H, _stream())
+          decay.data_ptr(), T, H, int(as_log), _stream())
 
 
 def delta_prepare(qk: torch.Tensor, k_col: int, z: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor, rows: torch.Tensor,
-                  b_col: int, beta: torch.Tensor, *, qk_heads: int, heads: int, head_dim: int, unit_eps: float, q_scale: float) -> None:
+                  b_col: int, beta: torch.Tensor, *, qk_heads: int, heads: int, head_dim: int, unit_eps: float, q_scale: float,
+                  as_log: bool = False) -> None:
     """In place: the q heads (columns 0 .. qk_heads * d of qk) and the k heads (from k_col) become unit vectors
-    x / sqrt(sum x^2 + unit_eps), q also times q_scale; z [T, heads * d] becomes exp(-exp(a_log[h]) softplus(z + dt_bias));
+    x / sqrt(sum x^2 + unit_eps), q also times q_scale; z [T, heads * d] becomes exp(-exp(a_log[h]) softplus(z + dt_bias)), as_log: its logarithm;
     beta[t, h] = sigmoid(rows[t, b_col + h])."""
     T = qk.shape[0]
     G, H, d = qk_heads, heads, head_dim
@@ -1191,7 +1196,8 @@ def delta_prepare(qk: torch.Tensor, k_col: int, z: torch.Tensor, dt_bias: torch.
     if rows.shape[0] != T or b_col + H > rows.shape[1] or k_col < G * d or k_col + G * d > qk.shape[1]:
         raise HipLibraryError("the rows are too short for the heads")
     _call("alice_delta_prepare", qk.data_ptr(), qk.shape[1], int(k_col), G, d, float(unit_eps), float(q_scale), z.data_ptr(),
-          dt_bias.data_ptr(), a_log.data_ptr(), rows.data_ptr(), rows.shape[1], int(b_col), beta.data_ptr(), T, H, _stream())
+          dt_bias.data_ptr(), a_log.data_ptr(), rows.data_ptr(), rows.shape[1], int(b_col), beta.data_ptr(), T, H,
+          int(as_log), _stream())
 
 
 def recurrence_columns(n_seqs: int, heads: int, head_dim: int, value_head_dim: int) -> int:
@@ -1229,6 +1235,48 @@ def matrix_recurrence(q, q_col: int, k, k_col: int, v, v_col: int, decay: torch.
           v.shape[1], int(v_col), decay.data_ptr(), int(per_row), b.data_ptr(), _opt(skip, "skip"), out.data_ptr(),
           ctx.cu_seqlens.data_ptr(), ctx.slots.data_ptr(), S.data_ptr(), int(ctx.n_seqs), int(n_slots), H, int(qk_heads), d, dv,
           int(bool(delta)), int(columns_per_wave), _stream())
+
+
+# Steps whose longest piece has at least this many tokens go by chunks: beyond what is captured into graphs, whose rounded
+# lengths would choose otherwise than the eager step (at 128 tokens the two ways are within 20 us of each other).
+RECURRENCE_CHUNKS_FROM = 257
+# The delta rule only up to this many (sequence, head, 16 columns): with more, the token-by-token kernel fills the chip and has
+# less to do (heads of 128, 8 pieces of 1,000 tokens: 468 us by chunks, 682 token by token; 32 of 64: 167 and 120).
+DELTA_CHUNKS_WAVES = 1024
+
+
+def recurrence_by_chunks(ctx, width: int, q_col: int, *, heads: int, qk_heads: int, head_dim: int, value_head_dim: int,
+                         delta: bool) -> bool:
+    """Whether a step takes recurrence_chunks: pieces long enough, and sizes (rows of `width` floats with the queries from
+    q_col) that its kernels cover."""
+    return (ctx.max_new >= RECURRENCE_CHUNKS_FROM and width % 4 == 0 and q_col % 4 == 0
+            and (not delta or ctx.n_seqs * heads * -(-value_head_dim // 16) <= DELTA_CHUNKS_WAVES)
+            and library().alice_recurrence_chunks_workspace(1, int(ctx.n_seqs), heads, qk_heads, head_dim, value_head_dim, int(delta)) > 0)
+
+
+def recurrence_chunks(q, q_col: int, k, k_col: int, v, v_col: int, log_decay: torch.Tensor, b: torch.Tensor, skip: Optional[torch.Tensor],
+                      out: torch.Tensor, ctx, S: torch.Tensor, *, heads: int, qk_heads: int, head_dim: int, value_head_dim: int,
+                      delta: bool) -> None:
+    """matrix_recurrence's result for pieces of many tokens, 16 tokens at a time (recurrent_chunks.hip); log_decay: the
+    decays' logarithms, [T, heads * d] with delta, else [T, heads]."""
+    H, d, dv = heads, head_dim, value_head_dim
+    T = out.shape[0]
+    for t_, nm in ((q, "q"), (k, "k"), (v, "v")):
+        _dev(t_, nm, torch.float32)
+        if t_.dim() != 2 or t_.shape[0] != T:
+            raise HipLibraryError(f"{nm} must be [T, width]")
+    _dev(log_decay, "log_decay", torch.float32, (T, H * d) if delta else (T, H))
+    _dev(b, "b", torch.float32, (T, H))
+    _opt(skip, "skip", torch.float32, (H,))
+    _dev(out, "out", torch.float32, (T, H * dv))
+    _step_arrays(ctx)
+    _dev(S, "S", torch.float32, (S.shape[0], H, d, dv))
+    need = library().alice_recurrence_chunks_workspace(T, int(ctx.n_seqs), H, int(qk_heads), d, dv, int(delta))
+    work = torch.empty((max(1, need),), dtype=torch.float32, device=out.device)
+    _call("alice_recurrence_chunks", q.data_ptr(), q.shape[1], int(q_col), k.data_ptr(), k.shape[1], int(k_col), v.data_ptr(),
+          v.shape[1], int(v_col), log_decay.data_ptr(), b.data_ptr(), _opt(skip, "skip"), out.data_ptr(), work.data_ptr(),
+          ctx.cu_seqlens.data_ptr(), ctx.slots.data_ptr(), S.data_ptr(), T, int(ctx.n_seqs), H, int(qk_heads), d, dv, int(bool(delta)),
+          _stream())
 
 
 def norm_gate(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, *, parts: int, eps: float, weight_shared: bool,

@@ -127,13 +127,19 @@ class ChannelDeltaMixer(Part):
         z = self.decay(rows[:, self.a_col:self.a_col + self.ra].to(act).contiguous(), torch.float32)
         gate = self.gate(rows[:, self.g_col:self.g_col + self.rg].to(act).contiguous(), torch.float32)
         beta = torch.empty((T, self.nH), dtype=torch.float32, device=dev)
+        # pieces of many tokens by chunks, which take the decays' logarithms
+        heads = dict(heads=self.nH, qk_heads=self.nKV, head_dim=self.d)
+        values = dict(value_head_dim=self.P, delta=True)
+        chunks = ops.recurrence_by_chunks(ctx, self.channels, 0, **values, **heads)
         ops.delta_prepare(conv, self.qk, z, self.small[n["dt_bias"]], self.small[n["A_log"]], rows, self.b_col, beta,
-                          qk_heads=self.nKV, heads=self.nH, head_dim=self.d, unit_eps=self.unit_eps, q_scale=self.d ** -0.5)
+                          unit_eps=self.unit_eps, q_scale=self.d ** -0.5, as_log=chunks, **heads)
         o = torch.empty((T, self.vw), dtype=torch.float32, device=dev)
-        ops.matrix_recurrence(conv, 0, conv, self.qk, conv, 2 * self.qk, z, beta, None, o, ctx, cache.state["S"],
-                              heads=self.nH, qk_heads=self.nKV, head_dim=self.d, value_head_dim=self.P, delta=True,
-                              decay_per_channel=True,
-                              columns_per_wave=ops.recurrence_columns(getattr(ctx, "rounded_seqs", 0) or ctx.n_seqs, self.nH, self.d, self.P))
+        args = (conv, 0, conv, self.qk, conv, 2 * self.qk, z, beta, None, o, ctx, cache.state["S"])
+        if chunks:
+            ops.recurrence_chunks(*args, **values, **heads)
+        else:
+            ops.matrix_recurrence(*args, decay_per_channel=True, **values, **heads,
+                                  columns_per_wave=ops.recurrence_columns(getattr(ctx, "rounded_seqs", 0) or ctx.n_seqs, self.nH, self.d, self.P))
         out = torch.empty((T, self.vw), dtype=act, device=dev)
         ops.norm_gate(o, self.small[n["norm"]], out, parts=self.nH, eps=self.eps, weight_shared=True, gate=gate, gate_col=0,
                       gate_act="sigmoid")

@@ -94,13 +94,18 @@ class StateSpaceMixer(Part):
         ops.short_conv(rows, self.inner, self.small[n["conv"]], self.small[n["conv_bias"]], cache.state.get("conv"), conv, ctx)
         step = torch.empty((T, self.nH), dtype=torch.float32, device=dev)
         decay = torch.empty_like(step)
-        ops.ssm_prepare(rows, self.dt_col, self.small[n["dt_bias"]], self.small[n["A_log"]], step, decay)
+        # pieces of many tokens by chunks, which take the decays' logarithms
+        b_col, c_col = self.inner, self.inner + self.G * self.N
+        heads = dict(heads=self.nH, qk_heads=self.G, head_dim=self.N, value_head_dim=self.P)
+        chunks = ops.recurrence_by_chunks(ctx, self.channels, c_col, delta=False, **heads)
+        ops.ssm_prepare(rows, self.dt_col, self.small[n["dt_bias"]], self.small[n["A_log"]], step, decay, as_log=chunks)
         y = torch.empty((T, self.inner), dtype=torch.float32, device=dev)
-        b_col = self.inner
-        ops.matrix_recurrence(conv, b_col + self.G * self.N, conv, b_col, conv, 0, decay, step, self.small[n["D"]], y, ctx,
-                              cache.state["S"], heads=self.nH, qk_heads=self.G, head_dim=self.N, value_head_dim=self.P,
-                              delta=False, decay_per_channel=False,
-                              columns_per_wave=ops.recurrence_columns(getattr(ctx, "rounded_seqs", 0) or ctx.n_seqs, self.nH, self.N, self.P))
+        args = (conv, c_col, conv, b_col, conv, 0, decay, step, self.small[n["D"]], y, ctx, cache.state["S"])
+        if chunks:
+            ops.recurrence_chunks(*args, delta=False, **heads)
+        else:
+            ops.matrix_recurrence(*args, delta=False, decay_per_channel=False, **heads,
+                                  columns_per_wave=ops.recurrence_columns(getattr(ctx, "rounded_seqs", 0) or ctx.n_seqs, self.nH, self.N, self.P))
         out = torch.empty((T, self.inner), dtype=self.precision.act, device=dev)
         ops.norm_gate(y, self.small[n["norm"]], out, parts=self.norm_groups, eps=self.eps, weight_shared=False,
                       gate=rows, gate_col=0, gate_act="silu")

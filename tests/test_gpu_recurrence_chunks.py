@@ -1,0 +1,85 @@
+"""The matrix recurrences by chunks of 16 tokens against the plain token-by-token scans in 64 bits."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from alice_llm_amd.hip import ops
+from plain import vifirax_plain as P
+from test_gpu_vifirax import DEV, _Ctx, max_err, rnd
+
+pytestmark = pytest.mark.gpu
+
+# two steps over three slots: pieces that end within a chunk, at its end and one token behind it, and single tokens
+STEPS = [([33, 16, 1, 47], [2, 0, 5, 3]), ([1, 17, 15, 64], [5, 0, 3, 2])]
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("strength", [0.05, 1.0, 30.0])
+@pytest.mark.parametrize("H,G,d,dv", [(4, 2, 8, 16), (3, 3, 12, 20), (2, 1, 64, 128), (1, 1, 136, 24), (2, 2, 200, 7), (70, 1, 16, 8), (2, 2, 256, 17)])
+def test_chunks_over_pieces_and_slots(delta, strength, H, G, d, dv):
+    """`strength`: the size of the decays' logarithms a token, from slow ones to such that a chunk's product underflows."""
+    per, total = H // G, {slot: 0 for _, slots in STEPS for slot in slots}
+    S = torch.full((6, H, d, dv), 3.0, device=DEV)
+    S[list(total)] = 0.0
+    state = {slot: None for slot in total}
+    skip = None if delta else rnd(H, seed=3)
+    for step, (lens, slots) in enumerate(STEPS):
+        T = sum(lens)
+        q, k, v = rnd(T, G * d + 4, seed=20 + step), rnd(T, G * d, seed=30 + step), rnd(T, H * dv, seed=40 + step)
+        if delta:
+            q[:, :G * d] = P.unit_vectors(q[:, :G * d].view(T, G, d)).reshape(T, G * d)
+            k = P.unit_vectors(k.view(T, G, d)).reshape(T, G * d)
+        log = -strength * rnd(T, H * d if delta else H, seed=50 + step).abs()
+        b = torch.sigmoid(rnd(T, H, seed=60 + step)) * (1.0 if delta else 2.0)
+        out = torch.full((T, H * dv), float("nan"), device=DEV)
+        ops.recurrence_chunks(q.to(DEV), 0, k.to(DEV), 0, v.to(DEV), 0, log.to(DEV), b.to(DEV), None if skip is None else skip.to(DEV),
+                              out, _Ctx(lens, slots), S, heads=H, qk_heads=G, head_dim=d, value_head_dim=dv, delta=delta)
+        at = 0
+        for n, slot in zip(lens, slots):
+            r = slice(at, at + n)
+            qh, kh = (x[r, :G * d].double().view(n, G, d).repeat_interleave(per, dim=1) for x in (q, k))
+            vh, decay = v[r].double().view(n, H, dv), torch.exp(log[r].double())
+            if delta:
+                ref, state[slot] = P.delta_rule_scan(qh, kh, vh, decay.view(n, H, d), b[r].double(), state[slot])
+            else:
+                # the plain scan takes step sizes and rates of one; the write's factor is given by scaling the values
+                dt = -log[r].double()
+                u = vh * (b[r].double() / dt)[:, :, None]
+                ref, state[slot] = P.state_space_scan(u, kh, qh, dt, torch.zeros(H).double(), torch.zeros(H).double(), state[slot])
+                ref = ref + skip.double()[None, :, None] * vh
+            # sums over a few hundred terms of order one and their products with queries of the same size
+            assert max_err(out[r], ref.reshape(n, H * dv)) < 2e-5 * max(1.0, float(ref.abs().max())), (step, slot)
+            assert max_err(S[slot], state[slot]) < 2e-5 * max(1.0, float(state[slot].abs().max())), (step, slot)
+            at += n
+    others = [i for i in range(6) if i not in total]
+    assert float((S[others] - 3.0).abs().max()) == 0.0                  # rows of other slots are untouched
+
+
+def test_sizes_outside_the_range_stay_with_the_token_by_token_kernel():
+    ctx = SimpleNamespace(max_new=ops.RECURRENCE_CHUNKS_FROM, n_seqs=1)
+    kw = dict(heads=2, qk_heads=2, value_head_dim=16, delta=True)
+    assert ops.recurrence_by_chunks(ctx, 64, 0, head_dim=16, **kw)
+    assert not ops.recurrence_by_chunks(ctx, 64, 0, head_dim=18, **kw) and not ops.recurrence_by_chunks(ctx, 63, 0, head_dim=16, **kw)
+    assert not ops.recurrence_by_chunks(SimpleNamespace(max_new=ops.RECURRENCE_CHUNKS_FROM - 1, n_seqs=1), 64, 0, head_dim=16, **kw)
+    many = SimpleNamespace(max_new=400, n_seqs=ops.DELTA_CHUNKS_WAVES // 2 + 1)
+    assert not ops.recurrence_by_chunks(many, 64, 0, head_dim=16, **kw)
+    assert ops.recurrence_by_chunks(many, 64, 0, head_dim=16, **dict(kw, delta=False))
+
+
+@pytest.mark.parametrize("delta", [False, True])
+def test_both_block_sizes_give_the_same(delta):
+    """Key sizes of 65 to 128 take eight waves a block, or four where there are 512 blocks and more: the same pieces alone
+    and 64 times over."""
+    H, d, dv, n = 2, 96, 64, 35
+    q, k, v = (rnd(n, H * w, seed=i).to(DEV) for i, w in ((1, d), (2, d), (3, dv)))
+    log, b = -rnd(n, H * d if delta else H, seed=4).abs().to(DEV), torch.sigmoid(rnd(n, H, seed=5)).to(DEV)
+    outs = []
+    for copies in (1, 64):
+        S, out = torch.zeros(copies, H, d, dv, device=DEV), torch.empty(copies * n, H * dv, device=DEV)
+        many = [x.repeat(copies, 1) for x in (q, k, v, log, b)]
+        ops.recurrence_chunks(many[0], 0, many[1], 0, many[2], 0, many[3], many[4], None, out, _Ctx([n] * copies, list(range(copies))), S,
+                              heads=H, qk_heads=H, head_dim=d, value_head_dim=dv, delta=delta)
+        outs.append((out.view(copies, n, H * dv), S))
+    (a, sa), (c, sc) = outs
+    assert (c - a).abs().max() < 1e-5 * a.abs().max() and (sc - sa).abs().max() < 1e-5 * sa.abs().max()
