@@ -350,6 +350,37 @@ __global__ __launch_bounds__(SB) void chunk_collect_kernel(const float* __restri
   });
 }
 
+// The thresholds by bisection over the whole row, for what a list could not settle; all threads of a block of ST call it.
+template <int VEC>
+__device__ __forceinline__ uint32_t whole_row_threshold(const float* __restrict__ row, int V, float inv_t, float m, uint32_t key_m,
+                                                        uint32_t thr, bool k_done, bool p_done, int top_k, float top_p, float* red,
+                                                        int* ired) {
+  if (!k_done) {
+    uint32_t lo = 0, hi = key_m;
+    while (lo < hi) {
+      const uint32_t mid = lo + (uint32_t)(((uint64_t)hi - lo + 1) >> 1);
+      int c = 0;
+      for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) { c += ok && order_key(x) >= mid; });
+      if (block_count(c, ired) >= top_k) lo = mid; else hi = mid - 1;
+    }
+    thr = lo;
+  }
+  if (!p_done) {
+    float z = 0.f;
+    for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) { if (ok && order_key(x) >= thr) z += expf(x - m); });
+    const float target = top_p * block_sum(z, red);
+    uint32_t lo = thr, hi = key_m;
+    while (lo < hi) {
+      const uint32_t mid = lo + (uint32_t)(((uint64_t)hi - lo + 1) >> 1);
+      float s = 0.f;
+      for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) { if (ok && order_key(x) >= mid) s += expf(x - m); });
+      if (block_sum(s, red) > target) lo = mid; else hi = mid - 1;
+    }
+    thr = lo;
+  }
+  return thr;
+}
+
 template <int VEC>
 __global__ __launch_bounds__(ST) void row_threshold_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t,
                                                            int top_k, float top_p) {
@@ -477,45 +508,17 @@ __global__ __launch_bounds__(ST) void row_threshold_kernel(const float* __restri
     __syncthreads();
     if (found[1]) { k_done = true; if (found[2]) { p_done = true; thr = found[0]; } else if (need_k) thr = found[0]; }
   }
-  // ---- the same over the whole row, for what the list could not settle
-  if (!k_done) {
-    uint32_t lo = 0, hi = key_m;
-    while (lo < hi) {
-      const uint32_t mid = lo + (uint32_t)(((uint64_t)hi - lo + 1) >> 1);
-      int c = 0;
-      for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) { c += ok && order_key(x) >= mid; });
-      if (block_count(c, ired) >= top_k) lo = mid; else hi = mid - 1;
-    }
-    thr = lo;
-  }
-  if (!p_done) {
-    float z = 0.f;
-    for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) { if (ok && order_key(x) >= thr) z += expf(x - m); });
-    const float target = top_p * block_sum(z, red);
-    uint32_t lo = thr, hi = key_m;
-    while (lo < hi) {
-      const uint32_t mid = lo + (uint32_t)(((uint64_t)hi - lo + 1) >> 1);
-      float s = 0.f;
-      for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) { if (ok && order_key(x) >= mid) s += expf(x - m); });
-      if (block_sum(s, red) > target) lo = mid; else hi = mid - 1;
-    }
-    thr = lo;
-  }
+  thr = whole_row_threshold<VEC>(row, V, inv_t, m, key_m, thr, k_done, p_done, top_k, top_p, red, ired);
   if (tid == 0) w.thr[b] = thr;
 }
 
-// The kept mass of every tile of the chunk (wave v takes the chunk's tiles v, v + 4, ...), and the last index with
-// a positive probability in it (-1: none).
+// The kept mass of the row's tiles t, t + step, ... below t_end (a wave), and the last index with a positive probability
+// in each (-1: none).
 template <int VEC>
-__global__ __launch_bounds__(SB) void tile_sum_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t,
-                                                      int filtered) {
-  const int b = blockIdx.y, c = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const float* row = logits + (size_t)b * V;
-  const float m = row_max(w, b);
-  const uint32_t thr = filtered ? w.thr[b] : 0u;
-  const int t_end = min(w.tiles, (c + 1) * w.tiles_per_chunk);
-  for (int t = c * w.tiles_per_chunk + wave; t < t_end; t += SB / 64) {
+__device__ __forceinline__ void tile_sums(const float* __restrict__ row, const SampleWork& w, int b, int V, float inv_t, float m,
+                                          uint32_t thr, int t, int t_end, int step) {
+  const int lane = threadIdx.x & 63;
+  for (; t < t_end; t += step) {
     float s = 0.f;
     int last_kept = -1;
     const int base = t * TILE;
@@ -548,57 +551,21 @@ __global__ __launch_bounds__(SB) void tile_sum_kernel(const float* __restrict__ 
   }
 }
 
-// Inverse CDF in index order: the running sums of the tiles (one thread, in order), the tile in which the sum
-// passes u times the total, and a scan of that tile, four consecutive elements per thread.
-__global__ __launch_bounds__(ST) void draw_kernel(const float* __restrict__ logits, int* __restrict__ out,
-                                                  const float* __restrict__ uniform, SampleWork w, int V, float inv_t,
-                                                  int filtered) {
-  __shared__ float wred[ST / 64];
-  __shared__ float prefix[1024];                          // inclusive running sums of up to 1024 tiles at a time
-  __shared__ int pick[2];
-  __shared__ float carry[2];
-  const int b = blockIdx.x;
-  const float* row = logits + (size_t)b * V;
+// (wave v takes the chunk's tiles v, v + 4, ...)
+template <int VEC>
+__global__ __launch_bounds__(SB) void tile_sum_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t,
+                                                      int filtered) {
+  const int b = blockIdx.y, c = blockIdx.x;
+  tile_sums<VEC>(logits + (size_t)b * V, w, b, V, inv_t, row_max(w, b), filtered ? w.thr[b] : 0u,
+                 c * w.tiles_per_chunk + (threadIdx.x >> 6), min(w.tiles, (c + 1) * w.tiles_per_chunk), SB / 64);
+}
+
+// The draw within the tile t_sel (-1: the row's last kept token) that the running sums chose, whose predecessors hold tile_before.
+// All threads of a block of ST call it, pick: two ints in shared memory.
+__device__ __forceinline__ void draw_in_tile(const float* __restrict__ row, int* __restrict__ out, int b, int V, float inv_t, float m,
+                                             uint32_t thr, int t_sel, int last_of_row, float target, float tile_before, float* wred,
+                                             int* pick) {
   const int tid = threadIdx.x;
-  const float m = row_max(w, b);
-  const uint32_t thr = filtered ? w.thr[b] : 0u;
-  const float u = uniform[b];
-  const float* tsum = w.tsum + (size_t)b * w.tiles;
-  int last_kept = -1;
-  for (int t = tid; t < w.tiles; t += ST) last_kept = max(last_kept, w.tlast[(size_t)b * w.tiles + t]);
-  if (tid == 0) { pick[0] = -1; pick[1] = -1; carry[0] = 0.f; carry[1] = 0.f; }
-  __syncthreads();
-  atomicMax(&pick[1], last_kept);
-  // the total first (groups of 1024 tiles), then the tile of the target
-  for (int sweep = 0; sweep < 2; ++sweep) {
-    const float target = u * carry[0];
-    float before_group = 0.f;
-    for (int t0 = 0; t0 < w.tiles; t0 += 1024) {
-      const int n = min(w.tiles - t0, 1024);
-      __syncthreads();
-      for (int t = tid; t < n; t += ST) prefix[t] = tsum[t0 + t];
-      __syncthreads();
-      if (tid == 0) {
-        float acc = before_group;
-        for (int t = 0; t < n; ++t) { acc += prefix[t]; prefix[t] = acc; }
-        if (sweep == 0) carry[0] = acc;
-      }
-      __syncthreads();
-      if (sweep == 1 || w.tiles <= 1024) {
-        const float tgt = sweep == 1 ? target : u * carry[0];
-        for (int t = tid; t < n; t += ST) {
-          const float lo = t == 0 ? before_group : prefix[t - 1];
-          if (tgt >= lo && tgt < prefix[t]) { pick[0] = t0 + t; carry[1] = lo; }   // at most one tile
-        }
-      }
-      before_group = prefix[n - 1];
-    }
-    if (w.tiles <= 1024) break;
-  }
-  __syncthreads();
-  const int t_sel = pick[0], last_of_row = pick[1];
-  const float target = u * carry[0];
-  const float tile_before = carry[1];
   __syncthreads();
   if (t_sel < 0) {                                       // u * total rounded up to the total: the last kept token
     if (tid == 0) out[b] = max(last_of_row, 0);
@@ -638,6 +605,341 @@ __global__ __launch_bounds__(ST) void draw_kernel(const float* __restrict__ logi
   __syncthreads();
   // the tile's sum by waves and by the scan can differ in the last bit: past the scan's end means the tile's last
   if (tid == 0) out[b] = pick[0] >= 0 ? pick[0] : max(pick[1], 0);
+}
+
+// Inverse CDF in index order: the running sums of the tiles (one thread, in order), the tile in which the sum
+// passes u times the total, and a scan of that tile, four consecutive elements per thread.
+// All threads of a block of ST call it.
+__device__ __forceinline__ void draw_from_tiles(const float* __restrict__ row, int* __restrict__ out, float u, const SampleWork& w, int b,
+                                                int V, float inv_t, float m, uint32_t thr, float* wred) {
+  __shared__ float prefix[1024];                          // inclusive running sums of up to 1024 tiles at a time
+  __shared__ int pick[2];
+  __shared__ float carry[2];
+  const int tid = threadIdx.x;
+  const float* tsum = w.tsum + (size_t)b * w.tiles;
+  int last_kept = -1;
+  for (int t = tid; t < w.tiles; t += ST) last_kept = max(last_kept, w.tlast[(size_t)b * w.tiles + t]);
+  if (tid == 0) { pick[0] = -1; pick[1] = -1; carry[0] = 0.f; carry[1] = 0.f; }
+  __syncthreads();
+  atomicMax(&pick[1], last_kept);
+  // the total first (groups of 1024 tiles), then the tile of the target
+  for (int sweep = 0; sweep < 2; ++sweep) {
+    const float target = u * carry[0];
+    float before_group = 0.f;
+    for (int t0 = 0; t0 < w.tiles; t0 += 1024) {
+      const int n = min(w.tiles - t0, 1024);
+      __syncthreads();
+      for (int t = tid; t < n; t += ST) prefix[t] = tsum[t0 + t];
+      __syncthreads();
+      if (tid == 0) {
+        float acc = before_group;
+        for (int t = 0; t < n; ++t) { acc += prefix[t]; prefix[t] = acc; }
+        if (sweep == 0) carry[0] = acc;
+      }
+      __syncthreads();
+      if (sweep == 1 || w.tiles <= 1024) {
+        const float tgt = sweep == 1 ? target : u * carry[0];
+        for (int t = tid; t < n; t += ST) {
+          const float lo = t == 0 ? before_group : prefix[t - 1];
+          if (tgt >= lo && tgt < prefix[t]) { pick[0] = t0 + t; carry[1] = lo; }   // at most one tile
+        }
+      }
+      before_group = prefix[n - 1];
+    }
+    if (w.tiles <= 1024) break;
+  }
+  __syncthreads();
+  draw_in_tile(row, out, b, V, inv_t, m, thr, pick[0], pick[1], u * carry[0], carry[1], wred, pick);
+}
+
+__global__ __launch_bounds__(ST) void draw_kernel(const float* __restrict__ logits, int* __restrict__ out,
+                                                  const float* __restrict__ uniform, SampleWork w, int V, float inv_t,
+                                                  int filtered) {
+  __shared__ float wred[ST / 64];
+  const int b = blockIdx.x;
+  draw_from_tiles(logits + (size_t)b * V, out, uniform[b], w, b, V, inv_t, row_max(w, b), filtered ? w.thr[b] : 0u, wred);
+}
+
+// ---- top-k of up to TOPK_MOST in one pass over the row
+//
+//   chunk_topk   the chunk's elements in registers; every thread's largest goes to shared memory, and the k-th largest of
+//                these 256 is a bound that at least k of the chunk's elements reach: what reaches it (about -256 ln(1 - k/256)
+//                elements where the large ones are spread) goes to the chunk's list with its index.  Whatever the row's k
+//                largest are, ties among them included, they are in the lists.
+//   row_topk     a block a row: the same bound once more over the lists' elements, then every survivor counts the larger ones
+//                (the threshold of top-k) and adds up the mass at and above itself (top-p, the same fixed point); the sums of
+//                the tiles from the kept elements alone, each lane's share in index order as tile_sum adds them (what it adds
+//                for the others is zero), and the draw.
+//
+// So a row is read once, and the tile of the draw once more.  Against five passes (64 rows of 256,000, top-k 50, top-p 0.95):
+// 22 + 23 us, 103 before: the one pass takes twice its reads' time (registers allow three waves a SIMD), row_topk the latency
+// of its phases.  Rows that the lists do not settle (one that holds no number or no finite maximum, lists that
+// outgrow their room because of ties or an uneven spread) take the bisection over the whole row within row_topk.
+constexpr int TOPK_MOST = 200;       // beyond, the bound of 256 maxima lets too much through
+constexpr int TOPK_LIST = 7168;      // elements of a row's lists in shared memory
+constexpr int TOPK_LEFT = 1024;      // survivors
+constexpr int TOPK_TILES = 128;      // tiles a row
+
+struct TopkShape {
+  int tiles, chunks, room;           // tiles a chunk, chunks a row, elements a chunk's list
+};
+// Fewer elements a chunk while 1,024 blocks are not reached and the lists' expected length fits; chunks of 0: not this way.
+__host__ inline TopkShape topk_shape(int B, int tiles, int top_k, int capg) {
+  if (top_k > TOPK_MOST || tiles > TOPK_TILES) return {0, 0, 0};
+  const float expected = -256.f * logf(1.f - top_k / 256.f) * 1.1f + 16.f;
+  int per = 1;
+  while (per < 4 && ((long)B * ceil_div(tiles, per) > 1024 || ceil_div(tiles, per) * expected > 0.9f * TOPK_LIST)) per *= 2;
+  const int chunks = ceil_div(tiles, per);
+  if (chunks * expected > 0.9f * TOPK_LIST) return {0, 0, 0};
+  return {per, chunks, capg / chunks};
+}
+
+// The k-th largest of n <= 256 keys in shared memory (0: fewer than k of them are above 0 keys of no element); every thread
+// of the block calls it, `mine` is the key of thread tid < 256.
+__device__ __forceinline__ uint32_t kth_of_256(const uint32_t* keys, uint32_t mine, int k, uint32_t* wmin, int n_waves) {
+  uint32_t v = 0xffffffffu;
+  if (threadIdx.x < 256) {
+    int larger = 0;
+    const uint4* k4 = reinterpret_cast<const uint4*>(keys);
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {
+      const uint4 x = k4[j];
+      larger += (x.x > mine) + (x.y > mine) + (x.z > mine) + (x.w > mine);
+    }
+    if (larger < k) v = mine;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = min(v, (uint32_t)__shfl_xor(v, o, 64));
+  if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = v;
+  __syncthreads();
+  for (int x = 0; x < n_waves; ++x) v = min(v, wmin[x]);
+  return v;
+}
+
+template <int VEC, int TILES>
+__global__ __launch_bounds__(SB) void chunk_topk_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t, int top_k,
+                                                        TopkShape sh) {
+  constexpr int NE = TILES * TILE / SB;                    // elements a thread
+  __shared__ __align__(16) uint32_t keys[SB];
+  __shared__ uint32_t wmin[SB / 64];
+  __shared__ int fill, odd;
+  const int b = blockIdx.y, c = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const float* row = logits + (size_t)b * V;
+  const int lo = c * TILES * TILE, hi = min(V, lo + TILES * TILE);
+  if (tid == 0) fill = odd = 0;
+  auto index = [&](int e) { return VEC == 4 ? lo + ((e >> 2) * SB + tid) * 4 + (e & 3) : lo + e * SB + tid; };
+  float x[NE];
+#pragma unroll
+  for (int e = 0; e < NE; e += 4) {
+    if constexpr (VEC == 4) {
+      const float4 v = *reinterpret_cast<const float4*>(row + min(index(e), V - 4));
+      x[e] = v.x; x[e + 1] = v.y; x[e + 2] = v.z; x[e + 3] = v.w;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[e + i] = row[min(index(e + i), V - 1)];
+    }
+  }
+  uint32_t key[NE], most = 0;                              // 0: no element
+  bool nan = false;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const float v = x[e] * inv_t;
+    nan = nan || v != v;                                   // (an element read twice at the row's end is looked at twice)
+    key[e] = order_key(v);
+  }
+  if (hi - lo < TILES * TILE) {
+#pragma unroll
+    for (int e = 0; e < NE; ++e) key[e] = index(e) < hi ? key[e] : 0u;
+  }
+#pragma unroll
+  for (int e = 0; e < NE; ++e) most = max(most, key[e]);
+  keys[tid] = most;
+  __syncthreads();
+  if (nan) odd = 1;
+  const uint32_t bound = max(kth_of_256(keys, most, top_k, wmin, SB / 64), 1u);
+  unsigned long long* list = w.cmass + (size_t)b * w.capg + (size_t)c * sh.room;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    if (key[e] >= bound) {
+      const int pos = atomicAdd(&fill, 1);
+      if (pos < sh.room) list[pos] = ((unsigned long long)key[e] << 32) | (uint32_t)index(e);
+    }
+  }
+  __syncthreads();
+  if (tid == 0) w.tlast[(size_t)b * w.tiles + c] = (odd || fill > sh.room) ? -1 : fill;
+}
+
+template <int VEC>
+__global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ logits, int* __restrict__ out,
+                                                      const float* __restrict__ uniform, SampleWork w, int V, float inv_t, int top_k,
+                                                      float top_p, TopkShape sh) {
+  __shared__ __align__(16) unsigned long long list[TOPK_LIST];       // then the tiles' sums by lane
+  __shared__ __align__(16) uint32_t lkey[TOPK_LEFT + 4];             // the survivors; 0 up to a multiple of four
+  __shared__ __align__(16) unsigned long long lmass[TOPK_LEFT + 4];
+  __shared__ __align__(16) int lat[TOPK_LEFT], lslot[TOPK_LEFT + 4];
+  __shared__ __align__(16) uint32_t keys[256];
+  __shared__ uint32_t wmin[ST / 64];
+  __shared__ unsigned long long wsum[ST / 64];
+  __shared__ int first[TOPK_TILES + 1], n_left, last_kept, rounds, pick[2];
+  __shared__ float red[17], wred[ST / 64], tsum[TOPK_TILES], prefix[TOPK_TILES], carry[2];
+  __shared__ int ired[ST / 64];
+  __shared__ uint32_t best;
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float* row = logits + (size_t)b * V;
+  const float u = uniform[b];
+  const int* counts = w.tlast + (size_t)b * w.tiles;
+  if (tid < sh.chunks) first[tid + 1] = counts[tid];
+  if (tid == 0) { first[0] = 0; n_left = 0; last_kept = -1; rounds = 0; best = 0; }
+  __syncthreads();
+  if (tid == 0) {
+    int at = 0;
+    bool fine = true;
+    for (int c = 0; c < sh.chunks; ++c) {
+      const int k = first[c + 1];
+      fine = fine && k >= 0;
+      at += max(k, 0);
+      first[c + 1] = at;
+    }
+    if (!fine) first[sh.chunks] = -1;
+  }
+  __syncthreads();
+  const int n = first[sh.chunks];
+  bool settled = n >= 1 && n <= TOPK_LIST;
+  uint32_t key_m = 0;
+  if (settled) {
+    for (int c = wave; c < sh.chunks; c += ST / 64) {
+      const unsigned long long* src = w.cmass + (size_t)b * w.capg + (size_t)c * sh.room;
+      for (int i = first[c] + lane; i < first[c + 1]; i += 64) list[i] = src[i - first[c]];
+    }
+    __syncthreads();
+    // the bound again: the largest of every four threads' elements, of these the k-th largest
+    uint32_t most = 0;
+    for (int i = tid; i < n; i += ST) most = max(most, (uint32_t)(list[i] >> 32));
+    most = max(most, (uint32_t)__shfl_xor(most, 1, 64));
+    most = max(most, (uint32_t)__shfl_xor(most, 2, 64));
+    if ((tid & 3) == 0) keys[tid >> 2] = most;
+    __syncthreads();
+    const uint32_t bound = kth_of_256(keys, tid < 256 ? keys[tid] : 0u, top_k, wmin, ST / 64);
+    for (int x = 0; x < 256; x += 64) key_m = max(key_m, keys[x + lane]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) key_m = max(key_m, (uint32_t)__shfl_xor(key_m, o, 64));
+    for (int i = tid; i < n; i += ST)
+      if ((uint32_t)(list[i] >> 32) >= bound) {
+        const int pos = atomicAdd(&n_left, 1);
+        if (pos < TOPK_LEFT) {
+          lkey[pos] = (uint32_t)(list[i] >> 32);
+          lat[pos] = (int)(uint32_t)list[i];
+        }
+      }
+    __syncthreads();
+    settled = n_left <= TOPK_LEFT && fabsf(key_value(key_m)) < INFINITY;
+  }
+  if (!settled) {                                          // the whole row, as the kernels for any k do it at worst
+    float lmax = -INFINITY;
+    for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) { lmax = fmaxf(lmax, ok ? x : -INFINITY); });
+    const float m = block_max(lmax, red);
+    const uint32_t thr = whole_row_threshold<VEC>(row, V, inv_t, m, order_key(m), 0u, false, top_p >= 1.f, top_k, top_p, red, ired);
+    __syncthreads();
+    tile_sums<VEC>(row, w, b, V, inv_t, m, thr, wave, w.tiles, ST / 64);
+    __syncthreads();
+    draw_from_tiles(row, out, u, w, b, V, inv_t, m, thr, wred);
+    return;
+  }
+  const float m = key_value(key_m);
+  const int nl = n_left, quads = (nl + 3) >> 2;
+  const uint32_t key = tid < nl ? lkey[tid] : 0u;
+  const int at = tid < nl ? lat[tid] : 0;
+  if (tid >= nl && tid < quads * 4) { lkey[tid] = 0; lmass[tid] = 0; lslot[tid] = -1; }
+  __syncthreads();
+  int larger = 0;
+  if (tid < nl) {
+#pragma unroll 4
+    for (int j = 0; j < quads; ++j) {
+      const uint4 o = reinterpret_cast<const uint4*>(lkey)[j];
+      larger += (o.x > key) + (o.y > key) + (o.z > key) + (o.w > key);
+    }
+  }
+  const bool kept_k = tid < nl && larger < top_k;
+  uint32_t thr = kept_k ? key : 0xffffffffu;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) thr = min(thr, (uint32_t)__shfl_xor(thr, o, 64));
+  const unsigned long long mass = kept_k ? fixed_mass(key_value(key), m) : 0ull;
+  const unsigned long long z_wave = wave_sum_u64(mass);
+  if (tid < nl) lmass[tid] = mass;
+  __syncthreads();                                         // (the first bound's minima have been read)
+  if (lane == 0) { wmin[wave] = thr; wsum[wave] = z_wave; }
+  __syncthreads();
+  unsigned long long z = 0;
+  for (int x = 0; x < ST / 64; ++x) { thr = min(thr, wmin[x]); z += wsum[x]; }
+  if (top_p < 1.f) {
+    // the largest key at and above which lies more than the target
+    const unsigned long long target = (unsigned long long)((double)top_p * (double)z);
+    unsigned long long above = 0;
+    if (kept_k) {
+#pragma unroll 2
+      for (int j = 0; j < quads; ++j) {
+        const uint4 o = reinterpret_cast<const uint4*>(lkey)[j];
+        const ulonglong2 m0 = reinterpret_cast<const ulonglong2*>(lmass)[2 * j], m1 = reinterpret_cast<const ulonglong2*>(lmass)[2 * j + 1];
+        above += (o.x >= key ? m0.x : 0ull) + (o.y >= key ? m0.y : 0ull) + (o.z >= key ? m1.x : 0ull) + (o.w >= key ? m1.y : 0ull);
+      }
+    }
+    if (kept_k && above > target) atomicMax(&best, key);
+    __syncthreads();
+    thr = best;
+  }
+  // the tiles' sums: a lane of tile_sum adds its elements in index order
+  float* lanes = reinterpret_cast<float*>(list);           // [tiles][64]
+  for (int i = tid; i < w.tiles * 64; i += ST) lanes[i] = 0.f;
+  const bool kept = tid < nl && key >= thr;
+  const float e = kept ? expf(key_value(key) - m) : 0.f;
+  const int slot = (at / TILE) * 64 + (VEC == 4 ? (at >> 2) & 63 : at & 63);
+  if (tid < nl) lslot[tid] = kept ? slot : -1;
+  __syncthreads();
+  int turn = 0;                                            // kept elements of the same lane before this one
+  if (kept) {
+#pragma unroll 4
+    for (int j = 0; j < quads; ++j) {
+      const int4 o = reinterpret_cast<const int4*>(lslot)[j];
+      if (o.x == slot) turn += lat[4 * j] < at;
+      if (o.y == slot) turn += lat[4 * j + 1] < at;
+      if (o.z == slot) turn += lat[4 * j + 2] < at;
+      if (o.w == slot) turn += lat[4 * j + 3] < at;
+    }
+    if (e > 0.f) atomicMax(&last_kept, at);
+    atomicMax(&rounds, turn + 1);
+  }
+  __syncthreads();
+  const int n_rounds = rounds;
+  for (int r = 0; r < n_rounds; ++r) {
+    if (kept && turn == r) lanes[slot] += e;
+    __syncthreads();
+  }
+  for (int t = wave; t < w.tiles; t += ST / 64) {
+    const float s = wave_sum(lanes[t * 64 + lane]);
+    if (lane == 0) tsum[t] = s;
+  }
+  if (tid == 0) { pick[0] = -1; pick[1] = -1; carry[1] = 0.f; }
+  __syncthreads();
+  // their running sums, in order (a wave: what a lane reads of the others costs no trip through memory)
+  if (wave == 0) {
+    float acc = 0.f, p0 = 0.f, p1 = 0.f;
+    const float s0 = lane < w.tiles ? tsum[lane] : 0.f, s1 = 64 + lane < w.tiles ? tsum[min(64 + lane, w.tiles - 1)] : 0.f;
+    for (int t = 0; t < w.tiles; ++t) {
+      acc += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t < 64 ? s0 : s1), t & 63));
+      if (lane == (t & 63)) { if (t < 64) p0 = acc; else p1 = acc; }
+    }
+    if (lane < w.tiles) prefix[lane] = p0;
+    if (64 + lane < w.tiles) prefix[64 + lane] = p1;
+    if (lane == 0) carry[0] = acc;
+  }
+  __syncthreads();
+  const float target = u * carry[0];
+  if (tid < w.tiles) {
+    const float lo = tid == 0 ? 0.f : prefix[tid - 1];
+    if (target >= lo && target < prefix[tid]) { pick[0] = tid; carry[1] = lo; }      // at most one tile
+  }
+  __syncthreads();
+  draw_in_tile(row, out, b, V, inv_t, m, thr, pick[0], last_kept, target, carry[1], wred, pick);
 }
 
 // How long a row's list may be: 32,768 candidates, fewer (down to what fits shared memory) when the lists of
@@ -776,6 +1078,25 @@ extern "C" int alice_sample(const float* logits, int* out, const float* uniform,
   const float inv_t = 1.f / temperature;
   const bool need_k = top_k > 0 && top_k < V, need_p = top_p < 1.f;
   const int filtered = need_k || need_p;
+  const bool vec = V % 4 == 0 && ((uintptr_t)logits & 15) == 0;
+  if (need_k) {                                            // a small k: the row is read once
+    const TopkShape sh = topk_shape(B, w.tiles, top_k, w.capg);
+    if (sh.chunks > 0) {
+#define GO(VEC)                                                                                             \
+  do {                                                                                                      \
+    const dim3 grid(sh.chunks, B);                                                                          \
+    if (sh.tiles == 4) chunk_topk_kernel<VEC, 4><<<grid, SB, 0, stream>>>(logits, w, V, inv_t, top_k, sh);  \
+    else if (sh.tiles == 2) chunk_topk_kernel<VEC, 2><<<grid, SB, 0, stream>>>(logits, w, V, inv_t, top_k, sh); \
+    else chunk_topk_kernel<VEC, 1><<<grid, SB, 0, stream>>>(logits, w, V, inv_t, top_k, sh);                \
+    ALICE_LAUNCH_CHECK();                                                                                   \
+    row_topk_kernel<VEC><<<B, ST, 0, stream>>>(logits, out, uniform, w, V, inv_t, top_k, top_p, sh);        \
+  } while (0)
+      if (vec) GO(4); else GO(1);
+#undef GO
+      ALICE_LAUNCH_CHECK();
+      return 0;
+    }
+  }
   const dim3 cgrid(w.chunks, B);
 #define GO(VEC)                                                                                                             \
   do {                                                                                                                      \
@@ -787,7 +1108,7 @@ extern "C" int alice_sample(const float* logits, int* out, const float* uniform,
     }                                                                                                                       \
     tile_sum_kernel<VEC><<<cgrid, SB, 0, stream>>>(logits, w, V, inv_t, filtered);                                          \
   } while (0)
-  if (V % 4 == 0 && ((uintptr_t)logits & 15) == 0) GO(4); else GO(1);
+  if (vec) GO(4); else GO(1);
 #undef GO
   ALICE_LAUNCH_CHECK();
   draw_kernel<<<B, ST, 0, stream>>>(logits, out, uniform, w, V, inv_t, filtered);
