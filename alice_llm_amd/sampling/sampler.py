@@ -10,6 +10,7 @@ from __future__ import annotations
 
 from typing import List, Optional, Sequence
 
+import numpy as np
 import torch
 
 from ..hip import ops
@@ -30,6 +31,30 @@ def uniform(seed: int, request: int, n: int) -> float:
     """The n-th uniform number in [0, 1) of request `request` under `seed`."""
     stream = splitmix64((seed & _M) ^ ((request * 0xD1B54A32D192ED03) & _M))
     return (splitmix64((stream + n) & _M) >> 40) / float(1 << 24)
+
+
+def _u64(x: Sequence[int]) -> np.ndarray:
+    try:
+        return np.array(x, dtype=np.int64).view(np.uint64)
+    except OverflowError:
+        return np.array([int(v) & _M for v in x], dtype=np.uint64)
+
+
+def _splitmix64_all(x: np.ndarray) -> np.ndarray:
+    x = x + np.uint64(0x9E3779B97F4A7C15)                    # arrays of 64-bit integers wrap
+    z = (x ^ (x >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    return z ^ (z >> np.uint64(31))
+
+
+def uniforms(seed: int, requests: Sequence[int], draws: Sequence[int]) -> torch.Tensor:
+    """uniform(seed, requests[i], draws[i]) for all i as float32 (24 bits: exact).  All at once from 24 rows on: 64 rows take
+    25 us so and 69 one by one, 8 rows 20 and 13."""
+    if len(requests) < 24:
+        return torch.tensor([uniform(seed, r, n) for r, n in zip(requests, draws)], dtype=torch.float32)
+    stream = _splitmix64_all((_u64(requests) * np.uint64(0xD1B54A32D192ED03)) ^ np.uint64(seed & _M))
+    drawn = _splitmix64_all(stream + _u64(draws)) >> np.uint64(40)
+    return torch.from_numpy((drawn.astype(np.float64) / float(1 << 24)).astype(np.float32))
 
 
 class Sampler:
@@ -56,7 +81,7 @@ class Sampler:
         how many tokens it has drawn before.  Returns int32 [B] on the GPU."""
         if self.greedy:
             return ops.argmax(logits)
-        u = torch.tensor([uniform(self.seed, r, n) for r, n in zip(requests, draws)], dtype=torch.float32)
+        u = uniforms(self.seed, requests, draws)
         return ops.sample(logits, self._upload(u, logits.device), self.temperature, self.top_k, self.top_p)
 
     def _upload(self, u: torch.Tensor, device) -> torch.Tensor:
