@@ -191,15 +191,22 @@ int alice_gla(const float* rows, int row_w, int q_col, int k_col, int v_col, int
 // state [slots, channels, taps - 1]; act 1: silu.  See recurrent.hip for this and the four entries below.
 int alice_short_conv(const float* rows, int row_w, int col0, int channels, int taps, const float* w, const float* bias,
                      float* state, float* out, int act, const int* cu_seqlens, const int* seq_of_token, const int* slots,
-                     int T, int n_seqs, hipStream_t stream);
-// step = softplus(rows[:, dt_col + h] + dt_bias[h]), decay = exp(-exp(a_log[h]) step) (as_log: its logarithm), both [T, H]
-int alice_ssm_prepare(const float* rows, int row_w, int dt_col, const float* dt_bias, const float* a_log, float* step,
-                      float* decay, int T, int H, int as_log, hipStream_t stream);
-// unit vectors of the q and k heads of qk [T, q (G d) | ... k at k_col (G d)] in place (q times q_scale); z [T, H d] turned
-// into decays exp(-exp(a_log[h]) softplus(z + dt_bias)) (as_log: their logarithms) in place; beta[t, h] = sigmoid(rows[t, b_col + h])
-int alice_delta_prepare(float* qk, int qk_w, int k_col, int G, int d, float unit_eps, float q_scale, float* z,
-                        const float* dt_bias, const float* a_log, const float* rows, int row_w, int b_col, float* beta,
-                        int T, int H, int as_log, hipStream_t stream);
+                     int T, int n_seqs, int form, hipStream_t stream);
+// (form, here and below: 1 by tokens, 2 by sequences, in one launch with the state; 3 channel by channel, taken for what 1 and 2 do not cover)
+// The convolution (with silu) and what else a state space takes from the rows: step = softplus(rows[:, dt_col + h] + dt_bias[h]),
+// decay = exp(-exp(a_log[h]) step) (as_log: its logarithm), both [T, H].
+int alice_ssm_enter(const float* rows, int row_w, int col0, int channels, int taps, const float* w, const float* bias, float* state,
+                    float* out, int dt_col, const float* dt_bias, const float* a_log, float* step, float* decay, int H, int as_log,
+                    const int* cu_seqlens, const int* seq_of_token, const int* slots, int T, int n_seqs, int form, hipStream_t stream);
+// The convolution (with silu) of the columns q | k | v and what else the delta rule takes from the rows: the q and k heads (G
+// of d each) as unit vectors x / sqrt(sum x^2 + unit_eps), q times q_scale; beta[t, h] = sigmoid(rows[t, b_col + h]); the columns
+// [low_col, + n0) and the n1 behind them to low0 [T, n0] and low1 [T, n1] in low_dtype.
+int alice_delta_enter(const float* rows, int row_w, int channels, int taps, const float* w, float* state, float* out, int G, int d,
+                      float unit_eps, float q_scale, int b_col, int H, float* beta, int low_col, int n0, int n1, void* low0, void* low1,
+                      int low_dtype, const int* cu_seqlens, const int* seq_of_token, const int* slots, int T, int n_seqs, int form,
+                      hipStream_t stream);
+// z [T, H d] turned into decays exp(-exp(a_log[h]) softplus(z + dt_bias)) (as_log: their logarithms) in place
+int alice_delta_decay(float* z, const float* dt_bias, const float* a_log, int T, int H, int d, int as_log, hipStream_t stream);
 // The matrix-state recurrence over a step's tokens (delta 0: S = diag(a) S + k (b v)^T; 1: the delta rule), o to out
 // [T, H dv] float32; q and k are shared by groups of H / qk_heads heads; decay [T, H d] (decay_per_row) or [T, H].
 int alice_matrix_recurrence(const float* q, int q_w, int q_col, const float* k, int k_w, int k_col, const float* v, int v_w,

@@ -72,9 +72,10 @@ def _declare(lib) -> None:
         "alice_attention_split_runs": [I],
         "alice_mix_heads": [P, P, P, I, F, P, I, I, I, I, I, I, P],
         "alice_qkv_prepare": [P, I, I, P, P, P, P, I, P, P, I, I, P, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, P],
-        "alice_short_conv": [P, I, I, I, I, P, P, P, P, I, P, P, P, I, I, P],
-        "alice_ssm_prepare": [P, I, I, P, P, P, P, I, I, I, P],
-        "alice_delta_prepare": [P, I, I, I, I, F, F, P, P, P, P, I, I, P, I, I, I, P],
+        "alice_short_conv": [P, I, I, I, I, P, P, P, P, I, P, P, P, I, I, I, P],
+        "alice_ssm_enter": [P, I, I, I, I, P, P, P, P, I, P, P, P, P, I, I, P, P, P, I, I, I, P],
+        "alice_delta_enter": [P, I, I, I, P, P, P, I, I, F, F, I, I, P, I, I, I, P, P, I, P, P, P, I, I, I, P],
+        "alice_delta_decay": [P, P, P, I, I, I, I, P],
         "alice_recurrence_chunks": [P, I, I, P, I, I, P, I, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P],
         "alice_matrix_recurrence": [P, I, I, P, I, I, P, I, I, P, I, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
         "alice_matrix_recurrence_columns": [I, I, I, I],
@@ -1135,11 +1136,19 @@ def _step_arrays(ctx) -> None:
         raise HipLibraryError("cu_seqlens and slots are too short for the step's sequences")
 
 
-def short_conv(rows: torch.Tensor, col0: int, weight: torch.Tensor, bias: Optional[torch.Tensor], state: Optional[torch.Tensor],
-               out: torch.Tensor, ctx, *, silu: bool = True) -> None:
-    """out[t, c] = act(bias[c] + sum_j weight[c, j] x[t - (taps - 1) + j, c]) with x = rows[:, col0 + c] (float32), over the
-    tokens of the token's own sequence; what lies before the step comes from state float32 [slots, channels, taps - 1]
-    (the last inputs of the sequence's earlier steps, zeros at its start), which then takes the step's last inputs."""
+# Steps whose longest piece has at most this many tokens take the convolution by sequences (with the state in the same
+# launch), longer ones by tokens: the same sums in the same order.  Eight sequences of 6,144 channels: 4 tokens each 5.1 us
+# by sequences and 13.0 by tokens, 8 tokens 8.2 and 11.8, 16 tokens 14.8 and 12.3.
+CONV_WALK_UP_TO = 8
+CONV_BY_TOKENS, CONV_BY_SEQUENCES, CONV_BY_CHANNELS = 1, 2, 3
+
+
+def _conv_form(ctx) -> int:
+    return CONV_BY_SEQUENCES if getattr(ctx, "max_new", CONV_WALK_UP_TO + 1) <= CONV_WALK_UP_TO else CONV_BY_TOKENS
+
+
+def _conv_checked(rows, col0, weight, bias, state, out, ctx):
+    """The sizes (T, channels, taps) of a convolution whose operands fit together."""
     T = rows.shape[0]
     if weight.dim() != 2:
         raise HipLibraryError("weight must be [channels, taps]")
@@ -1158,46 +1167,66 @@ def short_conv(rows: torch.Tensor, col0: int, weight: torch.Tensor, bias: Option
         if state is None or state.dim() != 3 or tuple(state.shape[1:]) != (C, taps - 1):
             raise HipLibraryError(f"state must be [slots, {C}, {taps - 1}]")
         _dev(state, "state", torch.float32)
+    return T, C, taps
+
+
+def short_conv(rows: torch.Tensor, col0: int, weight: torch.Tensor, bias: Optional[torch.Tensor], state: Optional[torch.Tensor],
+               out: torch.Tensor, ctx, *, silu: bool = True, form: Optional[int] = None) -> None:
+    """out[t, c] = act(bias[c] + sum_j weight[c, j] x[t - (taps - 1) + j, c]) with x = rows[:, col0 + c] (float32), over the
+    tokens of the token's own sequence; what lies before the step comes from state float32 [slots, channels, taps - 1]
+    (the last inputs of the sequence's earlier steps, zeros at its start), which then takes the step's last inputs.
+    form: CONV_BY_*; None: by the step's longest piece."""
+    T, C, taps = _conv_checked(rows, col0, weight, bias, state, out, ctx)
     _call("alice_short_conv", rows.data_ptr(), rows.shape[1], int(col0), C, taps, weight.data_ptr(), _opt(bias, "bias"),
           None if taps == 1 else state.data_ptr(), out.data_ptr(), int(bool(silu)), ctx.cu_seqlens.data_ptr(),
-          ctx.seq_of_token.data_ptr(), ctx.slots.data_ptr(), T, int(ctx.n_seqs), _stream())
+          ctx.seq_of_token.data_ptr(), ctx.slots.data_ptr(), T, int(ctx.n_seqs), form or _conv_form(ctx), _stream())
 
 
-def ssm_prepare(rows: torch.Tensor, dt_col: int, dt_bias: torch.Tensor, a_log: torch.Tensor, step: torch.Tensor,
-                decay: torch.Tensor, *, as_log: bool = False) -> None:
-    """step = softplus(rows[:, dt_col + h] + dt_bias[h]); decay = exp(-exp(a_log[h]) * step), as_log: its logarithm;
-    float32 [T, heads] each."""
-    T, H = step.shape
-    _dev(rows, "rows", torch.float32)
+def ssm_enter(rows: torch.Tensor, col0: int, weight: torch.Tensor, bias: Optional[torch.Tensor], state: Optional[torch.Tensor],
+              out: torch.Tensor, ctx, dt_col: int, dt_bias: torch.Tensor, a_log: torch.Tensor, step: torch.Tensor,
+              decay: torch.Tensor, *, as_log: bool = False, form: Optional[int] = None) -> None:
+    """short_conv with silu, and in the same launch step = softplus(rows[:, dt_col + h] + dt_bias[h]) and decay =
+    exp(-exp(a_log[h]) * step), as_log: its logarithm; float32 [T, heads] each."""
+    T, C, taps = _conv_checked(rows, col0, weight, bias, state, out, ctx)
+    H = step.shape[1]
     _dev(dt_bias, "dt_bias", torch.float32, (H,))
     _dev(a_log, "a_log", torch.float32, (H,))
-    _dev(step, "step", torch.float32)
+    _dev(step, "step", torch.float32, (T, H))
     _dev(decay, "decay", torch.float32, (T, H))
-    if rows.shape[0] != T or dt_col + H > rows.shape[1]:
+    if dt_col + H > rows.shape[1]:
         raise HipLibraryError("rows do not hold the step sizes")
-    _call("alice_ssm_prepare", rows.data_ptr(), rows.shape[1], int(dt_col), dt_bias.data_ptr(), a_log.data_ptr(), step.data_ptr(),
-          decay.data_ptr(), T, H, int(as_log), _stream())
+    _call("alice_ssm_enter", rows.data_ptr(), rows.shape[1], int(col0), C, taps, weight.data_ptr(), _opt(bias, "bias"),
+          None if taps == 1 else state.data_ptr(), out.data_ptr(), int(dt_col), dt_bias.data_ptr(), a_log.data_ptr(), step.data_ptr(),
+          decay.data_ptr(), H, int(as_log), ctx.cu_seqlens.data_ptr(), ctx.seq_of_token.data_ptr(), ctx.slots.data_ptr(), T,
+          int(ctx.n_seqs), form or _conv_form(ctx), _stream())
 
 
-def delta_prepare(qk: torch.Tensor, k_col: int, z: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor, rows: torch.Tensor,
-                  b_col: int, beta: torch.Tensor, *, qk_heads: int, heads: int, head_dim: int, unit_eps: float, q_scale: float,
-                  as_log: bool = False) -> None:
-    """In place: the q heads (columns 0 .. qk_heads * d of qk) and the k heads (from k_col) become unit vectors
-    x / sqrt(sum x^2 + unit_eps), q also times q_scale; z [T, heads * d] becomes exp(-exp(a_log[h]) softplus(z + dt_bias)), as_log: its logarithm;
-    beta[t, h] = sigmoid(rows[t, b_col + h])."""
-    T = qk.shape[0]
-    G, H, d = qk_heads, heads, head_dim
-    _dev(qk, "qk", torch.float32)
+def delta_enter(rows: torch.Tensor, weight: torch.Tensor, state: Optional[torch.Tensor], out: torch.Tensor, ctx, b_col: int,
+                beta: torch.Tensor, low_col: int, low0: torch.Tensor, low1: torch.Tensor, *, qk_heads: int, head_dim: int,
+                unit_eps: float, q_scale: float, form: Optional[int] = None) -> None:
+    """short_conv with silu over the columns q | k | v (from column 0), and in the same launch: the q and k heads (qk_heads of
+    head_dim each) become unit vectors x / sqrt(sum x^2 + unit_eps), q also times q_scale; beta[t, h] = sigmoid(rows[t, b_col + h]);
+    the columns from low_col to low0 and the ones behind them to low1, in their dtype."""
+    T, C, taps = _conv_checked(rows, 0, weight, None, state, out, ctx)
+    H = beta.shape[1]
+    _dev(beta, "beta", torch.float32, (T, H))
+    _dev(low0, "low0", None, (T, low0.shape[1]))
+    _dev(low1, "low1", low0.dtype, (T, low1.shape[1]))
+    if b_col + H > rows.shape[1] or low_col + low0.shape[1] + low1.shape[1] > rows.shape[1] or 2 * qk_heads * head_dim > C:
+        raise HipLibraryError("the rows are too short for the heads")
+    _call("alice_delta_enter", rows.data_ptr(), rows.shape[1], C, taps, weight.data_ptr(), None if taps == 1 else state.data_ptr(),
+          out.data_ptr(), int(qk_heads), int(head_dim), float(unit_eps), float(q_scale), int(b_col), H, beta.data_ptr(), int(low_col),
+          low0.shape[1], low1.shape[1], low0.data_ptr(), low1.data_ptr(), dtype_code(low0.dtype), ctx.cu_seqlens.data_ptr(),
+          ctx.seq_of_token.data_ptr(), ctx.slots.data_ptr(), T, int(ctx.n_seqs), form or _conv_form(ctx), _stream())
+
+
+def delta_decay(z: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor, *, heads: int, head_dim: int, as_log: bool = False) -> None:
+    """In place: z [T, heads * d] becomes exp(-exp(a_log[h]) softplus(z + dt_bias)), as_log: its logarithm."""
+    T, H, d = z.shape[0], heads, head_dim
     _dev(z, "z", torch.float32, (T, H * d))
     _dev(dt_bias, "dt_bias", torch.float32, (H * d,))
     _dev(a_log, "a_log", torch.float32, (H,))
-    _dev(rows, "rows", torch.float32)
-    _dev(beta, "beta", torch.float32, (T, H))
-    if rows.shape[0] != T or b_col + H > rows.shape[1] or k_col < G * d or k_col + G * d > qk.shape[1]:
-        raise HipLibraryError("the rows are too short for the heads")
-    _call("alice_delta_prepare", qk.data_ptr(), qk.shape[1], int(k_col), G, d, float(unit_eps), float(q_scale), z.data_ptr(),
-          dt_bias.data_ptr(), a_log.data_ptr(), rows.data_ptr(), rows.shape[1], int(b_col), beta.data_ptr(), T, H,
-          int(as_log), _stream())
+    _call("alice_delta_decay", z.data_ptr(), dt_bias.data_ptr(), a_log.data_ptr(), T, H, d, int(as_log), _stream())
 
 
 def recurrence_columns(n_seqs: int, heads: int, head_dim: int, value_head_dim: int) -> int:

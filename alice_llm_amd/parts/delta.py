@@ -122,17 +122,18 @@ class ChannelDeltaMixer(Part):
         T, n, dev, act = x.shape[0], self.names, self.proj.weight.device, self.precision.act
         rows = self.proj(x, torch.float32)                   # [T, q | k | v | b | a | g], nothing rounded
         conv = torch.empty((T, self.channels), dtype=torch.float32, device=dev)
-        ops.short_conv(rows, 0, self.conv_w, None, cache.state.get("conv"), conv, ctx)
-        # the second matrices of the decay and of the gate: their operands in the activation dtype
-        z = self.decay(rows[:, self.a_col:self.a_col + self.ra].to(act).contiguous(), torch.float32)
-        gate = self.gate(rows[:, self.g_col:self.g_col + self.rg].to(act).contiguous(), torch.float32)
         beta = torch.empty((T, self.nH), dtype=torch.float32, device=dev)
-        # pieces of many tokens by chunks, which take the decays' logarithms
+        # the operands of the decay's and of the gate's second matrix: in the activation dtype
+        low_a, low_g = (torch.empty((T, r), dtype=act, device=dev) for r in (self.ra, self.rg))
         heads = dict(heads=self.nH, qk_heads=self.nKV, head_dim=self.d)
         values = dict(value_head_dim=self.P, delta=True)
+        ops.delta_enter(rows, self.conv_w, cache.state.get("conv"), conv, ctx, self.b_col, beta, self.a_col, low_a, low_g,
+                        qk_heads=self.nKV, head_dim=self.d, unit_eps=self.unit_eps, q_scale=self.d ** -0.5)
+        z = self.decay(low_a, torch.float32)
+        gate = self.gate(low_g, torch.float32)
+        # pieces of many tokens by chunks, which take the decays' logarithms
         chunks = ops.recurrence_by_chunks(ctx, self.channels, 0, **values, **heads)
-        ops.delta_prepare(conv, self.qk, z, self.small[n["dt_bias"]], self.small[n["A_log"]], rows, self.b_col, beta,
-                          unit_eps=self.unit_eps, q_scale=self.d ** -0.5, as_log=chunks, **heads)
+        ops.delta_decay(z, self.small[n["dt_bias"]], self.small[n["A_log"]], heads=self.nH, head_dim=self.d, as_log=chunks)
         o = torch.empty((T, self.vw), dtype=torch.float32, device=dev)
         args = (conv, 0, conv, self.qk, conv, 2 * self.qk, z, beta, None, o, ctx, cache.state["S"])
         if chunks:

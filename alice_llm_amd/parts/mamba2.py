@@ -91,14 +91,14 @@ class StateSpaceMixer(Part):
         T, n, dev = x.shape[0], self.names, self.proj.weight.device
         rows = self.proj(x, torch.float32)                   # [T, z | x | B | C | dt], nothing rounded
         conv = torch.empty((T, self.channels), dtype=torch.float32, device=dev)
-        ops.short_conv(rows, self.inner, self.small[n["conv"]], self.small[n["conv_bias"]], cache.state.get("conv"), conv, ctx)
         step = torch.empty((T, self.nH), dtype=torch.float32, device=dev)
         decay = torch.empty_like(step)
         # pieces of many tokens by chunks, which take the decays' logarithms
         b_col, c_col = self.inner, self.inner + self.G * self.N
         heads = dict(heads=self.nH, qk_heads=self.G, head_dim=self.N, value_head_dim=self.P)
         chunks = ops.recurrence_by_chunks(ctx, self.channels, c_col, delta=False, **heads)
-        ops.ssm_prepare(rows, self.dt_col, self.small[n["dt_bias"]], self.small[n["A_log"]], step, decay, as_log=chunks)
+        ops.ssm_enter(rows, self.inner, self.small[n["conv"]], self.small[n["conv_bias"]], cache.state.get("conv"), conv, ctx,
+                      self.dt_col, self.small[n["dt_bias"]], self.small[n["A_log"]], step, decay, as_log=chunks)
         y = torch.empty((T, self.inner), dtype=torch.float32, device=dev)
         args = (conv, c_col, conv, b_col, conv, 0, decay, step, self.small[n["D"]], y, ctx, cache.state["S"])
         if chunks:
