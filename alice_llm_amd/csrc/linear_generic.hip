@@ -12,8 +12,9 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int BK = 32;       // inner elements a stage
-constexpr int LROW = BK + 4; // row length of a stage in LDS: 16-byte pieces of 16 neighbouring rows lie in different banks
+// Inner elements a stage; a row of a stage in LDS is eight 16-byte pieces, piece p of row r at p ^ (r / 2 % 8): the pieces that
+// 16 lanes read (one of 16 neighbouring rows) or write (two whole rows) at a time lie in different banks.
+constexpr int BK = 32;
 
 // Four neighbouring elements of a row as float32.  VEC: in one load (rows start at multiples of four elements on memory
 // aligned for them, K is a multiple of four); else one by one, none beyond the row's end.  Loads are unconditional: one
@@ -25,34 +26,37 @@ template <> __device__ __forceinline__ f32x4 load4<bf16_t>(const bf16_t* __restr
   return f32x4{bf16_bits_to_f32(w.x & 0xffffu), bf16_bits_to_f32(w.x >> 16), bf16_bits_to_f32(w.y & 0xffffu), bf16_bits_to_f32(w.y >> 16)};
 }
 template <typename T, bool VEC>
-__device__ __forceinline__ f32x4 load_row4(const T* __restrict__ row, int k, int K) {
-  if constexpr (VEC) return load4<T>(row + min(k, K - 4));
-  return f32x4{load_f32(row, min(k, K - 1)), load_f32(row, min(k + 1, K - 1)), load_f32(row, min(k + 2, K - 1)), load_f32(row, min(k + 3, K - 1))};
+__device__ __forceinline__ f32x4 load_row4(const T* __restrict__ row, int k, int end) {
+  if constexpr (VEC) return load4<T>(row + min(k, end - 4));
+  return f32x4{load_f32(row, min(k, end - 1)), load_f32(row, min(k + 1, end - 1)), load_f32(row, min(k + 2, end - 1)), load_f32(row, min(k + 3, end - 1))};
 }
 
 // More than 16 tokens: the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: 32-bit products and sums, the rate of the
 // vector unit's FMA at a quarter of its register reads).  A block of 2 x 2 waves takes 32 TM tokens by 32 TN rows of W, a
 // wave 16 TM by 16 TN; both operands go through LDS 32 inner elements at a time in two buffers (one barrier a stage), the
-// next stage on its way from memory meanwhile.  A lane reads 16-byte pieces: lane group g of a 16-element chunk holds the
+// stage after the next on its way from memory meanwhile.  Every LDS and memory instruction stands behind a product of the
+// same wave: with all of them ahead of a stage's products the waves of a SIMD fell into step and left the matrix unit idle
+// a quarter of the time.  A lane reads 16-byte pieces: lane group g of a 16-element chunk holds the
 // elements 4 g .. 4 g + 3 of its row, and product i of the chunk takes element i of every group, the same permutation of
 // the inner dimension on both sides.  W is the first operand, so that a lane ends up with four neighbouring outputs of a
 // token.  With GeGLU the first half of a wave's rows are gate rows, the second half the up rows of the same outputs.
 // blockIdx: the tiles of one set of W rows are neighbours on one XCD, whose L2 then serves W's rows to all of them.
 // split: slices of the inner dimension, slice z to Y + z M N (float32 sums that the residual add adds up).
 //
-// What bounds it: the matrix instruction (157 TFLOP/s at 256 CUs).  A product of 500 tokens with 18,432 x 2,304 rows
-// and GeGLU takes 438 us (97 TFLOP/s), the down product of 2,304 x 9,216 188 us (113) in slices, against 1,576 and
-// 1,444 us with a 64 x 64 tile of scalar FMAs, which read an LDS operand for every two of them.
+// What bounds it: the matrix instruction (157 TFLOP/s at 256 CUs and 2.4 GHz, 141 at the 2.15 GHz that it runs at under this
+// load; 512 tokens by 16,384 x 2,304 rows reach 129).  A product of 500 tokens with 18,432 x 2,304 rows and GeGLU takes
+// 350 us (122 TFLOP/s), the down product of 2,304 x 9,216 176 us (120) in slices; 438 and 188 with the instructions of a
+// stage ahead of its products, 1,576 and 1,444 with a 64 x 64 tile of scalar FMAs.
 template <typename TA, typename TW, typename TO, int TM, int TN, bool VEC>
 __global__ __launch_bounds__(256) void linear_mfma32_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y,
                                                             int M, int N, int K, int kslice, int mt, int nt, int epi, float param,
                                                             int full, int wide) {
   constexpr int BM = 32 * TM, BN = 32 * TN;
   constexpr int YROW = BN + 4;
-  static_assert(BM * YROW <= 2 * (BM + BN) * LROW, "the outputs do not fit where the operands were");
-  __shared__ __align__(16) float lds[2 * (BM + BN) * LROW];
-  auto As = reinterpret_cast<float (*)[BM][LROW]>(lds);
-  auto Bs = reinterpret_cast<float (*)[BN][LROW]>(lds + 2 * BM * LROW);
+  constexpr int STAGES = 2 * (BM + BN) * BK;
+  __shared__ __align__(16) float lds[STAGES > BM * YROW ? STAGES : BM * YROW];
+  auto As = reinterpret_cast<float (*)[BM][BK]>(lds);
+  auto Bs = reinterpret_cast<float (*)[BN][BK]>(lds + 2 * BM * BK);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
   const int wm = wave & 1, wn = wave >> 1;
 
@@ -65,15 +69,15 @@ __global__ __launch_bounds__(256) void linear_mfma32_kernel(const TA* __restrict
   const int n0 = nb * (geglu ? BN / 2 : BN);
   const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);
 
-  // loaders: 16-byte piece `id` of a stage is row id / 8, elements (id % 8) * 4
-  const int lk = (tid & 7) * 4;
+  // loaders: 16-byte piece `id` of a stage is row id / 8, elements (id % 8) * 4; lw, sw: where it is written, what is read (see BK)
+  const int lk = (tid & 7) * 4, lr = tid >> 3, lw = lk ^ (lr / 2 % 8 * 4), sw = c / 2 % 8 * 4;
   const TA* arow[TM];                                         // rows beyond the last are read as the last and not written
   const TW* wrow[TN];
 #pragma unroll
-  for (int j = 0; j < TM; ++j) arow[j] = A + (size_t)min(m0 + (tid >> 3) + 32 * j, M - 1) * K;
+  for (int j = 0; j < TM; ++j) arow[j] = A + (size_t)min(m0 + lr + 32 * j, M - 1) * K;
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int r = (tid >> 3) + 32 * j;
+    const int r = lr + 32 * j;
     int row = min(n0 + r, N - 1);
     if (geglu) {                                              // a wave's 16 TN rows: gate rows, then up rows of the same outputs
       const int w = r / (16 * TN), rr = r % (16 * TN), half = rr / (8 * TN);
@@ -81,61 +85,75 @@ __global__ __launch_bounds__(256) void linear_mfma32_kernel(const TA* __restrict
     }
     wrow[j] = W + (size_t)row * K;
   }
-  f32x4 pa[TM], pb[TN];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int j = 0; j < TM; ++j) pa[j] = load_row4<TA, VEC>(arow[j], k0 + lk, K);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) pb[j] = load_row4<TW, VEC>(wrow[j], k0 + lk, K);
+  f32x4 pa[TM], pb[TN];                                       // the stage on its way from memory
+  auto load = [&](int n, int k0) {                            // its n-th piece
+    if (n < TM) pa[n] = load_row4<TA, VEC>(arow[n], k0 + lk, k_end);
+    else pb[n - TM] = load_row4<TW, VEC>(wrow[n - TM], k0 + lk, k_end);
   };
-  auto stage = [&](int buf, int k0) {
-    if (k0 + BK > k_end) {                                    // the last stage of a slice: nothing beyond its end
+  auto clear_beyond = [&](int k0) {                           // the last stage of a slice: nothing beyond its end
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool in = k0 + lk + e < k_end;
+    for (int e = 0; e < 4; ++e) {
+      const bool in = k0 + lk + e < k_end;
 #pragma unroll
-        for (int j = 0; j < TM; ++j) pa[j][e] = in ? pa[j][e] : 0.f;
+      for (int j = 0; j < TM; ++j) pa[j][e] = in ? pa[j][e] : 0.f;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) pb[j][e] = in ? pb[j][e] : 0.f;
-      }
+      for (int j = 0; j < TN; ++j) pb[j][e] = in ? pb[j][e] : 0.f;
     }
-#pragma unroll
-    for (int j = 0; j < TM; ++j) *reinterpret_cast<f32x4*>(&As[buf][(tid >> 3) + 32 * j][lk]) = pa[j];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4*>(&Bs[buf][(tid >> 3) + 32 * j][lk]) = pb[j];
   };
-
+  auto write = [&](int n, int buf) {
+    if (n < TM) *reinterpret_cast<f32x4*>(&As[buf][lr + 32 * n][lw]) = pa[n];
+    else *reinterpret_cast<f32x4*>(&Bs[buf][lr + 32 * (n - TM)][lw]) = pb[n - TM];
+  };
+  f32x4 f0[TN + TM], f1[TN + TM];                             // operands of a stage's first and second 16 elements
+  auto read = [&](f32x4 (&f)[TN + TM], int n, int buf, int ch) {
+    if (n < TN) f[n] = *reinterpret_cast<const f32x4*>(&Bs[buf][(wn * TN + n) * 16 + c][(ch + g * 4) ^ sw]);
+    else f[n] = *reinterpret_cast<const f32x4*>(&As[buf][(wm * TM + n - TN) * 16 + c][(ch + g * 4) ^ sw]);
+  };
   f32x4 acc[TN][TM];
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // The products of 16 elements with one other instruction behind each (op(0) .. op(ops - 1)): it is issued while the product
+  // runs.
+  constexpr int PRODUCTS = 4 * TM * TN, PIECES = TM + TN, READS = TN + TM;
+  auto products = [&](const f32x4 (&f)[TN + TM], int ops, auto&& op) {
+#pragma unroll
+    for (int p = 0; p < PRODUCTS; ++p) {
+      const int e = p / (TN * TM), i = p / TM % TN, j = p % TM;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[i][e], f[TN + j][e], acc[i][j], 0, 0, 0);
+      if (p < ops) op(p);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int p = PRODUCTS; p < ops; ++p) op(p);
+  };
 
-  fetch(k_begin);
-  stage(0, k_begin);
-  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < PIECES; ++n) load(n, k_begin);
+  if (k_begin + BK > k_end) clear_beyond(k_begin);
+#pragma unroll
+  for (int n = 0; n < PIECES; ++n) write(n, 0);
+#pragma unroll
+  for (int n = 0; n < PIECES; ++n) load(n, k_begin + BK);
+  lds_barrier();
+#pragma unroll
+  for (int n = 0; n < READS; ++n) read(f0, n, 0, 0);
+  // Behind the first half's products: the reads for the second half, the next stage into the other buffer (whose last reads
+  // were ahead of the last barrier), the loads of the stage after it; behind the second half's: the next stage's first reads.
   int cur = 0;
   for (int k0 = k_begin; k0 < k_end; k0 += BK) {
-    const bool more = k0 + BK < k_end;
-    if (more) fetch(k0 + BK);
-#pragma unroll
-    for (int ch = 0; ch < BK; ch += 16) {
-      f32x4 wf[TN], xf[TM];
-#pragma unroll
-      for (int i = 0; i < TN; ++i) wf[i] = *reinterpret_cast<const f32x4*>(&Bs[cur][(wn * TN + i) * 16 + c][ch + g * 4]);
-#pragma unroll
-      for (int j = 0; j < TM; ++j) xf[j] = *reinterpret_cast<const f32x4*>(&As[cur][(wm * TM + j) * 16 + c][ch + g * 4]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int i = 0; i < TN; ++i)
-#pragma unroll
-          for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], xf[j][e], acc[i][j], 0, 0, 0);
-    }
-    if (more) stage(cur ^ 1, k0 + BK);                                 // read two stages ago, by waves that have passed a barrier since
-    __syncthreads();
+    if (k0 + 2 * BK > k_end) clear_beyond(k0 + BK);
+    products(f0, READS + 2 * PIECES, [&](int n) {
+      if (n < READS) read(f1, n, cur, 16);
+      else if (n < READS + PIECES) write(n - READS, cur ^ 1);
+      else load(n - READS - PIECES, k0 + 2 * BK);
+    });
+    lds_barrier();
+    products(f1, READS, [&](int n) { read(f0, n, cur ^ 1, 0); });
     cur ^= 1;
   }
+  __syncthreads();
 
   // The outputs go through LDS (the last barrier has passed): 16-byte pieces of a token's row, and the epilogue's functions stand
   // in the code for four elements and not for a lane's 16 TM TN / 4 (which took 16,000 instructions).
@@ -176,27 +194,34 @@ __global__ __launch_bounds__(256) void linear_mfma32_kernel(const TA* __restrict
   }
 }
 
-// Tile and number of slices for a product.  Estimated microseconds: rounds of blocks over the CUs times a block's products at
-// a CU's 0.61 TFLOP/s (less for small tiles, which read LDS more often, and for a CU with a single block, which waits for
-// its own barriers), not less than reading W takes; slices cost writing and reading their sums.
+// Tile and number of slices for a product.  Estimated microseconds: 8, and for every block that a CU gets its products at a CU's
+// rate (TFLOP/s, measured with 1 to 8 blocks a CU and K 576 and 2,304) and 1 more; not less than reading W takes; slices cost
+// writing and reading their sums.  The rates are close, so what decides is how evenly the tiles fill the CUs: 500 tokens with
+// GeGLU on 18,432 x 2,304 rows are 1,536 tiles of 64 x 96, six a CU, 350 us; 576 of 128 x 128, three for some, 504.  (A CU holds
+// two blocks of 128 x 128: a third one runs alone.)
+struct Tile {
+  int bm, bn;
+  float rate;
+};
+constexpr Tile TILES[] = {{128, 128, 0.510f}, {128, 64, 0.500f}, {64, 96, 0.492f}, {64, 64, 0.490f}, {32, 64, 0.460f}};
 struct Plan {
-  int tm, tn, split;
+  int tile, split;
 };
 Plan plan_mfma32(int M, int N, int K, bool geglu, int max_split) {
-  static const struct { int tm, tn; float eff; } tiles[] = {{4, 4, 0.85f}, {2, 4, 0.80f}, {2, 2, 0.70f}, {1, 2, 0.50f}};
-  Plan best{2, 2, 1};
+  Plan best{3, 1};
   float best_us = 1e30f;
-  for (const auto& t : tiles) {
-    const int mt = ceil_div(M, 32 * t.tm), nt = ceil_div(N, geglu ? 16 * t.tn : 32 * t.tn);
+  for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
+    const Tile& t = TILES[i];
+    const int mt = ceil_div(M, t.bm), nt = ceil_div(N, geglu ? t.bn / 2 : t.bn);
     for (int s = 1; s <= max_split; ++s) {
       const int ks = ceil_div(ceil_div(K, s), BK) * BK;
       if (s > 1 && (ks < 256 || (long)ks * (s - 1) >= K)) continue;      // no slice without elements
-      const float rounds = (float)ceil_div((long)mt * nt * s, 256);
-      const float block_us = 2.f * (32 * t.tm) * (32 * t.tn) * (float)ks / (0.614e6f * t.eff) + 2.f;
-      float us = rounds * block_us * (rounds < 2.f ? 1.25f : 1.f);
+      const int blocks = ceil_div((long)mt * nt * s, 256);
+      const float alone = i == 0 && blocks > 1 && blocks % 2 ? 0.5f : 0.f;
+      float us = 8.f + (blocks + alone) * (2.f * t.bm * t.bn * (float)ks / (1e6f * t.rate) + 1.f);
       us = fmaxf(us, (geglu ? 2.f : 1.f) * N * (float)K * 4.f / 4.5e6f);
       if (s > 1) us += 2.f * s * (float)M * N * 4.f / 4.0e6f;
-      if (us < best_us) { best_us = us; best = Plan{t.tm, t.tn, s}; }
+      if (us < best_us) { best_us = us; best = Plan{i, s}; }
     }
   }
   return best;
@@ -325,18 +350,19 @@ int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int
     if (q.split == split) p = q;
   }
   const int vec = K % 4 == 0 && ((uintptr_t)x & (4 * sizeof(TA) - 1)) == 0 && ((uintptr_t)w & (4 * sizeof(TW) - 1)) == 0;
-  if (!vec) p.tm = p.tn = 2;                                  // one tile for rows that are no multiples of four elements
+  if (!vec) p.tile = 3;                                       // one tile for rows that are no multiples of four elements
   const int kslice = ceil_div(ceil_div(K, split), BK) * BK;
-  const int BM = 32 * p.tm, cols = epi == ALICE_EPI_GEGLU ? 16 * p.tn : 32 * p.tn;
+  const int BM = TILES[p.tile].bm, cols = epi == ALICE_EPI_GEGLU ? TILES[p.tile].bn / 2 : TILES[p.tile].bn;
   const int mt = ceil_div(M, BM), nt = ceil_div(N, cols);
   ALICE_CHECK((long)mt * nt < (1l << 30), "linear: too many tiles for one launch");
   const int wide = N % 4 == 0 && ((uintptr_t)y & 15) == 0;
   dim3 grid(8 * ceil_div((long)mt * nt, 8), split);
 #define GO(TM, TN, VEC) linear_mfma32_kernel<TA, TW, TO, TM, TN, VEC><<<grid, 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, kslice, mt, nt, epi, epi_param, full, wide)
   if (!vec) GO(2, 2, false);
-  else if (p.tm == 4) GO(4, 4, true);
-  else if (p.tm == 2 && p.tn == 4) GO(2, 4, true);
-  else if (p.tm == 2) GO(2, 2, true);
+  else if (p.tile == 0) GO(4, 4, true);
+  else if (p.tile == 1) GO(4, 2, true);
+  else if (p.tile == 2) GO(2, 3, true);
+  else if (p.tile == 3) GO(2, 2, true);
   else GO(1, 2, true);
 #undef GO
   ALICE_LAUNCH_CHECK();
