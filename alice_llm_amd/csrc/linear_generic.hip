@@ -229,12 +229,13 @@ Plan plan_mfma32(int M, int N, int K, bool geglu, int max_split) {
 constexpr int MAX_SPLIT = 8;
 
 // Up to 16 tokens: the tokens are the columns of the same matrix instruction, the rows of W its rows.  A block takes 16 R rows
-// (with GeGLU 16 gate rows and the up rows of the same outputs), its four waves every fourth chunk of 32 inner elements of
+// (with GeGLU 8 gate rows and the up rows of the same outputs: twice the blocks of 16 and 16, and the registers for more of
+// them a CU), its four waves every fourth chunk of 32 inner elements of
 // its slice; their sums meet in LDS.  W goes straight from memory into the instruction's operand, 128 bytes of a row a
 // chunk, the next two chunks on their way while two are multiplied; the tokens' elements come through the L1.  A token's
 // result depends on no other token.
 //
-// What bounds it: reading W.  At 4 tokens (2B shape): gate and up (170 MB) 42 us, 4.1 TB/s, the output head (2.36 GB)
+// What bounds it: reading W.  At 4 tokens (2B shape): gate and up (170 MB) 41 us, 4.1 TB/s, the output head (2.36 GB)
 // 405 us, 5.8; a wave a row on FMAs, which read every token's elements again for every row, 49 and 652 us.
 template <typename T>
 __device__ __forceinline__ void load8(const T* __restrict__ p, f32x4* v);
@@ -254,12 +255,12 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(const TA* __restrict__
   constexpr int U = 2;                                        // chunks a step
   __shared__ __align__(16) f32x4 red[4][R][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
-  const bool geglu = R == 2 && epi == ALICE_EPI_GEGLU;
-  const int n0 = blockIdx.x * (geglu ? 16 : 16 * R);
+  const bool geglu = R == 1 && epi == ALICE_EPI_GEGLU;
+  const int n0 = blockIdx.x * (geglu ? 8 : 16 * R);
   const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);
   const TW* wrow[R];                                          // rows and tokens beyond the last are read as the last and not written
 #pragma unroll
-  for (int r = 0; r < R; ++r) wrow[r] = W + (size_t)(geglu ? r * N + min(n0 + c, N - 1) : min(n0 + r * 16 + c, N - 1)) * K + g * 8;
+  for (int r = 0; r < R; ++r) wrow[r] = W + (size_t)(geglu ? (c >> 3) * N + min(n0 + (c & 7), N - 1) : min(n0 + r * 16 + c, N - 1)) * K + g * 8;
   const TA* arow = A + (size_t)min(c, M - 1) * K + g * 8;
 
   f32x4 acc[R][2];
@@ -306,26 +307,36 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(const TA* __restrict__
 #pragma unroll
   for (int r = 0; r < R; ++r) red[wave][r][lane] = acc[r][0] + acc[r][1];
   __syncthreads();
-  if (wave >= (geglu ? 1 : R) || c >= M) return;
-  f32x4 v[R];
+  if (wave >= R) return;
+  f32x4 v = (red[0][wave][lane] + red[1][wave][lane]) + (red[2][wave][lane] + red[3][wave][lane]), up;
+  if (geglu) {                                                // the up rows of lane group g are with lane group g + 2
 #pragma unroll
-  for (int r = 0; r < R; ++r) v[r] = (red[0][r][lane] + red[1][r][lane]) + (red[2][r][lane] + red[3][r][lane]);
-  if (R == 2 && !geglu && wave == 1) v[0] = v[R - 1];
-  const int n = n0 + (geglu ? 0 : wave * 16) + g * 4;
+    for (int e = 0; e < 4; ++e) up[e] = __shfl_xor(v[e], 32, 64);
+    if (g >= 2) return;
+  }
+  if (c >= M) return;
+  const int n = n0 + wave * 16 + g * 4;
   TO* y = Y + (size_t)blockIdx.y * M * N + (size_t)c * N;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    if (n + e >= N) continue;
-    float o = v[0][e];
-    if (geglu) o = gated_act(o, v[R - 1][e], param, full);
+    if (n + e >= (geglu ? min(N, n0 + 8) : N)) continue;
+    float o = v[e];
+    if (geglu) o = gated_act(o, up[e], param, full);
     if (epi == ALICE_EPI_SOFTCAP) o = unary_act(o, param, full);
     store_f32(y, n + e, o);
   }
 }
 
-// Slices of the inner dimension for up to 16 tokens: two blocks a CU where the rows alone do not give them, slices of at
-// least 512 elements (2,304 rows by 9,216 and by 2,048 at 4 tokens: 16 us on average in four, 30 in one with a wave a row).
-int rows_split(int N, int K) { return max(1, min(min(ceil_div(512, ceil_div(N, 16)), K / 512), 8)); }
+// Slices of the inner dimension for up to 16 tokens: three blocks a CU where the rows alone do not give them, slices of at
+// least 256 elements, and rather a few more slices than uneven ones.  At 4 tokens 2,304 rows by 9,216 take 38 us whole, 24.1 in
+// four slices, 21.8 in six; by 2,048: 10.6, 8.1, 8.5 in six (uneven), 7.2 in eight; 4,096 rows by 2,304: 14.1, 12.4 in four, 10.8
+// in three.
+int rows_split(int N, int K) {
+  const int most = max(1, min(K / 256, 8)), least = min(ceil_div(768, ceil_div(N, 16)), most);
+  for (int s = least; s <= most; ++s)
+    if (K % (128 * s) == 0) return s;
+  return least;
+}
 bool rows_cover(int M, int K) { return M <= 16 && K % 8 == 0 && K >= 32; }
 
 template <typename TA, typename TW, typename TO>
@@ -333,7 +344,7 @@ int launch_rows(const void* x, const void* w, void* y, int M, int N, int K, int 
                 hipStream_t stream) {
   const int kslice = ceil_div(ceil_div(K, split), 128) * 128;
 #define GO(R, BLOCKS) linear_rows_kernel<TA, TW, TO, R><<<dim3(BLOCKS, split), 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, kslice, epi, epi_param, full)
-  if (epi == ALICE_EPI_GEGLU) GO(2, ceil_div(N, 16));
+  if (epi == ALICE_EPI_GEGLU) GO(1, ceil_div(N, 8));
   else if (N >= 16384) GO(2, ceil_div(N, 32));                // enough blocks: a token's elements serve 32 rows
   else GO(1, ceil_div(N, 16));
 #undef GO

@@ -16,7 +16,8 @@ DEV = "cuda"
 
 
 # ------------------------------------------------------------------ products
-@pytest.mark.parametrize("M,N,K", [(1, 64, 9216), (4, 16400, 72), (9, 64, 32), (13, 46, 1032), (16, 100, 2048), (17, 64, 40), (31, 33, 36), (33, 65, 68), (64, 128, 31), (129, 257, 96), (250, 2304, 2048), (500, 1000, 2308)])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 9216), (4, 16400, 72), (9, 64, 32), (13, 46, 1032), (16, 100, 2048), (17, 64, 40), (31, 33, 36), (33, 65, 68), (64, 128, 31), (129, 257, 96), (250, 2304, 2048), (500, 1000, 2308),
+                                   (257, 4002, 100), (250, 8202, 36), (250, 24004, 36)])
 @pytest.mark.parametrize("xdt,wdt", [("float32", "float32"), ("float32", "bfloat16"), ("bfloat16", "float32")])
 def test_products_at_the_edges_of_tiles_and_slices(M, N, K, xdt, wdt):
     x, w = rnd(M, K, seed=M, dtype=DT[xdt]), rnd(N, K, seed=N, scale=0.1, dtype=DT[wdt])
