@@ -227,6 +227,11 @@ Plan plan_mfma32(int M, int N, int K, bool geglu, int max_split) {
   return best;
 }
 constexpr int MAX_SPLIT = 8;
+// The number of tokens that the slices are planned for.  Their number decides in which order the sums of an output are added, and an
+// output must not depend on how a step is launched: steps of single tokens are captured with their number rounded up to a power of two
+// up to 64 and to a multiple of 64 beyond, short prompts to a multiple of 16.  Any number of tokens here gives what either rounding of it
+// gives.  (Numbers of tokens on two sides of a multiple of 64 may add in another order: rounding, no more.)
+int planned_tokens(int M) { return M <= 32 ? 32 : ceil_div(M, 64) * 64; }
 
 // Up to 16 tokens: the tokens are the columns of the same matrix instruction, the rows of W its rows.  A block takes 16 R rows
 // (with GeGLU 8 gate rows and the up rows of the same outputs: twice the blocks of 16 and 16, and the registers for more of
@@ -357,7 +362,7 @@ int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int
                  hipStream_t stream) {
   Plan p = plan_mfma32(M, N, K, epi == ALICE_EPI_GEGLU, 1);
   if (split > 1) {                                            // the tile that goes best with this many slices
-    const Plan q = plan_mfma32(M, N, K, false, MAX_SPLIT);
+    const Plan q = plan_mfma32(planned_tokens(M), N, K, false, MAX_SPLIT);
     if (q.split == split) p = q;
   }
   const int vec = K % 4 == 0 && ((uintptr_t)x & (4 * sizeof(TA) - 1)) == 0 && ((uintptr_t)w & (4 * sizeof(TW) - 1)) == 0;
@@ -384,7 +389,7 @@ int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int
 
 // Into how many slices of the inner dimension a product without an epilogue is best cut.
 int alice_linear_split_hint_generic(int M, int N, int K) {
-  return rows_cover(M, K) ? rows_split(N, K) : plan_mfma32(M, N, K, false, MAX_SPLIT).split;
+  return rows_cover(M, K) ? rows_split(N, K) : plan_mfma32(planned_tokens(M), N, K, false, MAX_SPLIT).split;
 }
 
 int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype,

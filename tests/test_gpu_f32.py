@@ -8,6 +8,7 @@ import torch
 import torch.nn.functional as F
 
 from alice_llm_amd.hip import ops
+from helpers import TINY, random_tokens
 from plain import gemma2_plain as P
 from test_gpu_kernels import DT, attention_case, close, rnd
 
@@ -52,6 +53,31 @@ def test_products_refuse_slices_with_an_epilogue_and_too_many():
         ops.linear(x, w, torch.empty(2, 16, 64, device=DEV), n_out=64, k_in=64, epilogue=ops.EPI_SOFTCAP, epi_param=1.0, split_k=2, full_precision=True)
     with pytest.raises(ops.HipLibraryError, match="slices"):
         ops.linear(x, w, torch.empty(9, 16, 64, device=DEV), n_out=64, k_in=64, split_k=9, full_precision=True)
+
+
+def test_sliced_products_add_in_one_order_in_captured_and_eager_steps():
+    """A layer whose output and down projections go in slices (which the tiny shapes are too narrow for): prompts whose token
+    count a captured step rounds up, and single tokens of 33 sequences, for which it takes 64 rows: the same bits."""
+    import alice_llm_amd as alice
+    raw = dict(TINY["tiny-a"][0], num_hidden_layers=1, hidden_size=2304, num_attention_heads=8, num_key_value_heads=4, head_dim=256,
+               intermediate_size=1024, query_pre_attn_scalar=256)
+    model = alice.Model.random(raw, seed=4, dtype="float32", fast=True)
+    eager, graph = (model.engine(max_tokens=64 * 70, max_seqs=40, use_graphs=g) for g in (False, True))
+    assert graph.capture_prompts
+    assert ops.linear_split_hint(49, 2304, 2048, ops.LAYOUT_ROW) > 1
+    for n in (49, 129, 200):
+        for seed in range(3):                                            # seen, captured, replayed
+            toks = random_tokens(256, n, seed)
+            a, b = ([e.open(1), e] for e in (eager, graph))
+            assert torch.equal(a[1].step(a[0], [toks], "last"), b[1].step(b[0], [toks], "last")), (n, seed)
+            eager.close(a[0]), graph.close(b[0])
+    slots = [e.open(33) for e in (eager, graph)]
+    first = [random_tokens(256, 2, 100 + i) for i in range(33)]
+    logits = [e.step(s, first, "last") for e, s in zip((eager, graph), slots)]
+    for _ in range(3):
+        ids = [[int(t)] for t in logits[0].argmax(dim=1)]
+        logits = [e.step(s, ids, "last") for e, s in zip((eager, graph), slots)]
+        assert torch.equal(*logits)
 
 
 # ------------------------------------------------------------------ attention
