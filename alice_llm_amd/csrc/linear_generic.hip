@@ -235,60 +235,80 @@ int planned_tokens(int M) { return M <= 32 ? 32 : ceil_div(M, 64) * 64; }
 
 // Up to 16 tokens: the tokens are the columns of the same matrix instruction, the rows of W its rows.  A block takes 16 R rows
 // (with GeGLU 8 gate rows and the up rows of the same outputs: twice the blocks of 16 and 16, and the registers for more of
-// them a CU), its four waves every fourth chunk of 32 inner elements of
+// them a CU), its NW waves every NW-th chunk of 32 inner elements of
 // its slice; their sums meet in LDS.  W goes straight from memory into the instruction's operand, 128 bytes of a row a
 // chunk, the next two chunks on their way while two are multiplied; the tokens' elements come through the L1.  A token's
-// result depends on no other token.
+// result depends on no other token, nor on how many there are.
+// WHOLE: rows of whole, aligned units of eight elements.  Else (any K, any address) the same loads without an alignment, and the
+// elements behind the last whole chunk one by one, by the wave whose turn it is: 2,304 rows by 2,305 at 4 tokens 9.0 us (by 2,304
+// 9.1; on the tile of 64 tokens 71).
 //
 // What bounds it: reading W.  At 4 tokens (2B shape): gate and up (170 MB) 41 us, 4.1 TB/s, the output head (2.36 GB)
 // 405 us, 5.8; a wave a row on FMAs, which read every token's elements again for every row, 49 and 652 us.
-template <typename T>
-__device__ __forceinline__ void load8(const T* __restrict__ p, f32x4* v);
-template <> __device__ __forceinline__ void load8<float>(const float* __restrict__ p, f32x4* v) {
-  v[0] = *reinterpret_cast<const f32x4*>(p);
-  v[1] = *reinterpret_cast<const f32x4*>(p + 4);
+template <bool ALIGNED>
+__device__ __forceinline__ f32x4 piece(const float* __restrict__ p) {
+  struct __attribute__((packed, aligned(4))) Any { f32x4 v; };
+  if constexpr (ALIGNED) return *reinterpret_cast<const f32x4*>(p);
+  return reinterpret_cast<const Any*>(p)->v;
 }
-template <> __device__ __forceinline__ void load8<bf16_t>(const bf16_t* __restrict__ p, f32x4* v) {
-  const uint4 w = *reinterpret_cast<const uint4*>(p);
+template <bool ALIGNED>
+__device__ __forceinline__ void load8(const float* __restrict__ p, f32x4* v) {
+  v[0] = piece<ALIGNED>(p);
+  v[1] = piece<ALIGNED>(p + 4);
+}
+template <bool ALIGNED>
+__device__ __forceinline__ void load8(const bf16_t* __restrict__ p, f32x4* v) {
+  struct __attribute__((packed, aligned(2))) Any { uint4 v; };
+  uint4 w;
+  if constexpr (ALIGNED) w = *reinterpret_cast<const uint4*>(p);
+  else w = reinterpret_cast<const Any*>(p)->v;
   v[0] = f32x4{bf16_bits_to_f32(w.x & 0xffffu), bf16_bits_to_f32(w.x >> 16), bf16_bits_to_f32(w.y & 0xffffu), bf16_bits_to_f32(w.y >> 16)};
   v[1] = f32x4{bf16_bits_to_f32(w.z & 0xffffu), bf16_bits_to_f32(w.z >> 16), bf16_bits_to_f32(w.w & 0xffffu), bf16_bits_to_f32(w.w >> 16)};
 }
 
-template <typename TA, typename TW, typename TO, int R>
-__global__ __launch_bounds__(256) void linear_rows_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y, int M,
-                                                          int N, int K, int kslice, int epi, float param, int full) {
-  constexpr int U = 2;                                        // chunks a step
-  __shared__ __align__(16) f32x4 red[4][R][64];
+template <typename TA, typename TW, typename TO, int R, int NW, bool WHOLE>
+__global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y, int M,
+                                                              int N, int K, int kslice, int epi, float param, int full) {
+  constexpr int U = 2, TURN = NW * 32;                        // chunks a step; elements from one of a wave's chunks to its next
+  __shared__ __align__(16) f32x4 red[NW][R][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
   const bool geglu = R == 1 && epi == ALICE_EPI_GEGLU;
   const int n0 = blockIdx.x * (geglu ? 8 : 16 * R);
   const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);
+  const int k_chunks = WHOLE ? K : K & ~31, k_stop = min(k_end, k_chunks);       // what is read in units of eight
   const TW* wrow[R];                                          // rows and tokens beyond the last are read as the last and not written
 #pragma unroll
-  for (int r = 0; r < R; ++r) wrow[r] = W + (size_t)(geglu ? (c >> 3) * N + min(n0 + (c & 7), N - 1) : min(n0 + r * 16 + c, N - 1)) * K + g * 8;
-  const TA* arow = A + (size_t)min(c, M - 1) * K + g * 8;
+  for (int r = 0; r < R; ++r) wrow[r] = W + (size_t)(geglu ? (c >> 3) * N + min(n0 + (c & 7), N - 1) : min(n0 + r * 16 + c, N - 1)) * K;
+  const TA* arow = A + (size_t)min(c, M - 1) * K;
 
   f32x4 acc[R][2];
 #pragma unroll
   for (int r = 0; r < R; ++r) acc[r][0] = acc[r][1] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 w[U][R][2], x[U][2], wn[U][R][2], xn[U][2];
-  const int k_last = K - 32;                                  // (K is a multiple of 8 and at least 32)
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = min(k0 + u * 128, k_last + 24 - g * 8);   // stays inside the row: lane group g reads k + 8 g .. + 7
+      const int k = min(k0 + u * TURN + g * 8, k_chunks - 8);         // stays inside the row
 #pragma unroll
-      for (int r = 0; r < R; ++r) load8<TW>(wrow[r] + k, wn[u][r]);
-      load8<TA>(arow + k, xn[u]);
+      for (int r = 0; r < R; ++r) load8<WHOLE>(wrow[r] + k, wn[u][r]);
+      load8<WHOLE>(arow + k, xn[u]);
     }
   };
+  auto multiply = [&](int u) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u][r][i][e], x[u][i][e], acc[r][e & 1], 0, 0, 0);
+  };
   int k0 = k_begin + wave * 32;
-  if (k0 < k_end) fetch(k0);
-  for (; k0 < k_end; k0 += U * 128) {
+  if (k0 < k_stop) fetch(k0);
+  for (; k0 < k_stop; k0 += U * TURN) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       // beyond the slice's end: zeros on both sides
-      const bool in = k0 + u * 128 + g * 8 < k_end;
+      const bool in = k0 + u * TURN + g * 8 < k_stop;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
 #pragma unroll
@@ -299,21 +319,36 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(const TA* __restrict__
         }
       }
     }
-    if (k0 + U * 128 < k_end) fetch(k0 + U * 128);
+    if (k0 + U * TURN < k_stop) fetch(k0 + U * TURN);
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) multiply(u);
+  }
+  if constexpr (!WHOLE) {
+    if (k_begin <= k_chunks && k_chunks < k_end && wave == (k_chunks - k_begin) / 32 % NW) {
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int e = 0; e < 4; ++e) {
+          const int k = k_chunks + g * 8 + i * 4 + e, kc = min(k, K - 1);
 #pragma unroll
-          for (int r = 0; r < R; ++r) acc[r][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u][r][i][e], x[u][i][e], acc[r][e & 1], 0, 0, 0);
+          for (int r = 0; r < R; ++r) {
+            const float v = load_f32(wrow[r], kc);
+            w[0][r][i][e] = k < K ? v : 0.f;
+          }
+          const float v = load_f32(arow, kc);
+          x[0][i][e] = k < K ? v : 0.f;
+        }
+      multiply(0);
+    }
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) red[wave][r][lane] = acc[r][0] + acc[r][1];
   __syncthreads();
   if (wave >= R) return;
   f32x4 v = (red[0][wave][lane] + red[1][wave][lane]) + (red[2][wave][lane] + red[3][wave][lane]), up;
+#pragma unroll
+  for (int j = 4; j < NW; j += 4)
+    v += (red[j][wave][lane] + red[j + 1][wave][lane]) + (red[j + 2][wave][lane] + red[j + 3][wave][lane]);
   if (geglu) {                                                // the up rows of lane group g are with lane group g + 2
 #pragma unroll
     for (int e = 0; e < 4; ++e) up[e] = __shfl_xor(v[e], 32, 64);
@@ -342,17 +377,28 @@ int rows_split(int N, int K) {
     if (K % (128 * s) == 0) return s;
   return least;
 }
-bool rows_cover(int M, int K) { return M <= 16 && K % 8 == 0 && K >= 32; }
 
 template <typename TA, typename TW, typename TO>
 int launch_rows(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split,
                 hipStream_t stream) {
   const int kslice = ceil_div(ceil_div(K, split), 128) * 128;
-#define GO(R, BLOCKS) linear_rows_kernel<TA, TW, TO, R><<<dim3(BLOCKS, split), 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, kslice, epi, epi_param, full)
-  if (epi == ALICE_EPI_GEGLU) GO(1, ceil_div(N, 8));
-  else if (N >= 16384) GO(2, ceil_div(N, 32));                // enough blocks: a token's elements serve 32 rows
-  else GO(1, ceil_div(N, 16));
+  const bool whole = K % 8 == 0 && K >= 32 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
+  const int by = epi == ALICE_EPI_GEGLU ? 8 : (N >= 16384 ? 32 : 16);      // many rows: a token's elements serve 32 of them
+  const dim3 grid(ceil_div(N, by), split);
+  // Four waves a block, eight where there are few blocks with long rows (2,304 rows by 9,216 in one slice, 2 tokens: 23.5 us, 29.0 with
+  // four; by 2,304 four are the better: 8.3 and 9.0).  A rule without the number of tokens: the sums are the same for all of them.
+  const bool eight = by != 32 && (long)grid.x * split <= 256 && kslice >= 4096;
+#define GO2(R, NW, WHOLE) linear_rows_kernel<TA, TW, TO, R, NW, WHOLE><<<grid, 64 * NW, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, kslice, epi, epi_param, full)
+#define GO(R, NW)                  \
+  do {                             \
+    if (whole) GO2(R, NW, true);   \
+    else GO2(R, NW, false);        \
+  } while (0)
+  if (by == 32) GO(2, 4);
+  else if (eight) GO(1, 8);
+  else GO(1, 4);
 #undef GO
+#undef GO2
   ALICE_LAUNCH_CHECK();
   return 0;
 }
@@ -389,7 +435,7 @@ int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int
 
 // Into how many slices of the inner dimension a product without an epilogue is best cut.
 int alice_linear_split_hint_generic(int M, int N, int K) {
-  return rows_cover(M, K) ? rows_split(N, K) : plan_mfma32(planned_tokens(M), N, K, false, MAX_SPLIT).split;
+  return M <= 16 ? rows_split(N, K) : plan_mfma32(planned_tokens(M), N, K, false, MAX_SPLIT).split;
 }
 
 int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype,
@@ -404,9 +450,8 @@ int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype,
   ALICE_CHECK(split_k >= 1 && split_k <= MAX_SPLIT, "linear: %d slices of the inner dimension are outside 1..%d", split_k, MAX_SPLIT);
   if (M == 0) return 0;
   int rc = 0;
-  const bool rows = rows_cover(M, K) && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
   DISPATCH_DTYPE(x_dtype, TA, DISPATCH_DTYPE(w_dtype, TW, DISPATCH_DTYPE(y_dtype, TO, {
-    rc = rows ? launch_rows<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream)
+    rc = M <= 16 ? launch_rows<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream)
               : launch_tiled<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
   })));
   return rc;

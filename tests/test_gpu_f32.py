@@ -17,7 +17,7 @@ DEV = "cuda"
 
 
 # ------------------------------------------------------------------ products
-@pytest.mark.parametrize("M,N,K", [(1, 64, 9216), (4, 16400, 72), (9, 64, 32), (13, 46, 1032), (16, 100, 2048), (17, 64, 40), (31, 33, 36), (33, 65, 68), (64, 128, 31), (129, 257, 96), (250, 2304, 2048), (500, 1000, 2308),
+@pytest.mark.parametrize("M,N,K", [(1, 64, 9216), (4, 16400, 72), (9, 64, 32), (13, 46, 1032), (3, 70, 33), (8, 2304, 2305), (16, 40, 9220), (5, 24, 30), (16, 100, 2048), (17, 64, 40), (31, 33, 36), (33, 65, 68), (64, 128, 31), (129, 257, 96), (250, 2304, 2048), (500, 1000, 2308),
                                    (257, 4002, 100), (250, 8202, 36), (250, 24004, 36)])
 @pytest.mark.parametrize("xdt,wdt", [("float32", "float32"), ("float32", "bfloat16"), ("bfloat16", "float32")])
 def test_products_at_the_edges_of_tiles_and_slices(M, N, K, xdt, wdt):
@@ -39,12 +39,28 @@ def test_products_at_the_edges_of_tiles_and_slices(M, N, K, xdt, wdt):
         close(out, F.gelu(g, approximate="tanh") * u, 4 * tol, 1e-5)
 
 
-def test_products_of_rows_that_are_not_aligned():
-    big = rnd(40 * 64 + 1, seed=3)
-    x, w = big[1:].view(40, 64), rnd(48 * 64 + 2, seed=4)[2:].view(48, 64)
-    y = torch.empty(40, 48, device=DEV)
-    ops.linear(x, w, y, n_out=48, k_in=64, full_precision=True)
-    close(y, x.double() @ w.double().T, 8 * 64 * 2 ** -24)
+@pytest.mark.parametrize("M", [1, 2, 16, 40])
+@pytest.mark.parametrize("K", [64, 4, 31, 97, 4101])
+def test_products_of_rows_that_are_not_aligned(M, K):
+    big = rnd(M * K + 1, seed=3)
+    for dt in (torch.float32, torch.bfloat16):
+        x, w = big[1:].view(M, K), rnd(48 * K + 3, seed=4).to(dt)[3:].view(48, K)
+        ref = x.double() @ w.double().T
+        for split in (1, 2, 8):
+            y = torch.empty(*((split,) if split > 1 else ()), M, 48, device=DEV)
+            ops.linear(x, w, y, n_out=48, k_in=K, split_k=split, full_precision=True)
+            close(y.sum(0) if split > 1 else y, ref, 8 * K * 2 ** -24)
+
+
+@pytest.mark.parametrize("N,K", [(64, 4101), (2304, 2305), (48, 20), (16400, 37)])
+def test_a_few_tokens_give_each_what_one_of_them_gives(N, K):
+    """Rows of any length, up to 16 tokens: a token's sums are added in the same order however many there are."""
+    x, w = rnd(16, K, seed=1), rnd(N, K, seed=2)
+    outs = []
+    for M in (2, 5, 16):
+        outs.append(torch.empty(M, N, device=DEV))
+        ops.linear(x[:M].contiguous(), w, outs[-1], n_out=N, k_in=K, full_precision=True)
+    assert torch.equal(outs[0], outs[2][:2]) and torch.equal(outs[1], outs[2][:5])
 
 
 def test_products_refuse_slices_with_an_epilogue_and_too_many():
