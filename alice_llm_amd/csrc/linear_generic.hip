@@ -233,7 +233,7 @@ constexpr int MAX_SPLIT = 8;
 // gives.  (Numbers of tokens on two sides of a multiple of 64 may add in another order: rounding, no more.)
 int planned_tokens(int M) { return M <= 32 ? 32 : ceil_div(M, 64) * 64; }
 
-// Up to 16 tokens: the tokens are the columns of the same matrix instruction, the rows of W its rows.  A block takes 16 R rows
+// 2 to 16 tokens: the tokens are the columns of the same matrix instruction, the rows of W its rows.  A block takes 16 R rows
 // (with GeGLU 8 gate rows and the up rows of the same outputs: twice the blocks of 16 and 16, and the registers for more of
 // them a CU), its NW waves every NW-th chunk of 32 inner elements of
 // its slice; their sums meet in LDS.  W goes straight from memory into the instruction's operand, 128 bytes of a row a
@@ -243,8 +243,8 @@ int planned_tokens(int M) { return M <= 32 ? 32 : ceil_div(M, 64) * 64; }
 // elements behind the last whole chunk one by one, by the wave whose turn it is: 2,304 rows by 2,305 at 4 tokens 9.0 us (by 2,304
 // 9.1; on the tile of 64 tokens 71).
 //
-// What bounds it: reading W.  At 4 tokens (2B shape): gate and up (170 MB) 41 us, 4.1 TB/s, the output head (2.36 GB)
-// 405 us, 5.8; a wave a row on FMAs, which read every token's elements again for every row, 49 and 652 us.
+// What bounds it: reading W.  At 4 tokens (2B shape): gate and up (170 MB) 34.6 us, 4.9 TB/s, the output head (2.36 GB)
+// 391 us, 6.0; a wave a row on FMAs, which read every token's elements again for every row, 39.5 and 632 us.
 template <bool ALIGNED>
 __device__ __forceinline__ f32x4 piece(const float* __restrict__ p) {
   struct __attribute__((packed, aligned(4))) Any { f32x4 v; };
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const TA* __restri
   }
 }
 
-// Slices of the inner dimension for up to 16 tokens: three blocks a CU where the rows alone do not give them, slices of at
+// Slices of the inner dimension for 2 to 16 tokens: three blocks a CU where the rows alone do not give them, slices of at
 // least 256 elements, and rather a few more slices than uneven ones.  At 4 tokens 2,304 rows by 9,216 take 38 us whole, 24.1 in
 // four slices, 21.8 in six; by 2,048: 10.6, 8.1, 8.5 in six (uneven), 7.2 in eight; 4,096 rows by 2,304: 14.1, 12.4 in four, 10.8
 // in three.
@@ -376,6 +376,57 @@ int rows_split(int N, int K) {
   for (int s = least; s <= most; ++s)
     if (K % (128 * s) == 0) return s;
   return least;
+}
+
+// One token: a wave a row of W (with GeGLU the gate row and the up row of an output) on FMAs, four elements a lane a step; the lanes'
+// sums meet in a fixed tree.  Any K, any address.  No column of the matrix instruction is idle: 18,432 rows by 2,304 with GeGLU
+// 25.9 us (31.7 as columns, which gain from 2 to 4 tokens on), 256,000 rows 373 (402), 2,304 by 9,216 16.3 (19.1 in slices).
+template <typename TA, typename TW, typename TO, bool GEGLU>
+__global__ __launch_bounds__(256) void linear_single_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y, int N,
+                                                            int K, int epi, float param, int full) {
+  constexpr int NR = GEGLU ? 2 : 1;
+  const int lane = threadIdx.x & 63, n = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (n >= N) return;
+  float acc[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) acc[r] = 0.f;
+  const int K4 = K & ~3;
+  for (int k = lane * 4; k < K4; k += 256) {
+    float w[NR][4];
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[r][e] = load_f32(W, (size_t)(n + r * N) * K + k + e);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = load_f32(A, k + e);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) acc[r] = fmaf(w[r][e], x, acc[r]);
+    }
+  }
+  if (lane < K - K4) {                                        // up to three elements behind the last whole group of four
+    const int k = K4 + lane;
+    const float x = load_f32(A, k);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) acc[r] = fmaf(load_f32(W, (size_t)(n + r * N) * K + k), x, acc[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < NR; ++r) acc[r] = wave_sum(acc[r]);
+  if (lane) return;
+  float o = acc[0];
+  if (GEGLU) o = gated_act(acc[0], acc[NR - 1], param, full);
+  if (epi == ALICE_EPI_SOFTCAP) o = unary_act(o, param, full);
+  store_f32(Y, n, o);
+}
+
+template <typename TA, typename TW, typename TO>
+int launch_single(const void* x, const void* w, void* y, int N, int K, int epi, float epi_param, int full, hipStream_t stream) {
+  if (epi == ALICE_EPI_GEGLU)
+    linear_single_kernel<TA, TW, TO, true><<<ceil_div(N, 4), 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, N, K, epi, epi_param, full);
+  else
+    linear_single_kernel<TA, TW, TO, false><<<ceil_div(N, 4), 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, N, K, epi, epi_param, full);
+  ALICE_LAUNCH_CHECK();
+  return 0;
 }
 
 template <typename TA, typename TW, typename TO>
@@ -435,6 +486,7 @@ int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int
 
 // Into how many slices of the inner dimension a product without an epilogue is best cut.
 int alice_linear_split_hint_generic(int M, int N, int K) {
+  if (M == 1) return 1;
   return M <= 16 ? rows_split(N, K) : plan_mfma32(planned_tokens(M), N, K, false, MAX_SPLIT).split;
 }
 
@@ -451,8 +503,9 @@ int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype,
   if (M == 0) return 0;
   int rc = 0;
   DISPATCH_DTYPE(x_dtype, TA, DISPATCH_DTYPE(w_dtype, TW, DISPATCH_DTYPE(y_dtype, TO, {
-    rc = M <= 16 ? launch_rows<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream)
-              : launch_tiled<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
+    if (M == 1 && split_k == 1) rc = launch_single<TA, TW, TO>(x, w, y, N, K, epi, epi_param, full_precision, stream);
+    else rc = M <= 16 ? launch_rows<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream)
+                      : launch_tiled<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
   })));
   return rc;
 }

@@ -190,7 +190,8 @@ class _PromptGraph:
         self.width = -(-engine.max_positions // engine.cache.page_size)
         n_groups = len(engine.cache.groups)
         B, T = n_seqs + (1 if spare else 0), tokens
-        sizes = [T, T, T, B, B, B + 1, B] + [B * self.width] * n_groups
+        # (logits of the real sequences alone: as many rows as an eager step of the same prompts has)
+        sizes = [T, T, T, B, n_seqs, B + 1, B] + [B * self.width] * n_groups
         self.offs = [0]
         for n in sizes:
             self.offs.append(self.offs[-1] + n)
@@ -232,7 +233,6 @@ class _PromptGraph:
             sh[o[1] + used:o[2]] = np.arange(pad)
             sh[o[2] + used:o[3]] = B
             sh[o[3] + B] = engine.cache.spare_slot
-            sh[o[4] + B] = T - 1
             sh[o[5] + B + 1] = T
             sh[o[6] + B] = pad
         rows = B + (1 if self.spare else 0)
