@@ -381,31 +381,23 @@ __device__ __forceinline__ uint32_t whole_row_threshold(const float* __restrict_
   return thr;
 }
 
+// The thresholds by bisection over the row's list of the n elements within the chosen distance of the maximum m (cut < 0: there is
+// none); list, list_mass: CAP elements of shared memory; z_row: (top-p alone) the whole row's mass.  All threads of a block of ST call it.
 template <int VEC>
-__global__ __launch_bounds__(ST) void row_threshold_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t,
-                                                           int top_k, float top_p) {
-  __shared__ float red[17];
-  __shared__ int ired[ST / 64];
-  __shared__ uint32_t list[CAP];
-  __shared__ unsigned long long list_mass[CAP];
-  __shared__ int tot[NCUT];
-  __shared__ unsigned long long z_sh[1 + NMC];
+__device__ __forceinline__ uint32_t list_threshold(const float* __restrict__ row, const SampleWork& w, int b, int V, float inv_t, float m,
+                                                   int cut, int n, unsigned long long z_row, int top_k, float top_p, uint32_t* list,
+                                                   unsigned long long* list_mass, float* red, int* ired) {
   __shared__ uint32_t found[3];                           // threshold, top-k done, top-p done
-  const int b = blockIdx.x;
-  const float* row = logits + (size_t)b * V;
+  __shared__ unsigned long long wsum[ST / 64];
+  __shared__ uint32_t wmin[ST / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const float m = row_max(w, b);
   const uint32_t key_m = order_key(m);
   const bool need_k = top_k > 0 && top_k < V, need_p = top_p < 1.f;
   uint32_t thr = 0;
   bool k_done = !need_k, p_done = !need_p;
   if (tid == 0) { found[0] = 0; found[1] = 0; found[2] = 0; }
-  const int cut = choose_cut(w, b, need_k, top_k, top_p, tot, z_sh);
-  const int n = cut >= 0 ? min(tot[cut], w.capg) : 0;
   if (cut >= 0 && n > CAP) {
     // a long list: the same bisections by the whole block over the list in memory
-    __shared__ unsigned long long wsum[ST / 64];
-    __shared__ uint32_t wmin[ST / 64];
     const uint32_t* gl = w.cand + (size_t)b * w.capg;
     unsigned long long* gm = w.cmass + (size_t)b * w.capg;
     auto block_sum_u64 = [&](unsigned long long v) {
@@ -445,7 +437,7 @@ __global__ __launch_bounds__(ST) void row_threshold_kernel(const float* __restri
       unsigned long long kept = 0;
       for (int j = tid; j < n; j += ST) if (gl[j] >= t) kept += gm[j];
       kept = block_sum_u64(kept);
-      const unsigned long long z = need_k ? kept : z_sh[0];
+      const unsigned long long z = need_k ? kept : z_row;
       const unsigned long long target = (unsigned long long)((double)top_p * (double)z);
       if (kept > target) {
         uint32_t lo = t, hi = key_m;
@@ -463,7 +455,6 @@ __global__ __launch_bounds__(ST) void row_threshold_kernel(const float* __restri
     for (int j = tid; j < n; j += ST) list[j] = w.cand[(size_t)b * w.capg + j];
     __syncthreads();
     if (wave == 0) {
-      const unsigned long long z_row = z_sh[0];
       uint32_t kmin = 0xffffffffu;
       for (int j = lane; j < n; j += 64) kmin = min(kmin, list[j]);
 #pragma unroll
@@ -508,8 +499,70 @@ __global__ __launch_bounds__(ST) void row_threshold_kernel(const float* __restri
     __syncthreads();
     if (found[1]) { k_done = true; if (found[2]) { p_done = true; thr = found[0]; } else if (need_k) thr = found[0]; }
   }
-  thr = whole_row_threshold<VEC>(row, V, inv_t, m, key_m, thr, k_done, p_done, top_k, top_p, red, ired);
-  if (tid == 0) w.thr[b] = thr;
+  return whole_row_threshold<VEC>(row, V, inv_t, m, key_m, thr, k_done, p_done, top_k, top_p, red, ired);
+}
+
+template <int VEC>
+__global__ __launch_bounds__(ST) void row_threshold_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t,
+                                                           int top_k, float top_p) {
+  __shared__ float red[17];
+  __shared__ int ired[ST / 64];
+  __shared__ uint32_t list[CAP];
+  __shared__ unsigned long long list_mass[CAP];
+  __shared__ int tot[NCUT];
+  __shared__ unsigned long long z_sh[1 + NMC];
+  const int b = blockIdx.x;
+  const float m = row_max(w, b);
+  const int cut = choose_cut(w, b, top_k > 0 && top_k < V, top_k, top_p, tot, z_sh);
+  const uint32_t thr = list_threshold<VEC>(logits + (size_t)b * V, w, b, V, inv_t, m, cut, cut >= 0 ? min(tot[cut], w.capg) : 0, z_sh[0],
+                                           top_k, top_p, list, list_mass, red, ired);
+  if (threadIdx.x == 0) w.thr[b] = thr;
+}
+
+// The same for one row by one block, which counts and collects for itself: for the few rows with a small k whose lists
+// of the one pass settle nothing.  Two passes over the row more than bisecting a list, thirty to sixty less than bisecting the row.
+template <int VEC>
+__device__ __forceinline__ uint32_t row_threshold_alone(const float* __restrict__ row, const SampleWork& w, int b, int V, float inv_t, float m,
+                                                        int top_k, float top_p, uint32_t* list, unsigned long long* list_mass, float* red,
+                                                        int* ired) {
+  __shared__ int filled;
+  const int tid = threadIdx.x, lane = tid & 63;
+  int cnt[NCUT];
+#pragma unroll
+  for (int j = 0; j < NCUT; ++j) cnt[j] = 0;
+  for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) {
+    const float d = ok ? m - x : INFINITY;
+#pragma unroll
+    for (int j = 0; j < NCUT; ++j) cnt[j] += d <= kCut[j];
+  });
+  if (tid == 0) filled = 0;
+  int cut = -1, n = 0;
+  float dcut = 0.f;
+#pragma unroll
+  for (int j = 0; j < NCUT; ++j) {
+    const int c = block_count(cnt[j], ired);
+    if (cut == -1 && c >= top_k) {
+      cut = c <= w.capg ? j : -2;
+      n = c;
+      dcut = kCut[j];
+    }
+  }
+  if (cut >= 0) {
+    uint32_t* out = w.cand + (size_t)b * w.capg;
+    for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) {
+      const bool in = ok && (m - x <= dcut);
+      const unsigned long long mask = __ballot(in);
+      if (mask) {
+        const int leader = __ffsll((long long)mask) - 1;
+        int base = 0;
+        if (lane == leader) base = atomicAdd(&filled, __popcll(mask));
+        base = __shfl(base, leader, 64);
+        if (in) out[base + __popcll(mask & ((1ull << lane) - 1ull))] = order_key(x);
+      }
+    });
+    __syncthreads();
+  }
+  return list_threshold<VEC>(row, w, b, V, inv_t, m, cut, n, 0ull, top_k, top_p, list, list_mass, red, ired);
 }
 
 // The kept mass of the row's tiles t, t + step, ... below t_end (a wave), and the last index with a positive probability
@@ -664,8 +717,10 @@ __global__ __launch_bounds__(ST) void draw_kernel(const float* __restrict__ logi
 //
 //   chunk_topk   the chunk's elements in registers; every thread's largest goes to shared memory, and the k-th largest of
 //                these 256 is a bound that at least k of the chunk's elements reach: what reaches it (about -256 ln(1 - k/256)
-//                elements where the large ones are spread) goes to the chunk's list with its index.  Whatever the row's k
-//                largest are, ties among them included, they are in the lists.
+//                elements where the large ones are spread) goes to the chunk's list with its index.  A chunk in which more do
+//                (ties at the bound: masked elements, most often) lists what lies above it and names the key it left out.
+//                Whatever the row's k largest are, ties among them included, they are in the lists if the k-th of what is
+//                listed lies above every key that a chunk left out; and what was left out does not matter if its mass is zero.
 //   row_topk     a block a row: the same bound once more over the lists' elements, then every survivor counts the larger ones
 //                (the threshold of top-k) and adds up the mass at and above itself (top-p, the same fixed point); the sums of
 //                the tiles from the kept elements alone, each lane's share in index order as tile_sum adds them (what it adds
@@ -673,8 +728,9 @@ __global__ __launch_bounds__(ST) void draw_kernel(const float* __restrict__ logi
 //
 // So a row is read once, and the tile of the draw once more.  Against five passes (64 rows of 256,000, top-k 50, top-p 0.95):
 // 22 + 23 us, 103 before: the one pass takes twice its reads' time (registers allow three waves a SIMD), row_topk the latency
-// of its phases.  Rows that the lists do not settle (one that holds no number or no finite maximum, lists that
-// outgrow their room because of ties or an uneven spread) take the bisection over the whole row within row_topk.
+// of its phases.  Rows that the lists do not settle (one that holds no number or no finite maximum, too many ties at the
+// threshold itself) are counted and collected by their one block as the kernels for any k do it.  One row of 256,000 with 1,000 elements
+// that are not masked: 34 us; with 5,120 ties at the top 158 (46 and 41 by the five passes).
 constexpr int TOPK_MOST = 200;       // beyond, the bound of 256 maxima lets too much through
 constexpr int TOPK_LIST = 7168;      // elements of a row's lists in shared memory
 constexpr int TOPK_LEFT = 1024;      // survivors
@@ -690,7 +746,7 @@ __host__ inline TopkShape topk_shape(int B, int tiles, int top_k, int capg) {
   int per = 1;
   while (per < 4 && ((long)B * ceil_div(tiles, per) > 1024 || ceil_div(tiles, per) * expected > 0.9f * TOPK_LIST)) per *= 2;
   const int chunks = ceil_div(tiles, per);
-  if (chunks * expected > 0.9f * TOPK_LIST) return {0, 0, 0};
+  if (chunks * expected > 0.9f * TOPK_LIST || expected * 1.1f > capg / chunks) return {0, 0, 0};
   return {per, chunks, capg / chunks};
 }
 
@@ -766,7 +822,51 @@ __global__ __launch_bounds__(SB) void chunk_topk_kernel(const float* __restrict_
     }
   }
   __syncthreads();
-  if (tid == 0) w.tlast[(size_t)b * w.tiles + c] = (odd || fill > sh.room) ? -1 : fill;
+  // More than there is room for (ties, most often those of masked elements, or large elements in few threads' places): what
+  // lies above the bound alone, if that fits, else above the chunk's k-th largest; the ones tied with it are left out,
+  // and the row is settled if its threshold lies above them.
+  uint32_t tie = 0;
+  int n = fill;
+  if (n > sh.room) {
+    __syncthreads();
+    auto count = [&](uint32_t from) {                      // the chunk's elements at and above a key
+      int k = 0;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) k += key[e] >= from;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) k += __shfl_xor(k, o, 64);
+      if (lane == 0) wmin[tid >> 6] = (uint32_t)k;
+      __syncthreads();
+      k = 0;
+      for (int x = 0; x < SB / 64; ++x) k += (int)wmin[x];
+      __syncthreads();
+      return k;
+    };
+    tie = bound;
+    if (count(bound + 1) > sh.room) {
+      uint32_t from = bound, to = 0xfffffffeu;             // at least top_k at and above `from`, fewer above `to`
+      while (from < to) {
+        const uint32_t mid = from + ((to - from) >> 1) + 1;
+        if (count(mid) >= top_k) from = mid; else to = mid - 1;
+      }
+      tie = count(from) > sh.room ? from : from - 1;       // (all of them fit: nothing is left out but what is below)
+    }
+    if (tid == 0) fill = 0;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      if (key[e] > tie) {
+        const int pos = atomicAdd(&fill, 1);
+        if (pos < sh.room) list[pos] = ((unsigned long long)key[e] << 32) | (uint32_t)index(e);
+      }
+    }
+    __syncthreads();
+    n = fill;
+  }
+  if (tid == 0) {
+    w.tlast[(size_t)b * w.tiles + c] = (odd || n > sh.room) ? -1 : n;
+    w.tsum[(size_t)b * w.tiles + c] = __uint_as_float(tie);
+  }
 }
 
 template <int VEC>
@@ -783,13 +883,18 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
   __shared__ int first[TOPK_TILES + 1], n_left, last_kept, rounds, pick[2];
   __shared__ float red[17], wred[ST / 64], tsum[TOPK_TILES], prefix[TOPK_TILES], carry[2];
   __shared__ int ired[ST / 64];
-  __shared__ uint32_t best;
+  __shared__ uint32_t best, tie;
   const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float* row = logits + (size_t)b * V;
   const float u = uniform[b];
   const int* counts = w.tlast + (size_t)b * w.tiles;
-  if (tid < sh.chunks) first[tid + 1] = counts[tid];
-  if (tid == 0) { first[0] = 0; n_left = 0; last_kept = -1; rounds = 0; best = 0; }
+  if (tid == 0) { first[0] = 0; n_left = 0; last_kept = -1; rounds = 0; best = 0; tie = 0; }
+  __syncthreads();
+  if (tid < sh.chunks) {
+    first[tid + 1] = counts[tid];
+    const uint32_t left_out = __float_as_uint(w.tsum[(size_t)b * w.tiles + tid]);
+    if (left_out) atomicMax(&tie, left_out);
+  }
   __syncthreads();
   if (tid == 0) {
     int at = 0;
@@ -834,43 +939,53 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
     __syncthreads();
     settled = n_left <= TOPK_LEFT && fabsf(key_value(key_m)) < INFINITY;
   }
-  if (!settled) {                                          // the whole row, as the kernels for any k do it at worst
+  float m = 0.f;
+  int nl = 0, quads = 0, at = 0;
+  uint32_t key = 0, thr = 0xffffffffu;
+  unsigned long long z = 0;
+  bool kept_k = false;
+  if (settled) {
+    m = key_value(key_m);
+    nl = n_left;
+    quads = (nl + 3) >> 2;
+    key = tid < nl ? lkey[tid] : 0u;
+    at = tid < nl ? lat[tid] : 0;
+    if (tid >= nl && tid < quads * 4) { lkey[tid] = 0; lmass[tid] = 0; lslot[tid] = -1; }
+    __syncthreads();
+    int larger = 0;
+    if (tid < nl) {
+#pragma unroll 4
+      for (int j = 0; j < quads; ++j) {
+        const uint4 o = reinterpret_cast<const uint4*>(lkey)[j];
+        larger += (o.x > key) + (o.y > key) + (o.z > key) + (o.w > key);
+      }
+    }
+    kept_k = tid < nl && larger < top_k;
+    if (kept_k) thr = key;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) thr = min(thr, (uint32_t)__shfl_xor(thr, o, 64));
+    const unsigned long long mass = kept_k ? fixed_mass(key_value(key), m) : 0ull;
+    const unsigned long long z_wave = wave_sum_u64(mass);
+    if (tid < nl) lmass[tid] = mass;
+    __syncthreads();                                       // (the first bound's minima have been read)
+    if (lane == 0) { wmin[wave] = thr; wsum[wave] = z_wave; }
+    __syncthreads();
+    for (int x = 0; x < ST / 64; ++x) { thr = min(thr, wmin[x]); z += wsum[x]; }
+    // what was left out is not among the k largest, or its mass is zero
+    settled = tie == 0 || (nl >= top_k && thr > tie) || expf(key_value(tie) - m) == 0.f;
+  }
+  if (!settled) {
     float lmax = -INFINITY;
     for_range<VEC, ST>(row, 0, V, inv_t, [&](int, float x, bool ok) { lmax = fmaxf(lmax, ok ? x : -INFINITY); });
     const float m = block_max(lmax, red);
-    const uint32_t thr = whole_row_threshold<VEC>(row, V, inv_t, m, order_key(m), 0u, false, top_p >= 1.f, top_k, top_p, red, ired);
+    static_assert(TOPK_LIST >= CAP + CAP / 2, "the lists of the bisection take the place of the chunks' lists");
+    const uint32_t thr = row_threshold_alone<VEC>(row, w, b, V, inv_t, m, top_k, top_p, reinterpret_cast<uint32_t*>(list + CAP), list, red, ired);
     __syncthreads();
     tile_sums<VEC>(row, w, b, V, inv_t, m, thr, wave, w.tiles, ST / 64);
     __syncthreads();
     draw_from_tiles(row, out, u, w, b, V, inv_t, m, thr, wred);
     return;
   }
-  const float m = key_value(key_m);
-  const int nl = n_left, quads = (nl + 3) >> 2;
-  const uint32_t key = tid < nl ? lkey[tid] : 0u;
-  const int at = tid < nl ? lat[tid] : 0;
-  if (tid >= nl && tid < quads * 4) { lkey[tid] = 0; lmass[tid] = 0; lslot[tid] = -1; }
-  __syncthreads();
-  int larger = 0;
-  if (tid < nl) {
-#pragma unroll 4
-    for (int j = 0; j < quads; ++j) {
-      const uint4 o = reinterpret_cast<const uint4*>(lkey)[j];
-      larger += (o.x > key) + (o.y > key) + (o.z > key) + (o.w > key);
-    }
-  }
-  const bool kept_k = tid < nl && larger < top_k;
-  uint32_t thr = kept_k ? key : 0xffffffffu;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) thr = min(thr, (uint32_t)__shfl_xor(thr, o, 64));
-  const unsigned long long mass = kept_k ? fixed_mass(key_value(key), m) : 0ull;
-  const unsigned long long z_wave = wave_sum_u64(mass);
-  if (tid < nl) lmass[tid] = mass;
-  __syncthreads();                                         // (the first bound's minima have been read)
-  if (lane == 0) { wmin[wave] = thr; wsum[wave] = z_wave; }
-  __syncthreads();
-  unsigned long long z = 0;
-  for (int x = 0; x < ST / 64; ++x) { thr = min(thr, wmin[x]); z += wsum[x]; }
   if (top_p < 1.f) {
     // the largest key at and above which lies more than the target
     const unsigned long long target = (unsigned long long)((double)top_p * (double)z);

@@ -20,8 +20,8 @@ def test_small_k_at_the_edges(B, V, top_k, top_p):
 
 
 def test_lists_that_outgrow_their_room_and_rows_without_a_finite_maximum():
-    """All large values in one thread's places, thousands of ties, masked rows and rows with an infinite logit beside an
-    ordinary row: each row gets what it gets alone."""
+    """All large values in one thread's places, thousands of ties, a masked row, one with a huge logit, with an infinite one and with
+    one that is no number, beside an ordinary row: each row gets what it gets alone."""
     V, g = 70000, torch.Generator().manual_seed(5)
     ordinary = rnd(1, V, seed=31, scale=2.0)
     uneven = rnd(1, V, seed=32, scale=0.1)
@@ -32,9 +32,47 @@ def test_lists_that_outgrow_their_room_and_rows_without_a_finite_maximum():
     masked[0, [5, 69999]] = torch.tensor([1.0, 0.5], device=DEV)
     top = rnd(1, V, seed=34)
     top[0, 777] = 1e30
+    odd = rnd(2, V, seed=35)
+    odd[0, 30000], odd[1, 40000] = math.inf, math.nan
     rows = torch.cat([ordinary, uneven, ties, masked, top])
     for top_k, top_p in ((20, 0.9), (3, 1.0), (150, 0.5)):
-        u = torch.rand(5, generator=g)
-        got = check_samples(rows, u, 1.0, top_k, top_p)
-        assert got == [ops.sample(rows[i:i + 1], u[i:i + 1].to(DEV), 1.0, top_k, top_p).item() for i in range(5)]
+        u = torch.rand(7, generator=g)
+        got = check_samples(rows, u[:5], 1.0, top_k, top_p)
+        both = torch.cat([odd[:1], rows, odd[1:]])
+        order = [5, 0, 1, 2, 3, 4, 6]
+        many = ops.sample(both, u[order].to(DEV), 1.0, top_k, top_p).tolist()
+        assert many[1:6] == got and all(0 <= t < V for t in many)
+        assert many == [ops.sample(both[i:i + 1], u[order[i]:order[i] + 1].to(DEV), 1.0, top_k, top_p).item() for i in range(7)]
         assert got[3] in (5, 69999) and got[4] == 777
+
+
+@pytest.mark.parametrize("mask", [-math.inf, -1e9, torch.finfo(torch.float32).min])
+@pytest.mark.parametrize("B,V", [(2, 70000), (1, 256000), (70, 66001)])
+def test_masked_rows_are_settled_without_their_masked_elements(mask, B, V):
+    """Chunks that hold nothing but masked elements, or few others: spread, side by side, in one thread's places, fewer than k of
+    them, in the last chunk alone, and as many as fill a list.  The draw is the plain one, and takes no longer than a row without a
+    mask does by more than the second look at the chunks (a row bisected whole takes fifty times as long)."""
+    g = torch.Generator().manual_seed(V)
+    spread = torch.randperm(V, generator=g)
+    base = rnd(B, V, seed=3, scale=3.0)
+    sets = [spread[:1000], torch.arange(5000, 6000), torch.arange(0, V, 1024), spread[:4], torch.arange(V - 90, V), torch.arange(V // 2),
+            spread[:V // 3], torch.arange(4)]
+
+    def time(rows, u, k):
+        ops.sample(rows, u, 0.8, k, 0.95)
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(5):
+            ops.sample(rows, u, 0.8, k, 0.95)
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b)
+
+    for keep in sets:
+        rows = torch.full_like(base, mask)
+        rows[:, keep.to(DEV)] = base[:, keep.to(DEV)]
+        for top_k in (5, 50, 150):
+            u = torch.rand(B, generator=g)
+            got = ops.sample(rows, u.to(DEV), 0.8, top_k, 0.95).tolist()
+            assert set(got) <= set(keep.tolist()) and got[:4] == check_samples(rows[:4], u[:4], 0.8, top_k, 0.95)
+            assert min(time(rows, u.to(DEV), top_k) for _ in range(3)) < 8 * time(base, u.to(DEV), top_k), (len(keep), top_k)
