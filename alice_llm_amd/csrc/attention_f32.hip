@@ -149,7 +149,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(F32Args a) {
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[i] = any ? expf(p[i] - m_new) : 0.f;
+      p[i] = any ? expf(p[i] - m_new) : (p[i] != p[i] ? p[i] : 0.f);      // (a maximum passes over what is no number: that stays)
       sum += p[i];
     }
     m_run = m_new;

@@ -135,6 +135,25 @@ def test_attention_keeps_values_that_are_no_numbers_to_the_queries_that_see_them
         assert (got - ref)[fine].abs().max() < 1e-5
 
 
+@pytest.mark.parametrize("at", [0, 15, 16, 40, 64])
+def test_attention_keeps_a_score_that_is_no_number(at):
+    """A key that is not a number: every query that sees it gets none, also where it is the one key of its tile that the query sees;
+    the queries before it and those behind the window see nothing of it.  As prompts, and the last positions as single tokens."""
+    nH, nKV, d, L, window = 4, 2, 64, 80, 30
+    q, kp, vp, bt, pos, seq, _, scale = attention_case("float32", nH, nKV, d, (L,), (L,), None, window, seed=8)
+    kp[int(bt[0, at // 64]), :, at % 64, 5] = math.nan
+    sees = torch.tensor([at <= i < at + window for i in range(L)])
+    for splits in (1, 2, 3):
+        out = torch.empty_like(q)
+        ops.attention_f32(q, kp, vp, out, ctx_of((L,), (L,), pos, seq), bt, num_heads=nH, scale=scale, softcap=None, window=window, splits=splits)
+        assert torch.equal(torch.isnan(out).all(1).cpu(), sees) and torch.equal(torch.isnan(out).any(1).cpu(), sees)
+        for i in (at, at + 1, min(L, at + window) - 1):
+            one = torch.empty_like(q[:1])
+            ops.attention_f32(q[i:i + 1].contiguous(), kp, vp, one, ctx_of((i + 1,), (1,), pos[i:i + 1].contiguous(), seq[:1]), bt, num_heads=nH,
+                              scale=scale, softcap=None, window=window, splits=splits)
+            assert torch.isnan(one).all(), i
+
+
 def test_attention_refuses_what_is_outside_its_range():
     q, kp, vp, bt, pos, seq, _, scale = attention_case("float32", 4, 2, 32, (20,), (20,), None, None, seed=8)
     with pytest.raises(ops.HipLibraryError, match="outside"):
