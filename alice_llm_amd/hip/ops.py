@@ -1648,8 +1648,10 @@ def attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, out: 
         return
     if out_layout != LAYOUT_ROW or sink is not None:
         raise HipLibraryError("only the matrix-core attention kernels write fragment order, and here only they take a sink")
-    # the 32-bit path at the matrix-core head sizes, without the terms that the generic kernel alone has
+    # the 32-bit path at the matrix-core head sizes, without the terms that the generic kernel alone has, on memory that can
+    # be read 16 bytes at a time
     if (q.dtype == torch.float32 and full_precision and bias_slopes is None and gate is None and k_pool.shape[3] == v_pool.shape[3]
+            and all(t.data_ptr() % 16 == 0 for t in (q, k_pool, v_pool, out))
             and library().alice_attention_f32_supported(num_heads, k_pool.shape[1], k_pool.shape[3], k_pool.shape[2])):
         attention_f32(q, k_pool, v_pool, out, ctx, block_table, num_heads=num_heads, scale=scale, softcap=softcap, window=window)
         return

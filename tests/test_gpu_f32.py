@@ -154,6 +154,17 @@ def test_attention_keeps_a_score_that_is_no_number(at):
             assert torch.isnan(one).all(), i
 
 
+def test_attention_takes_rows_that_are_not_aligned():
+    """The step's attention, as mixers call it, on queries and outputs at any address."""
+    for lens, new in (((70, 33), (70, 33)), ((70, 33), (1, 1))):
+        q, kp, vp, bt, pos, seq, ref, scale = attention_case("float32", 4, 2, 64, lens, new, 5.0, 20, seed=9)
+        shifted = [torch.empty(q.numel() + 1, device=DEV)[1:].view_as(q) for _ in range(2)]
+        shifted[0].copy_(q)
+        for q_, out in ((q, shifted[1]), (shifted[0], torch.empty_like(q))):
+            ops.attention(q_, kp, vp, out, ctx_of(lens, new, pos, seq), bt, num_heads=4, scale=scale, softcap=5.0, window=20, full_precision=True)
+            close(out, ref, 1e-5)
+
+
 def test_attention_refuses_what_is_outside_its_range():
     q, kp, vp, bt, pos, seq, _, scale = attention_case("float32", 4, 2, 32, (20,), (20,), None, None, seed=8)
     with pytest.raises(ops.HipLibraryError, match="outside"):
