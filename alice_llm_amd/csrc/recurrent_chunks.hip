@@ -75,6 +75,15 @@ __device__ __forceinline__ bool find_chunk(const ChunkArgs& a, int at, int& t0, 
   return false;
 }
 
+template <int N>
+__device__ __forceinline__ float tree_sum(float (&x)[N]) {
+#pragma unroll
+  for (int n = N / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; ++i) x[i] += x[i + n];
+  return x[0];
+}
+
 // ------------------------------------------------------------------------------------------ what does not depend on the state
 
 // State space: a block a (chunk, group of heads with one q and k, 16 of its heads).
@@ -104,8 +113,13 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(ChunkArgs a) {
   }
   const int t = tid / C, r = tid % C;
   float qk = 0.f;
-  if (r <= t)
-    for (int c = 0; c < d; ++c) qk = fmaf(qs[t][c], ks[r][c], qk);
+  if (r <= t) {                                               // sixteen sums: the error of one grows with the key size (zeros behind d)
+    float part[16] = {};
+    for (int c = 0; c < d; c += 16)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) part[e] = fmaf(qs[t][c + e], ks[r][c + e], part[e]);
+    qk = tree_sum(part);
+  }
   const int h0 = blockIdx.z * HB, nh = min(HB, per - h0);      // of the group's heads
   float* heads = a.work + (size_t)a.max_chunks * a.G * DP * C + ((size_t)blockIdx.x * a.H + grp * per + h0) * SS_HEAD;
   if (tid < nh) {
@@ -174,15 +188,20 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(ChunkArgs a) {
   for (int c = tid; c < DP; c += 256) o[3 * C * DP + c] = power(ls[C - 1][c]);
   // the pairs (t, r <= t): those off the diagonal by two threads, (t, r) for the lower half of the channels and its mirror image for
   // the upper half
-  const int t = tid / C, r = tid % C, ht = max(t, r), hr = min(t, r), mid = (d + 1) / 2;
-  float m = 0.f, p = 0.f;
+  const int t = tid / C, r = tid % C, ht = max(t, r), hr = min(t, r), mid = (d / 2 + 7) & ~7;
+  float m, p;
   {
+    float mp[8] = {}, pp[8] = {};                             // eight sums each: the error of one grows with the key size (zeros behind d)
     const int c1 = r < t ? mid : d;
-    for (int c = r > t ? mid : 0; c < c1; ++c) {
-      const float kk = ks[hr][c] * power(ls[ht][c] - ls[hr][c]);
-      m = fmaf(ks[ht][c], kk, m);
-      p = fmaf(qs[ht][c], kk, p);
-    }
+    for (int c = r > t ? mid : 0; c < c1; c += 8)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float kk = ks[hr][c + e] * power(ls[ht][c + e] - ls[hr][c + e]);
+        mp[e] = fmaf(ks[ht][c + e], kk, mp[e]);
+        pp[e] = fmaf(qs[ht][c + e], kk, pp[e]);
+      }
+    m = tree_sum(mp);
+    p = tree_sum(pp);
   }
   ms[t][r] = m;
   ps[t][r] = p;

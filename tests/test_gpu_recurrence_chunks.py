@@ -83,3 +83,49 @@ def test_both_block_sizes_give_the_same(delta):
         outs.append((out.view(copies, n, H * dv), S))
     (a, sa), (c, sc) = outs
     assert (c - a).abs().max() < 1e-5 * a.abs().max() and (sc - sa).abs().max() < 1e-5 * sa.abs().max()
+
+
+def scan64(q, k, v, decay, b, H, delta):
+    """Token by token in 64 bits: q, k [T, H, d], v [T, H, dv], decay [T, H, d or 1], b [T, H] -> [T, H dv], the state."""
+    q, k, v, decay, b = (x.double() for x in (q, k, v, decay, b))
+    S, out = q.new_zeros(H, q.shape[2], v.shape[2]), []
+    for t in range(len(q)):
+        S = decay[t][:, :, None] * S
+        u = v[t] - (torch.matmul(k[t][:, None], S)[:, 0] if delta else 0.0)
+        S = S + k[t][:, :, None] * (b[t][:, None] * u)[:, None]
+        out.append(torch.matmul(q[t][:, None], S).reshape(-1))
+    return torch.stack(out), S
+
+
+def case(T, H, d, dv, delta, strength, seed=0):
+    q, k, v = (rnd(T, H * w, seed=seed + i).to(DEV) for i, w in ((1, d), (2, d), (3, dv)))
+    if delta:
+        q, k = ((x.view(T, H, d) / x.view(T, H, d).norm(dim=-1, keepdim=True)).reshape(T, -1) for x in (q, k))
+    log, b = -strength * rnd(T, H * d if delta else H, seed=seed + 4).abs().to(DEV), torch.sigmoid(rnd(T, H, seed=seed + 5)).to(DEV)
+    return q, k, v, log, b
+
+
+def both_ways(T, H, d, dv, delta, q, k, v, log, b):
+    """(by chunks, token by token): out and state of each."""
+    kw, res = dict(heads=H, qk_heads=H, head_dim=d, value_head_dim=dv, delta=delta), []
+    for chunks in (True, False):
+        S, out = torch.zeros(1, H, d, dv, device=DEV), torch.empty(T, H * dv, device=DEV)
+        if chunks:
+            ops.recurrence_chunks(q, 0, k, 0, v, 0, log, b, None, out, _Ctx([T], [0]), S, **kw)
+        else:
+            ops.matrix_recurrence(q, 0, k, 0, v, 0, torch.exp(log), b, None, out, _Ctx([T], [0]), S, decay_per_channel=delta, **kw)
+        res.append((out, S[0]))
+    return res
+
+
+@pytest.mark.parametrize("delta,H,d,dv", [(False, 64, 128, 64), (True, 16, 128, 128), (True, 8, 64, 64), (False, 8, 256, 64)])
+@pytest.mark.parametrize("strength", [0.01, 0.1, 1.0, 5.0])
+def test_chunks_are_as_near_to_64_bits_as_token_by_token(delta, H, d, dv, strength):
+    """The 2-norms of the errors over 300 tokens: 0.6 to 1.25 of the token-by-token kernel's, which adds up a product with a key in as
+    many sums as it has lanes (1.7 to 3.2 with one sum over a key)."""
+    T = 300
+    args = case(T, H, d, dv, delta, strength)
+    q, k, v, log, b = args
+    ref, S = scan64(q.view(T, H, d), k.view(T, H, d), v.view(T, H, dv), torch.exp(log.double()).view(T, H, -1), b, H, delta)
+    (a, sa), (c, sc) = both_ways(T, H, d, dv, delta, *args)
+    assert (a - ref).norm() < 1.4 * (c - ref).norm() and (sa - S).norm() < 1.4 * (sc - S).norm()
