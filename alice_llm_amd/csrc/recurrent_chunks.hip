@@ -41,6 +41,10 @@ constexpr double LOG2E = 1.4426950408889634;
 // 2^x for a difference x <= 0 of two sums: the hardware's instruction (1 ulp), on an argument that was scaled in 64-bit
 __device__ __forceinline__ float power(double x) { return __builtin_amdgcn_exp2f((float)x); }
 
+// A decay's logarithm to base 2.  One so low that the decay is zero in 32 bits (minus infinity among them) counts as -10,000, so that
+// differences of sums with it stay finite; what is no number stays so.
+__device__ __forceinline__ double log2_decay(float l) { return (double)(l < -1e4f ? -1e4f : l) * LOG2E; }
+
 struct ChunkArgs {
   const float* q; int q_w, q_col;          // as in recurrent.hip
   const float* k; int k_w, k_col;
@@ -129,7 +133,7 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(ChunkArgs a) {
     for (int i = 0; i < C; ++i) {
       const size_t at = (size_t)(t0 + min(i, len - 1)) * a.H + h;
       const float x = a.log_decay[at], w = a.b[at];
-      l += i < len ? (double)x * LOG2E : 0.0;
+      l += i < len ? log2_decay(x) : 0.0;
       ls[tid][i] = l;
       bs[tid][i] = i < len ? w : 0.f;
     }
@@ -166,7 +170,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(ChunkArgs a) {
     const float lv = a.log_decay[(row * H + h) * d + min(c, d - 1)];
     qs[t][c] = in ? qv : 0.f;
     ks[t][c] = in ? kv : 0.f;
-    ls[t][c] = in ? (double)lv * LOG2E : 0.0;
+    ls[t][c] = in ? log2_decay(lv) : 0.0;
   }
   if (tid < C) bs[tid] = tid < len ? a.b[(size_t)(t0 + tid) * H + h] : 0.f;
   __syncthreads();

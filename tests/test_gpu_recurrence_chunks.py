@@ -129,3 +129,16 @@ def test_chunks_are_as_near_to_64_bits_as_token_by_token(delta, H, d, dv, streng
     ref, S = scan64(q.view(T, H, d), k.view(T, H, d), v.view(T, H, dv), torch.exp(log.double()).view(T, H, -1), b, H, delta)
     (a, sa), (c, sc) = both_ways(T, H, d, dv, delta, *args)
     assert (a - ref).norm() < 1.4 * (c - ref).norm() and (sa - S).norm() < 1.4 * (sc - S).norm()
+
+
+@pytest.mark.parametrize("delta", [False, True])
+def test_a_decay_of_zero_forgets(delta):
+    """Logarithms of minus infinity, and ones far below what 32 bits hold: the state before is gone, nothing else."""
+    T, H, d, dv = 70, 2, 12, 20
+    q, k, v, log, b = case(T, H, d, dv, delta, 0.3)
+    log[21], log[40], log[41] = -float("inf"), -3e38, -2e5
+    if delta:
+        log[52, 5] = -float("inf")
+    ref, S = scan64(q.view(T, H, d), k.view(T, H, d), v.view(T, H, dv), torch.exp(log.double()).view(T, H, -1), b, H, delta)
+    for out, state in both_ways(T, H, d, dv, delta, q, k, v, log, b):
+        assert (out - ref).abs().max() < 2e-5 and (state - S).abs().max() < 2e-5
