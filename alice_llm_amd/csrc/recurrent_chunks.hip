@@ -91,7 +91,7 @@ __device__ __forceinline__ float tree_sum(float (&x)[N]) {
 // ------------------------------------------------------------------------------------------ what does not depend on the state
 
 // State space: a block a (chunk, group of heads with one q and k, 16 of its heads).
-constexpr int HB = 16;
+constexpr int HB = 16;                     // (times C tokens: a block's threads)
 template <int DP>
 __global__ __launch_bounds__(256) void ssm_chunk_kernel(ChunkArgs a) {
   __shared__ float qs[C][DP + 1], ks[C][DP + 1];
@@ -126,16 +126,20 @@ __global__ __launch_bounds__(256) void ssm_chunk_kernel(ChunkArgs a) {
   }
   const int h0 = blockIdx.z * HB, nh = min(HB, per - h0);      // of the group's heads
   float* heads = a.work + (size_t)a.max_chunks * a.G * DP * C + ((size_t)blockIdx.x * a.H + grp * per + h0) * SS_HEAD;
+  {
+    const int hh = tid % HB, i = tid / HB;
+    const size_t at = (size_t)(t0 + min(i, len - 1)) * a.H + grp * per + h0 + min(hh, nh - 1);
+    const float x = a.log_decay[at], w = a.b[at];
+    ls[hh][i] = i < len ? log2_decay(x) : 0.0;
+    bs[hh][i] = i < len ? w : 0.f;
+  }
+  __syncthreads();
   if (tid < nh) {
-    const int h = grp * per + h0 + tid;
     double l = 0.0;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-      const size_t at = (size_t)(t0 + min(i, len - 1)) * a.H + h;
-      const float x = a.log_decay[at], w = a.b[at];
-      l += i < len ? log2_decay(x) : 0.0;
+      l += ls[tid][i];
       ls[tid][i] = l;
-      bs[tid][i] = i < len ? w : 0.f;
     }
   }
   __syncthreads();
