@@ -15,7 +15,8 @@
 // one product with the state between two states, and the read-outs off that chain.
 // Decays arrive as logarithms; their sums over a chunk are kept in 64-bit (base 2) and only differences of two of them (never
 // above zero) are exponentiated, so that no quotient of small products is ever formed.  32-bit everywhere else, as in the
-// token-by-token kernel.  (A value that is no finite number reaches every read-out of its chunk, also those of earlier tokens.)
+// token-by-token kernel.  What is no finite number reaches the tokens from its own on and no earlier one of its chunk: where
+// there is any, the products with a triangle of zeros are made token by token (lower_product).
 //
 // The walk: a wave holds TW tiles of 16 channels.  A tile of the state as it stands in the accumulators (lane group g: rows 4 g ..
 // 4 g + 3) is the second operand of the products with it, if product e takes channel 4 g + e of the group on both sides,
@@ -86,6 +87,29 @@ __device__ __forceinline__ float tree_sum(float (&x)[N]) {
 #pragma unroll
     for (int i = 0; i < n; ++i) x[i] += x[i + n];
   return x[0];
+}
+
+// o + L x for a chunk's lower triangle L (lane: row c, columns 4 g .. 4 g + 3) and rows x (lane: column c, rows 4 g .. 4 g + 3).  A zero of
+// the triangle would not keep an infinity out of an earlier row: if x holds one, or NaN, a token at a time, and the rows before it
+// get back what they had.
+__device__ __forceinline__ f32x4 lower_product(const float* L, const float* x, f32x4 o, int g) {
+  bool odd = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) odd = odd || !(fabsf(x[e]) < INFINITY);
+  if (__ballot(odd) == 0ull) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o = mfma(L[e], x[e], o);
+  } else {
+#pragma unroll 1
+    for (int t4 = 0; t4 < 4; ++t4)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {                           // token 4 t4 + e
+        const f32x4 after = mfma(g == t4 ? L[e] : 0.f, g == t4 ? x[e] : 0.f, o);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = g * 4 + i >= t4 * 4 + e ? after[i] : o[i];
+      }
+  }
+  return o;
 }
 
 // ------------------------------------------------------------------------------------------ what does not depend on the state
@@ -250,14 +274,18 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(ChunkArgs a) {
     P4[e] = ps[c][g * 4 + e];
   }
   for (int tile = wave; tile < DP / 16; tile += 4) {
-    f32x4 w = {0.f, 0.f, 0.f, 0.f}, q;
+    f32x4 q;
+    float k[4], w[4], minus[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      w = mfma(T4[e], ks[g * 4 + e][tile * 16 + c], w);
+      k[e] = ks[g * 4 + e][tile * 16 + c];
       q[e] = qs[g * 4 + e][tile * 16 + c];
+      minus[e] = -P4[e];
     }
+    const f32x4 w4 = lower_product(T4, k, f32x4{0.f, 0.f, 0.f, 0.f}, g);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) q = mfma(-P4[e], w[e], q);
+    for (int e = 0; e < 4; ++e) w[e] = w4[e];
+    q = lower_product(minus, w, q, g);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       o[(g * 4 + e) * DP + tile * 16 + c] = w[e];
@@ -266,17 +294,17 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(ChunkArgs a) {
   }
   float* tv = o + 3 * C * DP + DP;
   for (int tile = wave; tile < dvp / 16; tile += 4) {
-    f32x4 u = {0.f, 0.f, 0.f, 0.f}, y = u;
-    float v[4];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    float v[4], u[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float x = a.v[(size_t)(t0 + min(g * 4 + e, len - 1)) * a.v_w + a.v_col + h * a.dv + min(tile * 16 + c, a.dv - 1)];
       v[e] = g * 4 + e < len ? x : 0.f;
     }
+    const f32x4 u4 = lower_product(T4, v, zero, g);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) u = mfma(T4[e], v[e], u);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) y = mfma(P4[e], u[e], y);
+    for (int e = 0; e < 4; ++e) u[e] = u4[e];
+    const f32x4 y = lower_product(P4, u, zero, g);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       tv[(g * 4 + e) * dvp + tile * 16 + c] = u[e];
@@ -454,9 +482,8 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void recurrence_chunks_kernel(Chun
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] += fin.x[e];
     } else {
-      o *= fin.A;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o = mfma(fin.P[e], fin.x[e], o);
+      const float P[4] = {fin.P[0], fin.P[1], fin.P[2], fin.P[3]};
+      o = lower_product(P, fin.x, o * fin.A, g);
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = fmaf(skip, fin.x[e], o[e]);
     }

@@ -142,3 +142,26 @@ def test_a_decay_of_zero_forgets(delta):
     ref, S = scan64(q.view(T, H, d), k.view(T, H, d), v.view(T, H, dv), torch.exp(log.double()).view(T, H, -1), b, H, delta)
     for out, state in both_ways(T, H, d, dv, delta, q, k, v, log, b):
         assert (out - ref).abs().max() < 2e-5 and (state - S).abs().max() < 2e-5
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("what", ["q", "k", "v", "log", "b"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("d,dv", [(12, 20), (128, 64), (256, 16)])
+def test_what_is_no_finite_number_reaches_no_earlier_token(delta, what, value, d, dv):
+    """One such number in the first head at a chunk's first, middle and last token and at the last one of all: the outputs that it
+    reaches are those of the scan in 64 bits, and the others are what they are without it."""
+    if what == "log" and value == float("inf"):
+        value = -value                                                  # (no decay is above one; this one is zero: nothing is lost)
+    T, H = 70, 2
+    for at in (16, 21, 31, 69):
+        args = dict(zip(("q", "k", "v", "log", "b"), case(T, H, d, dv, delta, 0.3, seed=at)))
+        args[what][at, 0 if what == "b" or what == "log" and not delta else 3] = value
+        q, k, v, log, b = args.values()
+        ref, S = scan64(q.view(T, H, d), k.view(T, H, d), v.view(T, H, dv), torch.exp(log.double()).view(T, H, -1), b, H, delta)
+        fine, there = torch.isfinite(ref), torch.isfinite(S)
+        assert fine[:at].all() and fine[:, dv:].all()
+        out, state = both_ways(T, H, d, dv, delta, q, k, v, log, b)[0]
+        assert torch.equal(torch.isfinite(out), fine) and torch.equal(torch.isfinite(state), there), at
+        assert (out - ref)[fine].abs().max() < 2e-5 * max(1.0, float(ref[fine].abs().max()))
+        assert (state - S)[there].abs().max() < 2e-5 * max(1.0, float(S[there].abs().max()))
