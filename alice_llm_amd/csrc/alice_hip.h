@@ -4,7 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define ALICE_ABI_VERSION 15
+#define ALICE_ABI_VERSION 16
 
 #define ALICE_EPI_NONE 0
 #define ALICE_EPI_GEGLU 1     // W = [gate; up] stacked; epi_param 0: y = gelu_tanh(gate x) * (up x); epi_param = limit > 0:
@@ -215,12 +215,12 @@ int alice_matrix_recurrence(const float* q, int q_w, int q_col, const float* k, 
                             int d, int dv, int delta, int columns, hipStream_t stream);
 // The same over pieces of many tokens, 16 at a time on the 32-bit matrix instruction (recurrent_chunks.hip); log_decay: the
 // decays' logarithms, [T, H d] with delta, else [T, H]; work: alice_recurrence_chunks_workspace floats (0: sizes outside
-// its range).
+// its range; never more than 256 MB and a chunk of every sequence: a longer step goes in runs); longest: tokens of the longest sequence.
 long alice_recurrence_chunks_workspace(int T, int n_seqs, int H, int qk_heads, int d, int dv, int delta);
 int alice_recurrence_chunks(const float* q, int q_w, int q_col, const float* k, int k_w, int k_col, const float* v, int v_w,
                             int v_col, const float* log_decay, const float* b, const float* skip, float* out, float* work,
-                            const int* cu_seqlens, const int* slots, float* S, int T, int n_seqs, int H, int qk_heads, int d,
-                            int dv, int delta, hipStream_t stream);
+                            const int* cu_seqlens, const int* slots, float* S, int T, int n_seqs, int longest, int H, int qk_heads,
+                            int d, int dv, int delta, hipStream_t stream);
 // (columns: value columns a wave, 4, 8 or 16; 0: by the step's size, the rule of alice_matrix_recurrence_columns)
 int alice_matrix_recurrence_columns(int n_seqs, int H, int d, int dv);
 // Rows of `width` in `parts` equal parts, each RMS-normed and multiplied by a weight (w_shared: of a part's length);

@@ -58,7 +58,8 @@ struct ChunkArgs {
   const int* cu_seqlens; const int* slots;
   float* S;                                // [slots, H, d, dv]
   int n_seqs, H, G, d, dv;
-  long max_chunks;
+  int first, run;                          // of every sequence the chunks first .. first + run - 1
+  long max_chunks;                         // of all sequences
 };
 
 // Floats of the workspace.  State space: a chunk and group K^T [DP][16]; a chunk and head A [16], (A_n / A_r) b [16], P [16][16].
@@ -66,13 +67,15 @@ struct ChunkArgs {
 constexpr int SS_HEAD = 2 * C + C * C;
 __host__ __device__ __forceinline__ int delta_head(int DP, int dv) { return 3 * C * DP + DP + 2 * C * ((dv + 15) & ~15); }
 
-// Which 16 tokens chunk `at` is: the chunks are dealt to the sequences in order.
+// How many chunks of a run are a sequence's of n tokens.
+__device__ __forceinline__ int run_chunks(const ChunkArgs& a, int n) { return min(max((n + C - 1) / C - a.first, 0), a.run); }
+// Which 16 tokens chunk `at` of the run is: the chunks are dealt to the sequences in order.
 __device__ __forceinline__ bool find_chunk(const ChunkArgs& a, int at, int& t0, int& len) {
   for (int s = 0; s < a.n_seqs; ++s) {
-    const int b = a.cu_seqlens[s], n = a.cu_seqlens[s + 1] - b, nc = (n + C - 1) / C;
+    const int b = a.cu_seqlens[s], n = a.cu_seqlens[s + 1] - b, nc = run_chunks(a, n);
     if (at < nc) {
-      t0 = b + at * C;
-      len = min(C, n - at * C);
+      t0 = b + (a.first + at) * C;
+      len = min(C, n - (a.first + at) * C);
       return true;
     }
     at -= nc;
@@ -331,11 +334,12 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void recurrence_chunks_kernel(Chun
   __shared__ __align__(16) f32x4 part[2][NW][64];             // (delta) of a chunk's W S, twice
   const int h = blockIdx.x, s = blockIdx.y, v0 = blockIdx.z * 16, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, g = lane >> 4;
-  const int t0 = a.cu_seqlens[s], t1 = a.cu_seqlens[s + 1];
-  if (t1 <= t0) return;
+  const int n = run_chunks(a, a.cu_seqlens[s + 1] - a.cu_seqlens[s]);
+  if (n <= 0) return;
+  const int t0 = a.cu_seqlens[s] + a.first * C, t1 = min(a.cu_seqlens[s + 1], t0 + n * C);
   size_t chunk0 = 0;                                          // this sequence's first chunk in the workspace
-  for (int i = 0; i < s; ++i) chunk0 += (a.cu_seqlens[i + 1] - a.cu_seqlens[i] + C - 1) / C;
-  const int H = a.H, d = a.d, dv = a.dv, n = (t1 - t0 + C - 1) / C, last = t1 - 1, grp = h / (H / a.G), dvp = (dv + 15) & ~15;
+  for (int i = 0; i < s; ++i) chunk0 += run_chunks(a, a.cu_seqlens[i + 1] - a.cu_seqlens[i]);
+  const int H = a.H, d = a.d, dv = a.dv, last = t1 - 1, grp = h / (H / a.G), dvp = (dv + 15) & ~15;
   const int col = min(v0 + c, dv - 1);
   const bool col_ok = v0 + c < dv;
   float* Sh = a.S + ((size_t)a.slots[s] * H + h) * d * dv;
@@ -564,35 +568,57 @@ int launch(const ChunkArgs& a, int delta, hipStream_t stream) {
   return 0;
 }
 
+// The workspace holds a step's chunks at once up to WORK_MOST floats (256 MB: 6,400 tokens with 16 heads of 128 x 128 under the delta rule,
+// 41 KB a token; the state space takes 5 KB a token with 64 heads).  A longer step goes in runs of that many chunks, each with the
+// state that the one before left: the same numbers, and a microsecond or two a run.
+constexpr long WORK_MOST = 1l << 26;
+struct Runs {
+  int run;                                 // chunks of every sequence a run
+  long chunks;                             // chunks of all sequences a run, at most
+};
+long chunk_floats(int H, int G, int d, int dv, int delta) {
+  return delta ? (long)H * delta_head(padded(d), dv) : G * (long)padded(d) * C + H * (long)SS_HEAD;
+}
+Runs runs_of(int T, int n_seqs, int H, int G, int d, int dv, int delta) {
+  const long all = (long)T / C + n_seqs, fit = WORK_MOST / chunk_floats(H, G, d, dv, delta);
+  if (all <= fit) return {T / C + 1, all};
+  const long run = fit / n_seqs > 1 ? fit / n_seqs : 1;
+  return {(int)run, run * n_seqs < all ? run * n_seqs : all};
+}
+
 }  // namespace
 
 // Float32 workspace of alice_recurrence_chunks for a step of T tokens in n_seqs sequences; 0 where the sizes are outside
 // its range (key sizes that are no multiples of four: the queries are read 16 bytes at a time).
 extern "C" long alice_recurrence_chunks_workspace(int T, int n_seqs, int H, int qk_heads, int d, int dv, int delta) {
   if (T < 0 || dv < 1 || n_seqs < 1 || H < 1 || qk_heads < 1 || H % qk_heads || d < 4 || d > 256 || d % 4 || H > 65535 || n_seqs > 65535) return 0;
-  const long chunks = (long)T / C + n_seqs;
-  const int DP = padded(d);
-  if (delta) return chunks * H * delta_head(DP, dv);
-  return chunks * (qk_heads * (long)DP * C + H * (long)SS_HEAD);
+  return runs_of(T, n_seqs, H, qk_heads, d, dv, delta).chunks * chunk_floats(H, qk_heads, d, dv, delta);
 }
 
+// longest: tokens of the longest sequence.
 extern "C" int alice_recurrence_chunks(const float* q, int q_w, int q_col, const float* k, int k_w, int k_col, const float* v, int v_w,
                                        int v_col, const float* log_decay, const float* b, const float* skip, float* out, float* work,
-                                       const int* cu_seqlens, const int* slots, float* S, int T, int n_seqs, int H, int qk_heads, int d,
-                                       int dv, int delta, hipStream_t stream) {
+                                       const int* cu_seqlens, const int* slots, float* S, int T, int n_seqs, int longest, int H,
+                                       int qk_heads, int d, int dv, int delta, hipStream_t stream) {
   ALICE_CHECK(q && k && v && log_decay && b && out && work && cu_seqlens && slots && S, "recurrence_chunks: a pointer is missing");
-  ALICE_CHECK(T >= 0 && n_seqs >= 0 && dv >= 1 && ceil_div(dv, 16) <= 65535, "recurrence_chunks: bad sizes");
+  ALICE_CHECK(T >= 0 && n_seqs >= 0 && longest >= 0 && longest <= T && dv >= 1 && ceil_div(dv, 16) <= 65535, "recurrence_chunks: bad sizes");
   if (n_seqs == 0 || T == 0) return 0;
   ALICE_CHECK(alice_recurrence_chunks_workspace(T, n_seqs, H, qk_heads, d, dv, delta) > 0, "recurrence_chunks: heads %d / %d of size %d are outside this kernel's range", H, qk_heads, d);
   ALICE_CHECK(q_col >= 0 && k_col >= 0 && v_col >= 0 && q_col + qk_heads * d <= q_w && k_col + qk_heads * d <= k_w && v_col + H * dv <= v_w,
               "recurrence_chunks: the rows are too short for the heads");
   ALICE_CHECK(((uintptr_t)q & 15) == 0 && q_w % 4 == 0 && q_col % 4 == 0 && ((uintptr_t)work & 15) == 0, "recurrence_chunks: operands are not aligned");
-  ChunkArgs a{q, q_w, q_col, k, k_w, k_col, v, v_w, v_col, log_decay, b, skip, out, work, cu_seqlens, slots, S, n_seqs, H, qk_heads, d, dv,
-              (long)T / C + n_seqs};
-  ALICE_CHECK(a.max_chunks < (1l << 31), "recurrence_chunks: too many chunks for one launch");
-  if (d <= 64) return launch<4, 1>(a, delta, stream);
-  // Eight waves a block while the blocks are few (2,048 tokens: 131 against 138 us, state space 81 against 91), four where several
-  // blocks share a CU (8 sequences of 1,000: 503 against 534 us with the preparation, 295 against 344).
-  if (d <= 128) return (long)H * n_seqs * ceil_div(dv, 16) < 512 ? launch<8, 1>(a, delta, stream) : launch<4, 2>(a, delta, stream);
-  return launch<8, 2>(a, delta, stream);
+  const Runs r = runs_of(T, n_seqs, H, qk_heads, d, dv, delta);
+  ALICE_CHECK(r.chunks < (1l << 31), "recurrence_chunks: too many chunks for one launch");
+  for (int first = 0; first * C < longest; first += r.run) {
+    const ChunkArgs a{q, q_w, q_col, k, k_w, k_col, v, v_w, v_col, log_decay, b, skip, out, work, cu_seqlens, slots, S, n_seqs, H, qk_heads, d,
+                      dv, first, r.run, r.chunks};
+    int rc;
+    // Eight waves a block while the blocks are few (2,048 tokens: 131 against 138 us, state space 81 against 91), four where several
+    // blocks share a CU (8 sequences of 1,000: 503 against 534 us with the preparation, 295 against 344).
+    if (d <= 64) rc = launch<4, 1>(a, delta, stream);
+    else if (d <= 128) rc = (long)H * n_seqs * ceil_div(dv, 16) < 512 ? launch<8, 1>(a, delta, stream) : launch<4, 2>(a, delta, stream);
+    else rc = launch<8, 2>(a, delta, stream);
+    if (rc) return rc;
+  }
+  return 0;
 }

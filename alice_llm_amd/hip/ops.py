@@ -19,7 +19,7 @@ EPI_NONE, EPI_GEGLU, EPI_SOFTCAP = 0, 1, 2
 LAYOUT_ROW, LAYOUT_FRAG16 = 0, 1
 KV_ROW, KV_FRAGMENT = 0, 1
 LINEAR_AUTO, LINEAR_GENERIC, LINEAR_SKINNY, LINEAR_MFMA, LINEAR_TILED_W16, LINEAR_TILED_W32 = 0, 1, 2, 3, 4, 5
-ABI_VERSION = 15
+ABI_VERSION = 16
 GATED_SILU = -1.0        # epi_param of EPI_GEGLU that picks silu(gate) * up
 UNARY_RELU2 = -1.0       # epi_param of EPI_SOFTCAP that picks the square of max(y, 0) instead of the capped form
 UNARY_SILU = -2.0        # likewise y * sigmoid(y)
@@ -76,7 +76,7 @@ def _declare(lib) -> None:
         "alice_ssm_enter": [P, I, I, I, I, P, P, P, P, I, P, P, P, P, I, I, P, P, P, I, I, I, P],
         "alice_delta_enter": [P, I, I, I, P, P, P, I, I, F, F, I, I, P, I, I, I, P, P, I, P, P, P, I, I, I, P],
         "alice_delta_decay": [P, P, P, I, I, I, I, P],
-        "alice_recurrence_chunks": [P, I, I, P, I, I, P, I, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P],
+        "alice_recurrence_chunks": [P, I, I, P, I, I, P, I, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
         "alice_matrix_recurrence": [P, I, I, P, I, I, P, I, I, P, I, P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
         "alice_matrix_recurrence_columns": [I, I, I, I],
         "alice_norm_gate": [P, I, I, P, I, I, I, I, P, I, F, P, I, I, P],
@@ -1304,8 +1304,8 @@ def recurrence_chunks(q, q_col: int, k, k_col: int, v, v_col: int, log_decay: to
     work = torch.empty((max(1, need),), dtype=torch.float32, device=out.device)
     _call("alice_recurrence_chunks", q.data_ptr(), q.shape[1], int(q_col), k.data_ptr(), k.shape[1], int(k_col), v.data_ptr(),
           v.shape[1], int(v_col), log_decay.data_ptr(), b.data_ptr(), _opt(skip, "skip"), out.data_ptr(), work.data_ptr(),
-          ctx.cu_seqlens.data_ptr(), ctx.slots.data_ptr(), S.data_ptr(), T, int(ctx.n_seqs), H, int(qk_heads), d, dv, int(bool(delta)),
-          _stream())
+          ctx.cu_seqlens.data_ptr(), ctx.slots.data_ptr(), S.data_ptr(), T, int(ctx.n_seqs), min(T, int(getattr(ctx, "max_new", T))), H,
+          int(qk_heads), d, dv, int(bool(delta)), _stream())
 
 
 def norm_gate(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, *, parts: int, eps: float, weight_shared: bool,

@@ -165,3 +165,27 @@ def test_what_is_no_finite_number_reaches_no_earlier_token(delta, what, value, d
         assert torch.equal(torch.isfinite(out), fine) and torch.equal(torch.isfinite(state), there), at
         assert (out - ref)[fine].abs().max() < 2e-5 * max(1.0, float(ref[fine].abs().max()))
         assert (state - S)[there].abs().max() < 2e-5 * max(1.0, float(S[there].abs().max()))
+
+
+@pytest.mark.parametrize("delta,H,d,dv,lens", [(True, 512, 256, 16, [300]), (True, 300, 256, 20, [40, 230, 7, 129]), (False, 4096, 64, 4, [1500]),
+                                              (False, 3000, 64, 4, [900, 33, 600])])
+def test_a_step_beyond_the_workspace_goes_in_runs(delta, H, d, dv, lens):
+    """More chunks than 256 MB hold: in runs, with the token-by-token kernel's result, and from no more memory."""
+    T, G = sum(lens), 1
+    per = ops.library().alice_recurrence_chunks_workspace(16, 1, H, G, d, dv, int(delta)) // 2
+    need = ops.library().alice_recurrence_chunks_workspace(T, len(lens), H, G, d, dv, int(delta))
+    assert need <= 1 << 26 and need < per * sum(-(-n // 16) for n in lens)
+    q, k, v = (rnd(T, w, seed=i).to(DEV) for i, w in ((1, G * d), (2, G * d), (3, H * dv)))
+    q, k = (x / x.norm(dim=1, keepdim=True) for x in (q, k))
+    log, b = -0.3 * rnd(T, H * d if delta else H, seed=4).abs().to(DEV), torch.sigmoid(rnd(T, H, seed=5)).to(DEV)
+    ctx, kw, res = _Ctx(lens, list(range(len(lens)))), dict(heads=H, qk_heads=G, head_dim=d, value_head_dim=dv, delta=delta), []
+    for chunks in (True, False):
+        S, out = torch.zeros(len(lens), H, d, dv, device=DEV), torch.full((T, H * dv), float("nan"), device=DEV)
+        if chunks:
+            ctx.max_new = max(lens)
+            ops.recurrence_chunks(q, 0, k, 0, v, 0, log, b, None, out, ctx, S, **kw)
+        else:
+            ops.matrix_recurrence(q, 0, k, 0, v, 0, torch.exp(log), b, None, out, ctx, S, decay_per_channel=delta, **kw)
+        res.append((out, S))
+    for x, y in zip(*res):
+        assert (x - y).abs().max() < 2e-5 * max(1.0, float(y.abs().max()))
