@@ -525,6 +525,45 @@ def test_long_decoding_from_the_first_token(name, dtype):
     assert_close(got, ref, dtype)
 
 
+@pytest.mark.parametrize("name,dtype", CASES)
+def test_pieces_by_chunks_then_single_tokens(name, dtype, monkeypatch):
+    """Pieces of 257 and more tokens, by chunks where a layer's sizes allow it: a whole prompt, one on top of a short piece and in a batch
+    with shorter ones, each followed by single tokens on the state that the chunks left."""
+    model, plain = pair(name, dtype)
+    calls, old = [], ops.recurrence_chunks
+    monkeypatch.setattr(ops, "recurrence_chunks", lambda *a, **k: (calls.append(k["delta"]), old(*a, **k)))
+    V = plain.config["vocab"]
+    toks = [random_tokens(V, n, 70 + n) for n in (320, 60, 300)]
+    refs = [plain.forward(t) for t in toks]
+    eng = model.engine(max_tokens=64 * 16, max_seqs=3)
+    for cuts in ([300], [5, 258], [257, 40]):
+        s = eng.open(1)
+        got, at = [], 0
+        for c in cuts + [1] * 6:
+            got.append(eng.step(s, [toks[0][at:at + c]], "all"))
+            at += c
+        eng.close(s)
+        assert_close(torch.cat(got), refs[0][:at], dtype, cuts)
+    slots = eng.open(3)
+    got = [eng.step(slots, [t[:-4] for t in toks], "last")] + [eng.step(slots, [[t[j]] for t in toks], "last") for j in range(-4, 0)]
+    eng.close(slots)
+    for i, ref in enumerate(refs):
+        assert_close(torch.stack([g[i] for g in got]), ref[-5:], dtype, i)
+    kinds = {"mamba2": False, "channel_delta": True}
+    sized = [kinds[l["type"]] for l in plain.config["layers"] if l["type"] in kinds and _by_chunks(l)]
+    assert calls == sized * 4
+    if name in ("vx-a", "vx-b"):
+        assert set(calls) == {False, True}
+
+
+def _by_chunks(layer):
+    m = layer["mixer"]
+    if layer["type"] == "mamba2":
+        inner, keys = m["heads"] * m["vdim"], m["groups"] * m["state"]
+        return m["state"] % 4 == 0 and (inner + 2 * keys) % 4 == 0 and (inner + keys) % 4 == 0
+    return m["dim"] % 4 == 0 and (2 * m["kv_heads"] * m["dim"] + m["heads"] * m["vdim"]) % 4 == 0
+
+
 @pytest.mark.parametrize("name", list(VIFIRAX))
 def test_captured_steps_equal_eager_ones(name):
     model, plain = pair(name, "bfloat16")
