@@ -18,9 +18,11 @@
 //
 // What bounds it: the vector instructions of the softmax and of the moves through LDS, some 300 for every 32 MFMA of a step, and
 // few waves (a prompt of 2,048 tokens and 16 heads is two blocks a CU).  So blocks wholly inside every query's range skip the
-// masks, the exponents are powers of two, and the output is rescaled only when a maximum has outgrown the base by 2^8:
-// 2,048 tokens, 16 heads of 128 on 4 kv heads 129 -> 116 us, 8 prompts of 1,000 164 -> 150, 16 heads of 64 87 -> 76.  Loads two
-// steps ahead gave nothing (132).
+// masks, the exponents are powers of two, and the output is rescaled only in blocks where a column's maximum grows:
+// 2,048 tokens, 16 heads of 128 on 4 kv heads 128 -> 117 us, 8 prompts of 1,000 164 -> 153, 16 heads of 64 87 -> 77.  Keys of 256 leave a
+// SIMD one wave, and a branch there costs more than what it skips: 8 heads of 256 186 -> 154 us without the two, 177 with the
+// masks' one, 183 with both.  Loads two steps ahead gave nothing.  A base that lags behind the maximum by up to 2^8 (115 us) rounds the
+// largest weight too, which as the maximum's own is 1: the error against 64 bits rose by 4 to 20 % (peaked scores).
 #include "common.h"
 #include "alice_hip.h"
 
@@ -59,7 +61,6 @@ struct TiledArgs {
 
 constexpr int KT = 32;        // keys a step
 constexpr float LOG2E = 1.44269504088896341f;
-constexpr float RAISE = 8.f;  // by how much (base 2) the maximum must outgrow the exponents' base before that follows
 constexpr int VPAD = 40;      // row length of the transposed values in LDS (32 keys and a pad against bank conflicts)
 
 template <int DP, int DVP, int HPW>
@@ -68,6 +69,7 @@ __global__ __launch_bounds__(256) void attn_tiled_kernel(TiledArgs a) {
   constexpr int KROW = DP + 8;
   constexpr int NKC = DP / 64, NVC = DVP / 64;          // 16-byte pieces of keys / values a thread moves a step
   constexpr int NBUF = (DP + DVP <= 384) ? 2 : 1;        // two buffers where they fit the static LDS limit
+  constexpr bool BRANCHES = DP < 256;                    // around what a block of keys does not need (see above)
   __shared__ __align__(16) bf16_t Ks[NBUF][KT][KROW];
   __shared__ __align__(16) bf16_t Vt[NBUF][DVP][VPAD];
 
@@ -213,7 +215,7 @@ __global__ __launch_bounds__(256) void attn_tiled_kernel(TiledArgs a) {
       }
       // Which of the lane's eight keys its query sees (the same for every head); most blocks lie wholly inside every
       // query's range (a column without a query takes what comes, nothing of it is stored).
-      const bool all_seen = __all(!valid || (key0 >= lo_q && key0 + KT - 1 <= qpos)) != 0;
+      const bool all_seen = BRANCHES && __all(!valid || (key0 >= lo_q && key0 + KT - 1 <= qpos)) != 0;
       bool vis[8];
       bool any = all_seen;
       if (!all_seen) {
@@ -243,10 +245,10 @@ __global__ __launch_bounds__(256) void attn_tiled_kernel(TiledArgs a) {
           for (int j = 0; j < 8; ++j) m_t = fmaxf(m_t, sc[j]);
           m_t = fmaxf(m_t, __shfl_xor(m_t, 16, 64));
           m_t = fmaxf(m_t, __shfl_xor(m_t, 32, 64));
-          // The base follows the maximum only when that has outgrown it by RAISE: weights reach 2^RAISE at most, which 32-bit
-          // sums and bfloat16 operands hold as well as weights up to 1, and the output is rescaled in a few blocks only.
-          const bool raise = m_t > m_run[hh] + RAISE;
-          if (__any(raise)) {
+          // The base is the running maximum, so that the largest weight is 1 and not rounded; the output is rescaled in the blocks
+          // only where some column's maximum grows.
+          const bool raise = m_t > m_run[hh];
+          if (!BRANCHES || __any(raise)) {
             const float corr = raise ? exp2f_fast(m_run[hh] - m_t) : 1.f;       // m_run = -inf gives 0
             if (raise) m_run[hh] = m_t;
             l_run[hh] *= corr;
