@@ -96,6 +96,41 @@ def test_sliced_products_add_in_one_order_in_captured_and_eager_steps():
         assert torch.equal(*logits)
 
 
+@pytest.mark.parametrize("family", ["novotar", "vazilorn"])
+def test_sliced_products_through_the_residual_adds(family, monkeypatch):
+    """Down projections in slices ahead of an add of several branches (from 256 rows on) and of one with a norm element by element:
+    prompts and single tokens of a batch, against the plain model."""
+    import helpers
+    from test_gpu_novotar import assert_close
+    from plain import novotar_plain, vazilorn_plain
+    raw = {"novotar": helpers._nv_c, "vazilorn": helpers._vz_a}[family]()
+    for layer in raw["layers"]:
+        if layer["mlp"] is not None and layer["mlp"]["kind"] == "dense":
+            layer["mlp"] = dict(layer["mlp"], ff=2048)
+    cfg, t = {"novotar": helpers.novotar_tensors, "vazilorn": helpers.vazilorn_tensors}[family](raw, 5)
+    plain = {"novotar": novotar_plain.PlainNovotar, "vazilorn": vazilorn_plain.PlainVazilorn}[family](raw, {k: v.double() for k, v in t.items()})
+    model = helpers.model_from_tensors(cfg, {k: v.to(DEV) for k, v in t.items()}, "float32")
+    added, old = set(), {}
+    for name in ("add_branches", "add_dyntanh"):
+        old[name] = getattr(ops, name)
+    monkeypatch.setattr(ops, "add_branches", lambda x, many, *a, **k: (added.update(("many", b[0].shape[0]) for b in many if b[0].dim() == 3),
+                                                                       old["add_branches"](x, many, *a, **k)))
+    monkeypatch.setattr(ops, "add_dyntanh", lambda *a, **k: (added.add(("pointwise", k.get("n_partials", 1))), old["add_dyntanh"](*a, **k)))
+    toks = [random_tokens(raw["vocab"], n, n) for n in (70, 300, 9)]
+    refs = [plain.forward(x) for x in toks]
+    eng = model.engine(max_tokens=64 * 16, max_seqs=3)
+    for x, ref in zip(toks, refs):
+        s = eng.open(1)
+        assert_close(eng.step(s, [x], "all"), ref, "float32", len(x))
+        eng.close(s)
+    slots = eng.open(3)
+    got = [eng.step(slots, [x[:-2] for x in toks], "last")] + [eng.step(slots, [[x[j]] for x in toks], "last") for j in (-2, -1)]
+    for i, ref in enumerate(refs):
+        assert_close(torch.stack([g[i] for g in got]), ref[-3:], "float32", i)
+    kind = {"novotar": "many", "vazilorn": "pointwise"}[family]
+    assert any(k == kind and n > 1 for k, n in added)
+
+
 # ------------------------------------------------------------------ attention
 def ctx_of(lens, new, pos, seq):
     cu = [0]
