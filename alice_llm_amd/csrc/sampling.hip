@@ -61,8 +61,7 @@ __global__ __launch_bounds__(ST) void argmax_kernel(const float* __restrict__ va
 
 __device__ __forceinline__ int block_count(int v, int* ired) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_reduce(v, [](int a, int b) { return a + b; });
   __syncthreads();
   if (lane == 0) ired[wid] = v;
   __syncthreads();
@@ -127,15 +126,7 @@ __device__ __forceinline__ unsigned long long fixed_mass(float x, float m) {
 }
 
 __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v) {
-  uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    unsigned long long other = ((unsigned long long)__shfl_xor(hi, o, 64) << 32) | __shfl_xor(lo, o, 64);
-    v += other;
-    lo = (uint32_t)v;
-    hi = (uint32_t)(v >> 32);
-  }
-  return v;
+  return wave_reduce(v, [](unsigned long long a, unsigned long long b) { return a + b; });
 }
 
 // Where a row's intermediate results live (all arrays are per row; `chunks` and `tiles` per row).
@@ -240,10 +231,7 @@ __global__ __launch_bounds__(SB) void chunk_count_kernel(const float* __restrict
     for (int i = 0; i <= NMC; ++i) mass[i] = wave_sum_u64(mass[i]);
   }
 #pragma unroll
-  for (int j = 0; j < NCUT; ++j) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) cnt[j] += __shfl_xor(cnt[j], o, 64);
-  }
+  for (int j = 0; j < NCUT; ++j) cnt[j] = wave_reduce(cnt[j], [](int a, int b) { return a + b; });
   if (lane == 0) {
 #pragma unroll
     for (int j = 0; j < NCUT; ++j) wave_cnt[wave][j] = cnt[j];
@@ -329,8 +317,7 @@ __global__ __launch_bounds__(SB) void chunk_collect_kernel(const float* __restri
   {
     int mine = 0;
     for (int cc = threadIdx.x; cc < c; cc += SB) mine += w.pcnt[((size_t)b * w.chunks + cc) * NCUT + cut];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, 64);
+    mine = wave_reduce(mine, [](int a, int b) { return a + b; });
     if (lane == 0 && mine) atomicAdd(&before, mine);
   }
   __syncthreads();
@@ -415,8 +402,7 @@ __device__ __forceinline__ uint32_t list_threshold(const float* __restrict__ row
       kmin = min(kmin, key);
       if (need_p) gm[j] = fixed_mass(key_value(key), m);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) kmin = min(kmin, (uint32_t)__shfl_xor(kmin, o, 64));
+    kmin = wave_reduce(kmin, [](uint32_t a, uint32_t b) { return min(a, b); });
     if (lane == 0) wmin[wave] = kmin;
     __syncthreads();                                      // also: the masses are written
     for (int x = 0; x < ST / 64; ++x) kmin = min(kmin, wmin[x]);
@@ -457,8 +443,7 @@ __device__ __forceinline__ uint32_t list_threshold(const float* __restrict__ row
     if (wave == 0) {
       uint32_t kmin = 0xffffffffu;
       for (int j = lane; j < n; j += 64) kmin = min(kmin, list[j]);
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) kmin = min(kmin, (uint32_t)__shfl_xor(kmin, o, 64));
+      kmin = wave_reduce(kmin, [](uint32_t a, uint32_t b) { return min(a, b); });
       uint32_t t = kmin;
       if (need_k) {
         uint32_t lo = kmin, hi = key_m;                   // count(list >= lo) = n >= k
@@ -595,8 +580,7 @@ __device__ __forceinline__ void tile_sums(const float* __restrict__ row, const S
       for (int i = base + lane; i < min(V, base + TILE); i += 64) take(i, row[i] * inv_t);
     }
     s = wave_sum(s);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) last_kept = max(last_kept, __shfl_xor(last_kept, o, 64));
+    last_kept = wave_reduce(last_kept, [](int a, int b) { return max(a, b); });
     if (lane == 0) {
       w.tsum[(size_t)b * w.tiles + t] = s;
       w.tlast[(size_t)b * w.tiles + t] = last_kept;
@@ -764,8 +748,7 @@ __device__ __forceinline__ uint32_t kth_of_256(const uint32_t* keys, uint32_t mi
     }
     if (larger < k) v = mine;
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = min(v, (uint32_t)__shfl_xor(v, o, 64));
+  v = wave_reduce(v, [](uint32_t a, uint32_t b) { return min(a, b); });
   if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = v;
   __syncthreads();
   for (int x = 0; x < n_waves; ++x) v = min(v, wmin[x]);
@@ -833,8 +816,7 @@ __global__ __launch_bounds__(SB) void chunk_topk_kernel(const float* __restrict_
       int k = 0;
 #pragma unroll
       for (int e = 0; e < NE; ++e) k += key[e] >= from;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) k += __shfl_xor(k, o, 64);
+      k = wave_reduce(k, [](int a, int b) { return a + b; });
       if (lane == 0) wmin[tid >> 6] = (uint32_t)k;
       __syncthreads();
       k = 0;
@@ -926,8 +908,7 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
     __syncthreads();
     const uint32_t bound = kth_of_256(keys, tid < 256 ? keys[tid] : 0u, top_k, wmin, ST / 64);
     for (int x = 0; x < 256; x += 64) key_m = max(key_m, keys[x + lane]);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) key_m = max(key_m, (uint32_t)__shfl_xor(key_m, o, 64));
+    key_m = wave_reduce(key_m, [](uint32_t a, uint32_t b) { return max(a, b); });
     for (int i = tid; i < n; i += ST)
       if ((uint32_t)(list[i] >> 32) >= bound) {
         const int pos = atomicAdd(&n_left, 1);
@@ -962,8 +943,7 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
     }
     kept_k = tid < nl && larger < top_k;
     if (kept_k) thr = key;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) thr = min(thr, (uint32_t)__shfl_xor(thr, o, 64));
+    thr = wave_reduce(thr, [](uint32_t a, uint32_t b) { return min(a, b); });
     const unsigned long long mass = kept_k ? fixed_mass(key_value(key), m) : 0ull;
     const unsigned long long z_wave = wave_sum_u64(mass);
     if (tid < nl) lmass[tid] = mass;
