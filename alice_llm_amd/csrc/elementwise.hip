@@ -251,6 +251,153 @@ __global__ void add_norm_regs_kernel(float* __restrict__ resid, const float* __r
   }
 }
 
+// The same with four consecutive elements a thread at a time (E4 such groups, H a multiple of 4, operands on 16 bytes):
+// a block a row, for the widths and addresses that models have.  What a step of single tokens waits for here is a chain of
+// latencies, not bytes: the kernel's start, one round trip to memory for everything (a few vector loads a thread, all
+// issued before the first use: 9 instead of 36 for a row of 2,304 in six partial sums), and two sums over the row.  A sum
+// is a butterfly in registers, one value a wave through LDS and one barrier that waits for LDS alone: the store of the
+// new residual row is still on its way when the second sum is taken.  (Per launch in a captured 2B decode step 5.8 us with one
+// element at a time, 3.9 this way: the step of eight sequences 1,952 -> 1,865 us, of one 1,810 -> 1,744.)
+__device__ __forceinline__ float row_sum_lds(float v, float* red) {        // `red`: 16 floats of its own for every call
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  v = wave_sum(v);
+  if (lane == 0) red[wid] = v;
+  lds_barrier();
+  return wave_sum(lane < nw ? red[lane] : 0.f);
+}
+__device__ __forceinline__ float4 operator+(const float4& a, const float4& b) { return float4{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w}; }
+__device__ __forceinline__ float square_sum(const float4& a) { return (a.x * a.x + a.y * a.y) + (a.z * a.z + a.w * a.w); }
+template <typename TW> struct raw4_of;
+template <> struct raw4_of<float> { typedef float4 type; };
+template <> struct raw4_of<bf16_t> { typedef uint2 type; };
+__device__ __forceinline__ float4 raw4_to_f32(const float4& v) { return v; }
+__device__ __forceinline__ float4 raw4_to_f32(const uint2& v) {
+  return float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)};
+}
+
+template <typename TW, typename TO, bool FULL, bool LN, int E4>
+__global__ __launch_bounds__(1024) void add_norm_row_kernel(float* __restrict__ resid, const float* __restrict__ branch, int n_partials,
+                                                            size_t partial_stride, const TW* __restrict__ w_post,
+                                                            const TW* __restrict__ w_pre, const TW* __restrict__ b_pre,
+                                                            TO* __restrict__ out, const int* __restrict__ rows, int H, float eps_post,
+                                                            float eps_pre, float off_post, float off_pre, int out_layout) {
+  typedef typename raw4_of<TW>::type RW;
+  constexpr int CMAX = E4 == 1 ? 8 : 4;                      // partial sums in flight per element (registers)
+  __shared__ float red[3][16];
+  const int r = blockIdx.x;
+  const size_t src = (size_t)(rows ? rows[r] : r) * H;
+  int e[E4];
+  bool ok[E4];
+#pragma unroll
+  for (int j = 0; j < E4; ++j) {
+    const int i = (threadIdx.x + j * blockDim.x) * 4;
+    ok[j] = i < H;
+    e[j] = min(i, H - 4);                                    // clamped: loads are unconditional
+  }
+  // ---- loads
+  const float4 zero4 = {0.f, 0.f, 0.f, 0.f};
+  float4 xv[E4], bv[E4], t[CMAX][E4];
+  RW wq[E4], wp[E4], bq[E4];
+#pragma unroll
+  for (int j = 0; j < E4; ++j) xv[j] = *reinterpret_cast<const float4*>(resid + src + e[j]);
+  if (branch) {
+#pragma unroll
+    for (int p = 0; p < CMAX; ++p) {
+      if (p < n_partials) {
+#pragma unroll
+        for (int j = 0; j < E4; ++j) t[p][j] = *reinterpret_cast<const float4*>(branch + (size_t)p * partial_stride + src + e[j]);
+      }
+    }
+    if (w_post) {
+#pragma unroll
+      for (int j = 0; j < E4; ++j) wp[j] = *reinterpret_cast<const RW*>(w_post + e[j]);
+    }
+  }
+  if (w_pre) {
+#pragma unroll
+    for (int j = 0; j < E4; ++j) wq[j] = *reinterpret_cast<const RW*>(w_pre + e[j]);
+    if (LN) {
+#pragma unroll
+      for (int j = 0; j < E4; ++j) bq[j] = *reinterpret_cast<const RW*>(b_pre + e[j]);
+    }
+  }
+  // ---- arithmetic
+  if (branch) {
+#pragma unroll
+    for (int j = 0; j < E4; ++j) bv[j] = zero4;
+    // partial sums are added in their order, CMAX at a time
+    for (int p0 = 0; p0 < n_partials; p0 += CMAX) {
+      if (p0 > 0) {
+#pragma unroll
+        for (int p = 0; p < CMAX; ++p) {
+          if (p0 + p < n_partials) {
+#pragma unroll
+            for (int j = 0; j < E4; ++j) t[p][j] = *reinterpret_cast<const float4*>(branch + (size_t)(p0 + p) * partial_stride + src + e[j]);
+          }
+        }
+      }
+#pragma unroll
+      for (int p = 0; p < CMAX; ++p) {
+        if (p0 + p < n_partials) {
+#pragma unroll
+          for (int j = 0; j < E4; ++j) bv[j] = bv[j] + t[p][j];
+        }
+      }
+    }
+    if (w_post) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < E4; ++j) ss += ok[j] ? square_sum(bv[j]) : 0.f;
+      const float mean = row_sum_lds(ss, red[0]) / (float)H;
+      const float inv_b = FULL ? 1.f / sqrtf(mean + eps_post) : rsqrtf(mean + eps_post);
+#pragma unroll
+      for (int j = 0; j < E4; ++j) {
+        const float4 w = raw4_to_f32(wp[j]);
+        bv[j] = float4{bv[j].x * inv_b * (off_post + w.x), bv[j].y * inv_b * (off_post + w.y), bv[j].z * inv_b * (off_post + w.z),
+                       bv[j].w * inv_b * (off_post + w.w)};
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < E4; ++j) {
+      xv[j] = xv[j] + bv[j];
+      if (ok[j]) *reinterpret_cast<float4*>(resid + src + e[j]) = xv[j];
+    }
+  }
+  if (!out) return;
+  float inv = 1.f;
+  if (w_pre) {
+    if (LN) {
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < E4; ++j) sum += ok[j] ? (xv[j].x + xv[j].y) + (xv[j].z + xv[j].w) : 0.f;
+      const float mu = row_sum_lds(sum, red[2]) / (float)H;
+#pragma unroll
+      for (int j = 0; j < E4; ++j) xv[j] = float4{xv[j].x - mu, xv[j].y - mu, xv[j].z - mu, xv[j].w - mu};
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < E4; ++j) ss += ok[j] ? square_sum(xv[j]) : 0.f;
+    const float mean = row_sum_lds(ss, red[1]) / (float)H;
+    inv = FULL ? 1.f / sqrtf(mean + eps_pre) : rsqrtf(mean + eps_pre);
+  }
+#pragma unroll
+  for (int j = 0; j < E4; ++j) {
+    if (!ok[j]) continue;
+    float4 o = xv[j];
+    if (w_pre) {
+      const float4 w = raw4_to_f32(wq[j]);
+      o = float4{o.x * inv * (off_pre + w.x), o.y * inv * (off_pre + w.y), o.z * inv * (off_pre + w.z), o.w * inv * (off_pre + w.w)};
+      if (LN) o = o + raw4_to_f32(bq[j]);
+    }
+    const size_t at = out_index(out_layout, r, e[j], H);     // four consecutive elements are neighbours in both layouts
+    if constexpr (sizeof(TO) == 4) {
+      *reinterpret_cast<float4*>((float*)out + at) = o;
+    } else {
+      *reinterpret_cast<uint2*>((bf16_t*)out + at) = uint2{pack_bf16x2(o.x, o.y), pack_bf16x2(o.z, o.w)};
+    }
+  }
+}
+
 // The same operation for many rows (prompts): one wave per row, four rows a block, four consecutive
 // elements a lane at a time (H a multiple of 4, at most 256 * K4); or, for rows too wide for one wave's
 // registers, two waves per row (WPR = 2, at most 512 * K4 elements: the first wave takes the first 256 * K4),
@@ -408,6 +555,9 @@ extern "C" int alice_add_norm(float* resid, const float* branch, int n_partials,
 #define ROWS(TW, TO, FULL, LN, K4, WPR) add_norm_rows_kernel<TW, TO, FULL, LN, K4, WPR><<<ceil_div(T, 4 / WPR), 256, 0, stream>>>( \
     resid, branch, n_partials, (size_t)partial_stride, (const TW*)w_post, (const TW*)w_pre, (const TW*)b_pre, (TO*)out, T, H,   \
     eps_post, eps_pre, off_post, off_pre, out_layout)
+  // Fewer rows, or a gather: four elements a thread where width and addresses allow it.
+  const bool by_four = aligned && H % 4 == 0 && H <= 8192 && (partial_stride % 4 == 0 || !branch);
+  const int threads4 = ceil_div(ceil_div(H, H <= 4096 ? 4 : 8), 64) * 64;
 #define LAUNCH(TW, TO, FULL, LN)                                                                     \
   do {                                                                                               \
     if (k4 > 0 && k4 <= 4) ROWS(TW, TO, FULL, LN, 4, 1);                                             \
@@ -415,6 +565,8 @@ extern "C" int alice_add_norm(float* resid, const float* branch, int n_partials,
     else if (k4 > 9 && k4 <= 16) ROWS(TW, TO, FULL, LN, 16, 1);                                      \
     else if (k4 > 16 && k4 <= 18) ROWS(TW, TO, FULL, LN, 9, 2);                                      \
     else if (k4 > 18) ROWS(TW, TO, FULL, LN, 16, 2);                                                 \
+    else if (by_four && H <= 4096) add_norm_row_kernel<TW, TO, FULL, LN, 1><<<T, threads4, 0, stream>>>(ARGS); \
+    else if (by_four) add_norm_row_kernel<TW, TO, FULL, LN, 2><<<T, threads4, 0, stream>>>(ARGS);    \
     else if (ept == 1) add_norm_regs_kernel<TW, TO, FULL, LN, 1><<<T, threads, 0, stream>>>(ARGS);   \
     else if (ept == 2) add_norm_regs_kernel<TW, TO, FULL, LN, 2><<<T, threads, 0, stream>>>(ARGS);   \
     else if (ept == 4) add_norm_regs_kernel<TW, TO, FULL, LN, 4><<<T, threads, 0, stream>>>(ARGS);   \
