@@ -88,25 +88,17 @@ struct Core {
 
   // The fragments of one block of 32 keys: kpage/vpage point at the page of one kv head, kb is the block
   // within the page (0/1).
-  // ONCE: the tile is read once per step by one wave (single tokens): loaded with the streaming hint.
-  template <bool ONCE = false>
-  __device__ __forceinline__ static u32x4 load_tile(const bf16_t* p) {
-    if constexpr (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-    else return *reinterpret_cast<const u32x4*>(p);
-  }
-  template <bool ONCE = false>
   __device__ __forceinline__ static void load_k(const bf16_t* __restrict__ kpage, int kb, int lane, u32x4 (&kf)[2][DT]) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
-        kf[t][dt] = load_tile<ONCE>(kpage + ((size_t)((kb * 2 + t) * DT + dt) * 64 + lane) * 8);
+        kf[t][dt] = *reinterpret_cast<const u32x4*>(kpage + ((size_t)((kb * 2 + t) * DT + dt) * 64 + lane) * 8);
   }
-  template <bool ONCE = false>
   __device__ __forceinline__ static void load_v(const bf16_t* __restrict__ vpage, int kb, int lane, u32x4 (&vf)[2 * DT]) {
 #pragma unroll
     for (int t = 0; t < 2 * DT; ++t)
-      vf[t] = load_tile<ONCE>(vpage + ((size_t)(kb * 2 * DT + t) * 64 + lane) * 8);
+      vf[t] = *reinterpret_cast<const u32x4*>(vpage + ((size_t)(kb * 2 * DT + t) * 64 + lane) * 8);
   }
 
   // Scores of one block of 32 keys from loaded key fragments; key0 is the absolute position of its first
@@ -592,21 +584,143 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 4 ? 2 : 1) void attn_prefi
   }
 }
 
-// ---------------------------------------------------------------- single tokens, keys split over blocks
+// ---------------------------------------------------------------- single tokens
+// One wave's walk over blocks of 32 keys for the 16 query columns (the heads of a kv head's group).  One set of fragments,
+// refilled as it is used up: the next block's keys are asked for when this block's scores are done, its values when this
+// block's values have been added, so that loads are in flight all the time and the loop's body stands in the program once.
+// That matters as much as the loads: a step launches this kernel once a layer, its instructions come from memory every time, and
+// each jump to a place not yet fetched costs about 0.2 us (two sets of fragments in an unrolled loop, with masked and unmasked
+// blocks apart, were 1,740 instructions and lines where this is 1,000; with a tail of their own for the last blocks they were
+// 3,100 and took 2 us more a launch).  So the mask is always applied, and what is asked for behind a wave's last block is a tile
+// that lies in the cache: a load under a branch makes the compiler wait for everything in flight.  The queries wait in LDS,
+// the tiles' addresses are the wave's, and 250 registers are enough.  A launch over 2,100 keys of one sequence (4 kv heads
+// of 256) 9.0 -> 7.9 us, of eight 16.2 -> 15.3, over 300 keys of one 7.6 -> 5.3, with the splits that decode_splits() chose and
+// chooses.  What bounds it now: 54 bytes a nanosecond and CU, and 6.3 TB/s in all (537 MB in 85 us).  Eight waves a block
+// were no faster; the step's key blocks dealt evenly to all waves, with a kernel that combines a sequence's parts, took 53
+// instead of 55-57 us for 64 sequences of 64 to 2,048 keys, but 89 instead of 83 for 64 of 2,048 and 21 instead of 17 for 64 of 300.
+static __device__ __align__(16) uint32_t g_idle[4096];       // read in place of a block that there is not: 16 KB
+
+template <int DT>
+struct Walk {
+  u32x4 kf[2][DT], vf[2 * DT];
+  f32x4 o[2 * DT];
+  float m, l;
+
+  __device__ __forceinline__ void begin() {
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int t = 0; t < 2 * DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  __device__ __forceinline__ void start_at_sink(float v, int lane) {         // see Core
+    m = v * LOG2E;
+    l = lane < 16 ? 1.f : 0.f;
+  }
+  // (the tile's address is the wave's, the lane's place in it an offset of 32 bits: no address registers a tile)
+  __device__ __forceinline__ static u32x4 tile(const bf16_t* __restrict__ p, unsigned lane) {
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p) + lane);
+  }
+  __device__ __forceinline__ void load_k(const bf16_t* __restrict__ p, int lane) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) kf[t][dt] = tile(p + (t * DT + dt) * 512, lane);
+  }
+  __device__ __forceinline__ void load_v(const bf16_t* __restrict__ p, int lane) {
+#pragma unroll
+    for (int t = 0; t < 2 * DT; ++t) vf[t] = tile(p + t * 512, lane);
+  }
+  // The block whose first key is key0, seen by the query at `pos`; next_k and next_v: the next block's tiles, or g_idle.
+  template <bool SOFTCAP>
+  __device__ __forceinline__ void step(const u32x4* __restrict__ ql, int key0, int pos, int window, ScoreConsts k, const bf16_t* next_k,
+                                       const bf16_t* next_v, int lane) {
+    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const u32x4 q = ql[dt * 64 + lane];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) s[t] = mfma16(kf[t][dt], q, s[t]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load_k(next_k, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    // key visible iff lo <= key <= pos, i.e. (unsigned)(key - lo) <= (unsigned)(pos - lo)
+    const int lo = window > 0 ? max(pos + 1 - window, 0) : 0;
+    const unsigned span = (unsigned)(pos - lo);
+    const int rel0 = key0 + (lane >> 4) * 4 - lo;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v = s[t][i] * k.c_in;
+        if (SOFTCAP) v = fmaf(-2.f * k.c_out, rcp_fast(exp2_fast(v) + 1.f), k.c_out);
+        v = ((unsigned)(rel0 + t * 16 + i) <= span) ? v : -INFINITY;
+        s[t][i] = v;
+        mx = fmaxf(mx, v);
+      }
+    const float seen = col_max(mx);                          // the base follows as in Core::softmax_step
+    const bool raise = seen > m + RAISE;
+    const float m_new = raise ? seen : m;
+    const float base = (m_new == -INFINITY) ? 0.f : m_new;
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float e = exp2_fast(s[t][i] - base);
+        s[t][i] = e;
+        sum += e;
+      }
+    const u32x4 p = {pack2(s[0][0], s[0][1]), pack2(s[0][2], s[0][3]), pack2(s[1][0], s[1][1]), pack2(s[1][2], s[1][3])};
+    if (__any(raise)) {
+      const float corr = raise ? exp2_fast(m - base) : 1.f;
+      l *= corr;
+#pragma unroll
+      for (int t = 0; t < 2 * DT; ++t) o[t] *= corr;
+    }
+    l += sum;
+    m = m_new;
+#pragma unroll
+    for (int t = 0; t < 2 * DT; ++t) o[t] = mfma16(vf[t], p, o[t]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_v(next_v, lane);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // The queries of 16 columns (columns without a head: the first head's, never stored) on their way to LDS as fragments; PARTS
+  // waves share them.
+  template <int PARTS>
+  struct Queries {
+    static constexpr int N = (DT + PARTS - 1) / PARTS;
+    u32x4 r[N];
+    __device__ __forceinline__ void load(const bf16_t* __restrict__ rows, bool head_ok, int part, int lane) {
+      const bf16_t* qrow = rows + (size_t)(head_ok ? lane & 15 : 0) * (DT * 32) + (lane >> 4) * 8;
+#pragma unroll
+      for (int i = 0; i < N; ++i) r[i] = *reinterpret_cast<const u32x4*>(qrow + min(part + i * PARTS, DT - 1) * 32);
+    }
+    __device__ __forceinline__ void store(u32x4* __restrict__ ql, int part, int lane) const {
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (DT % PARTS == 0 || part + i * PARTS < DT) ql[(part + i * PARTS) * 64 + lane] = r[i];
+    }
+  };
+};
+
+// Keys split over blocks.
 // grid: (sequences, kv heads, splits).  The query tile's 16 columns are the query heads of the kv head's
-// group (group <= 16).  The sequence's 32-key blocks are dealt out in contiguous runs to the
-// splits * 4 waves; every wave keeps a running (max, sum, output); the block's four waves are combined
-// in LDS in the order 0, 1, 2, 3 and the split's result goes to `parts`:
+// group (group <= 16).  The sequence's 32-key blocks go to the splits in even runs, a split's to its NW waves likewise; every
+// wave keeps a running (max, sum, output); the block's waves are combined in LDS in their order and the split's result goes to `parts`:
 // [sequence][head][split][4 + D] = (max, sum, two unused, unnormalised output).  With one split the output is final.
 template <int DT, bool SOFTCAP>
-__global__ __launch_bounds__(256) void attn_decode_kernel(
+__global__ __launch_bounds__(256, 2) void attn_decode_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
     bf16_t* __restrict__ out, float* __restrict__ parts, const int* __restrict__ context_lens,
     const int* __restrict__ block_table, int bt_stride, int nH, int nKV, float scale, float cap, int window, int splits,
     int out_layout, const float* __restrict__ sink) {
-  constexpr int D = DT * 32;
-  __shared__ float sm[4][16], sl[4][16];
-  extern __shared__ __align__(16) float so[];            // [4 waves][group][D + 4]
+  constexpr int D = DT * 32, NW = 4;
+  __shared__ float sm[NW][16], sl[NW][16];
+  extern __shared__ __align__(16) float so[];            // [NW waves][group][D + 4]
+  __shared__ __align__(16) u32x4 ql[DT * 64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
   const int b = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
@@ -615,70 +729,55 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   const int first_key = window > 0 ? max(0, pos + 1 - window) : 0;
   const int kb_first = first_key >> 5, kb_last = pos >> 5;
   const int n_blocks = kb_last - kb_first + 1;
-  const int workers = splits * 4, me = split * 4 + wave;
-  const int per = (n_blocks + workers - 1) / workers;
-  const int my_first = kb_first + me * per, my_last = min(kb_last, my_first + per - 1);
+  const int run0 = split * n_blocks / splits, run = (split + 1) * n_blocks / splits - run0;
+  const int my_first = kb_first + run0 + wave * run / NW, my_last = kb_first + run0 + (wave + 1) * run / NW - 1;
   const int* bt = block_table + (size_t)b * bt_stride;
   const size_t page_elems = (size_t)64 * D;
 
-  Core<DT, 1> c;
-  c.init();
+  Walk<DT> c;
   const ScoreConsts sc(scale, cap);
   const bool head_ok = col < group;
-  int cpos[1] = {head_ok ? pos : -1};
-  if (sink && me == 0 && head_ok) c.start_at_sink(0, sink[kvh * group + col], lane);
-  {
-    const bf16_t* qrow = q + ((size_t)b * nH + kvh * group + (head_ok ? col : 0)) * D;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      c.q[0][dt] = u32x4{0u, 0u, 0u, 0u};
-      if (head_ok) c.q[0][dt] = *reinterpret_cast<const u32x4*>(qrow + dt * 32 + g * 8);
-    }
+  typename Walk<DT>::template Queries<NW> qs;
+  qs.load(q + ((size_t)b * nH + kvh * group) * D, head_ok, wave, lane);
+  __builtin_amdgcn_sched_barrier(0);
+  // Page numbers are read one step before the tiles they name, through the scalar cache (the indices are the same for the
+  // whole wave): a wait for them is no wait for the tiles in flight.
+  auto page_of = [&](int kb32) { return bt[max(min(kb32, my_last), 0) >> 1]; };
+  const bf16_t* idle = reinterpret_cast<const bf16_t*>(g_idle);
+  auto tiles = [&](const bf16_t* pool, int kb32, int page) {
+    return kb32 <= my_last ? pool + ((size_t)page * nKV + kvh) * page_elems + (size_t)(kb32 & 1) * (DT * 1024) : idle;
+  };
+  int page = page_of(my_first), page_next = page_of(my_first + 1);
+  c.load_k(tiles(k_pool, my_first, page), lane);
+  __builtin_amdgcn_sched_barrier(0);
+  c.load_v(tiles(v_pool, my_first, page), lane);
+  __builtin_amdgcn_sched_barrier(0);
+  qs.store(ql, wave, lane);
+  c.begin();
+  if (sink && split == 0 && wave == 0 && head_ok) c.start_at_sink(sink[kvh * group + col], lane);
+  lds_barrier();
+  for (int kb32 = my_first; kb32 <= my_last; ++kb32) {
+    page = page_next;
+    page_next = page_of(kb32 + 2);
+    c.template step<SOFTCAP>(ql, kb32 << 5, pos, window, sc, tiles(k_pool, kb32 + 1, page), tiles(v_pool, kb32 + 1, page), lane);
   }
-  // Two sets of fragment registers: while one block of keys is computed, the next one's loads are in flight.
-  // The page numbers are read one step before the tiles they name, through the scalar cache (the indices are
-  // the same for the whole wave): a wait for them is no wait for the tiles in flight.
-  {
-    u32x4 kf0[2][DT], vf0[2 * DT], kf1[2][DT], vf1[2 * DT];
-    auto page_of = [&](int kb32) { return bt[min(kb32, my_last) >> 1]; };
-    auto fetch = [&](int kb32, int page, u32x4 (&kf)[2][DT], u32x4 (&vf)[2 * DT]) {
-      Core<DT, 1>::template load_k<true>(k_pool + ((size_t)page * nKV + kvh) * page_elems, kb32 & 1, lane, kf);
-      Core<DT, 1>::template load_v<true>(v_pool + ((size_t)page * nKV + kvh) * page_elems, kb32 & 1, lane, vf);
-    };
-    int page_a = 0, page_b = 0;
-    if (my_first <= my_last) {
-      page_a = page_of(my_first);
-      page_b = page_of(my_first + 1);
-      fetch(my_first, page_a, kf0, vf0);
-    }
-    for (int kb32 = my_first; kb32 <= my_last; kb32 += 2) {
-      if (kb32 + 1 <= my_last) fetch(kb32 + 1, page_b, kf1, vf1);
-      page_a = page_of(kb32 + 2);
-      page_b = page_of(kb32 + 3);
-      c.template compute<SOFTCAP>(kf0, vf0, kb32 << 5, cpos, window, sc, lane);
-      if (kb32 + 1 <= my_last) {
-        if (kb32 + 2 <= my_last) fetch(kb32 + 2, page_a, kf0, vf0);
-        c.template compute<SOFTCAP>(kf1, vf1, (kb32 + 1) << 5, cpos, window, sc, lane);
-      }
-    }
-  }
-  // combine the four waves
-  c.finish();
-  if (g == 0) { sm[wave][col] = c.m[0]; sl[wave][col] = c.l[0]; }
+  // combine the waves
+  c.l = col_sum(c.l);
+  if (g == 0) { sm[wave][col] = c.m; sl[wave][col] = c.l; }
   if (head_ok) {
 #pragma unroll
     for (int t = 0; t < 2 * DT; ++t)
-      *reinterpret_cast<f32x4*>(&so[((size_t)wave * group + col) * (D + 4) + t * 16 + g * 4]) = c.o[0][t];
+      *reinterpret_cast<f32x4*>(&so[((size_t)wave * group + col) * (D + 4) + t * 16 + g * 4]) = c.o[t];
   }
-  __syncthreads();
-  // thread -> (head column hc, dims): 256 threads cover 16 columns x D dims
-  for (int idx = threadIdx.x; idx < 16 * D; idx += 256) {
+  lds_barrier();
+  for (int idx = threadIdx.x; idx < group * D; idx += 64 * NW) {
     const int hc = idx / D, e = idx % D;
-    if (hc >= group) continue;
-    float mm = fmaxf(fmaxf(sm[0][hc], sm[1][hc]), fmaxf(sm[2][hc], sm[3][hc]));
+    float mm = sm[0][hc];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) mm = fmaxf(mm, sm[w][hc]);
     float acc = 0.f, ll = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float f = (sm[w][hc] == -INFINITY) ? 0.f : exp2_fast(sm[w][hc] - mm);     // maxima are base-2 exponents
       acc += so[((size_t)w * group + hc) * (D + 4) + e] * f;
       ll += sl[w][hc] * f;

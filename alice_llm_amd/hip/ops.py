@@ -1498,18 +1498,26 @@ def attention_mfma_supported(head_dim: int) -> bool:
     return bool(library().alice_attention_mfma_supported(int(head_dim)))
 
 
-def decode_splits(n_seqs: int, num_kv_heads: int, max_context: int) -> int:
-    """Into how many blocks the keys of a sequence are split for single-token attention.  At most as many as fill
-    the chip (about a thousand waves); among those, the fewest that leave a wave the fewest 32-key blocks to walk
-    through one after the other, but no fewer than two (125 blocks of keys: 16 splits of four waves walk two each,
-    15 splits three)."""
-    n_blocks = -(-max_context // 32)
-    cap = max(1, min(-(-1024 // max(1, n_seqs * num_kv_heads * 4)), 64))
-    best, best_per = 1, -(-n_blocks // 4)
-    for s in range(2, cap + 1):
-        per = -(-n_blocks // (4 * s))
-        if 2 <= per < best_per:
-            best, best_per = s, per
+def decode_splits(n_seqs: int, num_kv_heads: int, max_context: int, head_dim: int = 256) -> int:
+    """Into how many blocks the keys of a sequence are split for single-token attention: the cheapest in microseconds by what
+    was measured on the 2B, 9B and 27B shapes (1 to 32 sequences of 100 to 6,000 keys), among those that leave a CU one block.
+    A block takes 0.57 us for every 32 keys of head size 256 (what a CU reads) and 0.5 a round of its four waves, all blocks
+    together read 6.5 TB/s (the shorter of the two is not quite hidden), and the output projection pays for every split
+    that it combines (up to 16 splits of 16 sequences; beyond, a kernel of its own combines them).  Captured steps name
+    the context rounded up to 512: half of that is taken off.  Against the earlier rule, at least two rounds a wave: a 2B
+    step of one sequence at 2,048 keys 1,719 -> 1,660 us, of four at 300 1,726 -> 1,620, of eight at 500 1,742 -> 1,685."""
+    n_blocks = -(-max(max_context - 256, min(max_context, 256)) // 32)
+    size = head_dim / 256
+    whole = n_seqs * num_kv_heads * n_blocks * 32768 * size / 6.5e6
+    best, best_cost = 1, None
+    for s in range(1, max(1, min(256 // max(1, n_seqs * num_kv_heads), 64, n_blocks)) + 1):
+        run = -(-n_blocks // s)
+        block = 0.57 * size * run + 0.5 * -(-run // 4)
+        cost = max(whole, block) + 0.3 * min(whole, block)
+        if s > 1:
+            cost += (0.12 + 0.05 * n_seqs) * s if n_seqs <= 16 and s <= 16 else 9.0 + 0.02 * s
+        if best_cost is None or cost < best_cost:
+            best, best_cost = s, cost
     return best
 
 
@@ -1570,7 +1578,7 @@ def attention_decode(q, k_pool, v_pool, out, context_lens, block_table, *, num_h
         raise HipLibraryError(f"{max_context} keys are beyond the block table {tuple(block_table.shape)}")
     if splits is None:
         reach = max_context if not window else min(max_context, window + 32)
-        splits = decode_splits(B, nKV, reach)
+        splits = decode_splits(B, nKV, reach, d)
     if out is None and splits < 2:
         raise HipLibraryError("attention_decode: without an output buffer the keys must be split")
     parts = (torch.empty((library().alice_attention_decode_workspace(B, num_heads, d, splits),), dtype=torch.float32,
@@ -1590,10 +1598,10 @@ def attention_decode(q, k_pool, v_pool, out, context_lens, block_table, *, num_h
     return parts, splits
 
 
-def decode_attention_splits(n_seqs: int, num_kv_heads: int, max_context: int, window: Optional[int]) -> int:
+def decode_attention_splits(n_seqs: int, num_kv_heads: int, max_context: int, window: Optional[int], head_dim: int = 256) -> int:
     """The number of key splits that attention_decode picks by itself for a step."""
     reach = max_context if not window else min(max_context, window + 32)
-    return decode_splits(n_seqs, num_kv_heads, reach)
+    return decode_splits(n_seqs, num_kv_heads, reach, head_dim)
 
 
 def linear_parts_slices(M: int, n_out: int, num_heads: int, head_dim: int, splits: int) -> int:
