@@ -238,7 +238,7 @@ int planned_tokens(int M) { return M <= 32 ? 32 : ceil_div(M, 64) * 64; }
 // them a CU), its NW waves every NW-th chunk of 32 inner elements of
 // its slice; their sums meet in LDS.  W goes straight from memory into the instruction's operand, 128 bytes of a row a
 // chunk, the next two chunks on their way while two are multiplied; the tokens' elements come through the L1.  A token's
-// result depends on no other token, nor on how many there are.
+// result depends on no other token, nor on how many there are (as long as this kernel takes them).
 // WHOLE: rows of whole, aligned units of eight elements.  Else (any K, any address) the same loads without an alignment, and the
 // elements behind the last whole chunk one by one, by the wave whose turn it is: 2,304 rows by 2,305 at 4 tokens 9.0 us (by 2,304
 // 9.1; on the tile of 64 tokens 71).
@@ -429,6 +429,160 @@ int launch_single(const void* x, const void* w, void* y, int N, int K, int epi, 
   return 0;
 }
 
+// Up to 4 tokens on FMAs, where rows are whole units of four elements at aligned addresses: a wave takes four rows of W (with GeGLU
+// the gate and up rows of two outputs), its lanes 1 KB of a row at a time, and every element that it reads serves all tokens, whose
+// elements wait in LDS.  The matrix instruction above leaves 12 or more of its 16 columns idle at so few, and its operand order
+// reads W in pieces of 128 bytes of a row; here a load is a whole kilobyte, with the streaming hint (gate and up 35.4 -> 33.7 us,
+// the output head 394 -> 357; the 128-byte pieces get slower by it), and two of every row are on their way while two
+// are multiplied.  The tokens' elements are asked for ahead of W's first (33.7 -> 30.2 us: a block's start is what its CU waits for).
+// What bounds it: reading W, at 6.6 TB/s where it is long.  4 tokens, 2B shape, matrix instruction and this: q, k, v 12.6 and
+// 8.9 us, output projection 7.2 (8 slices) and 6.3 (3), gate and up 40.0 and 30.2, down 21.6 and 17.1, head 404 and 353; five to
+// eight tokens gain nothing by it (42 us for gate and up, 468 for the head).
+// Which products a token's sum adds, and in which order, depends on K and the slices alone: a lane's elements in their order, then
+// the lanes over the distances 32, 16 .. 1.  That is the order of the kernel for one token as well (the same bits), not that of the
+// matrix instruction: the fifth token of a step changes the others' sums by rounding.
+constexpr int FEW_MT = 4, FEW_R = 4, FEW_SEG = 256, FEW_KC = 2560;       // tokens, rows a wave, elements a step, elements of a token that a block keeps (whole steps of two)
+
+template <typename T> __device__ __forceinline__ f32x4 load_four(const T* p);
+template <> __device__ __forceinline__ f32x4 load_four<float>(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+template <> __device__ __forceinline__ f32x4 load_four<bf16_t>(const bf16_t* p) {
+  const uint2 v = *reinterpret_cast<const uint2*>(p);
+  return f32x4{bf16_bits_to_f32(v.x & 0xffffu), bf16_bits_to_f32(v.x >> 16), bf16_bits_to_f32(v.y & 0xffffu), bf16_bits_to_f32(v.y >> 16)};
+}
+
+__device__ __forceinline__ f32x4 load_once(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p)); }
+__device__ __forceinline__ f32x4 load_once(const bf16_t* p) { return load_four(p); }
+
+// V sums over the 64 lanes at once: a step over lane distance d adds the partner's value, and while several values are left each half of
+// the lanes goes on with half of them.  Lane l ends with the sums of values first + 0 .. V / 8 - 1, first = V/2 (l / 32) + V/4 (l / 16 % 2)
+// + V/8 (l / 8 % 2).
+template <int V>
+__device__ __forceinline__ int sums_by_lane(float (&v)[V], int lane) {
+  static_assert(V >= 8, "three halvings");
+  auto bits = [](float x) { return __float_as_uint(x); };
+#pragma unroll
+  for (int i = 0; i < V / 2; ++i) {
+    auto p = __builtin_amdgcn_permlane32_swap(bits(v[i]), bits(v[i + V / 2]), false, false);
+    v[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < V / 4; ++i) {
+    auto p = __builtin_amdgcn_permlane16_swap(bits(v[i]), bits(v[i + V / 4]), false, false);
+    v[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < V / 8; ++i) {
+    const bool upper = lane & 8;
+    const float give = upper ? v[i] : v[i + V / 8], keep = upper ? v[i + V / 8] : v[i];
+    v[i] = keep + __uint_as_float(dpp_move<DPP_ROR8>(bits(give)));
+  }
+#pragma unroll
+  for (int i = 0; i < V / 8; ++i) {
+    v[i] += __uint_as_float(dpp_move<0x1B>(dpp_move<0x141>(bits(v[i]))));    // lane ^ 4: mirrored in its eight, then in its four
+    v[i] += __uint_as_float(dpp_move<DPP_XOR2>(bits(v[i])));
+    v[i] += __uint_as_float(dpp_move<DPP_XOR1>(bits(v[i])));
+  }
+  return (lane >> 5) * (V / 2) + ((lane >> 4) & 1) * (V / 4) + ((lane >> 3) & 1) * (V / 8);
+}
+
+template <typename TA, typename TW, typename TO, bool GEGLU>
+__global__ __launch_bounds__(256) void linear_few_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y, int M, int N,
+                                                         int K, int kslice, int kc, int epi, float param, int full) {
+  constexpr int MT = FEW_MT, R = FEW_R, U = 2, P = (FEW_KC + 1023) / 1024;   // P: rounds of the block over a chunk's elements
+  extern __shared__ __align__(16) float xs[];                 // [MT][kc]: the tokens' elements of a chunk, zeros behind the slice
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n0 = (blockIdx.x * 4 + wave) * (GEGLU ? R / 2 : R);
+  const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);
+  const TW* wrow[R];                                          // rows beyond the last are read as the last and not written
+#pragma unroll
+  for (int r = 0; r < R; ++r) wrow[r] = W + (size_t)(GEGLU ? (r & 1) * N + min(n0 + (r >> 1), N - 1) : min(n0 + r, N - 1)) * K;
+  float acc[MT * R];
+#pragma unroll
+  for (int i = 0; i < MT * R; ++i) acc[i] = 0.f;
+  f32x4 w[U][R];
+  auto fetch = [&](int k, f32x4 (&to)[R]) {                   // unconditional: behind the slice its last four elements
+#pragma unroll
+    for (int r = 0; r < R; ++r) to[r] = load_once(wrow[r] + min(k + lane * 4, k_end - 4));
+  };
+  // The tokens' elements of a chunk through registers into LDS: the first chunk's are asked for before W's first, which are on
+  // their way while the block meets.
+  f32x4 v[P][MT];
+  auto load_x = [&](int c0) {
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) v[p][m] = load_four(A + (size_t)min(m, M - 1) * K + min(c0 + p * 1024 + tid * 4, k_end - 4));
+  };
+  load_x(k_begin);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) fetch(k_begin + u * FEW_SEG, w[u]);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int c0 = k_begin; c0 < k_end; c0 += kc) {
+    if (c0 > k_begin) {
+      load_x(c0);
+      lds_barrier();
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int k = p * 1024 + tid * 4;
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        if (k < kc) *reinterpret_cast<f32x4*>(xs + m * kc + k) = c0 + k < k_end ? v[p][m] : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    lds_barrier();
+    const int stop = min(k_end - c0, kc);
+    for (int s = 0; s < stop; s += U * FEW_SEG) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = s + u * FEW_SEG;
+        if (k < stop) {                                       // (the same for the whole block)
+          if (k + FEW_SEG > stop) {                           // what was read again behind the end: zeros
+#pragma unroll
+            for (int r = 0; r < R; ++r) w[u][r] = k + lane * 4 < stop ? w[u][r] : f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(xs + m * kc + k + lane * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int r = 0; r < R; ++r) acc[m * R + r] = fmaf(w[u][r][e], x[e], acc[m * R + r]);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(c0 + k + U * FEW_SEG, w[u]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  const int first = sums_by_lane<MT * R>(acc, lane);
+  if (lane & 7) return;
+  TO* y = Y + (size_t)blockIdx.y * M * N;
+#pragma unroll
+  for (int i = 0; i < MT * R / 8; i += GEGLU ? 2 : 1) {
+    const int m = (first + i) / R, r = (first + i) % R, n = n0 + (GEGLU ? r >> 1 : r);
+    if (m >= M || n >= N) continue;
+    float o = acc[i];
+    if (GEGLU) o = gated_act(acc[i], acc[i + 1], param, full);
+    if (epi == ALICE_EPI_SOFTCAP) o = unary_act(o, param, full);
+    store_f32(y, (size_t)m * N + n, o);
+  }
+}
+
+template <typename TA, typename TW, typename TO>
+int launch_few(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split, hipStream_t stream) {
+  const int kslice = ceil_div(ceil_div(K, split), 128) * 128;
+  const int kc = min(ceil_div(kslice, FEW_SEG) * FEW_SEG, FEW_KC);
+  const dim3 grid(ceil_div(N, (epi == ALICE_EPI_GEGLU ? 2 : 4) * FEW_R), split);
+  const size_t lds = (size_t)FEW_MT * kc * sizeof(float);
+#define GO(GEGLU) linear_few_kernel<TA, TW, TO, GEGLU><<<grid, 256, lds, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, kslice, kc, epi, epi_param, full)
+  if (epi == ALICE_EPI_GEGLU) GO(true); else GO(false);
+#undef GO
+  ALICE_LAUNCH_CHECK();
+  return 0;
+}
+
 template <typename TA, typename TW, typename TO>
 int launch_rows(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split,
                 hipStream_t stream) {
@@ -484,9 +638,34 @@ int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int
 
 }  // namespace
 
-// Into how many slices of the inner dimension a product without an epilogue is best cut.
+// Whether up to 4 tokens go on FMAs: rows of whole units of four elements, at addresses of such units, and long enough that the
+// block's start does not outweigh them (65,536 rows by 256: 22.7 us, 16.2 on the matrix instruction; by 1,024 and more it is faster).
+static bool few_by_fours(const void* x, int x_dtype, const void* w, int w_dtype, int K) {
+  auto unit = [](int dtype) { return dtype == DT_F32 ? 15u : 7u; };
+  return K % 4 == 0 && K >= 1024 && ((uintptr_t)x & unit(x_dtype)) == 0 && ((uintptr_t)w & unit(w_dtype)) == 0;
+}
+
+// Slices for one token: W is read at 6.6 TB/s with three blocks a CU, at three quarters of that with few; the busiest CU reads
+// its blocks' rows at 40 GB/s or less; a slice more costs the add behind it 0.2 us.  (2,304 rows by 2,048: 3 or 4 slices, 6.3 and
+// 6.8 us; by 9,216: 6, 17.1, 24.4 whole; 3,584 by 14,336: 4, 38.0, 40.7 whole; 8,192 by 3,584: 1.)
+static int single_split(int N, int K) {
+  const int blocks = ceil_div(N, 4 * FEW_R);
+  int best = 1;
+  float best_us = 1e30f;
+  for (int s = 1; s <= MAX_SPLIT; ++s) {
+    const int ks = ceil_div(ceil_div(K, s), 128) * 128;
+    if (s > 1 && (ks < 512 || (long)ks * (s - 1) >= K)) continue;
+    const float full = fminf(1.f, 0.75f + 0.25f * blocks * s / 768.f);
+    const float us = fmaxf((float)N * K * 4e-6f / (6.6f * full), ceil_div((long)blocks * s, 256) * (float)ks * 64.f / 40e3f) + 0.2f * s;
+    if (us < best_us) { best_us = us; best = s; }
+  }
+  return best;
+}
+
+// Into how many slices of the inner dimension a product without an epilogue is best cut (for 2 to 16 tokens one
+// number, whatever captured steps round theirs to).
 int alice_linear_split_hint_generic(int M, int N, int K) {
-  if (M == 1) return 1;
+  if (M == 1) return K % 4 == 0 && K >= 1024 ? single_split(N, K) : 1;
   return M <= 16 ? rows_split(N, K) : plan_mfma32(planned_tokens(M), N, K, false, MAX_SPLIT).split;
 }
 
@@ -503,7 +682,13 @@ int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype,
   if (M == 0) return 0;
   int rc = 0;
   DISPATCH_DTYPE(x_dtype, TA, DISPATCH_DTYPE(w_dtype, TW, DISPATCH_DTYPE(y_dtype, TO, {
-    if (M == 1 && split_k == 1) rc = launch_single<TA, TW, TO>(x, w, y, N, K, epi, epi_param, full_precision, stream);
+    // (slices of 256 elements: 8.2 us, 7.2 on the matrix instruction)
+    const bool few = M <= FEW_MT && few_by_fours(x, x_dtype, w, w_dtype, K) && ceil_div(K, split_k) >= 512;
+    // One token: the same sums either way; a wave a row is the faster start (1,000 x 1,024: 3.6 and 4.5 us, 3,584 x 4,096: 14.1 and
+    // 14.9), four rows a wave read longer matrices faster (8,192 x 3,584: 22.3 and 21.3, gate and up 34.5 and 30.4).
+    const bool large = (size_t)N * K * sizeof(TW) * (epi == ALICE_EPI_GEGLU ? 2 : 1) >= ((size_t)80 << 20);
+    if (M == 1 && split_k == 1 && !(few && large)) rc = launch_single<TA, TW, TO>(x, w, y, N, K, epi, epi_param, full_precision, stream);
+    else if (few) rc = launch_few<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
     else rc = M <= 16 ? launch_rows<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream)
                       : launch_tiled<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
   })));

@@ -1,0 +1,84 @@
+"""32-bit products of up to four tokens: at the edges of the rows a wave takes, the elements a step and the chunk that a block
+keeps, in slices that end anywhere, against 64 bits and against the kernel for rows of any address."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from alice_llm_amd.hip import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+DT = {"float32": torch.float32, "bfloat16": torch.bfloat16}
+
+
+def rnd(*shape, seed=0, scale=1.0, dtype=torch.float32):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=g) * scale).to(dtype).to(DEV)
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,K", [(1, 1024), (17, 1028), (70, 2560), (46, 2564), (33, 5120), (18, 9220), (2304, 2048)])
+@pytest.mark.parametrize("xdt,wdt", [("float32", "float32"), ("float32", "bfloat16"), ("bfloat16", "float32")])
+def test_few_tokens(M, N, K, xdt, wdt):
+    x, w = rnd(M, K, seed=M, dtype=DT[xdt]), rnd(N, K, seed=N, scale=0.1, dtype=DT[wdt])
+    ref, tol = x.double() @ w.double().T, 8 * 0.1 * K * 2 ** -24           # (as in test_gpu_f32.py)
+    moved = torch.empty(N * K + 1, dtype=w.dtype, device=DEV)[1:].view(N, K).copy_(w)
+    for split in {1, 2, 3, 7, 8, ops.linear_split_hint(M, N, K, ops.LAYOUT_ROW)}:
+        outs = []
+        for wt in (w, moved):
+            y = torch.full((split, M, N) if split > 1 else (M, N), float("nan"), device=DEV)
+            ops.linear(x, wt, y, n_out=N, k_in=K, split_k=split, full_precision=True)
+            outs.append(y.sum(0) if split > 1 else y)
+            assert (outs[-1].double() - ref).abs().max() <= tol, split
+    if N % 2 == 0:
+        out = torch.full((M, N // 2), float("nan"), device=DEV)
+        ops.linear(x, w, out, n_out=N // 2, k_in=K, epilogue=ops.EPI_GEGLU, full_precision=True)
+        want = F.gelu(ref[:, :N // 2], approximate="tanh") * ref[:, N // 2:]
+        assert ((out.double() - want).abs() <= 4 * tol + 1e-5 * want.abs()).all()
+    capped = torch.full((M, N), float("nan"), device=DEV)
+    ops.linear(x, w, capped, n_out=N, k_in=K, epilogue=ops.EPI_SOFTCAP, epi_param=5.0, full_precision=True)
+    assert (capped.double() - 5 * torch.tanh(ref / 5)).abs().max() <= tol + 1e-5
+
+
+def test_a_token_gets_the_same_with_and_without_others():
+    """One token (a wave a row, or four rows a wave in large matrices) and four: the same bits."""
+    for N, K in ((40, 1028), (8200, 2560)):
+        x, w = rnd(4, K, seed=1), rnd(N, K, seed=2)
+        outs = []
+        for M in (1, 2, 4):
+            outs.append(torch.empty(M, N, device=DEV))
+            ops.linear(x[:M].contiguous(), w, outs[-1], n_out=N, k_in=K, full_precision=True)
+        assert torch.equal(outs[0], outs[2][:1]) and torch.equal(outs[1], outs[2][:2])
+
+
+def test_weights_that_are_no_numbers_stay_in_their_rows():
+    """What is read again behind a row's end is not multiplied: a last element that is infinite reaches its own product alone."""
+    x, w = rnd(3, 1028, seed=1), rnd(12, 1028, seed=2)
+    x[:, -1] = 0.0
+    x[1, -1] = 1.0
+    w[5, -1] = float("inf")
+    y = torch.empty(3, 12, device=DEV)
+    ops.linear(x, w, y, n_out=12, k_in=1028, full_precision=True)
+    want = x.double() @ w.double().T
+    assert torch.equal(torch.isnan(y).cpu(), torch.isnan(want).cpu()) and torch.equal(torch.isinf(y).cpu(), torch.isinf(want).cpu())
+
+
+def test_short_prompts_captured_and_eagerly():
+    """Prompts of two to five tokens at a width whose products take this kernel, which a captured step of sixteen rows does not: the
+    same up to the order of sums (K = 1,024: logits of order 1, 32-bit)."""
+    import alice_llm_amd as alice
+    from helpers import TINY, random_tokens
+    raw = dict(TINY["tiny-a"][0], num_hidden_layers=1, hidden_size=1024, intermediate_size=1024)
+    model = alice.Model.random(raw, seed=4, dtype="float32", fast=True)
+    eager, graph = (model.engine(max_tokens=64 * 8, max_seqs=2, use_graphs=g) for g in (False, True))
+    assert graph.capture_prompts
+    for n in (2, 3, 4, 5):
+        replayed = []
+        toks = random_tokens(256, n, n)
+        for _ in range(4):                                               # seen, captured, replayed
+            a, b = eager.open(1), graph.open(1)
+            want = eager.step(a, [toks], "last")
+            replayed.append(graph.step(b, [toks], "last"))
+            assert (replayed[-1] - want).abs().max() < 1e-5
+            eager.close(a), graph.close(b)
+        assert torch.equal(replayed[2], replayed[3])
