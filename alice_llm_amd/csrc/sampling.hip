@@ -70,7 +70,7 @@ __device__ __forceinline__ int block_count(int v, int* ired) {
   return t;
 }
 
-// Inclusive prefix sum over the block in thread order; `excl` gets the previous thread's inclusive sum (bit for bit).
+// Inclusive prefix sum over a block of ST in thread order; `excl` gets the previous thread's inclusive sum (bit for bit).
 __device__ __forceinline__ float block_inclusive_scan(float v, float* wred, float* excl) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
@@ -82,8 +82,9 @@ __device__ __forceinline__ float block_inclusive_scan(float v, float* wred, floa
   __syncthreads();
   if (lane == 63) wred[wid] = v;
   __syncthreads();
-  float before = 0.f;
-  for (int w = 0; w < wid; ++w) before += wred[w];
+  float before = 0.f;                                      // (all the waves' sums at once: what is not before this wave adds zero)
+#pragma unroll
+  for (int w = 0; w < ST / 64 - 1; ++w) before += w < wid ? wred[w] : 0.f;
   // the thread before lane 0 is lane 63 of the wave before: its inclusive sum is (sum of waves < wid-1) + wred[wid-1],
   // which is how `before` was built
   *excl = lane == 0 ? before : before + prev;
@@ -597,11 +598,11 @@ __global__ __launch_bounds__(SB) void tile_sum_kernel(const float* __restrict__ 
                  c * w.tiles_per_chunk + (threadIdx.x >> 6), min(w.tiles, (c + 1) * w.tiles_per_chunk), SB / 64);
 }
 
-// The draw within the tile t_sel (-1: the row's last kept token) that the running sums chose, whose predecessors hold tile_before.
+// The draw within the tile t_sel (-1: the row's last kept token) that the running sums chose, whose predecessors hold tile_before;
+// e: the probabilities of the thread's four elements, 0 for what is not kept.
 // All threads of a block of ST call it, pick: two ints in shared memory.
-__device__ __forceinline__ void draw_in_tile(const float* __restrict__ row, int* __restrict__ out, int b, int V, float inv_t, float m,
-                                             uint32_t thr, int t_sel, int last_of_row, float target, float tile_before, float* wred,
-                                             int* pick) {
+__device__ __forceinline__ void draw_in_tile(const float (&e)[4], int* __restrict__ out, int b, int t_sel, int last_of_row, float target,
+                                             float tile_before, float* wred, int* pick) {
   const int tid = threadIdx.x;
   __syncthreads();
   if (t_sel < 0) {                                       // u * total rounded up to the total: the last kept token
@@ -610,15 +611,10 @@ __device__ __forceinline__ void draw_in_tile(const float* __restrict__ row, int*
   }
   if (tid == 0) { pick[0] = -1; pick[1] = -1; }
   const int base = t_sel * TILE + tid * 4;
-  float e[4], mine = 0.f;
+  float mine = 0.f;
   int my_last = -1;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    e[j] = 0.f;
-    if (base + j < V) {
-      float x = row[base + j] * inv_t;
-      if (order_key(x) >= thr) e[j] = expf(x - m);
-    }
     if (e[j] > 0.f) my_last = base + j;
     mine += e[j];
   }
@@ -686,7 +682,19 @@ __device__ __forceinline__ void draw_from_tiles(const float* __restrict__ row, i
     if (w.tiles <= 1024) break;
   }
   __syncthreads();
-  draw_in_tile(row, out, b, V, inv_t, m, thr, pick[0], pick[1], u * carry[0], carry[1], wred, pick);
+  const int tile = pick[0];
+  float e[4] = {0.f, 0.f, 0.f, 0.f};
+  if (tile >= 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = tile * TILE + tid * 4 + j;
+      if (i < V) {
+        const float x = row[i] * inv_t;
+        if (order_key(x) >= thr) e[j] = expf(x - m);
+      }
+    }
+  }
+  draw_in_tile(e, out, b, tile, pick[1], u * carry[0], carry[1], wred, pick);
 }
 
 __global__ __launch_bounds__(ST) void draw_kernel(const float* __restrict__ logits, int* __restrict__ out,
@@ -699,20 +707,22 @@ __global__ __launch_bounds__(ST) void draw_kernel(const float* __restrict__ logi
 
 // ---- top-k of up to TOPK_MOST in one pass over the row
 //
-//   chunk_topk   the chunk's elements in registers; every thread's largest goes to shared memory, and the k-th largest of
-//                these 256 is a bound that at least k of the chunk's elements reach: what reaches it (about -256 ln(1 - k/256)
-//                elements where the large ones are spread) goes to the chunk's list with its index.  A chunk in which more do
+//   chunk_topk   the chunk's elements in registers; the largest of every 256th part goes to shared memory, and one of these
+//                that at least k reach (and at most (256 - k) / 16 more, ties apart) is a bound that at least k of the chunk's
+//                elements reach: what reaches it (about -256 ln(1 - k/256) elements where the large ones are spread, and less than
+//                topk_shape() expects) goes to the chunk's list with its index.  A chunk in which more do
 //                (ties at the bound: masked elements, most often) lists what lies above it and names the key it left out.
 //                Whatever the row's k largest are, ties among them included, they are in the lists if the k-th of what is
 //                listed lies above every key that a chunk left out; and what was left out does not matter if its mass is zero.
 //   row_topk     a block a row: the same bound once more over the lists' elements, then every survivor counts the larger ones
 //                (the threshold of top-k) and adds up the mass at and above itself (top-p, the same fixed point); the sums of
 //                the tiles from the kept elements alone, each lane's share in index order as tile_sum adds them (what it adds
-//                for the others is zero), and the draw.
+//                for the others is zero), and the draw, in which the drawn tile is put together from the kept elements too.
 //
-// So a row is read once, and the tile of the draw once more.  Against five passes (64 rows of 256,000, top-k 50, top-p 0.95):
-// 22 + 23 us, 103 before: the one pass takes twice its reads' time (registers allow three waves a SIMD), row_topk the latency
-// of its phases.  Rows that the lists do not settle (one that holds no number or no finite maximum, too many ties at the
+// So a row is read once.  64 rows of 256,000, top-k 50, top-p 0.95: 15 + 12 us (22 + 23 before the bound was found by counting,
+// and before all threads took part in what the survivors do; five passes over the row 103).  Back to back 8 rows take 19 us
+// (32), one 17 (25), 64 of 32,768 16 (26).  The one pass takes 1.6 times its reads' time, row_topk the latency of some twenty
+// phases, 0.5 us each, most of it for instructions that no launch before left in the CU's cache.  Rows that the lists do not settle (one that holds no number or no finite maximum, too many ties at the
 // threshold itself) are counted and collected by their one block as the kernels for any k do it.  One row of 256,000 with 1,000 elements
 // that are not masked: 34 us; with 5,120 ties at the top 158 (46 and 41 by the five passes).
 constexpr int TOPK_MOST = 200;       // beyond, the bound of 256 maxima lets too much through
@@ -734,48 +744,55 @@ __host__ inline TopkShape topk_shape(int B, int tiles, int top_k, int capg) {
   return {per, chunks, capg / chunks};
 }
 
-// The k-th largest of n <= 256 keys in shared memory (0: fewer than k of them are above 0 keys of no element); every thread
-// of the block calls it, `mine` is the key of thread tid < 256.
-__device__ __forceinline__ uint32_t kth_of_256(const uint32_t* keys, uint32_t mine, int k, uint32_t* wmin, int n_waves) {
-  uint32_t v = 0xffffffffu;
-  if (threadIdx.x < 256) {
-    int larger = 0;
-    const uint4* k4 = reinterpret_cast<const uint4*>(keys);
-#pragma unroll 8
-    for (int j = 0; j < 64; ++j) {
-      const uint4 x = k4[j];
-      larger += (x.x > mine) + (x.y > mine) + (x.z > mine) + (x.w > mine);
-    }
-    if (larger < k) v = mine;
+// A bound that at least k (1 <= k <= 256) of 256 keys in shared memory reach, and few more where the keys are spread: bit by bit
+// below what all keys have in common, by counting the lanes at and above, until k to k + (256 - k) / 16 are left, or (ties)
+// the k-th largest itself.  It is one of the keys.  One wave's work: sixteen that did the same were in each other's way and took
+// 4 us, every key against every other by four waves 2.9.
+__device__ __forceinline__ uint32_t bound_of_256(const uint32_t* keys, int k, uint32_t* largest) {
+  const uint4 v = reinterpret_cast<const uint4*>(keys)[threadIdx.x & 63];
+  auto smaller = [](uint32_t a, uint32_t b) { return min(a, b); };
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(wave_reduce(max(max(v.x, v.y), max(v.z, v.w)), [](uint32_t a, uint32_t b) { return max(a, b); }));
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(wave_reduce(min(min(v.x, v.y), min(v.z, v.w)), smaller));
+  *largest = hi;
+  if (hi == lo) return hi;
+  const int top = 31 - __builtin_clz(hi ^ lo), enough = k + (256 - k) / 16;
+  uint32_t t = hi & ~((2u << top) - 1u);                   // all keys reach it
+  for (int bit = top; bit >= 0; --bit) {
+    const uint32_t c = t | (1u << bit);
+    const int n = __popcll(__ballot(v.x >= c)) + __popcll(__ballot(v.y >= c)) + __popcll(__ballot(v.z >= c)) + __popcll(__ballot(v.w >= c));
+    if (n < k) continue;
+    t = c;
+    if (n <= enough) break;
   }
-  v = wave_reduce(v, [](uint32_t a, uint32_t b) { return min(a, b); });
-  if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = v;
-  __syncthreads();
-  for (int x = 0; x < n_waves; ++x) v = min(v, wmin[x]);
-  return v;
+  return wave_reduce(min(min(v.x >= t ? v.x : ~0u, v.y >= t ? v.y : ~0u), min(v.z >= t ? v.z : ~0u, v.w >= t ? v.w : ~0u)), smaller);
 }
 
+// 32 elements a thread, so that a CU holds all its blocks of a large step at once (with 64 and 256 threads a fourth
+// block had to wait for a first: 64 rows of 256,000 took 22 us, and take 15).
+template <int TILES>
+constexpr int topk_threads() { return TILES == 4 ? 512 : 256; }
+
 template <int VEC, int TILES>
-__global__ __launch_bounds__(SB) void chunk_topk_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t, int top_k,
+__global__ __launch_bounds__(topk_threads<TILES>(), 6) void chunk_topk_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t, int top_k,
                                                         TopkShape sh) {
-  constexpr int NE = TILES * TILE / SB;                    // elements a thread
-  __shared__ __align__(16) uint32_t keys[SB];
-  __shared__ uint32_t wmin[SB / 64];
+  constexpr int NT = topk_threads<TILES>(), NE = TILES * TILE / NT;      // threads, elements a thread
+  __shared__ __align__(16) uint32_t keys[256];
+  __shared__ uint32_t wmin[NT / 64];
   __shared__ int fill, odd;
   const int b = blockIdx.y, c = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const float* row = logits + (size_t)b * V;
   const int lo = c * TILES * TILE, hi = min(V, lo + TILES * TILE);
   if (tid == 0) fill = odd = 0;
-  auto index = [&](int e) { return VEC == 4 ? lo + ((e >> 2) * SB + tid) * 4 + (e & 3) : lo + e * SB + tid; };
+  auto index = [&](int e, int t) { return VEC == 4 ? lo + ((e >> 2) * NT + t) * 4 + (e & 3) : lo + e * NT + t; };
   float x[NE];
 #pragma unroll
   for (int e = 0; e < NE; e += 4) {
     if constexpr (VEC == 4) {
-      const float4 v = *reinterpret_cast<const float4*>(row + min(index(e), V - 4));
+      const float4 v = *reinterpret_cast<const float4*>(row + min(index(e, tid), V - 4));
       x[e] = v.x; x[e + 1] = v.y; x[e + 2] = v.z; x[e + 3] = v.w;
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[e + i] = row[min(index(e + i), V - 1)];
+      for (int i = 0; i < 4; ++i) x[e + i] = row[min(index(e + i, tid), V - 1)];
     }
   }
   uint32_t key[NE], most = 0;                              // 0: no element
@@ -787,24 +804,49 @@ __global__ __launch_bounds__(SB) void chunk_topk_kernel(const float* __restrict_
     key[e] = order_key(v);
   }
   if (hi - lo < TILES * TILE) {
+    int t = tid;
+    asm volatile("" : "+v"(t));
 #pragma unroll
-    for (int e = 0; e < NE; ++e) key[e] = index(e) < hi ? key[e] : 0u;
+    for (int e = 0; e < NE; ++e) key[e] = index(e, t) < hi ? key[e] : 0u;
   }
 #pragma unroll
   for (int e = 0; e < NE; ++e) most = max(most, key[e]);
-  keys[tid] = most;
+  constexpr int PER = NT / 256;                            // threads a maximum
+  if constexpr (PER >= 2) most = max(most, dpp_move<DPP_XOR1>(most));
+  if constexpr (PER >= 4) most = max(most, dpp_move<DPP_XOR2>(most));
+  if (tid % PER == 0) keys[tid / PER] = most;
   __syncthreads();
   if (nan) odd = 1;
-  const uint32_t bound = max(kth_of_256(keys, most, top_k, wmin, SB / 64), 1u);
-  unsigned long long* list = w.cmass + (size_t)b * w.capg + (size_t)c * sh.room;
-#pragma unroll
-  for (int e = 0; e < NE; ++e) {
-    if (key[e] >= bound) {
-      const int pos = atomicAdd(&fill, 1);
-      if (pos < sh.room) list[pos] = ((unsigned long long)key[e] << 32) | (uint32_t)index(e);
-    }
+  if (tid < 64) {
+    uint32_t largest;
+    const uint32_t from = bound_of_256(keys, top_k, &largest);
+    if (tid == 0) wmin[0] = max(from, 1u);
   }
-  __syncthreads();
+  lds_barrier();
+  const uint32_t bound = wmin[0];
+  unsigned long long* list = w.cmass + (size_t)b * w.capg + (size_t)c * sh.room;
+  // What reaches a key goes to the list: a wave counts its elements, takes their places at once and fills them in turn.
+  auto put = [&](uint32_t from) {
+    int n = 0;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) n += __popcll(__ballot(key[e] >= from));
+    int at = 0;
+    if (lane == 0 && n > 0) at = atomicAdd(&fill, n);
+    at = __builtin_amdgcn_readfirstlane(at);
+    asm volatile("" : "+v"(from));                         // (the masks of all elements are not kept: no registers for them)
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      const unsigned long long mask = __ballot(key[e] >= from);
+      if (mask == 0) continue;
+      const int pos = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+      int at_index = tid;
+      asm volatile("" : "+v"(at_index));                   // (nor their indices)
+      if (key[e] >= from && pos < sh.room) list[pos] = ((unsigned long long)key[e] << 32) | (uint32_t)index(e, at_index);
+      at += __popcll(mask);
+    }
+  };
+  put(bound);
+  lds_barrier();
   // More than there is room for (ties, most often those of masked elements, or large elements in few threads' places): what
   // lies above the bound alone, if that fits, else above the chunk's k-th largest; the ones tied with it are left out,
   // and the row is settled if its threshold lies above them.
@@ -820,7 +862,7 @@ __global__ __launch_bounds__(SB) void chunk_topk_kernel(const float* __restrict_
       if (lane == 0) wmin[tid >> 6] = (uint32_t)k;
       __syncthreads();
       k = 0;
-      for (int x = 0; x < SB / 64; ++x) k += (int)wmin[x];
+      for (int x = 0; x < NT / 64; ++x) k += (int)wmin[x];
       __syncthreads();
       return k;
     };
@@ -835,13 +877,7 @@ __global__ __launch_bounds__(SB) void chunk_topk_kernel(const float* __restrict_
     }
     if (tid == 0) fill = 0;
     __syncthreads();
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      if (key[e] > tie) {
-        const int pos = atomicAdd(&fill, 1);
-        if (pos < sh.room) list[pos] = ((unsigned long long)key[e] << 32) | (uint32_t)index(e);
-      }
-    }
+    put(tie + 1);
     __syncthreads();
     n = fill;
   }
@@ -855,60 +891,69 @@ template <int VEC>
 __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ logits, int* __restrict__ out,
                                                       const float* __restrict__ uniform, SampleWork w, int V, float inv_t, int top_k,
                                                       float top_p, TopkShape sh) {
-  __shared__ __align__(16) unsigned long long list[TOPK_LIST];       // then the tiles' sums by lane
+  __shared__ __align__(16) unsigned long long list[TOPK_LIST];       // then the tiles' sums by lane and the drawn tile
   __shared__ __align__(16) uint32_t lkey[TOPK_LEFT + 4];             // the survivors; 0 up to a multiple of four
   __shared__ __align__(16) unsigned long long lmass[TOPK_LEFT + 4];
-  __shared__ __align__(16) int lat[TOPK_LEFT], lslot[TOPK_LEFT + 4];
-  __shared__ __align__(16) uint32_t keys[256];
-  __shared__ uint32_t wmin[ST / 64];
-  __shared__ unsigned long long wsum[ST / 64];
-  __shared__ int first[TOPK_TILES + 1], n_left, last_kept, rounds, pick[2];
-  __shared__ float red[17], wred[ST / 64], tsum[TOPK_TILES], prefix[TOPK_TILES], carry[2];
+  __shared__ __align__(16) int lat[TOPK_LEFT + 4], lslot[TOPK_LEFT + 4];
+  __shared__ __align__(16) uint32_t keys[256], wmin[ST / 64];
+  __shared__ __align__(16) unsigned long long wsum[ST / 64];
+  __shared__ int n_left, last_kept, rounds, pick[2];
+  __shared__ __align__(16) float red[17], wred[ST / 64], tsum[TOPK_TILES];
+  __shared__ float carry[2];
   __shared__ int ired[ST / 64];
-  __shared__ uint32_t best, tie;
-  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ uint32_t best;
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const float* row = logits + (size_t)b * V;
   const float u = uniform[b];
+  // where the chunks' lists go, by every wave for itself: lane c has chunk c and 64 + c
   const int* counts = w.tlast + (size_t)b * w.tiles;
-  if (tid == 0) { first[0] = 0; n_left = 0; last_kept = -1; rounds = 0; best = 0; tie = 0; }
-  __syncthreads();
-  if (tid < sh.chunks) {
-    first[tid + 1] = counts[tid];
-    const uint32_t left_out = __float_as_uint(w.tsum[(size_t)b * w.tiles + tid]);
-    if (left_out) atomicMax(&tie, left_out);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int at = 0;
-    bool fine = true;
-    for (int c = 0; c < sh.chunks; ++c) {
-      const int k = first[c + 1];
-      fine = fine && k >= 0;
-      at += max(k, 0);
-      first[c + 1] = at;
+  const uint32_t* left_out = reinterpret_cast<const uint32_t*>(w.tsum + (size_t)b * w.tiles);
+  const int c0 = lane < sh.chunks ? counts[lane] : 0, c1 = 64 + lane < sh.chunks ? counts[64 + lane] : 0;
+  const uint32_t t0 = lane < sh.chunks ? left_out[lane] : 0u, t1 = 64 + lane < sh.chunks ? left_out[64 + lane] : 0u;
+  if (tid < TOPK_TILES) tsum[tid] = 0.f;
+  if (tid == 0) { n_left = 0; last_kept = -1; rounds = 0; best = 0; pick[0] = -1; pick[1] = -1; carry[1] = 0.f; }
+  const uint32_t tie = wave_reduce(max(t0, t1), [](uint32_t a, uint32_t b) { return max(a, b); });
+  bool settled = !__any(c0 < 0 || c1 < 0);
+  auto scan = [&](int v) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int before = __shfl_up(v, o, 64);
+      v += lane >= o ? before : 0;
     }
-    if (!fine) first[sh.chunks] = -1;
-  }
-  __syncthreads();
-  const int n = first[sh.chunks];
-  bool settled = n >= 1 && n <= TOPK_LIST;
+    return v;
+  };
+  const int s0 = scan(max(c0, 0)), s1 = sh.chunks > 64 ? scan(max(c1, 0)) : 0;
+  const int n0 = __builtin_amdgcn_readlane(s0, 63), n = n0 + __builtin_amdgcn_readlane(s1, 63);
+  settled = settled && n >= 1 && n <= TOPK_LIST;
   uint32_t key_m = 0;
   if (settled) {
-    for (int c = wave; c < sh.chunks; c += ST / 64) {
-      const unsigned long long* src = w.cmass + (size_t)b * w.capg + (size_t)c * sh.room;
-      for (int i = first[c] + lane; i < first[c + 1]; i += 64) list[i] = src[i - first[c]];
-    }
-    __syncthreads();
-    // the bound again: the largest of every four threads' elements, of these the k-th largest
+    // the lists' elements, several waves a chunk where there are few; the bound again: the largest of every four threads'
+    // elements, of these the k-th largest
+    constexpr int NW = ST / 64;
+    const int share = max(NW / sh.chunks, 1), sub = wave % share;
     uint32_t most = 0;
-    for (int i = tid; i < n; i += ST) most = max(most, (uint32_t)(list[i] >> 32));
-    most = max(most, (uint32_t)__shfl_xor(most, 1, 64));
-    most = max(most, (uint32_t)__shfl_xor(most, 2, 64));
+    for (int c = wave / share; c < sh.chunks; c += NW / share) {
+      const int end = c < 64 ? __builtin_amdgcn_readlane(s0, c) : n0 + __builtin_amdgcn_readlane(s1, c - 64);
+      const int len = c < 64 ? __builtin_amdgcn_readlane(c0, c) : __builtin_amdgcn_readlane(c1, c - 64);
+      const unsigned long long* src = w.cmass + (size_t)b * w.capg + (size_t)c * sh.room;
+      for (int i = sub * 64 + lane; i < len; i += share * 64) {
+        const unsigned long long el = src[i];
+        list[end - len + i] = el;
+        most = max(most, (uint32_t)(el >> 32));
+      }
+    }
+    most = max(most, dpp_move<DPP_XOR1>(most));
+    most = max(most, dpp_move<DPP_XOR2>(most));
     if ((tid & 3) == 0) keys[tid >> 2] = most;
     __syncthreads();
-    const uint32_t bound = kth_of_256(keys, tid < 256 ? keys[tid] : 0u, top_k, wmin, ST / 64);
-    for (int x = 0; x < 256; x += 64) key_m = max(key_m, keys[x + lane]);
-    key_m = wave_reduce(key_m, [](uint32_t a, uint32_t b) { return max(a, b); });
+    if (wave == 0) {
+      uint32_t largest;
+      const uint32_t from = bound_of_256(keys, top_k, &largest);
+      if (lane == 0) { wmin[0] = from; wmin[1] = largest; }
+    }
+    __syncthreads();
+    const uint32_t bound = wmin[0];
+    key_m = wmin[1];
     for (int i = tid; i < n; i += ST)
       if ((uint32_t)(list[i] >> 32) >= bound) {
         const int pos = atomicAdd(&n_left, 1);
@@ -920,36 +965,49 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
     __syncthreads();
     settled = n_left <= TOPK_LEFT && fabsf(key_value(key_m)) < INFINITY;
   }
+  // 2^split threads a survivor look at the others, so that all 1,024 have work (a thread a survivor: of the 23 us that this
+  // kernel took 12 went into a few waves' loops over the others)
   float m = 0.f;
-  int nl = 0, quads = 0, at = 0;
+  int nl = 0, quads = 0, at = 0, split = 0, who = 0, part = 0;
   uint32_t key = 0, thr = 0xffffffffu;
   unsigned long long z = 0;
-  bool kept_k = false;
+  bool kept_k = false, first = false;                      // first: of the threads of a survivor
+  auto all_parts = [&](uint32_t v) {                       // their sum, in all of them
+    if (split >= 1) v += dpp_move<DPP_XOR1>(v);
+    if (split >= 2) v += dpp_move<DPP_XOR2>(v);
+    if (split >= 3) v += dpp_move<DPP_HALF_MIRROR>(v);     // (the quads of 8 lanes are uniform by now)
+    return v;
+  };
   if (settled) {
     m = key_value(key_m);
     nl = n_left;
     quads = (nl + 3) >> 2;
-    key = tid < nl ? lkey[tid] : 0u;
-    at = tid < nl ? lat[tid] : 0;
-    if (tid >= nl && tid < quads * 4) { lkey[tid] = 0; lmass[tid] = 0; lslot[tid] = -1; }
+    split = nl <= ST / 8 ? 3 : nl <= ST / 4 ? 2 : nl <= ST / 2 ? 1 : 0;
+    who = tid >> split;
+    part = tid & ((1 << split) - 1);
+    first = part == 0 && who < nl;
+    key = who < nl ? lkey[who] : 0u;
+    at = who < nl ? lat[who] : 0;
+    if (tid >= nl && tid < quads * 4) { lkey[tid] = 0; lmass[tid] = 0; lslot[tid] = -1; lat[tid] = 0; }
     __syncthreads();
-    int larger = 0;
-    if (tid < nl) {
+    uint32_t larger = 0;
+    if (who < nl) {
 #pragma unroll 4
-      for (int j = 0; j < quads; ++j) {
+      for (int j = part; j < quads; j += 1 << split) {
         const uint4 o = reinterpret_cast<const uint4*>(lkey)[j];
         larger += (o.x > key) + (o.y > key) + (o.z > key) + (o.w > key);
       }
     }
-    kept_k = tid < nl && larger < top_k;
+    larger = all_parts(larger);
+    kept_k = who < nl && (int)larger < top_k;
     if (kept_k) thr = key;
     thr = wave_reduce(thr, [](uint32_t a, uint32_t b) { return min(a, b); });
-    const unsigned long long mass = kept_k ? fixed_mass(key_value(key), m) : 0ull;
+    const unsigned long long mass = kept_k && first ? fixed_mass(key_value(key), m) : 0ull;
     const unsigned long long z_wave = wave_sum_u64(mass);
-    if (tid < nl) lmass[tid] = mass;
-    __syncthreads();                                       // (the first bound's minima have been read)
+    if (first) lmass[who] = mass;
     if (lane == 0) { wmin[wave] = thr; wsum[wave] = z_wave; }
     __syncthreads();
+#pragma unroll
     for (int x = 0; x < ST / 64; ++x) { thr = min(thr, wmin[x]); z += wsum[x]; }
     // what was left out is not among the k largest, or its mass is zero
     settled = tie == 0 || (nl >= top_k && thr > tie) || expf(key_value(tie) - m) == 0.f;
@@ -966,75 +1024,86 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
     draw_from_tiles(row, out, u, w, b, V, inv_t, m, thr, wred);
     return;
   }
+  float* lanes = reinterpret_cast<float*>(list);           // [tiles][64]: the tiles' sums by lane, then the drawn tile's elements
+  static_assert(sizeof(list) >= (TOPK_TILES * 64 + TILE) * sizeof(float) && TILE == 4 * ST, "both lie where the lists were");
+  float4* drawn = reinterpret_cast<float4*>(lanes + TOPK_TILES * 64);
+  for (int i = tid; i < w.tiles * 16; i += ST) reinterpret_cast<float4*>(lanes)[i] = float4{0.f, 0.f, 0.f, 0.f};
+  drawn[tid] = float4{0.f, 0.f, 0.f, 0.f};
   if (top_p < 1.f) {
     // the largest key at and above which lies more than the target
     const unsigned long long target = (unsigned long long)((double)top_p * (double)z);
     unsigned long long above = 0;
     if (kept_k) {
 #pragma unroll 2
-      for (int j = 0; j < quads; ++j) {
+      for (int j = part; j < quads; j += 1 << split) {
         const uint4 o = reinterpret_cast<const uint4*>(lkey)[j];
         const ulonglong2 m0 = reinterpret_cast<const ulonglong2*>(lmass)[2 * j], m1 = reinterpret_cast<const ulonglong2*>(lmass)[2 * j + 1];
         above += (o.x >= key ? m0.x : 0ull) + (o.y >= key ? m0.y : 0ull) + (o.z >= key ? m1.x : 0ull) + (o.w >= key ? m1.y : 0ull);
       }
     }
-    if (kept_k && above > target) atomicMax(&best, key);
+    // (three pieces of 21 bits and one more: their sums over eight parts stay below 32 bits)
+    unsigned long long sum = 0;
+#pragma unroll
+    for (int p = 0; p < 64; p += 21) sum += (unsigned long long)all_parts((uint32_t)(above >> p) & 0x1fffffu) << p;
+    if (kept_k && first && sum > target) atomicMax(&best, key);
     __syncthreads();
     thr = best;
   }
   // the tiles' sums: a lane of tile_sum adds its elements in index order
-  float* lanes = reinterpret_cast<float*>(list);           // [tiles][64]
-  for (int i = tid; i < w.tiles * 64; i += ST) lanes[i] = 0.f;
-  const bool kept = tid < nl && key >= thr;
+  const bool kept = who < nl && key >= thr;
   const float e = kept ? expf(key_value(key) - m) : 0.f;
   const int slot = (at / TILE) * 64 + (VEC == 4 ? (at >> 2) & 63 : at & 63);
-  if (tid < nl) lslot[tid] = kept ? slot : -1;
+  if (first) lslot[who] = kept ? slot : -1;
   __syncthreads();
-  int turn = 0;                                            // kept elements of the same lane before this one
+  uint32_t turn = 0;                                       // kept elements of the same lane before this one
   if (kept) {
-#pragma unroll 4
-    for (int j = 0; j < quads; ++j) {
-      const int4 o = reinterpret_cast<const int4*>(lslot)[j];
-      if (o.x == slot) turn += lat[4 * j] < at;
-      if (o.y == slot) turn += lat[4 * j + 1] < at;
-      if (o.z == slot) turn += lat[4 * j + 2] < at;
-      if (o.w == slot) turn += lat[4 * j + 3] < at;
+#pragma unroll 2
+    for (int j = part; j < quads; j += 1 << split) {
+      const int4 o = reinterpret_cast<const int4*>(lslot)[j], i = reinterpret_cast<const int4*>(lat)[j];
+      turn += ((o.x == slot) & (i.x < at)) + ((o.y == slot) & (i.y < at)) + ((o.z == slot) & (i.z < at)) + ((o.w == slot) & (i.w < at));
     }
+  }
+  turn = all_parts(turn);
+  if (kept && first) {
     if (e > 0.f) atomicMax(&last_kept, at);
-    atomicMax(&rounds, turn + 1);
+    atomicMax(&rounds, (int)turn + 1);
   }
   __syncthreads();
   const int n_rounds = rounds;
   for (int r = 0; r < n_rounds; ++r) {
-    if (kept && turn == r) lanes[slot] += e;
+    if (kept && first && (int)turn == r) lanes[slot] += e;
     __syncthreads();
   }
   for (int t = wave; t < w.tiles; t += ST / 64) {
     const float s = wave_sum(lanes[t * 64 + lane]);
     if (lane == 0) tsum[t] = s;
   }
-  if (tid == 0) { pick[0] = -1; pick[1] = -1; carry[1] = 0.f; }
   __syncthreads();
-  // their running sums, in order (a wave: what a lane reads of the others costs no trip through memory)
-  if (wave == 0) {
-    float acc = 0.f, p0 = 0.f, p1 = 0.f;
-    const float s0 = lane < w.tiles ? tsum[lane] : 0.f, s1 = 64 + lane < w.tiles ? tsum[min(64 + lane, w.tiles - 1)] : 0.f;
-    for (int t = 0; t < w.tiles; ++t) {
-      acc += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t < 64 ? s0 : s1), t & 63));
-      if (lane == (t & 63)) { if (t < 64) p0 = acc; else p1 = acc; }
+  // their running sums in order: every thread adds up what lies before its tile and zeros, all in registers at once
+  float total = 0.f, before = 0.f;
+  const int mine = tid & (TOPK_TILES - 1);
+#pragma unroll
+  for (int t0 = 0; t0 < TOPK_TILES; t0 += 64) {
+    if (t0 >= w.tiles) break;
+    float4 s[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) s[t] = reinterpret_cast<const float4*>(tsum + t0)[t];
+#pragma unroll
+    for (int t = 0; t < 64; ++t) {
+      const float x = reinterpret_cast<const float*>(s)[t];
+      total += x;
+      before += t0 + t < mine ? x : 0.f;
     }
-    if (lane < w.tiles) prefix[lane] = p0;
-    if (64 + lane < w.tiles) prefix[64 + lane] = p1;
-    if (lane == 0) carry[0] = acc;
   }
+  const float target = u * total;
+  if (tid < w.tiles && target >= before && target < before + tsum[tid]) { pick[0] = tid; carry[1] = before; }      // at most one tile
   __syncthreads();
-  const float target = u * carry[0];
-  if (tid < w.tiles) {
-    const float lo = tid == 0 ? 0.f : prefix[tid - 1];
-    if (target >= lo && target < prefix[tid]) { pick[0] = tid; carry[1] = lo; }      // at most one tile
-  }
+  const int tile = pick[0];
+  if (kept && first && at / TILE == tile) reinterpret_cast<float*>(drawn)[at & (TILE - 1)] = e;
   __syncthreads();
-  draw_in_tile(row, out, b, V, inv_t, m, thr, pick[0], last_kept, target, carry[1], wred, pick);
+  const float4 own = drawn[tid];
+  const float ex[4] = {own.x, own.y, own.z, own.w};
+  draw_in_tile(ex, out, b, tile, last_kept, target, carry[1], wred, pick);
 }
 
 // How long a row's list may be: 32,768 candidates, fewer (down to what fits shared memory) when the lists of
@@ -1180,9 +1249,9 @@ extern "C" int alice_sample(const float* logits, int* out, const float* uniform,
 #define GO(VEC)                                                                                             \
   do {                                                                                                      \
     const dim3 grid(sh.chunks, B);                                                                          \
-    if (sh.tiles == 4) chunk_topk_kernel<VEC, 4><<<grid, SB, 0, stream>>>(logits, w, V, inv_t, top_k, sh);  \
-    else if (sh.tiles == 2) chunk_topk_kernel<VEC, 2><<<grid, SB, 0, stream>>>(logits, w, V, inv_t, top_k, sh); \
-    else chunk_topk_kernel<VEC, 1><<<grid, SB, 0, stream>>>(logits, w, V, inv_t, top_k, sh);                \
+    if (sh.tiles == 4) chunk_topk_kernel<VEC, 4><<<grid, topk_threads<4>(), 0, stream>>>(logits, w, V, inv_t, top_k, sh);  \
+    else if (sh.tiles == 2) chunk_topk_kernel<VEC, 2><<<grid, topk_threads<2>(), 0, stream>>>(logits, w, V, inv_t, top_k, sh); \
+    else chunk_topk_kernel<VEC, 1><<<grid, topk_threads<1>(), 0, stream>>>(logits, w, V, inv_t, top_k, sh);                \
     ALICE_LAUNCH_CHECK();                                                                                   \
     row_topk_kernel<VEC><<<B, ST, 0, stream>>>(logits, out, uniform, w, V, inv_t, top_k, top_p, sh);        \
   } while (0)

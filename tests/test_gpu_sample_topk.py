@@ -76,3 +76,19 @@ def test_masked_rows_are_settled_without_their_masked_elements(mask, B, V):
             got = ops.sample(rows, u.to(DEV), 0.8, top_k, 0.95).tolist()
             assert set(got) <= set(keep.tolist()) and got[:4] == check_samples(rows[:4], u[:4], 0.8, top_k, 0.95)
             assert min(time(rows, u.to(DEV), top_k) for _ in range(3)) < 8 * time(base, u.to(DEV), top_k), (len(keep), top_k)
+
+
+@pytest.mark.parametrize("ties", [100, 128, 129, 257, 513, 1000, 1030])
+@pytest.mark.parametrize("V", [40000, 300001])
+def test_as_many_tied_at_the_threshold_as_change_the_shares_of_a_survivor(ties, V):
+    """The rows' block gives a survivor 8, 4, 2 or 1 of its threads; ties at the threshold are all kept, many of them in one lane's
+    share of a tile."""
+    g = torch.Generator().manual_seed(ties)
+    logits = rnd(4, V, seed=ties, scale=0.5).clamp_(max=1.9)
+    logits[0, torch.randperm(V, generator=g)[:ties].to(DEV)] = 3.0
+    logits[1, 4000:4000 + ties] = 3.0
+    logits[2, torch.arange(ties, device=DEV) * 8] = 3.0
+    logits[3, V - ties:] = 3.0
+    logits[:, 17] = 4.0
+    for top_k, top_p in ((2, 1.0), (20, 0.6)):
+        check_samples(logits, torch.rand(4, generator=g), 0.7, top_k, top_p)
