@@ -377,6 +377,12 @@ int alice_argmax_static(const float* logits, int* out, int B, int V, hipStream_t
 long alice_sample_workspace(int B, int V);
 int alice_sample(const float* logits, int* out, const float* uniform, void* work, int B, int V, float temperature,
                  int top_k, float top_p, hipStream_t stream);
+// The same with the draws[i]-th uniform number of request requests[i] under `seed` for row i (host arrays; the stream of
+// numbers of sampling/sampler.py), for at most ALICE_SAMPLE_HELD_ROWS rows.
+enum { ALICE_SAMPLE_HELD_ROWS = 256 };
+int alice_sample_drawn(const float* logits, int* out, unsigned long long seed, const unsigned long long* requests,
+                       const unsigned long long* draws, void* work, int B, int V, float temperature, int top_k, float top_p,
+                       hipStream_t stream);
 
 #ifdef __cplusplus
 }

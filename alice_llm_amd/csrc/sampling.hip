@@ -697,9 +697,16 @@ __device__ __forceinline__ void draw_from_tiles(const float* __restrict__ row, i
   draw_in_tile(e, out, b, tile, pick[1], u * carry[0], carry[1], wred, pick);
 }
 
+// The rows' uniform numbers as the launch's own argument: no copy to the device, no buffer that has to outlive the call.
+struct HeldUniforms {
+  float v[ALICE_SAMPLE_HELD_ROWS];
+  __device__ __forceinline__ float operator[](int b) const { return v[b]; }
+};
+
+// Uniforms: const float* in device memory, or HeldUniforms.
+template <class Uniforms>
 __global__ __launch_bounds__(ST) void draw_kernel(const float* __restrict__ logits, int* __restrict__ out,
-                                                  const float* __restrict__ uniform, SampleWork w, int V, float inv_t,
-                                                  int filtered) {
+                                                  const Uniforms uniform, SampleWork w, int V, float inv_t, int filtered) {
   __shared__ float wred[ST / 64];
   const int b = blockIdx.x;
   draw_from_tiles(logits + (size_t)b * V, out, uniform[b], w, b, V, inv_t, row_max(w, b), filtered ? w.thr[b] : 0u, wred);
@@ -887,9 +894,9 @@ __global__ __launch_bounds__(topk_threads<TILES>(), 6) void chunk_topk_kernel(co
   }
 }
 
-template <int VEC>
+template <int VEC, class Uniforms>
 __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ logits, int* __restrict__ out,
-                                                      const float* __restrict__ uniform, SampleWork w, int V, float inv_t, int top_k,
+                                                      const Uniforms uniform, SampleWork w, int V, float inv_t, int top_k,
                                                       float top_p, TopkShape sh) {
   __shared__ __align__(16) unsigned long long list[TOPK_LIST];       // then the tiles' sums by lane and the drawn tile
   __shared__ __align__(16) uint32_t lkey[TOPK_LEFT + 4];             // the survivors; 0 up to a multiple of four
@@ -1219,8 +1226,10 @@ extern "C" long alice_sample_workspace(int B, int V) {
   return rows * chunks * 2 * (1 + NMC) + rows * capg * 2 + rows * chunks + rows * chunks * NCUT + rows * capg + rows + rows * tiles * 2 + 16;
 }
 
-extern "C" int alice_sample(const float* logits, int* out, const float* uniform, void* work, int B, int V,
-                            float temperature, int top_k, float top_p, hipStream_t stream) {
+namespace {
+template <class Uniforms>
+int sample_launch(const float* logits, int* out, const Uniforms& uniform, void* work, int B, int V, float temperature, int top_k,
+                  float top_p, hipStream_t stream) {
   ALICE_CHECK(B >= 0 && V >= 1, "sample: bad sizes B=%d V=%d", B, V);
   ALICE_CHECK(temperature > 0.f, "sample: temperature must be positive (use argmax for greedy)");
   ALICE_CHECK(top_k >= 0 && top_p > 0.f, "sample: top_k must not be negative and top_p must be positive");
@@ -1278,4 +1287,34 @@ extern "C" int alice_sample(const float* logits, int* out, const float* uniform,
   draw_kernel<<<B, ST, 0, stream>>>(logits, out, uniform, w, V, inv_t, filtered);
   ALICE_LAUNCH_CHECK();
   return 0;
+}
+
+uint64_t splitmix64(uint64_t x) {
+  x += 0x9E3779B97F4A7C15ull;
+  uint64_t z = x;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
+}  // namespace
+
+extern "C" int alice_sample(const float* logits, int* out, const float* uniform, void* work, int B, int V,
+                            float temperature, int top_k, float top_p, hipStream_t stream) {
+  return sample_launch(logits, out, uniform, work, B, V, temperature, top_k, top_p, stream);
+}
+
+// The same for at most ALICE_SAMPLE_HELD_ROWS rows, row i with the draws[i]-th uniform number of request requests[i] under
+// `seed` (host arrays; read before the call returns).  Against numbers made as an array, copied through a pinned buffer and
+// read from device memory, 64 rows of 256,000: the host's part of a call 36 -> 12 us, and a copy fewer on the stream.
+extern "C" int alice_sample_drawn(const float* logits, int* out, unsigned long long seed, const unsigned long long* requests,
+                                  const unsigned long long* draws, void* work, int B, int V, float temperature, int top_k, float top_p,
+                                  hipStream_t stream) {
+  ALICE_CHECK(B >= 0 && B <= ALICE_SAMPLE_HELD_ROWS, "sample: %d rows are more than a launch holds the uniform numbers of", B);
+  ALICE_CHECK(B == 0 || (requests && draws), "sample: the rows' requests or draws are missing");
+  HeldUniforms u = {};
+  for (int i = 0; i < B; ++i) {
+    const uint64_t row = splitmix64(seed ^ (requests[i] * 0xD1B54A32D192ED03ull));
+    u.v[i] = (float)(splitmix64(row + draws[i]) >> 40) / (float)(1 << 24);             // 24 bits: exact
+  }
+  return sample_launch(logits, out, u, work, B, V, temperature, top_k, top_p, stream);
 }

@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+from array import array
 from typing import Optional
 
 import torch
@@ -108,6 +109,7 @@ def _declare(lib) -> None:
         "alice_argmax_chunks": [I, I],
         "alice_sample_workspace": [I, I],
         "alice_sample": [P, P, P, P, I, I, F, I, F, P],
+        "alice_sample_drawn": [P, P, ctypes.c_ulonglong, P, P, P, I, I, F, I, F, P],
     }
     for name, args in sigs.items():
         fn = getattr(lib, name)
@@ -1826,6 +1828,14 @@ def sample(logits: torch.Tensor, uniform: torch.Tensor, temperature: float, top_
     if out is None:
         out = torch.empty((B,), dtype=torch.int32, device=logits.device)
     _dev(out, "out", torch.int32, (B,))
+    work = _sample_workspace(logits)
+    _call("alice_sample", logits.data_ptr(), out.data_ptr(), uniform.data_ptr(), work.data_ptr(), B, V,
+          float(temperature), int(top_k), float(top_p), _stream())
+    return out
+
+
+def _sample_workspace(logits: torch.Tensor) -> torch.Tensor:
+    B, V = logits.shape
     key = (logits.device, B, V)
     work = _sample_work.get(key)
     if work is None:
@@ -1833,6 +1843,21 @@ def sample(logits: torch.Tensor, uniform: torch.Tensor, temperature: float, top_
             _sample_work.clear()
         work = _sample_work[key] = torch.empty((library().alice_sample_workspace(B, V) + 1) // 2, dtype=torch.int64,
                                                device=logits.device)
-    _call("alice_sample", logits.data_ptr(), out.data_ptr(), uniform.data_ptr(), work.data_ptr(), B, V,
-          float(temperature), int(top_k), float(top_p), _stream())
+    return work
+
+
+SAMPLE_HELD_ROWS = 256           # ALICE_SAMPLE_HELD_ROWS
+
+
+def sample_drawn(logits: torch.Tensor, seed: int, requests: array, draws: array, temperature: float, top_k: int = 0,
+                 top_p: float = 1.0) -> torch.Tensor:
+    """sample() of at most SAMPLE_HELD_ROWS rows whose uniform numbers the launch makes itself: row i takes the draws[i]-th of
+    request requests[i] under `seed` (arrays of unsigned 64-bit integers on the host)."""
+    _dev(logits, "logits", torch.float32)
+    B, V = logits.shape
+    if len(requests) != B or len(draws) != B or requests.typecode != "Q" or draws.typecode != "Q":
+        raise HipLibraryError(f"requests and draws must be arrays of {B} unsigned 64-bit integers")
+    out = torch.empty((B,), dtype=torch.int32, device=logits.device)
+    _call("alice_sample_drawn", logits.data_ptr(), out.data_ptr(), seed & 0xFFFFFFFFFFFFFFFF, requests.buffer_info()[0],
+          draws.buffer_info()[0], _sample_workspace(logits).data_ptr(), B, V, float(temperature), int(top_k), float(top_p), _stream())
     return out

@@ -1,10 +1,12 @@
 """Top-k of up to 200 in one pass over the row: against the plain sampler, at the edges of chunks, tiles and lists."""
 import math
+import random
 
 import pytest
 import torch
 
 from alice_llm_amd.hip import ops
+from alice_llm_amd.sampling.sampler import Sampler, uniforms
 from test_gpu_kernels import DEV, check_samples, rnd
 
 pytestmark = pytest.mark.gpu
@@ -92,3 +94,22 @@ def test_as_many_tied_at_the_threshold_as_change_the_shares_of_a_survivor(ties, 
     logits[:, 17] = 4.0
     for top_k, top_p in ((2, 1.0), (20, 0.6)):
         check_samples(logits, torch.rand(4, generator=g), 0.7, top_k, top_p)
+
+
+@pytest.mark.parametrize("n", [1, 30, 256, 257])
+@pytest.mark.parametrize("seed", [0, -3, 2 ** 70 + 5])
+def test_uniform_numbers_made_by_the_launch_are_those_of_the_sampler(n, seed):
+    """Rows whose numbers the launch makes itself, and those that go the other way (many rows, numbers of another type or below 0),
+    draw as they do with the sampler's own numbers."""
+    rng = random.Random(n)
+    logits = rnd(n, 5000, seed=n)
+    draws = [rng.randrange(10000) for _ in range(n)]
+    for requests in ([rng.randrange(2 ** 64) for _ in range(n)], [-1] * n, [2 ** 64 + 3] * n, [True] * n):
+        u = uniforms(seed, requests, draws).to(DEV)
+        for top_k, top_p in ((0, 1.0), (50, 0.9), (0, 0.9)):
+            assert Sampler(0.9, top_k, top_p, seed=seed)(logits, requests, draws).tolist() == ops.sample(logits, u, 0.9, top_k, top_p).tolist()
+    if n > 1:
+        with pytest.raises(ops.HipLibraryError):
+            Sampler(0.9, seed=seed)(logits, [1] * (n - 1), [1] * (n - 1))
+    with pytest.raises(TypeError):
+        Sampler(0.9, seed=seed)(logits, [1.5] * n, draws)
