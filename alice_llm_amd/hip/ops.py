@@ -1643,8 +1643,11 @@ def attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, out: 
             raise HipLibraryError("the matrix-core attention kernels take no score bias: lay the cache out row-major")
         nKV = k_pool.shape[1]
         if ctx.is_decode and num_heads // nKV <= 16:
+            # (split as a captured step of these sequences is, so that eager and captured steps add in one order)
+            splits = decode_attention_splits(getattr(ctx, "rounded_seqs", 0) or q.shape[0], nKV,
+                                             getattr(ctx, "rounded_context", 0) or ctx.max_context, window, k_pool.shape[3])
             res = attention_decode(q, k_pool, v_pool, out, ctx.context_lens, block_table, num_heads=num_heads,
-                                   max_context=ctx.max_context, scale=scale, softcap=softcap, window=window,
+                                   max_context=ctx.max_context, scale=scale, softcap=softcap, window=window, splits=splits,
                                    out_layout=out_layout, gate=gate, sink=sink)
             if gate is not None and res[2]:
                 return                                         # gated where the key splits were combined

@@ -248,7 +248,9 @@ class Attention(Part):
         # splits itself (one kernel fewer a layer).
         if (ctx.is_decode and self.kv_layout == ops.KV_FRAGMENT and self.o.layout == ops.LAYOUT_FRAG16
                 and not self.n_gate and self.nH // self.nKV <= 16 and getattr(ctx, "fragment_activations", False)):
-            splits = ops.decode_attention_splits(T, self.nKV, ctx.max_context, self.window, self.d)
+            # (of the sizes that a captured step of these sequences has, so that eager and captured steps add in one order)
+            splits = ops.decode_attention_splits(getattr(ctx, "rounded_seqs", 0) or T, self.nKV,
+                                                 getattr(ctx, "rounded_context", 0) or ctx.max_context, self.window, self.d)
             slices = ops.linear_parts_slices(T, self.o.n, self.nH, self.d, splits) if splits > 1 else 0
             if slices > 0:
                 parts, _ = ops.attention_decode(q, cache.k, cache.v, None, ctx.context_lens, cache.block_table,
