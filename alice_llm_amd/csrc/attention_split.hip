@@ -2,21 +2,25 @@
 // alice_attention_masked, the keys split over blocks: 32-bit arithmetic on operands of either dtype (the decode kernel
 // of the mixers that the matrix-core decode kernel does not take, and of the true 32-bit path).
 //
-// A block takes one token, one kv head and one run of 256 visible keys, a thread one key: it has the whole key row
-// on its way from memory at once (16-byte loads), and scores it against every query head of the kv head's group,
-// whose queries lie in LDS; the key row is read once for the group.  The block's maximum and sum a head come from
-// two barriers; then the threads turn to the values: a thread owns 16 bytes of the value row's width for a share of
-// the keys, with one accumulator set a head, the shares meet by lane swaps and through LDS.  With per-value-head
-// outputs the second phase runs once for every kv head's values.  Each block leaves (maximum, sum, unnormalised
-// output) per head; attn_split_combine_kernel merges the runs in their order, adds the sink to the denominator,
-// turns the output back where the values were cached turned, applies gate and factor, and writes the result (or
-// the per-value-head outputs in float32 for the mix of the heads that follows).
+// A block takes one token, one kv head and one run of 256 visible keys, a wave 32 of them.  A key row is read by as many lanes as
+// it has pieces of 16 bytes, so that a wave's load covers whole rows (a lane a row, each load touching 64 lines of which it used
+// 16 bytes, moved them several times); a lane holds its piece of the group's queries in registers, its partial products meet
+// by lane moves, and the key row serves the whole group.  The block's maximum and sum a head come from two barriers; then the
+// threads turn to the values: a thread owns 16 bytes of the value row's width for a share of the keys, with one accumulator set
+// a head, eight loads on their way at a time and the first eight asked for before the scores; the shares meet by lane
+// moves and through LDS, four heads at a time.  With per-value-head outputs the second phase runs once for every kv head's values.
+// Each block leaves (maximum, sum, unnormalised output) per head; attn_split_combine_kernel merges the runs in their order, adds the
+// sink to the denominator, turns the output back where the values were cached turned, applies gate and factor, and writes the
+// result (or the per-value-head outputs in float32 for the mix of the heads that follows).
+// Eight sequences of 500 to 1,500 keys, 16 heads on 4 kv heads of 128 in bfloat16: 25 us before, 12 now, of which reading is 3:
+// what bounds it is the chain of waits (place, key, score, maximum, sum, value), one block on a CU.
 #include "common.h"
 #include "alice_hip.h"
 
 namespace {
 
 constexpr int KEYS = 256;
+constexpr int WAVES = 8, NT = 64 * WAVES, WKEYS = KEYS / WAVES;      // of a block; keys a wave scores
 
 struct SplitArgs {
   const int* positions;
@@ -43,90 +47,184 @@ template <> __device__ __forceinline__ void unpack16<bf16_t>(const uint4& w, flo
   }
 }
 
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) { return __uint_as_float(dpp_move<CTRL>(__float_as_uint(v))); }
+// v and the value of the lane 16 (32) away, added
+__device__ __forceinline__ float sum_over_16(float v) {
+  auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+}
+__device__ __forceinline__ float sum_over_32(float v) {
+  auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+}
+
+// (128 registers let a second block work while one waits; the widest groups need more)
 template <typename T, int PER>
-__global__ __launch_bounds__(256) void attn_split_kernel(const T* __restrict__ q, const T* __restrict__ k_pool,
-                                                         const T* __restrict__ v_pool, SplitArgs a) {
+__global__ __launch_bounds__(NT, PER <= 8 ? 4 : 2) void attn_split_kernel(const T* __restrict__ q, const T* __restrict__ k_pool,
+                                                            const T* __restrict__ v_pool, SplitArgs a) {
   constexpr bool FULL = sizeof(T) == 4;
   constexpr int VEC = 16 / sizeof(T);
-  __shared__ __align__(16) float qs[PER][256];
+  constexpr int HG = PER < 4 ? PER : 4;               // heads that meet in LDS at a time
+  constexpr int UK = PER >= 8 ? 4 : 8, UV = UK;       // loads of keys, of values on their way at a time
+  constexpr int OWN = PER >= 4 ? PER / 4 : 1;         // heads of a key whose sums a lane ends up with
   __shared__ float ps[PER][KEYS];
   __shared__ int rows_of[KEYS];                       // the row of each of the block's keys in kv head 0's part of its page
-  __shared__ float wred[4][PER];
-  __shared__ __align__(16) float ored[4][256];
+  __shared__ float wred[WAVES][PER];
+  __shared__ __align__(16) float ored[WAVES][HG][256];
 
-  const int t = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int t = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int d = a.d, dv = a.dv, per = a.nH / a.nKV, h0 = kvh * per;
+  const int n_vh = a.value_heads > 0 ? a.value_heads : 1;
   const int pos = a.positions[t];
   const int* bt = a.block_table + (size_t)a.seq_of_token[t] * a.bt_stride;
   const int start = a.chunk > 0 ? (pos / a.chunk) * a.chunk : (a.window > 0 ? max(0, pos + 1 - a.window) : 0);
   const int n_first = (a.keep_first > 0 && a.window > 0 && a.chunk == 0) ? min(a.keep_first, start) : 0;
   const int n_keys = n_first + pos + 1 - start;
   const int v0 = split * KEYS, nk = max(0, min(KEYS, n_keys - v0));
-
-  // the group's queries (rows beyond the group stay zero)
-  for (int i = tid; i < PER * d; i += 256) {
-    const int hh = i / d, e = i % d;
-    qs[hh][e] = hh < per ? load_f32(q + ((size_t)t * a.nH + h0 + hh) * d, e) : 0.f;
+  if (nk == 0) {                                      // a run behind this token's keys
+    for (int i = tid; i < per; i += NT) {
+      float* ml = a.part_ml + (((size_t)t * a.nH + h0 + i) * a.n_splits + split) * 2;
+      ml[0] = -INFINITY;
+      ml[1] = 0.f;
+    }
+    for (int i = tid; i < per * n_vh * dv; i += NT)
+      a.part_o[(((size_t)t * a.nH + h0) * n_vh + i / dv) * a.n_splits * dv + (size_t)split * dv + i % dv] = 0.f;
+    return;
   }
   // this thread's key
   const bool has = tid < nk;
   const int vi = v0 + tid;
   const int kp = has ? (vi < n_first ? vi : start + (vi - n_first)) : 0;
-  const int row0 = has ? bt[kp / a.page_size] * a.nKV * a.page_size + kp % a.page_size : 0;
-  rows_of[tid] = row0;
+  if (has) rows_of[tid] = bt[kp / a.page_size] * a.nKV * a.page_size + kp % a.page_size;
+  // this lane's piece of the group's queries (zero beyond the group and beside the row)
+  const int EK = d / VEC;
+  int row_log = 2;                                    // lanes a row: a power of two, at least 4
+  while ((1 << row_log) < EK) ++row_log;
+  const int piece = lane & ((1 << row_log) - 1), key_of = lane >> row_log, KL = 64 >> row_log;
+  const bool in_row = piece < EK;
+  const int k_at = min(piece, EK - 1) * VEC;
+  float qf[PER][VEC];
+#pragma unroll
+  for (int hh = 0; hh < PER; ++hh) {
+    const uint4 w = *reinterpret_cast<const uint4*>(q + ((size_t)t * a.nH + h0 + min(hh, per - 1)) * d + k_at);
+    unpack16<T>(w, qf[hh]);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) qf[hh][e] = in_row && hh < per ? qf[hh][e] : 0.f;
+  }
   __syncthreads();
-  float dot[PER];
+  // Loads are clamped to the block's keys, not left out: what a branch surrounds the compiler waits for at its end.
+  const int key0 = wave * WKEYS, all_loads = WKEYS >> (6 - row_log);
+  const int loads = nk > key0 ? min((nk - key0 + KL - 1) >> (6 - row_log), all_loads) : 0;
+  auto load_keys = [&](uint4 (&w)[UK], int j) {
 #pragma unroll
-  for (int hh = 0; hh < PER; ++hh) dot[hh] = 0.f;
-  if (has) {
-    const T* krow = k_pool + ((size_t)row0 + (size_t)kvh * a.page_size) * d;
-    for (int c0 = 0; c0 < d; c0 += 8 * VEC) {           // eight loads on their way at a time
-      uint4 w[8];
+    for (int u = 0; u < UK; ++u) {
+      const int i = min(key0 + min(j + u, all_loads - 1) * KL + key_of, nk - 1);
+      w[u] = *reinterpret_cast<const uint4*>(k_pool + ((size_t)rows_of[i] + (size_t)kvh * a.page_size) * d + k_at);
+    }
+  };
+  const int EC = dv / VEC;
+  int EC2 = 1;
+  while (EC2 < EC) EC2 <<= 1;
+  const int KG = NT / EC2, ec = tid & (EC2 - 1), kg = tid / EC2;
+  auto load_values = [&](uint4 (&w)[UV], int z, int i0) {    // of the keys i0 + kg, i0 + kg + KG, ..
+    const int vh = a.value_heads > 0 ? z : kvh, at = min(ec, EC - 1) * VEC;
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (c0 + j * VEC < d) w[j] = *reinterpret_cast<const uint4*>(krow + c0 + j * VEC);
+    for (int u = 0; u < UV; ++u)
+      w[u] = *reinterpret_cast<const uint4*>(v_pool + ((size_t)rows_of[min(i0 + u * KG + kg, nk - 1)] + (size_t)vh * a.page_size) * dv + at);
+  };
+  uint4 kw[UK], vw[UV];
+  load_keys(kw, 0);
+  load_values(vw, 0, 0);
+  // A lane's partial products meet over the row's lanes: over the first two distances each lane keeps half of the heads and hands
+  // the other half over, then every lane's own heads are summed over the rest.
+  const bool odd1 = lane & 1, odd2 = lane & 2;
+  const int own0 = PER >= 4 ? (odd1 ? PER / 2 : 0) + (odd2 ? PER / 4 : 0) : PER == 2 && odd1 ? 1 : 0;
+  auto score_keys = [&](const uint4 (&w)[UK], int j) {
+    float sum[UK][OWN];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (c0 + j * VEC >= d) break;
-        float kf[VEC];
-        unpack16<T>(w[j], kf);
+    for (int u = 0; u < UK; ++u) {
+      const uint4 x = in_row ? w[u] : uint4{0u, 0u, 0u, 0u};
+      float kf[VEC], dot[PER];
+      unpack16<T>(x, kf);
 #pragma unroll
-        for (int i = 0; i < VEC; i += 4) {
+      for (int hh = 0; hh < PER; ++hh) {
+        dot[hh] = qf[hh][0] * kf[0];
 #pragma unroll
-          for (int hh = 0; hh < PER; ++hh) {
-            const float4 qq = *reinterpret_cast<const float4*>(&qs[hh][c0 + j * VEC + i]);
-            dot[hh] = fmaf(qq.x, kf[i], dot[hh]);
-            dot[hh] = fmaf(qq.y, kf[i + 1], dot[hh]);
-            dot[hh] = fmaf(qq.z, kf[i + 2], dot[hh]);
-            dot[hh] = fmaf(qq.w, kf[i + 3], dot[hh]);
-          }
+        for (int e = 1; e < VEC; ++e) dot[hh] = fmaf(qf[hh][e], kf[e], dot[hh]);
+      }
+      if constexpr (PER >= 2) {
+#pragma unroll
+        for (int i = 0; i < PER / 2; ++i) {
+          const float mine = odd1 ? dot[i + PER / 2] : dot[i], other = odd1 ? dot[i] : dot[i + PER / 2];
+          dot[i] = mine + lane_move<DPP_XOR1>(other);
         }
+      } else {
+        dot[0] += lane_move<DPP_XOR1>(dot[0]);
+      }
+      if constexpr (PER >= 4) {
+#pragma unroll
+        for (int i = 0; i < PER / 4; ++i) {
+          const float mine = odd2 ? dot[i + PER / 4] : dot[i], other = odd2 ? dot[i] : dot[i + PER / 4];
+          dot[i] = mine + lane_move<DPP_XOR2>(other);
+        }
+      } else {
+        dot[0] += lane_move<DPP_XOR2>(dot[0]);
+      }
+#pragma unroll
+      for (int i = 0; i < OWN; ++i) sum[u][i] = dot[i];
+    }
+    auto meet = [&](auto partner_sum) {
+#pragma unroll
+      for (int u = 0; u < UK; ++u)
+#pragma unroll
+        for (int i = 0; i < OWN; ++i) sum[u][i] = partner_sum(sum[u][i]);
+    };
+    if (row_log == 3) {
+      meet([](float v) { return v + lane_move<DPP_ROR12>(v); });                          // (from the lane 4 on: right in the row's first four)
+    } else if (row_log >= 4) {
+      meet([](float v) { v += lane_move<DPP_ROR8>(v); return v + lane_move<DPP_ROR4>(v); });
+    }
+    if (row_log >= 5) meet([](float v) { return sum_over_16(v); });
+    if (row_log >= 6) meet([](float v) { return sum_over_32(v); });
+    if (piece < 4) {
+#pragma unroll
+      for (int u = 0; u < UK; ++u) {
+        if (j + u >= loads) break;
+#pragma unroll
+        for (int i = 0; i < OWN; ++i) ps[own0 + i][key0 + (j + u) * KL + key_of] = sum[u][i];
       }
     }
+  };
+  for (int j = 0; j < loads; j += UK) {
+    score_keys(kw, j);
+    if (j + UK < loads) load_keys(kw, j + UK);
   }
+  lds_barrier();
   // scores, the block's maximum a head, the weights and their sum
   float sc[PER];
 #pragma unroll
   for (int hh = 0; hh < PER; ++hh) {
-    float s = dot[hh] * a.scale;
+    float s = has ? ps[hh][tid & (KEYS - 1)] * a.scale : 0.f;
     if (a.slopes && hh < per) s = fmaf(a.slopes[h0 + hh], (float)(kp - pos), s);
     sc[hh] = has ? s : -INFINITY;
     const float m = wave_max(sc[hh]);
     if (lane == 0) wred[wave][hh] = m;
   }
-  __syncthreads();
+  lds_barrier();
   float mx[PER];
 #pragma unroll
-  for (int hh = 0; hh < PER; ++hh) mx[hh] = fmaxf(fmaxf(wred[0][hh], wred[1][hh]), fmaxf(wred[2][hh], wred[3][hh]));
-  __syncthreads();
+  for (int hh = 0; hh < PER; ++hh) mx[hh] = fmaxf(fmaxf(wred[0][hh], wred[1][hh]), fmaxf(wred[2][hh], wred[3][hh]));   // (the waves of KEYS threads)
+  lds_barrier();
 #pragma unroll
   for (int hh = 0; hh < PER; ++hh) {
     const float p = has ? (FULL ? expf(sc[hh] - mx[hh]) : __expf(sc[hh] - mx[hh])) : 0.f;
-    ps[hh][tid] = p;
+    if (tid < KEYS) ps[hh][tid] = p;
     const float s = wave_sum(p);
     if (lane == 0) wred[wave][hh] = s;
   }
-  __syncthreads();
+  lds_barrier();
 #pragma unroll
   for (int hh = 0; hh < PER; ++hh) {
     if (tid == hh && hh < per) {
@@ -136,57 +234,63 @@ __global__ __launch_bounds__(256) void attn_split_kernel(const T* __restrict__ q
     }
   }
   // values: thread (kg, ec) takes the keys kg, kg + KG, .. and 16 bytes of the row's width
-  const int EC = dv / VEC;
-  int EC2 = 1;
-  while (EC2 < EC) EC2 <<= 1;
-  const int KG = 256 / EC2, ec = tid % EC2, kg = tid / EC2;
-  const int n_vh = a.value_heads > 0 ? a.value_heads : 1;
   for (int z = 0; z < n_vh; ++z) {
-    const int vh = a.value_heads > 0 ? z : kvh;
     float acc[PER][VEC];
 #pragma unroll
     for (int hh = 0; hh < PER; ++hh)
 #pragma unroll
       for (int i = 0; i < VEC; ++i) acc[hh][i] = 0.f;
-    if (ec < EC) {
-      for (int i = kg; i < nk; i += KG) {
-        const uint4 w = *reinterpret_cast<const uint4*>(v_pool + ((size_t)rows_of[i] + (size_t)vh * a.page_size) * dv + ec * VEC);
-        float vf[VEC];
-        unpack16<T>(w, vf);
+    auto add_values = [&](const uint4 (&w)[UV], int i0) {
 #pragma unroll
-        for (int hh = 0; hh < PER; ++hh) {
-          const float p = ps[hh][i];
+      for (int u = 0; u < UV; ++u) {
+        const int i = i0 + u * KG + kg;
+        if (i < nk) {
+          float vf[VEC];
+          unpack16<T>(w[u], vf);
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) acc[hh][e] = fmaf(p, vf[e], acc[hh][e]);
+          for (int hh = 0; hh < PER; ++hh) {
+            const float p = ps[hh][i];
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) acc[hh][e] = fmaf(p, vf[e], acc[hh][e]);
+          }
         }
       }
+    };
+    for (int i0 = 0; i0 < nk; i0 += UV * KG) {
+      if (z > 0 || i0 > 0) load_values(vw, z, i0);
+      add_values(vw, i0);
     }
-    // the shares of the keys meet: lane swaps within a wave, then the four waves through LDS, a head at a time
+    // the shares of the keys meet: lane moves within a wave, then the waves through LDS
+    auto meet = [&](auto partner_sum) {
 #pragma unroll
-    for (int hh = 0; hh < PER; ++hh) {
-      if (hh >= per) break;
+      for (int hh = 0; hh < PER; ++hh)
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        float v = acc[hh][e];
-        for (int off = EC2; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
-        acc[hh][e] = v;
+        for (int e = 0; e < VEC; ++e) acc[hh][e] = partner_sum(acc[hh][e]);
+    };
+    if (EC2 <= 1) meet([](float v) { return v + lane_move<DPP_XOR1>(v); });
+    if (EC2 <= 2) meet([](float v) { return v + lane_move<DPP_XOR2>(v); });
+    if (EC2 <= 4) meet([](float v) { return v + __shfl_xor(v, 4, 64); });
+    if (EC2 <= 8) meet([](float v) { return v + lane_move<DPP_ROR8>(v); });
+    if (EC2 <= 16) meet([](float v) { return sum_over_16(v); });
+    if (EC2 <= 32) meet([](float v) { return sum_over_32(v); });
+#pragma unroll
+    for (int g0 = 0; g0 < PER; g0 += HG) {
+      if (g0 >= per) break;
+      lds_barrier();                                    // ored is free again
+      if (lane < EC2 && ec < EC) {
+#pragma unroll
+        for (int hh = 0; hh < HG; ++hh)
+#pragma unroll
+          for (int e = 0; e < VEC; e += 4)
+            *reinterpret_cast<float4*>(&ored[wave][hh][ec * VEC + e]) = float4{acc[g0 + hh][e], acc[g0 + hh][e + 1], acc[g0 + hh][e + 2], acc[g0 + hh][e + 3]};
       }
-      __syncthreads();                                    // ored is free again
-      if (EC2 >= 64) {                                    // a wave holds one share only: the waves hold KG = 4 / (EC2 / 64) shares
-        if (ec < EC)
+      lds_barrier();
+      for (int i = tid; i < min(HG, per - g0) * dv; i += NT) {
+        const int hh = i / dv, e = i - hh * dv;
+        float o = ored[0][hh][e];
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) ored[kg % 4][(size_t)ec * VEC + e] = (kg < 4) ? acc[hh][e] : 0.f;
-      } else if (lane < EC2 && ec < EC) {
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) ored[wave][ec * VEC + e] = acc[hh][e];
-      }
-      __syncthreads();
-      const int shares = EC2 >= 64 ? KG : 4;
-      float* po = a.part_o + ((((size_t)t * a.nH + h0 + hh) * n_vh + z) * a.n_splits + split) * dv;
-      for (int e = tid; e < dv; e += 256) {
-        float o = 0.f;
-        for (int s = 0; s < shares; ++s) o += ored[s][e];
-        po[e] = o;
+        for (int x = 1; x < WAVES; ++x) o += ored[x][hh][e];
+        a.part_o[((((size_t)t * a.nH + h0 + g0 + hh) * n_vh + z) * a.n_splits + split) * dv + e] = o;
       }
     }
   }
@@ -297,7 +401,7 @@ extern "C" int alice_attention_split(const void* q, int dtype, const void* k_poo
               bias_slopes, part_ml, part_o};
   const int per = nH / nKV;
   dim3 grid(T, nKV, runs);
-#define GO(TT, PER) attn_split_kernel<TT, PER><<<grid, 256, 0, stream>>>((const TT*)q, (const TT*)k_pool, (const TT*)v_pool, a)
+#define GO(TT, PER) attn_split_kernel<TT, PER><<<grid, NT, 0, stream>>>((const TT*)q, (const TT*)k_pool, (const TT*)v_pool, a)
 #define BY_PER(TT)                 \
   do {                             \
     if (per <= 1) GO(TT, 1);       \

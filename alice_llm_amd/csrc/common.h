@@ -55,7 +55,7 @@ template <> __device__ __forceinline__ float round_to<bf16_t>(float v) { return 
 // eight sequences with its 53 norms 1,973 and 1,952 us.)
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_move(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true); }
-constexpr int DPP_ROR8 = 0x128, DPP_ROR4 = 0x124, DPP_XOR2 = 0x4E, DPP_XOR1 = 0xB1, DPP_HALF_MIRROR = 0x141;
+constexpr int DPP_ROR12 = 0x12C, DPP_ROR8 = 0x128, DPP_ROR4 = 0x124, DPP_XOR2 = 0x4E, DPP_XOR1 = 0xB1, DPP_HALF_MIRROR = 0x141;
 
 template <typename T, typename F>
 __device__ __forceinline__ T wave_reduce(T v, F op) {
