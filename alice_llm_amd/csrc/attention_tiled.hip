@@ -19,7 +19,10 @@
 // What bounds it: the vector instructions of the softmax and of the moves through LDS, some 300 for every 32 MFMA of a step, and
 // few waves (a prompt of 2,048 tokens and 16 heads is two blocks a CU).  So blocks wholly inside every query's range skip the
 // masks, the exponents are powers of two, and the output is rescaled only in blocks where a column's maximum grows:
-// 2,048 tokens, 16 heads of 128 on 4 kv heads 128 -> 117 us, 8 prompts of 1,000 164 -> 153, 16 heads of 64 87 -> 77.  Keys of 256 leave a
+// 2,048 tokens, 16 heads of 128 on 4 kv heads 128 -> 117 us, 8 prompts of 1,000 164 -> 153, 16 heads of 64 87 -> 77.  Loads
+// without branches from places that are offsets to the step's page, values turned by an exchange between two lanes and half as many
+// stores to LDS, the maximum by lane swaps: 117 -> 105 us, four prompts of 2,047 279 -> 222, 8,192 tokens 940 -> 763, 16 heads of
+// 64 79 -> 67, 8 of 256 153 -> 147 (the same bits).  What bounds a single prompt now is its longest chain of steps, 64 of 1.6 us.  Keys of 256 leave a
 // SIMD one wave, and a branch there costs more than what it skips: 8 heads of 256 186 -> 154 us without the two, 177 with the
 // masks' one, 183 with both.  Loads two steps ahead gave nothing.  A base that lags behind the maximum by up to 2^8 (115 us) rounds the
 // largest weight too, which as the maximum's own is 1: the error against 64 bits rose by 4 to 20 % (peaked scores).
@@ -37,6 +40,15 @@ __device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
 }
 
 __device__ __forceinline__ float exp2f_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// A reduction over the lanes 16, 32 and 48 away, in each of them.
+template <typename F>
+__device__ __forceinline__ float four_lanes(float v, F op) {
+  auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(x[0]), __uint_as_float(x[1]));
+  auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return op(__uint_as_float(y[0]), __uint_as_float(y[1]));
+}
 
 struct TiledArgs {
   const bf16_t* q;
@@ -64,7 +76,7 @@ constexpr float LOG2E = 1.44269504088896341f;
 constexpr int VPAD = 40;      // row length of the transposed values in LDS (32 keys and a pad against bank conflicts)
 
 template <int DP, int DVP, int HPW>
-__global__ __launch_bounds__(256) void attn_tiled_kernel(TiledArgs a) {
+__global__ __launch_bounds__(256, HPW == 1 && DP + DVP <= 256 ? 3 : 1) void attn_tiled_kernel(TiledArgs a) {
   constexpr int KS = DP / 32, ET = DVP / 16;
   constexpr int KROW = DP + 8;
   constexpr int NKC = DP / 64, NVC = DVP / 64;          // 16-byte pieces of keys / values a thread moves a step
@@ -138,26 +150,25 @@ __global__ __launch_bounds__(256) void attn_tiled_kernel(TiledArgs a) {
     const int key0 = (step < n_first ? step : t_lo + step - n_first) * KT;
     return (one_page && step < n_steps) ? bt[key0 >> a.page_shift] : 0;
   };
+  // Keys beyond the block's last one are its last one again (none of the queries sees them), dimensions beyond the head's are
+  // left out when the pieces go to LDS: no load stands under a branch, and in one page a thread's place is an offset to the step's.
   u32x4 pk[NKC], pv[NVC];
   auto fetch = [&](int step, int page) {
-    const int key0 = (step < n_first ? step : t_lo + step - n_first) * KT;
+    const int key0 = (step < n_first ? step : t_lo + step - n_first) * KT, last = p_last - key0;
+    const size_t at = one_page ? (size_t)page * a.nKV * a.page_size + (key0 & (a.page_size - 1)) : 0;
+    const bf16_t* kb = a.k_pool + (at + (size_t)kvh * a.page_size) * D;
+    const bf16_t* vb = a.v_pool + (at + (size_t)vh * a.page_size) * DV;
 #pragma unroll
     for (int n = 0; n < NKC; ++n) {
-      const int id = tid + n * 256, key = id / (DP / 8), dim = (id % (DP / 8)) * 8, kp = key0 + key;
-      pk[n] = u32x4{0u, 0u, 0u, 0u};
-      if (dim < D && kp <= p_last) {
-        const size_t row = one_page ? ((size_t)page * a.nKV + kvh) * a.page_size + (kp & (a.page_size - 1)) : row_of(kp, kvh);
-        pk[n] = *reinterpret_cast<const u32x4*>(a.k_pool + row * D + dim);
-      }
+      const int id = tid + n * 256, key = min(id / (DP / 8), last), dim = min((id % (DP / 8)) * 8, D - 8);
+      if (one_page) pk[n] = *reinterpret_cast<const u32x4*>(kb + (unsigned)(key * D + dim));
+      else pk[n] = *reinterpret_cast<const u32x4*>(a.k_pool + row_of(key0 + key, kvh) * D + dim);
     }
 #pragma unroll
     for (int n = 0; n < NVC; ++n) {
-      const int id = tid + n * 256, key = id % KT, e = (id / KT) * 8, kp = key0 + key;     // neighbouring lanes: neighbouring keys
-      pv[n] = u32x4{0u, 0u, 0u, 0u};
-      if (e < DV && kp <= p_last) {
-        const size_t row = one_page ? ((size_t)page * a.nKV + vh) * a.page_size + (kp & (a.page_size - 1)) : row_of(kp, vh);
-        pv[n] = *reinterpret_cast<const u32x4*>(a.v_pool + row * DV + e);
-      }
+      const int id = tid + n * 256, key = min(id % KT, last), e = min((id / KT) * 8, DV - 8);             // neighbouring lanes: neighbouring keys
+      if (one_page) pv[n] = *reinterpret_cast<const u32x4*>(vb + (unsigned)(key * DV + e));
+      else pv[n] = *reinterpret_cast<const u32x4*>(a.v_pool + row_of(key0 + key, vh) * DV + e);
     }
   };
 
@@ -171,21 +182,25 @@ __global__ __launch_bounds__(256) void attn_tiled_kernel(TiledArgs a) {
     for (int et = 0; et < ET; ++et) oT[hh][et] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  auto stage = [&](int buf) {                           // what was fetched goes into LDS
+  // What was fetched goes into LDS.  The values are turned on the way: two neighbouring lanes hold the same elements of two
+  // neighbouring keys, which lie side by side in the order of the score tiles' rows; they exchange halves, and each stores four
+  // words of two keys (eight stores of one key each before).
+  const bool odd = tid & 1;
+  const uint32_t halves = odd ? 0x03020706u : 0x05040100u;
+  auto stage = [&](int buf) {
 #pragma unroll
     for (int n = 0; n < NKC; ++n) {
       const int id = tid + n * 256, key = id / (DP / 8), dim = (id % (DP / 8)) * 8;
-      *reinterpret_cast<u32x4*>(&Ks[buf][key][dim]) = pk[n];
+      *reinterpret_cast<u32x4*>(&Ks[buf][key][dim]) = dim < D ? pk[n] : u32x4{0u, 0u, 0u, 0u};
     }
 #pragma unroll
     for (int n = 0; n < NVC; ++n) {
-      const int id = tid + n * 256, key = id % KT, e = (id / KT) * 8;
-      const int col = ((key & 15) >> 2) * 8 + (key & 3) + 4 * (key >> 4);       // the order of the score tiles' rows
-      const uint32_t w[4] = {pv[n][0], pv[n][1], pv[n][2], pv[n][3]};
+      const int id = tid + n * 256, key = id % KT, e = (id / KT) * 8, pair = key & ~1;
+      const int col = ((pair & 15) >> 2) * 8 + (pair & 3) + 4 * (pair >> 4);     // the order of the score tiles' rows
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        Vt[buf][e + 2 * i][col].bits = (uint16_t)(w[i] & 0xffffu);
-        Vt[buf][e + 2 * i + 1][col].bits = (uint16_t)(w[i] >> 16);
+        const uint32_t own = e < DV ? pv[n][i] : 0u, other = dpp_move<DPP_XOR1>(own);
+        *reinterpret_cast<uint32_t*>(&Vt[buf][e + 2 * i + odd][col]) = __builtin_amdgcn_perm(other, own, halves);
       }
     }
   };
@@ -243,8 +258,7 @@ __global__ __launch_bounds__(256) void attn_tiled_kernel(TiledArgs a) {
           }
 #pragma unroll
           for (int j = 0; j < 8; ++j) m_t = fmaxf(m_t, sc[j]);
-          m_t = fmaxf(m_t, __shfl_xor(m_t, 16, 64));
-          m_t = fmaxf(m_t, __shfl_xor(m_t, 32, 64));
+          m_t = four_lanes(m_t, [](float x, float y) { return fmaxf(x, y); });
           // The base is the running maximum, so that the largest weight is 1 and not rounded; the output is rescaled in the blocks
           // only where some column's maximum grows.
           const bool raise = m_t > m_run[hh];
@@ -287,8 +301,7 @@ __global__ __launch_bounds__(256) void attn_tiled_kernel(TiledArgs a) {
   for (int hh = 0; hh < HPW; ++hh) {
     const int h = h0 + hh;
     float l_tot = l_run[hh];
-    l_tot += __shfl_xor(l_tot, 16, 64);
-    l_tot += __shfl_xor(l_tot, 32, 64);
+    l_tot = four_lanes(l_tot, [](float x, float y) { return x + y; });
     float factor = 1.f;
     if (a.sink) {                                       // one more term of the denominator, without a value
       const float sk = a.sink[h] * LOG2E;
