@@ -731,7 +731,7 @@ __global__ __launch_bounds__(ST) void draw_kernel(const float* __restrict__ logi
 // (32), one 17 (25), 64 of 32,768 16 (26).  The one pass takes 1.6 times its reads' time, row_topk the latency of some twenty
 // phases, 0.5 us each, most of it for instructions that no launch before left in the CU's cache.  Rows that the lists do not settle (one that holds no number or no finite maximum, too many ties at the
 // threshold itself) are counted and collected by their one block as the kernels for any k do it.  One row of 256,000 with 1,000 elements
-// that are not masked: 34 us; with 5,120 ties at the top 158 (46 and 41 by the five passes).
+// that are not masked: 22 us (32 before); with 5,120 ties at the top 168 (175; 41 by the five passes).
 constexpr int TOPK_MOST = 200;       // beyond, the bound of 256 maxima lets too much through
 constexpr int TOPK_LIST = 7168;      // elements of a row's lists in shared memory
 constexpr int TOPK_LEFT = 1024;      // survivors
