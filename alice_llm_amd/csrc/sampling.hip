@@ -918,7 +918,9 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
   const int c0 = lane < sh.chunks ? counts[lane] : 0, c1 = 64 + lane < sh.chunks ? counts[64 + lane] : 0;
   const uint32_t t0 = lane < sh.chunks ? left_out[lane] : 0u, t1 = 64 + lane < sh.chunks ? left_out[64 + lane] : 0u;
   if (tid < TOPK_TILES) tsum[tid] = 0.f;
+  if (tid < 256) keys[tid] = 0;
   if (tid == 0) { n_left = 0; last_kept = -1; rounds = 0; best = 0; pick[0] = -1; pick[1] = -1; carry[1] = 0.f; }
+  lds_barrier();                                           // (the counts are on their way)
   const uint32_t tie = wave_reduce(max(t0, t1), [](uint32_t a, uint32_t b) { return max(a, b); });
   bool settled = !__any(c0 < 0 || c1 < 0);
   auto scan = [&](int v) {
@@ -934,11 +936,11 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
   settled = settled && n >= 1 && n <= TOPK_LIST;
   uint32_t key_m = 0;
   if (settled) {
-    // the lists' elements, several waves a chunk where there are few; the bound again: the largest of every four threads'
-    // elements, of these the k-th largest
+    // the lists' elements, several waves a chunk where there are few; the bound again, from the largest of 256 groups.  A group
+    // is by the place in all lists one after the other, not by the thread that moves an element: where not every wave has a chunk's
+    // share (6, 9 .. 15 chunks) fewer threads than 4 k may move all, and a bound that every element reaches settles nothing.
     constexpr int NW = ST / 64;
     const int share = max(NW / sh.chunks, 1), sub = wave % share;
-    uint32_t most = 0;
     for (int c = wave / share; c < sh.chunks; c += NW / share) {
       const int end = c < 64 ? __builtin_amdgcn_readlane(s0, c) : n0 + __builtin_amdgcn_readlane(s1, c - 64);
       const int len = c < 64 ? __builtin_amdgcn_readlane(c0, c) : __builtin_amdgcn_readlane(c1, c - 64);
@@ -946,12 +948,9 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
       for (int i = sub * 64 + lane; i < len; i += share * 64) {
         const unsigned long long el = src[i];
         list[end - len + i] = el;
-        most = max(most, (uint32_t)(el >> 32));
+        atomicMax(&keys[(end - len + i) / 4 % 256], (uint32_t)(el >> 32));
       }
     }
-    most = max(most, dpp_move<DPP_XOR1>(most));
-    most = max(most, dpp_move<DPP_XOR2>(most));
-    if ((tid & 3) == 0) keys[tid >> 2] = most;
     __syncthreads();
     if (wave == 0) {
       uint32_t largest;
