@@ -233,6 +233,9 @@ constexpr int MAX_SPLIT = 8;
 // gives.  (Numbers of tokens on two sides of a multiple of 64 may add in another order: rounding, no more.)
 int planned_tokens(int M) { return M <= 32 ? 32 : ceil_div(M, 64) * 64; }
 
+// Elements a slice of up to 16 tokens' products.
+int slice_of(int K, int split) { return ceil_div(ceil_div(K, split), 128) * 128; }
+
 // 2 to 16 tokens: the tokens are the columns of the same matrix instruction, the rows of W its rows.  A block takes 16 R rows
 // (with GeGLU 8 gate rows and the up rows of the same outputs: twice the blocks of 16 and 16, and the registers for more of
 // them a CU), its NW waves every NW-th chunk of 32 inner elements of
@@ -379,19 +382,20 @@ int rows_split(int N, int K) {
 }
 
 // One token: a wave a row of W (with GeGLU the gate row and the up row of an output) on FMAs, four elements a lane a step; the lanes'
-// sums meet in a fixed tree.  Any K, any address.  No column of the matrix instruction is idle: 18,432 rows by 2,304 with GeGLU
+// sums meet in a fixed tree.  Any K, any address, any slices.  No column of the matrix instruction is idle: 18,432 rows by 2,304 with GeGLU
 // 25.9 us (31.7 as columns, which gain from 2 to 4 tokens on), 256,000 rows 373 (402), 2,304 by 9,216 16.3 (19.1 in slices).
 template <typename TA, typename TW, typename TO, bool GEGLU>
 __global__ __launch_bounds__(256) void linear_single_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y, int N,
-                                                            int K, int epi, float param, int full) {
+                                                            int K, int kslice, int epi, float param, int full) {
   constexpr int NR = GEGLU ? 2 : 1;
   const int lane = threadIdx.x & 63, n = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (n >= N) return;
+  const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);       // (a slice begins at a multiple of 128)
   float acc[NR];
 #pragma unroll
   for (int r = 0; r < NR; ++r) acc[r] = 0.f;
-  const int K4 = K & ~3;
-  for (int k = lane * 4; k < K4; k += 256) {
+  const int K4 = k_end & ~3;
+  for (int k = k_begin + lane * 4; k < K4; k += 256) {
     float w[NR][4];
 #pragma unroll
     for (int r = 0; r < NR; ++r)
@@ -404,7 +408,7 @@ __global__ __launch_bounds__(256) void linear_single_kernel(const TA* __restrict
       for (int r = 0; r < NR; ++r) acc[r] = fmaf(w[r][e], x, acc[r]);
     }
   }
-  if (lane < K - K4) {                                        // up to three elements behind the last whole group of four
+  if (k_begin < k_end && lane < k_end - K4) {                 // up to three elements behind the last whole group of four
     const int k = K4 + lane;
     const float x = load_f32(A, k);
 #pragma unroll
@@ -416,15 +420,16 @@ __global__ __launch_bounds__(256) void linear_single_kernel(const TA* __restrict
   float o = acc[0];
   if (GEGLU) o = gated_act(acc[0], acc[NR - 1], param, full);
   if (epi == ALICE_EPI_SOFTCAP) o = unary_act(o, param, full);
-  store_f32(Y, n, o);
+  store_f32(Y, (size_t)blockIdx.y * N + n, o);
 }
 
 template <typename TA, typename TW, typename TO>
-int launch_single(const void* x, const void* w, void* y, int N, int K, int epi, float epi_param, int full, hipStream_t stream) {
-  if (epi == ALICE_EPI_GEGLU)
-    linear_single_kernel<TA, TW, TO, true><<<ceil_div(N, 4), 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, N, K, epi, epi_param, full);
-  else
-    linear_single_kernel<TA, TW, TO, false><<<ceil_div(N, 4), 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, N, K, epi, epi_param, full);
+int launch_single(const void* x, const void* w, void* y, int N, int K, int epi, float epi_param, int full, int split, hipStream_t stream) {
+  const int kslice = slice_of(K, split);
+  const dim3 grid(ceil_div(N, 4), split);
+#define GO(GEGLU) linear_single_kernel<TA, TW, TO, GEGLU><<<grid, 256, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, N, K, kslice, epi, epi_param, full)
+  if (epi == ALICE_EPI_GEGLU) GO(true); else GO(false);
+#undef GO
   ALICE_LAUNCH_CHECK();
   return 0;
 }
@@ -572,7 +577,7 @@ __global__ __launch_bounds__(256) void linear_few_kernel(const TA* __restrict__ 
 
 template <typename TA, typename TW, typename TO>
 int launch_few(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split, hipStream_t stream) {
-  const int kslice = ceil_div(ceil_div(K, split), 128) * 128;
+  const int kslice = slice_of(K, split);
   const int kc = min(ceil_div(kslice, FEW_SEG) * FEW_SEG, FEW_KC);
   const dim3 grid(ceil_div(N, (epi == ALICE_EPI_GEGLU ? 2 : 4) * FEW_R), split);
   const size_t lds = (size_t)FEW_MT * kc * sizeof(float);
@@ -586,7 +591,7 @@ int launch_few(const void* x, const void* w, void* y, int M, int N, int K, int e
 template <typename TA, typename TW, typename TO>
 int launch_rows(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split,
                 hipStream_t stream) {
-  const int kslice = ceil_div(ceil_div(K, split), 128) * 128;
+  const int kslice = slice_of(K, split);
   const bool whole = K % 8 == 0 && K >= 32 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
   const int by = epi == ALICE_EPI_GEGLU ? 8 : (N >= 16384 ? 32 : 16);      // many rows: a token's elements serve 32 of them
   const dim3 grid(ceil_div(N, by), split);
@@ -638,11 +643,14 @@ int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int
 
 }  // namespace
 
-// Whether up to 4 tokens go on FMAs: rows of whole units of four elements, at addresses of such units, and long enough that the
-// block's start does not outweigh them (65,536 rows by 256: 22.7 us, 16.2 on the matrix instruction; by 1,024 and more it is faster).
-static bool few_by_fours(const void* x, int x_dtype, const void* w, int w_dtype, int K) {
+// Whether up to 4 tokens go on FMAs, by the inner dimension: rows of whole units of four elements, long enough that the
+// block's start does not outweigh them (65,536 rows by 256: 22.7 us, 16.2 on the matrix instruction; by 1,024 and more it is faster), and
+// slices that are (of 256 elements: 8.2 us, 7.2 on the matrix instruction).  The rule of the slices and that of the launch ask here.
+static bool few_by_length(int K, int split) { return K % 4 == 0 && K >= 1024 && (split == 1 || slice_of(K, split) >= 512); }
+// And by the operands: at addresses of such units.
+static bool few_by_fours(const void* x, int x_dtype, const void* w, int w_dtype, int K, int split) {
   auto unit = [](int dtype) { return dtype == DT_F32 ? 15u : 7u; };
-  return K % 4 == 0 && K >= 1024 && ((uintptr_t)x & unit(x_dtype)) == 0 && ((uintptr_t)w & unit(w_dtype)) == 0;
+  return few_by_length(K, split) && ((uintptr_t)x & unit(x_dtype)) == 0 && ((uintptr_t)w & unit(w_dtype)) == 0;
 }
 
 // Slices for one token: W is read at 6.6 TB/s with three blocks a CU, at three quarters of that with few; the busiest CU reads
@@ -653,8 +661,8 @@ static int single_split(int N, int K) {
   int best = 1;
   float best_us = 1e30f;
   for (int s = 1; s <= MAX_SPLIT; ++s) {
-    const int ks = ceil_div(ceil_div(K, s), 128) * 128;
-    if (s > 1 && (ks < 512 || (long)ks * (s - 1) >= K)) continue;
+    const int ks = slice_of(K, s);
+    if (s > 1 && (!few_by_length(K, s) || (long)ks * (s - 1) >= K)) continue;
     const float full = fminf(1.f, 0.75f + 0.25f * blocks * s / 768.f);
     const float us = fmaxf((float)N * K * 4e-6f / (6.6f * full), ceil_div((long)blocks * s, 256) * (float)ks * 64.f / 40e3f) + 0.2f * s;
     if (us < best_us) { best_us = us; best = s; }
@@ -665,7 +673,7 @@ static int single_split(int N, int K) {
 // Into how many slices of the inner dimension a product without an epilogue is best cut (for 2 to 16 tokens one
 // number, whatever captured steps round theirs to).
 int alice_linear_split_hint_generic(int M, int N, int K) {
-  if (M == 1) return K % 4 == 0 && K >= 1024 ? single_split(N, K) : 1;
+  if (M == 1) return few_by_length(K, 1) ? single_split(N, K) : 1;
   return M <= 16 ? rows_split(N, K) : plan_mfma32(planned_tokens(M), N, K, false, MAX_SPLIT).split;
 }
 
@@ -682,12 +690,12 @@ int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype,
   if (M == 0) return 0;
   int rc = 0;
   DISPATCH_DTYPE(x_dtype, TA, DISPATCH_DTYPE(w_dtype, TW, DISPATCH_DTYPE(y_dtype, TO, {
-    // (slices of 256 elements: 8.2 us, 7.2 on the matrix instruction)
-    const bool few = M <= FEW_MT && few_by_fours(x, x_dtype, w, w_dtype, K) && ceil_div(K, split_k) >= 512;
+    const bool few = M <= FEW_MT && few_by_fours(x, x_dtype, w, w_dtype, K, split_k);
     // One token: the same sums either way; a wave a row is the faster start (1,000 x 1,024: 3.6 and 4.5 us, 3,584 x 4,096: 14.1 and
     // 14.9), four rows a wave read longer matrices faster (8,192 x 3,584: 22.3 and 21.3, gate and up 34.5 and 30.4).
     const bool large = (size_t)N * K * sizeof(TW) * (epi == ALICE_EPI_GEGLU ? 2 : 1) >= ((size_t)80 << 20);
-    if (M == 1 && split_k == 1 && !(few && large)) rc = launch_single<TA, TW, TO>(x, w, y, N, K, epi, epi_param, full_precision, stream);
+    // (In slices, which are planned for four rows a wave, a wave a row takes what that does not: operands at any address.)
+    if (M == 1 && !(few && (large || split_k > 1))) rc = launch_single<TA, TW, TO>(x, w, y, N, K, epi, epi_param, full_precision, split_k, stream);
     else if (few) rc = launch_few<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
     else rc = M <= 16 ? launch_rows<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream)
                       : launch_tiled<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);

@@ -40,6 +40,25 @@ def test_few_tokens(M, N, K, xdt, wdt):
     assert (capped.double() - 5 * torch.tanh(ref / 5)).abs().max() <= tol + 1e-5
 
 
+@pytest.mark.parametrize("N,K,split", [(48, 1280, None), (700, 1408, None), (48, 1920, None), (64, 2304, None), (2304, 2048, 8), (40, 1030, 3), (40, 2000, 5)])
+def test_slices_of_one_token(N, K, split):
+    """A slice of one token's product is the product of that slice's elements, bit for bit: in the slices that the library plans
+    (of which some end just below 512 elements) and in any others, at aligned and at odd addresses."""
+    x, w = rnd(1, K, seed=1), rnd(N, K, seed=2, scale=0.1)
+    moved = torch.empty(N * K + 1, device=DEV)[1:].view(N, K).copy_(w)
+    split = split or ops.linear_split_hint(1, N, K, ops.LAYOUT_ROW)
+    assert split > 1
+    step = -(-(-(-K // split)) // 128) * 128
+    for wt in (w, moved):
+        y = torch.full((split, 1, N), float("nan"), device=DEV)
+        ops.linear(x, wt, y, n_out=N, k_in=K, split_k=split, full_precision=True)
+        for s in range(split):
+            part, a, b = torch.zeros(1, N, device=DEV), s * step, min(K, (s + 1) * step)
+            if a < b:
+                ops.linear(x[:, a:b].contiguous(), w[:, a:b].contiguous(), part, n_out=N, k_in=b - a, full_precision=True)
+            assert torch.equal(y[s], part), s
+
+
 def test_a_token_gets_the_same_with_and_without_others():
     """One token (a wave a row, or four rows a wave in large matrices) and four: the same bits."""
     for N, K in ((40, 1028), (8200, 2560)):
