@@ -241,7 +241,8 @@ int slice_of(int K, int split) { return ceil_div(ceil_div(K, split), 128) * 128;
 // them a CU), its NW waves every NW-th chunk of 32 inner elements of
 // its slice; their sums meet in LDS.  W goes straight from memory into the instruction's operand, 128 bytes of a row a
 // chunk, the next two chunks on their way while two are multiplied; the tokens' elements come through the L1.  A token's
-// result depends on no other token, nor on how many there are (as long as this kernel takes them).
+// result depends on no other token, nor on how many there are.  (The rows that this kernel takes are those that few_by_fours() does not,
+// whatever the number of tokens.)
 // WHOLE: rows of whole, aligned units of eight elements.  Else (any K, any address) the same loads without an alignment, and the
 // elements behind the last whole chunk one by one, by the wave whose turn it is: 2,304 rows by 2,305 at 4 tokens 9.0 us (by 2,304
 // 9.1; on the tile of 64 tokens 71).
@@ -441,11 +442,11 @@ int launch_single(const void* x, const void* w, void* y, int N, int K, int epi, 
 // the output head 394 -> 357; the 128-byte pieces get slower by it), and two of every row are on their way while two
 // are multiplied.  The tokens' elements are asked for ahead of W's first (33.7 -> 30.2 us: a block's start is what its CU waits for).
 // What bounds it: reading W, at 6.6 TB/s where it is long.  4 tokens, 2B shape, matrix instruction and this: q, k, v 12.6 and
-// 8.9 us, output projection 7.2 (8 slices) and 6.3 (3), gate and up 40.0 and 30.2, down 21.6 and 17.1, head 404 and 353; five to
-// eight tokens gain nothing by it (42 us for gate and up, 468 for the head).
+// 8.9 us, output projection 7.2 (8 slices) and 6.3 (3), gate and up 40.0 and 30.2, down 21.6 and 17.1, head 404 and 353; more tokens in
+// one block gain nothing by it (eight: 42 us for gate and up, 468 for the head), but four a block do where there are few blocks.
 // Which products a token's sum adds, and in which order, depends on K and the slices alone: a lane's elements in their order, then
-// the lanes over the distances 32, 16 .. 1.  That is the order of the kernel for one token as well (the same bits), not that of the
-// matrix instruction: the fifth token of a step changes the others' sums by rounding.
+// the lanes over the distances 32, 16 .. 1.  That is the order of the kernel for one token as well, and of those for 5 to 16 tokens below
+// (the same bits).
 constexpr int FEW_MT = 4, FEW_R = 4, FEW_SEG = 256, FEW_KC = 2560;       // tokens, rows a wave, elements a step, elements of a token that a block keeps (whole steps of two)
 
 template <typename T> __device__ __forceinline__ f32x4 load_four(const T* p);
@@ -496,6 +497,7 @@ __global__ __launch_bounds__(256) void linear_few_kernel(const TA* __restrict__ 
   constexpr int MT = FEW_MT, R = FEW_R, U = 2, P = (FEW_KC + 1023) / 1024;   // P: rounds of the block over a chunk's elements
   extern __shared__ __align__(16) float xs[];                 // [MT][kc]: the tokens' elements of a chunk, zeros behind the slice
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m0 = blockIdx.z * MT;                             // this block's tokens are m0 .. m0 + MT - 1, as far as there are so many
   const int n0 = (blockIdx.x * 4 + wave) * (GEGLU ? R / 2 : R);
   const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);
   const TW* wrow[R];                                          // rows beyond the last are read as the last and not written
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(256) void linear_few_kernel(const TA* __restrict__ 
 #pragma unroll
     for (int p = 0; p < P; ++p)
 #pragma unroll
-      for (int m = 0; m < MT; ++m) v[p][m] = load_four(A + (size_t)min(m, M - 1) * K + min(c0 + p * 1024 + tid * 4, k_end - 4));
+      for (int m = 0; m < MT; ++m) v[p][m] = load_four(A + (size_t)min(m0 + m, M - 1) * K + min(c0 + p * 1024 + tid * 4, k_end - 4));
   };
   load_x(k_begin);
   __builtin_amdgcn_sched_barrier(0);
@@ -566,7 +568,7 @@ __global__ __launch_bounds__(256) void linear_few_kernel(const TA* __restrict__ 
   TO* y = Y + (size_t)blockIdx.y * M * N;
 #pragma unroll
   for (int i = 0; i < MT * R / 8; i += GEGLU ? 2 : 1) {
-    const int m = (first + i) / R, r = (first + i) % R, n = n0 + (GEGLU ? r >> 1 : r);
+    const int m = m0 + (first + i) / R, r = (first + i) % R, n = n0 + (GEGLU ? r >> 1 : r);
     if (m >= M || n >= N) continue;
     float o = acc[i];
     if (GEGLU) o = gated_act(acc[i], acc[i + 1], param, full);
@@ -579,11 +581,266 @@ template <typename TA, typename TW, typename TO>
 int launch_few(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split, hipStream_t stream) {
   const int kslice = slice_of(K, split);
   const int kc = min(ceil_div(kslice, FEW_SEG) * FEW_SEG, FEW_KC);
-  const dim3 grid(ceil_div(N, (epi == ALICE_EPI_GEGLU ? 2 : 4) * FEW_R), split);
+  const dim3 grid(ceil_div(N, (epi == ALICE_EPI_GEGLU ? 2 : 4) * FEW_R), split, ceil_div(M, FEW_MT));
   const size_t lds = (size_t)FEW_MT * kc * sizeof(float);
 #define GO(GEGLU) linear_few_kernel<TA, TW, TO, GEGLU><<<grid, 256, lds, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, kslice, kc, epi, epi_param, full)
   if (epi == ALICE_EPI_GEGLU) GO(true); else GO(false);
 #undef GO
+  ALICE_LAUNCH_CHECK();
+  return 0;
+}
+
+// 5 to 16 tokens where the kernel above takes up to 4: the same sums, bit for bit, on the matrix instruction for 16 blocks of 4 rows by
+// 4 tokens (v_mfma_f32_4x4x1_16b_f32: one 32-bit FMA an element a block, none of it idle).  So a token's result does not hang on how
+// many others its step has, up to 16 of them, nor on the rounded size of a captured step.  A lane holds four elements of row lane % 4 for
+// block lane / 4: block b of the 64 elements number a of every 256 adds what lane 16 a + b adds there.
+// Two kernels share that, and where few blocks are all there is the kernel above takes four tokens a block (launch_more() chooses).
+// Against the instruction for 16 columns, which adds in another order (rows x elements, slices; us at 8 and 16 tokens, before and after):
+// 256,000 x 2,304: 402 -> 385 and 463 -> 457; 2,304 x 9,216, 6: 22.9 -> 18.9 and 27.4 -> 21.9; 28,672 x 3,584 with GeGLU 83 -> 76 and
+// 101 -> 84; 18,432 x 2,304 with GeGLU 39.7 -> 38.7 and 47.9 -> 48.7; 4,096 x 2,304: 12.7 -> 10.2 and 12.9 -> 13.9; 2,048 x 2,048: 10.7 -> 6.7
+// and 11.1 -> 8.7; 65,536 x 1,024: 53.2 -> 55.1 and 59.6 -> 62.5.  The error against 64 bits falls from 3e-7 to 1.3e-7 of the result.
+template <typename T> struct Four;
+template <> struct Four<float> { typedef f32x4 type; };
+template <> struct Four<bf16_t> { typedef uint2 type; };
+__device__ __forceinline__ f32x4 four_f32(const f32x4& v) { return v; }
+__device__ __forceinline__ f32x4 four_f32(const uint2& v) {
+  return f32x4{bf16_bits_to_f32(v.x & 0xffffu), bf16_bits_to_f32(v.x >> 16), bf16_bits_to_f32(v.y & 0xffffu), bf16_bits_to_f32(v.y >> 16)};
+}
+__device__ __forceinline__ f32x4 four_once(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p)); }
+__device__ __forceinline__ uint2 four_once(const bf16_t* p) { return *reinterpret_cast<const uint2*>(p); }
+
+// The sum of a tile over the accumulators a and blocks b, in the order of the kernel above (its lanes' distances 32 and 16: a; 8, 4, 2, 1: b), and
+// its outputs: `v` holds rows n_first .. + 3 (with GeGLU the gate rows of outputs n_first and n_first + 1, then their up rows) of token
+// m_first + lane % 4.
+template <typename TO, bool GEGLU>
+__device__ __forceinline__ void finish_tile(f32x4 v, TO* __restrict__ y, int m_first, int n_first, int M, int N, int epi, float param, int full, int lane) {
+  auto bits = [](float f) { return __float_as_uint(f); };
+  float h[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto p = __builtin_amdgcn_permlane32_swap(bits(v[i]), bits(v[i + 2]), false, false);
+    h[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+  const auto p = __builtin_amdgcn_permlane16_swap(bits(h[0]), bits(h[1]), false, false);
+  float o = __uint_as_float(p[0]) + __uint_as_float(p[1]);                  // row lane / 16 of the four
+  o += __uint_as_float(dpp_move<DPP_ROR8>(bits(o)));
+  o += __uint_as_float(dpp_move<0x1B>(dpp_move<0x141>(bits(o))));           // lane ^ 4
+  const int m = m_first + (lane & 3);
+  int n = n_first + (lane >> 4);
+  bool mine = (lane & 12) == 0 && m < M;
+  if (GEGLU) {
+    const auto q = __builtin_amdgcn_permlane32_swap(bits(o), bits(o), false, false);
+    o = gated_act(o, __uint_as_float(q[1]), param, full);
+    n = n_first + ((lane >> 4) & 1);
+    mine = mine && lane < 32;
+  }
+  if (epi == ALICE_EPI_SOFTCAP) o = unary_act(o, param, full);
+  if (mine && n < N) store_f32(y, (size_t)m * N + n, o);
+}
+
+// Many blocks: a wave takes 8 rows of W (with GeGLU the gate and up rows of 4 outputs), four steps of 64 elements on their way, an
+// accumulator set for each a; the tokens' elements wait in LDS, four tokens' pieces side by side, the next chunk's in registers.
+// What bounds it: reading W, in pieces of 256 bytes of four rows with neighbouring lanes in different rows (5.2 to 6.2 TB/s).
+// NT threads a block: with 512 fewer blocks ask for the tokens' elements (256,000 x 2,304 at 16 tokens 473 -> 450).
+constexpr int some_chunk(int MT) { return MT == 8 ? 768 : 512; }       // elements of a token that a block keeps
+
+template <typename TA, typename TW, typename TO, bool GEGLU, int MT, int NT>
+__global__ __launch_bounds__(NT, MT == 8 ? 3 : 2) void linear_some_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y, int M,
+                                                                          int N, int K, int kslice, int epi, float param, int full) {
+  constexpr int NX = MT / 4, R = 2, U = 4, SEG = 64, KC = some_chunk(MT), P = KC / NT;     // a round of the block: NT elements of four tokens
+  static_assert(KC % NT == 0 && KC % (U * SEG) == 0, "whole rounds, whole turns");
+  typedef typename Four<TA>::type X4;
+  typedef typename Four<TW>::type W4;
+  __shared__ __align__(16) f32x4 xs[NX * KC];                 // [token / 4][element / 4][token % 4]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i4 = lane & 3, blk = lane >> 2;
+  const int n0 = (blockIdx.x * (NT / 64) + wave) * (GEGLU ? 2 * R : 4 * R);
+  const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);
+  const TW* wrow[R];                                          // rows beyond the last are read as the last and not written
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    wrow[r] = W + (size_t)(GEGLU ? (i4 >> 1) * N + min(n0 + 2 * r + (i4 & 1), N - 1) : min(n0 + 4 * r + i4, N - 1)) * K;
+  f32x4 acc[4][R][NX];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int x = 0; x < NX; ++x) acc[a][r][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+  W4 w[U][R];
+  X4 v[NX][P];
+  auto fetch = [&](int u, int k) {                            // unconditional: behind the slice its last four elements
+    const int at = min(k + blk * 4, k_end - 4);
+#pragma unroll
+    for (int r = 0; r < R; ++r) w[u][r] = four_once(wrow[r] + at);
+  };
+  auto load_x = [&](int c0) {
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+        v[x][p] = *reinterpret_cast<const X4*>(A + (size_t)min(4 * x + (tid & 3), M - 1) * K + min(c0 + p * NT + (tid >> 2) * 4, k_end - 4));
+  };
+  load_x(k_begin);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) fetch(u, k_begin + u * SEG);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int c0 = k_begin; c0 < k_end; c0 += KC) {
+    if (c0 > k_begin) lds_barrier();
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const int k = p * NT + (tid >> 2) * 4;
+        xs[x * KC + k + (tid & 3)] = c0 + k < k_end ? four_f32(v[x][p]) : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    if (c0 + KC < k_end) load_x(c0 + KC);
+    lds_barrier();
+    const int stop = min(k_end - c0, KC);
+    for (int s = 0; s < stop; s += U * SEG) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = s + u * SEG;
+        if (k < stop) {                                       // (the same for the whole block)
+          f32x4 wf[R];
+#pragma unroll
+          for (int r = 0; r < R; ++r) wf[r] = four_f32(w[u][r]);
+          if (k + SEG > stop) {                               // what was read again behind the end: zeros
+#pragma unroll
+            for (int r = 0; r < R; ++r) wf[r] = k + blk * 4 < stop ? wf[r] : f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+#pragma unroll
+          for (int x = 0; x < NX; ++x) {
+            const f32x4 xv = xs[x * KC + k + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int r = 0; r < R; ++r) acc[u][r][x] = __builtin_amdgcn_mfma_f32_4x4x1f32(wf[r][e], xv[e], acc[u][r][x], 0, 0, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(u, c0 + k + U * SEG);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  TO* y = Y + (size_t)blockIdx.y * M * N;
+#pragma unroll
+  for (int x = 0; x < NX; ++x)
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      finish_tile<TO, GEGLU>((acc[0][r][x] + acc[2][r][x]) + (acc[1][r][x] + acc[3][r][x]), y, 4 * x, n0 + (GEGLU ? 2 : 4) * r, M, N, epi, param, full, lane);
+}
+
+// Fewer blocks: the four waves share 16 rows of W (with GeGLU the gate and up rows of 8 outputs), a wave the 64 elements number a of every
+// 256; W and the tokens' elements come straight from memory, two steps of each, and the accumulators meet in LDS.  4,096 x 2,304 at 8 and 16 tokens
+// 10.2 and 13.7 us, 13.7 and 17.1 by the kernel above; 2,304 x 9,216 whole 27 and 36 (44 and 54); with three blocks a CU and more it is the slower.
+template <typename TA, typename TW, typename TO, bool GEGLU, int MT>
+__global__ __launch_bounds__(256, MT == 8 ? 4 : 3) void linear_quarters_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y, int M,
+                                                                               int N, int K, int kslice, int epi, float param, int full) {
+  constexpr int NX = MT / 4, R = 4, U = 2, TURN = 8;          // TURN: tiles that meet at a time
+  static_assert(R * NX % TURN == 0, "whole turns");
+  typedef typename Four<TA>::type X4;
+  typedef typename Four<TW>::type W4;
+  __shared__ __align__(16) f32x4 red[4][TURN][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i4 = lane & 3, blk = lane >> 2;
+  const int n0 = blockIdx.x * (GEGLU ? 2 * R : 4 * R);
+  const int k_begin = blockIdx.y * kslice, k_end = min(K, k_begin + kslice);
+  const TW* wrow[R];                                          // rows and tokens beyond the last are read as the last and not written
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    wrow[r] = W + (size_t)(GEGLU ? (i4 >> 1) * N + min(n0 + 2 * r + (i4 & 1), N - 1) : min(n0 + 4 * r + i4, N - 1)) * K;
+  const TA* xrow[NX];
+#pragma unroll
+  for (int x = 0; x < NX; ++x) xrow[x] = A + (size_t)min(4 * x + i4, M - 1) * K;
+  f32x4 acc[R][NX];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int x = 0; x < NX; ++x) acc[r][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+  W4 w[U][R];
+  X4 v[U][NX];
+  auto fetch = [&](int u, int k) {                            // unconditional: behind the slice its last four elements
+    const int at = min(k + blk * 4, k_end - 4);
+#pragma unroll
+    for (int x = 0; x < NX; ++x) v[u][x] = *reinterpret_cast<const X4*>(xrow[x] + at);
+#pragma unroll
+    for (int r = 0; r < R; ++r) w[u][r] = four_once(wrow[r] + at);
+  };
+  const int k0 = k_begin + wave * 64;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    fetch(u, k0 + u * 256);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (int s = k0; s < k_end; s += U * 256) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = s + u * 256;
+      if (k < k_end) {                                        // (the same for the whole wave)
+        f32x4 wf[R], xf[NX];
+#pragma unroll
+        for (int r = 0; r < R; ++r) wf[r] = four_f32(w[u][r]);
+#pragma unroll
+        for (int x = 0; x < NX; ++x) xf[x] = four_f32(v[u][x]);
+        if (k + 64 > k_end) {                                 // what was read again behind the end: zeros on both sides
+          const bool in = k + blk * 4 < k_end;
+#pragma unroll
+          for (int r = 0; r < R; ++r) wf[r] = in ? wf[r] : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int x = 0; x < NX; ++x) xf[x] = in ? xf[x] : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int x = 0; x < NX; ++x)
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[r][x] = __builtin_amdgcn_mfma_f32_4x4x1f32(wf[r][e], xf[x][e], acc[r][x], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(u, k + U * 256);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  TO* y = Y + (size_t)blockIdx.y * M * N;
+#pragma unroll
+  for (int t0 = 0; t0 < R * NX; t0 += TURN) {
+    if (t0 > 0) lds_barrier();
+#pragma unroll
+    for (int t = 0; t < TURN; ++t) red[wave][t][lane] = acc[(t0 + t) / NX][(t0 + t) % NX];
+    lds_barrier();
+    for (int t = wave; t < TURN; t += 4)
+      finish_tile<TO, GEGLU>((red[0][t][lane] + red[2][t][lane]) + (red[1][t][lane] + red[3][t][lane]), y, (t0 + t) % NX * 4,
+                             n0 + (GEGLU ? 2 : 4) * ((t0 + t) / NX), M, N, epi, param, full, lane);
+  }
+}
+
+// The three ways give the same bits, so the rule may look at the number of tokens.  Blocks of 16 rows and four tokens that find a CU
+// each, or two and a short way, go as up to four tokens do (1,024 x 2,048 at 16 tokens 6.2 us, 14.2 with 8 rows a wave; 2,048 x 2,048 at 16 8.7
+// and 11.4 in quarters); up to 256 blocks of 16 rows in quarters; more with 8 rows a wave.  There, beyond 8 tokens, eight waves a block
+// where their blocks fill one round of the CUs (216 blocks: 22.6 -> 21.5) or many with a long way (448: 87.6 -> 83.6; 151,936 x 1,024: 138.6, and 149.8
+// with eight); not with a second round that is nearly empty (288: 48.7 -> 55.8), nor where half the CUs get none (108: 8.5 -> 12.3).
+template <typename TA, typename TW, typename TO>
+int launch_more(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split, hipStream_t stream) {
+  const int kslice = slice_of(K, split), rows = epi == ALICE_EPI_GEGLU ? 2 * N : N;
+  const int blocks16 = ceil_div(rows, 16) * split, by_four = blocks16 * ceil_div(M, FEW_MT), blocks64 = ceil_div(rows, 64) * split;
+  if (by_four <= 256 || (by_four <= 512 && kslice <= 2048)) return launch_few<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full, split, stream);
+  const bool quarters = blocks16 <= 256, wide = M > 8 && ((blocks64 > 160 && blocks64 <= 256) || (blocks64 >= 400 && kslice >= 2048));
+  const dim3 grid(ceil_div(rows, quarters ? 16 : wide ? 64 : 32), split);
+#define GO3(NAME, THREADS, ...) NAME<TA, TW, TO, __VA_ARGS__><<<grid, THREADS, 0, stream>>>((const TA*)x, (const TW*)w, (TO*)y, M, N, K, kslice, epi, epi_param, full)
+#define GO2(GEGLU)                                                           \
+  do {                                                                       \
+    if (quarters && M <= 8) GO3(linear_quarters_kernel, 256, GEGLU, 8);      \
+    else if (quarters) GO3(linear_quarters_kernel, 256, GEGLU, 16);          \
+    else if (M <= 8) GO3(linear_some_kernel, 256, GEGLU, 8, 256);            \
+    else if (M <= 12 && !wide) GO3(linear_some_kernel, 256, GEGLU, 12, 256); \
+    else if (M <= 12) GO3(linear_some_kernel, 512, GEGLU, 12, 512);          \
+    else if (!wide) GO3(linear_some_kernel, 256, GEGLU, 16, 256);            \
+    else GO3(linear_some_kernel, 512, GEGLU, 16, 512);                       \
+  } while (0)
+  if (epi == ALICE_EPI_GEGLU) GO2(true); else GO2(false);
+#undef GO2
+#undef GO3
   ALICE_LAUNCH_CHECK();
   return 0;
 }
@@ -643,7 +900,7 @@ int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int
 
 }  // namespace
 
-// Whether up to 4 tokens go on FMAs, by the inner dimension: rows of whole units of four elements, long enough that the
+// Whether up to 4 tokens go on FMAs (and up to 16 as those do), by the inner dimension: rows of whole units of four elements, long enough that the
 // block's start does not outweigh them (65,536 rows by 256: 22.7 us, 16.2 on the matrix instruction; by 1,024 and more it is faster), and
 // slices that are (of 256 elements: 8.2 us, 7.2 on the matrix instruction).  The rule of the slices and that of the launch ask here.
 static bool few_by_length(int K, int split) { return K % 4 == 0 && K >= 1024 && (split == 1 || slice_of(K, split) >= 512); }
@@ -690,13 +947,14 @@ int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype,
   if (M == 0) return 0;
   int rc = 0;
   DISPATCH_DTYPE(x_dtype, TA, DISPATCH_DTYPE(w_dtype, TW, DISPATCH_DTYPE(y_dtype, TO, {
-    const bool few = M <= FEW_MT && few_by_fours(x, x_dtype, w, w_dtype, K, split_k);
+    const bool few = M <= 16 && few_by_fours(x, x_dtype, w, w_dtype, K, split_k);
     // One token: the same sums either way; a wave a row is the faster start (1,000 x 1,024: 3.6 and 4.5 us, 3,584 x 4,096: 14.1 and
     // 14.9), four rows a wave read longer matrices faster (8,192 x 3,584: 22.3 and 21.3, gate and up 34.5 and 30.4).
     const bool large = (size_t)N * K * sizeof(TW) * (epi == ALICE_EPI_GEGLU ? 2 : 1) >= ((size_t)80 << 20);
     // (In slices, which are planned for four rows a wave, a wave a row takes what that does not: operands at any address.)
     if (M == 1 && !(few && (large || split_k > 1))) rc = launch_single<TA, TW, TO>(x, w, y, N, K, epi, epi_param, full_precision, split_k, stream);
-    else if (few) rc = launch_few<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
+    else if (few && M <= FEW_MT) rc = launch_few<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
+    else if (few) rc = launch_more<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
     else rc = M <= 16 ? launch_rows<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream)
                       : launch_tiled<TA, TW, TO>(x, w, y, M, N, K, epi, epi_param, full_precision, split_k, stream);
   })));
