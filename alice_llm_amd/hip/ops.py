@@ -1505,9 +1505,12 @@ def decode_splits(n_seqs: int, num_kv_heads: int, max_context: int, head_dim: in
     was measured on the 2B, 9B and 27B shapes (1 to 32 sequences of 100 to 6,000 keys), among those that leave a CU one block.
     A block takes 0.57 us for every 32 keys of head size 256 (what a CU reads) and 0.5 a round of its four waves, all blocks
     together read 6.5 TB/s (the shorter of the two is not quite hidden), and the output projection pays for every split
-    that it combines (up to 16 splits of 16 sequences; beyond, a kernel of its own combines them).  Captured steps name
-    the context rounded up to 512: half of that is taken off.  Against the earlier rule, at least two rounds a wave: a 2B
-    step of one sequence at 2,048 keys 1,719 -> 1,660 us, of four at 300 1,726 -> 1,620, of eight at 500 1,742 -> 1,685."""
+    that it combines (up to 16 splits of 16 sequences; beyond, a kernel of its own combines them, in 6 us and 0.1 a split).  Captured
+    steps name the context rounded up to 512: half of that is taken off.  Against the earlier rule, at least two rounds a wave: a 2B
+    step of one sequence at 2,048 keys 1,719 -> 1,660 us, of four at 300 1,726 -> 1,620, of eight at 500 1,742 -> 1,685.
+    Over 684 shapes (1 to 16 kv heads of 64, 128 and 256, 1 to 64 sequences of 512 to 16,384 keys, four lengths each) the times that it
+    chooses are 3 % above the best ones and 11 % below those of the earlier kernel and rule; five are 3 % or more above those, by up
+    to 9 %: one or two kv heads of many keys, where 24 to 32 splits would be a little better than 16."""
     n_blocks = -(-max(max_context - 256, min(max_context, 256)) // 32)
     size = head_dim / 256
     whole = n_seqs * num_kv_heads * n_blocks * 32768 * size / 6.5e6
@@ -1517,7 +1520,7 @@ def decode_splits(n_seqs: int, num_kv_heads: int, max_context: int, head_dim: in
         block = 0.57 * size * run + 0.5 * -(-run // 4)
         cost = max(whole, block) + 0.3 * min(whole, block)
         if s > 1:
-            cost += (0.12 + 0.05 * n_seqs) * s if n_seqs <= 16 and s <= 16 else 9.0 + 0.02 * s
+            cost += (0.12 + 0.05 * n_seqs) * s if n_seqs <= 16 and s <= 16 else 6.0 + 0.1 * s
         if best_cost is None or cost < best_cost:
             best, best_cost = s, cost
     return best
