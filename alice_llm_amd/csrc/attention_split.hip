@@ -60,13 +60,14 @@ __device__ __forceinline__ float sum_over_32(float v) {
 }
 
 // (128 registers let a second block work while one waits; the widest groups need more)
-template <typename T, int PER>
+// U: loads of keys, of values on their way at a time, no more than a wave has of its rows.
+template <typename T, int PER, int U>
 __global__ __launch_bounds__(NT, PER <= 8 ? 4 : 2) void attn_split_kernel(const T* __restrict__ q, const T* __restrict__ k_pool,
                                                             const T* __restrict__ v_pool, SplitArgs a) {
   constexpr bool FULL = sizeof(T) == 4;
   constexpr int VEC = 16 / sizeof(T);
   constexpr int HG = PER < 4 ? PER : 4;               // heads that meet in LDS at a time
-  constexpr int UK = PER >= 8 ? 4 : 8, UV = UK;       // loads of keys, of values on their way at a time
+  constexpr int UK = U, UV = U;
   constexpr int OWN = PER >= 4 ? PER / 4 : 1;         // heads of a key whose sums a lane ends up with
   __shared__ float ps[PER][KEYS];
   __shared__ int rows_of[KEYS];                       // the row of each of the block's keys in kv head 0's part of its page
@@ -401,19 +402,30 @@ extern "C" int alice_attention_split(const void* q, int dtype, const void* k_poo
               bias_slopes, part_ml, part_o};
   const int per = nH / nKV;
   dim3 grid(T, nKV, runs);
-#define GO(TT, PER) attn_split_kernel<TT, PER><<<grid, NT, 0, stream>>>((const TT*)q, (const TT*)k_pool, (const TT*)v_pool, a)
-#define BY_PER(TT)                 \
-  do {                             \
-    if (per <= 1) GO(TT, 1);       \
-    else if (per <= 2) GO(TT, 2);  \
-    else if (per <= 4) GO(TT, 4);  \
-    else if (per <= 8) GO(TT, 8);  \
-    else GO(TT, 16);               \
+  // A wave's 32 keys are that many loads of whole rows, half as many as lanes read a row, and so are a thread's values: what is asked for
+  // beyond is a row that was read (32 sequences of 2,000 keys in bfloat16, 8 own kv heads of 32: 32.1 us with eight loads of which six
+  // are such, 23.8 with two; 16 of 64: 67.6 with eight, 59.9 with four).
+  const int piece = 16 / (dtype == DT_F32 ? 4 : 2), widest = max(ceil_div(d, piece), ceil_div(dv, piece));
+#define GO2(TT, PER, U) attn_split_kernel<TT, PER, U><<<grid, NT, 0, stream>>>((const TT*)q, (const TT*)k_pool, (const TT*)v_pool, a)
+#define GO(TT, PER, MOST)                            \
+  do {                                               \
+    if (widest <= 4) GO2(TT, PER, 2);                \
+    else if (widest <= 8) GO2(TT, PER, 4);           \
+    else GO2(TT, PER, MOST);                         \
+  } while (0)
+#define BY_PER(TT)                    \
+  do {                                \
+    if (per <= 1) GO(TT, 1, 8);       \
+    else if (per <= 2) GO(TT, 2, 8);  \
+    else if (per <= 4) GO(TT, 4, 8);  \
+    else if (per <= 8) GO(TT, 8, 4);  \
+    else GO(TT, 16, 4);               \
   } while (0)
   if (dtype == DT_F32) BY_PER(float);
   else BY_PER(bf16_t);
 #undef BY_PER
 #undef GO
+#undef GO2
   ALICE_LAUNCH_CHECK();
   CombineArgs c{positions, nH, nKV, dv, runs, n_vh, part_ml, part_o, sink, vrot_cos, vrot_sin, gate, gate_stride, gate_mode, out_scale, out32};
   dim3 g2(T, nH, out32 ? nKV : 1);
