@@ -23,7 +23,7 @@ struct Branches {
 // result) issued together.
 template <typename TW, typename TO, bool FULL, int EPT>
 __global__ __launch_bounds__(1024) void add_branches_kernel(float* __restrict__ resid, Branches a, TO* __restrict__ out, int H) {
-  __shared__ float red[17];
+  __shared__ float red[16];
   const size_t row = (size_t)blockIdx.x * H;
   float v[ALICE_MAX_BRANCHES][EPT];
   float x[EPT];

@@ -49,7 +49,7 @@ __global__ __launch_bounds__(THREADS) void attn_generic_kernel(
     int dv, const T* __restrict__ gate, int gate_stride, AttnExtras x) {
   __shared__ float qs[256];
   __shared__ float sc[CHUNK];
-  __shared__ float red[17];
+  __shared__ float red[16];
   __shared__ float part[THREADS];
 
   const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;

@@ -50,7 +50,8 @@ template <> __device__ __forceinline__ float round_to<bf16_t>(float v) { return 
 // A reduction over the 64 lanes, every lane gets the result: the butterfly over lane distances 32, 16, 8, 4, 2, 1 by lane-swap
 // and DPP moves, a few cycles each, where a shuffle goes through the LDS unit (about 60 cycles a step, one waiting for the
 // other).  The same partners in the same order as shuffles by 32 .. 1, so sums have the same bits: after the step over 8 a
-// row of 16 lanes repeats itself every 8, which makes a rotation by 4 the exchange over 4.  All 64 lanes take part.
+// row of 16 lanes repeats itself every 8, which makes a rotation by 4 the exchange over 4.  All 64 lanes must be active: a swap
+// with a lane that is not leaves a lane its own value twice, and the sum is wrong in every lane.
 // (Before and after, everything else equal: the draw behind 64 rows of 256,000 logits 49.2 and 47.2 us, a 2B decode step of
 // eight sequences with its 53 norms 1,973 and 1,952 us.)
 template <int CTRL>
@@ -89,7 +90,7 @@ __device__ __forceinline__ T wave_reduce(T v, F op) {
 __device__ __forceinline__ float wave_sum(float v) { return wave_reduce(v, [](float a, float b) { return a + b; }); }
 __device__ __forceinline__ float wave_max(float v) { return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); }); }
 
-// Sum over a block of up to 1024 threads (whole waves); every thread gets the result.  `red` holds 17 floats.  Every wave adds
+// Sum over a block of up to 1024 threads (whole waves); every thread gets the result.  `red` holds 16 floats, one a wave.  Every wave adds
 // up the waves' sums by itself: one barrier fewer than through the first wave.
 __device__ __forceinline__ float block_sum(float v, float* red) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;

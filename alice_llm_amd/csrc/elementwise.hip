@@ -67,7 +67,7 @@ __global__ void add_norm_kernel(float* __restrict__ resid, const float* __restri
                                 const TW* __restrict__ w_post, const TW* __restrict__ w_pre, const TW* __restrict__ b_pre,
                                 TO* __restrict__ out, const int* __restrict__ rows, int H,
                                 float eps_post, float eps_pre, float off_post, float off_pre, int out_layout) {
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int r = blockIdx.x;
   const size_t src = (size_t)(rows ? rows[r] : r) * H;
   float* x = resid + src;
@@ -153,7 +153,7 @@ __global__ void add_norm_regs_kernel(float* __restrict__ resid, const float* __r
                                      TO* __restrict__ out, const int* __restrict__ rows, int H,
                                      float eps_post, float eps_pre, float off_post, float off_pre, int out_layout) {
   typedef typename raw_of<TW>::type RW;
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int r = blockIdx.x;
   const size_t src = (size_t)(rows ? rows[r] : r) * H;
   int idx[EPT];

@@ -157,7 +157,7 @@ template <typename TW, typename TO>
 __global__ __launch_bounds__(256) void gla_finish_kernel(const float* __restrict__ o32, const float* __restrict__ rows, int row_w,
                                                          int g_col, const TW* __restrict__ norm_w, float eps, float out_scale,
                                                          TO* __restrict__ out, int H, int dv) {
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int t = blockIdx.x, h = blockIdx.y;
   const float* o = o32 + ((size_t)t * H + h) * dv;
   float ss = 0.f;

@@ -26,7 +26,7 @@ __global__ __launch_bounds__(PREP_THREADS) void latent_prepare_kernel(
     const float* __restrict__ wc, float eps, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
     const int* __restrict__ positions, const int* __restrict__ seq_of_token, const int* __restrict__ block_table,
     int bt_stride, int page_size, int n_pages, TO* __restrict__ a_out, TO* __restrict__ k_pool) {
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int t = blockIdx.x, tid = threadIdx.x;
   const float* row = rows + (size_t)t * row_w;
   float s = 0.f;
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(LA_THREADS) void latent_attention_kernel(
     int page_size, float scale, int window, int DG) {
   extern __shared__ float lds[];                      // q [R + r], then the partial outputs [G][R]
   __shared__ float sc[LA_CHUNK];
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int D = R + r;
   float* qs = lds;
   float* part = lds + D;

@@ -52,7 +52,7 @@ __global__ __launch_bounds__(THREADS) void mlstm_step_kernel(
   float* ks = qs + d;              // d
   float* vs = ks + d;              // dv
   float* part = vs + dv;           // THREADS * MAXC
-  __shared__ float red[17];
+  __shared__ float red[16];
 
   const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const int t0 = cu_seqlens[s], t1 = cu_seqlens[s + 1];
@@ -477,7 +477,7 @@ __global__ __launch_bounds__(THREADS) void mlstm_cols_kernel(
   float* ks = qs + d;              // d
   float* ns = ks + d;              // d
   float* part = ns + d;            // 4 * 64
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = blockIdx.z * 64 + lane;
   const bool col = c < dv;
@@ -556,7 +556,7 @@ __global__ __launch_bounds__(THREADS) void mlstm_head_kernel(
   float* qs = lds;                 // d
   float* ks = qs + d;              // d
   float* ns = ks + d;              // d
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int s = blockIdx.x, h = blockIdx.y, c = threadIdx.x;
   const bool col = c < dv;
   const int t0 = cu_seqlens[s], t1 = cu_seqlens[s + 1];
@@ -617,7 +617,7 @@ __global__ void mlstm_finish_kernel(const float* __restrict__ work, const float*
                                     const float* __restrict__ proj, int row_w,
                                     const void* __restrict__ norm_w, int norm_dtype, TO* __restrict__ out,
                                     int H, int d, int dv, float eps) {
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int t = blockIdx.x, h = blockIdx.y;
   const float* o = work + (size_t)t * H * dv + h * dv;
   const float* g = proj + (size_t)t * row_w + 2 * H * d + H * dv + h * dv;

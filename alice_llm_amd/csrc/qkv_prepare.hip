@@ -26,7 +26,7 @@ namespace {
 template <typename TI>
 __global__ __launch_bounds__(256) void projection_rms_kernel(const TI* __restrict__ rows, int row_w, const float* __restrict__ bias,
                                                              float* __restrict__ inv, int n_q, int n_k, float eps) {
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int t = blockIdx.x, part = blockIdx.y;
   const int c0 = part ? n_q : 0, n = part ? n_k : n_q;
   const TI* row = rows + (size_t)t * row_w;

@@ -459,7 +459,7 @@ template <typename TO, typename TG>
 __global__ __launch_bounds__(1024) void norm_gate_kernel(const float* __restrict__ x, int width, int parts, const TG* __restrict__ gate,
                                                         int gate_w, int gate_col, int gate_act, const float* __restrict__ w,
                                                         int w_shared, float eps, TO* __restrict__ out) {
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int t = blockIdx.x, g = blockIdx.y, n = width / parts;
   const float* xr = x + (size_t)t * width + (size_t)g * n;
   const TG* gr = gate ? gate + (size_t)t * gate_w + gate_col + (size_t)g * n : nullptr;
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(LANES > 256 ? LANES : 256) void norm_gate_regs_kern
                                                                                   int gate_act, const float* __restrict__ w, int w_shared,
                                                                                   float eps, TO* __restrict__ out) {
   constexpr int THREADS = LANES > 256 ? LANES : 256, PPB = THREADS / LANES;
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int lane = threadIdx.x % LANES, n = width / parts;
   const long p = (long)blockIdx.x * PPB + threadIdx.x / LANES;       // (token, part); beyond the last: computed on it, not stored
   const bool in = p < rows;

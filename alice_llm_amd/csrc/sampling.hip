@@ -188,7 +188,7 @@ __device__ __forceinline__ float row_max(const SampleWork& w, int b) {
 
 template <int VEC>
 __global__ __launch_bounds__(SB) void chunk_max_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t) {
-  __shared__ float red[17];
+  __shared__ float red[16];
   const int b = blockIdx.y, c = blockIdx.x;
   const float* row = logits + (size_t)b * V;
   const int lo = c * w.tiles_per_chunk * TILE, hi = min(V, lo + w.tiles_per_chunk * TILE);
@@ -491,7 +491,7 @@ __device__ __forceinline__ uint32_t list_threshold(const float* __restrict__ row
 template <int VEC>
 __global__ __launch_bounds__(ST) void row_threshold_kernel(const float* __restrict__ logits, SampleWork w, int V, float inv_t,
                                                            int top_k, float top_p) {
-  __shared__ float red[17];
+  __shared__ float red[16];
   __shared__ int ired[ST / 64];
   __shared__ uint32_t list[CAP];
   __shared__ unsigned long long list_mass[CAP];
@@ -905,7 +905,7 @@ __global__ __launch_bounds__(ST) void row_topk_kernel(const float* __restrict__ 
   __shared__ __align__(16) uint32_t keys[256], wmin[ST / 64];
   __shared__ __align__(16) unsigned long long wsum[ST / 64];
   __shared__ int n_left, last_kept, rounds, pick[2];
-  __shared__ __align__(16) float red[17], wred[ST / 64], tsum[TOPK_TILES];
+  __shared__ __align__(16) float red[16], wred[ST / 64], tsum[TOPK_TILES];
   __shared__ float carry[2];
   __shared__ int ired[ST / 64];
   __shared__ uint32_t best;
