@@ -247,8 +247,8 @@ int slice_of(int K, int split) { return ceil_div(ceil_div(K, split), 128) * 128;
 // elements behind the last whole chunk one by one, by the wave whose turn it is: 2,304 rows by 2,305 at 4 tokens 9.0 us (by 2,304
 // 9.1; on the tile of 64 tokens 71).
 //
-// What bounds it: reading W.  At 4 tokens (2B shape): gate and up (170 MB) 34.6 us, 4.9 TB/s, the output head (2.36 GB)
-// 391 us, 6.0; a wave a row on FMAs, which read every token's elements again for every row, 39.5 and 632 us.
+// What bounds it: reading W, in pieces of 128 bytes of a row.  With weights that no cache holds, at 4 tokens: 2,304 rows by 2,048 in eight
+// slices 7.0 us; the rows that the kernels below take now: gate and up of the 2B shape (170 MB) 37.4, 4.5 TB/s, the output head (2.36 GB) 400, 5.9.
 template <bool ALIGNED>
 __device__ __forceinline__ f32x4 piece(const float* __restrict__ p) {
   struct __attribute__((packed, aligned(4))) Any { f32x4 v; };
@@ -372,9 +372,10 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const TA* __restri
 }
 
 // Slices of the inner dimension for 2 to 16 tokens: three blocks a CU where the rows alone do not give them, slices of at
-// least 256 elements, and rather a few more slices than uneven ones.  At 4 tokens 2,304 rows by 9,216 take 38 us whole, 24.1 in
-// four slices, 21.8 in six; by 2,048: 10.6, 8.1, 8.5 in six (uneven), 7.2 in eight; 4,096 rows by 2,304: 14.1, 12.4 in four, 10.8
-// in three.
+// least 256 elements, and rather a few more slices than uneven ones.  At 4 tokens, on this kernel, 2,304 rows by 9,216 take 38 us whole,
+// 24.1 in four slices, 21.8 in six; by 2,048: 10.6, 8.1, 8.5 in six (uneven), 7.2 in eight; 4,096 rows by 2,304: 14.1, 12.4 in four, 10.8
+// in three.  On the kernels below, with weights that no cache holds: by 9,216 22.8 whole, 18.4 in four, 16.6 in six, 17.6 in eight; by 2,048 7.0
+// whole, 6.2 in three, 6.8 in four: the eight of 256 elements that this rule plans, here, are 7.0.
 int rows_split(int N, int K) {
   const int most = max(1, min(K / 256, 8)), least = min(ceil_div(768, ceil_div(N, 16)), most);
   for (int s = least; s <= most; ++s)
@@ -383,8 +384,9 @@ int rows_split(int N, int K) {
 }
 
 // One token: a wave a row of W (with GeGLU the gate row and the up row of an output) on FMAs, four elements a lane a step; the lanes'
-// sums meet in a fixed tree.  Any K, any address, any slices.  No column of the matrix instruction is idle: 18,432 rows by 2,304 with GeGLU
-// 25.9 us (31.7 as columns, which gain from 2 to 4 tokens on), 256,000 rows 373 (402), 2,304 by 9,216 16.3 (19.1 in slices).
+// sums meet in a fixed tree.  Any K, any address, any slices.  No column of the matrix instruction is idle.  With weights that no cache holds:
+// 3,584 rows by 4,096 14.1 us, 8,192 by 2,304 15.0 (5 TB/s); beyond some 80 MB four rows a wave are the faster (below): 18,432 by 2,304 with
+// GeGLU 33.5 us, 256,000 by 2,304 382.
 template <typename TA, typename TW, typename TO, bool GEGLU>
 __global__ __launch_bounds__(256) void linear_single_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TO* __restrict__ Y, int N,
                                                             int K, int kslice, int epi, float param, int full) {
@@ -441,9 +443,10 @@ int launch_single(const void* x, const void* w, void* y, int N, int K, int epi, 
 // reads W in pieces of 128 bytes of a row; here a load is a whole kilobyte, with the streaming hint (gate and up 35.4 -> 33.7 us,
 // the output head 394 -> 357; the 128-byte pieces get slower by it), and two of every row are on their way while two
 // are multiplied.  The tokens' elements are asked for ahead of W's first (33.7 -> 30.2 us: a block's start is what its CU waits for).
-// What bounds it: reading W, at 6.6 TB/s where it is long.  4 tokens, 2B shape, matrix instruction and this: q, k, v 12.6 and
-// 8.9 us, output projection 7.2 (8 slices) and 6.3 (3), gate and up 40.0 and 30.2, down 21.6 and 17.1, head 404 and 353; more tokens in
-// one block gain nothing by it (eight: 42 us for gate and up, 468 for the head), but four a block do where there are few blocks.
+// What bounds it: reading W, at 6.6 TB/s where it is long.  4 tokens, 2B shape, weights that no cache holds, matrix instruction and
+// this: q, k, v 12.4 and 8.7 us, gate and up 37.4 and 29.5, down (six slices) 21.6 and 16.6, head 400 and 355 (the output projection
+// goes in slices that are too short for it); more tokens in one block gain nothing by it (eight: 42 us for gate and up, 468 for the head),
+// but four a block do where there are few blocks.
 // Which products a token's sum adds, and in which order, depends on K and the slices alone: a lane's elements in their order, then
 // the lanes over the distances 32, 16 .. 1.  That is the order of the kernel for one token as well, and of those for 5 to 16 tokens below
 // (the same bits).
@@ -911,8 +914,9 @@ static bool few_by_fours(const void* x, int x_dtype, const void* w, int w_dtype,
 }
 
 // Slices for one token: W is read at 6.6 TB/s with three blocks a CU, at three quarters of that with few; the busiest CU reads
-// its blocks' rows at 40 GB/s or less; a slice more costs the add behind it 0.2 us.  (2,304 rows by 2,048: 3 or 4 slices, 6.3 and
-// 6.8 us; by 9,216: 6, 17.1, 24.4 whole; 3,584 by 14,336: 4, 38.0, 40.7 whole; 8,192 by 3,584: 1.)
+// its blocks' rows at 40 GB/s or less; a slice more costs the add behind it 0.2 us.  (Planned and measured, weights that no cache holds:
+// 2,304 rows by 2,048 whole, 7.2 us, 6.2 and 0.6 for the add in three; by 9,216 in 6, 16.8, 24.5 whole; 3,584 by 14,336 in 4, 35.3, 39.2 whole;
+// 8,192 by 3,584 in 2, 21.8, 20.7 whole.)
 static int single_split(int N, int K) {
   const int blocks = ceil_div(N, 4 * FEW_R);
   int best = 1;
@@ -948,8 +952,9 @@ int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype,
   int rc = 0;
   DISPATCH_DTYPE(x_dtype, TA, DISPATCH_DTYPE(w_dtype, TW, DISPATCH_DTYPE(y_dtype, TO, {
     const bool few = M <= 16 && few_by_fours(x, x_dtype, w, w_dtype, K, split_k);
-    // One token: the same sums either way; a wave a row is the faster start (1,000 x 1,024: 3.6 and 4.5 us, 3,584 x 4,096: 14.1 and
-    // 14.9), four rows a wave read longer matrices faster (8,192 x 3,584: 22.3 and 21.3, gate and up 34.5 and 30.4).
+    // One token: the same sums either way; a wave a row is the faster start (weights that no cache holds: 1,000 x 1,024 4.0 and 4.4 us, 3,584 x
+    // 4,096 14.1 and 14.8), four rows a wave read longer matrices faster (8,192 x 3,584: 21.8 and 21.0, 12,288 x 2,304 23.0 and 20.1, gate and
+    // up of the 2B shape 33.5 and 29.4); between 50 and 80 MB it goes either way by 4 %.
     const bool large = (size_t)N * K * sizeof(TW) * (epi == ALICE_EPI_GEGLU ? 2 : 1) >= ((size_t)80 << 20);
     // (In slices, which are planned for four rows a wave, a wave a row takes what that does not: operands at any address.)
     if (M == 1 && !(few && (large || split_k > 1))) rc = launch_single<TA, TW, TO>(x, w, y, N, K, epi, epi_param, full_precision, split_k, stream);
