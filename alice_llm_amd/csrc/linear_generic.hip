@@ -7,6 +7,7 @@
 // stacked (llama3.rs:14519-14534); softcap cap * tanh(y / cap) (llama3.rs:14606-14611).
 #include "common.h"
 #include "alice_hip.h"
+#include "linear_thirds.h"
 
 namespace {
 
@@ -206,14 +207,14 @@ struct Tile {
 constexpr Tile TILES[] = {{128, 128, 0.510f}, {128, 64, 0.500f}, {64, 96, 0.492f}, {64, 64, 0.490f}, {32, 64, 0.460f}};
 struct Plan {
   int tile, split;
+  float us;
 };
-Plan plan_mfma32(int M, int N, int K, bool geglu, int max_split) {
-  Plan best{3, 1};
-  float best_us = 1e30f;
+Plan plan_mfma32(int M, int N, int K, bool geglu, int min_split, int max_split) {
+  Plan best{3, min_split, 1e30f};
   for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
     const Tile& t = TILES[i];
     const int mt = ceil_div(M, t.bm), nt = ceil_div(N, geglu ? t.bn / 2 : t.bn);
-    for (int s = 1; s <= max_split; ++s) {
+    for (int s = min_split; s <= max_split; ++s) {
       const int ks = ceil_div(ceil_div(K, s), BK) * BK;
       if (s > 1 && (ks < 256 || (long)ks * (s - 1) >= K)) continue;      // no slice without elements
       const int blocks = ceil_div((long)mt * nt * s, 256);
@@ -221,7 +222,7 @@ Plan plan_mfma32(int M, int N, int K, bool geglu, int max_split) {
       float us = 8.f + (blocks + alone) * (2.f * t.bm * t.bn * (float)ks / (1e6f * t.rate) + 1.f);
       us = fmaxf(us, (geglu ? 2.f : 1.f) * N * (float)K * 4.f / 4.5e6f);
       if (s > 1) us += 2.f * s * (float)M * N * 4.f / 4.0e6f;
-      if (us < best_us) { best_us = us; best = Plan{i, s}; }
+      if (us < best.us) best = Plan{i, s, us};
     }
   }
   return best;
@@ -232,6 +233,12 @@ constexpr int MAX_SPLIT = 8;
 // up to 64 and to a multiple of 64 beyond, short prompts to a multiple of 16.  Any number of tokens here gives what either rounding of it
 // gives.  (Numbers of tokens on two sides of a multiple of 64 may add in another order: rounding, no more.)
 int planned_tokens(int M) { return M <= 32 ? 32 : ceil_div(M, 64) * 64; }
+static_assert(THIRDS_BK == BK, "both ways cut the inner dimension into the same slices");
+// Whether a product goes in thirds on the bfloat16 instruction: where that is estimated to be faster.  Both estimates are within a tenth of
+// what measures, and where they are that close either way will do.  (2B shape, the 32-bit instruction and thirds: 500 tokens gate and up 356
+// and 232 us, down 177 and 117, q, k, v 84 and 58, output 40 and 34; 128 tokens 105 and 75, 87 and 42, 32 and 38 (stays), 16 and 15; 32 tokens
+// 48 and 46, 28 and 23, 31 and 30, 8 and 8.)
+bool in_thirds(const ThirdsPlan& t, const Plan& p) { return t.us < p.us; }
 
 // Elements a slice of up to 16 tokens' products.
 int slice_of(int K, int split) { return ceil_div(ceil_div(K, split), 128) * 128; }
@@ -876,15 +883,18 @@ int launch_rows(const void* x, const void* w, void* y, int M, int N, int K, int 
 template <typename TA, typename TW, typename TO>
 int launch_tiled(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int full, int split,
                  hipStream_t stream) {
-  Plan p = plan_mfma32(M, N, K, epi == ALICE_EPI_GEGLU, 1);
-  if (split > 1) {                                            // the tile that goes best with this many slices
-    const Plan q = plan_mfma32(planned_tokens(M), N, K, false, MAX_SPLIT);
-    if (q.split == split) p = q;
-  }
+  const bool geglu = epi == ALICE_EPI_GEGLU;
   const int vec = K % 4 == 0 && ((uintptr_t)x & (4 * sizeof(TA) - 1)) == 0 && ((uintptr_t)w & (4 * sizeof(TW) - 1)) == 0;
+  Plan p = plan_mfma32(planned_tokens(M), N, K, geglu, split, split);         // the tile that goes best with this many slices
+  if constexpr (sizeof(TA) == 4 && sizeof(TW) == 4 && sizeof(TO) == 4) {
+    const ThirdsPlan t = alice_linear_thirds_plan(planned_tokens(M), N, K, geglu, split, split);
+    if (vec && in_thirds(t, p))
+      return alice_linear_thirds((const float*)x, (const float*)w, (float*)y, M, N, K, epi, epi_param, full, t, stream);
+  }
+  if (split == 1) p = plan_mfma32(M, N, K, geglu, 1, 1);      // (no tile changes the order of the sums)
   if (!vec) p.tile = 3;                                       // one tile for rows that are no multiples of four elements
   const int kslice = ceil_div(ceil_div(K, split), BK) * BK;
-  const int BM = TILES[p.tile].bm, cols = epi == ALICE_EPI_GEGLU ? TILES[p.tile].bn / 2 : TILES[p.tile].bn;
+  const int BM = TILES[p.tile].bm, cols = geglu ? TILES[p.tile].bn / 2 : TILES[p.tile].bn;
   const int mt = ceil_div(M, BM), nt = ceil_div(N, cols);
   ALICE_CHECK((long)mt * nt < (1l << 30), "linear: too many tiles for one launch");
   const int wide = N % 4 == 0 && ((uintptr_t)y & 15) == 0;
@@ -935,7 +945,16 @@ static int single_split(int N, int K) {
 // number, whatever captured steps round theirs to).
 int alice_linear_split_hint_generic(int M, int N, int K) {
   if (M == 1) return few_by_length(K, 1) ? single_split(N, K) : 1;
-  return M <= 16 ? rows_split(N, K) : plan_mfma32(planned_tokens(M), N, K, false, MAX_SPLIT).split;
+  if (M <= 16) return rows_split(N, K);
+  const Plan p = plan_mfma32(planned_tokens(M), N, K, false, 1, MAX_SPLIT);
+  const ThirdsPlan t = alice_linear_thirds_plan(planned_tokens(M), N, K, false, 1, MAX_SPLIT);
+  return K % 4 == 0 && in_thirds(t, p) ? t.split : p.split;
+}
+
+// The tile of a product of more than 16 tokens that goes in thirds, -1 if it goes on the 32-bit instruction (float32 and aligned operands).
+extern "C" int alice_linear_thirds_tile(int M, int N, int K, int geglu, int split) {
+  const ThirdsPlan t = alice_linear_thirds_plan(planned_tokens(M), N, K, geglu != 0, split, split);
+  return M > 16 && K % 4 == 0 && in_thirds(t, plan_mfma32(planned_tokens(M), N, K, geglu != 0, split, split)) ? t.tile : -1;
 }
 
 int alice_linear_generic(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype,

@@ -1,0 +1,337 @@
+// 32-bit products of more than 16 tokens on the bfloat16 matrix instruction: y[M, N] = x[M, K] . W[N, K]^T, all float32
+// (gguf.rs:4063-4074; GeGLU llama3.rs:14519-14534, softcap llama3.rs:14606-14611), with 32-bit sums and no less precision than
+// 32-bit products have.
+//
+// A float32 is the sum of three bfloat16 numbers: each takes the next eight bits of the mantissa, rounded to nearest, and what it
+// leaves is exact.  Of the nine products of two such sums the six largest are taken, every one of them exact in 32 bits; the three
+// left out are at most 2^-23 of the whole product and of either sign.  The six go into one float32 accumulator, the smallest first.
+// An accumulator is rounded six times for 32 inner elements instead of 32 times, and that outweighs what is left out: against
+// 64 bits the error is 0.3 to 0.6 of the 32-bit instruction's (normal numbers, K 64 / 2,304 / 9,216 / 16,384: 0.46, 5.1, 6.0 (three
+// slices) and 13.8e-7 of the result's norm; 1.44, 8.6, 9.9 and 22.9), that of the 2B shape's logits after a prompt of 500 tokens 1.6e-6
+// instead of 2.8e-6.
+#include "common.h"
+#include "alice_hip.h"
+#include "linear_thirds.h"
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int BK = THIRDS_BK;                                 // inner elements a stage: one product's
+
+__device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// Eight elements of a row as three times eight bfloat16 numbers.
+__device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float x = v[i >> 1][(i & 1) * 2], y = v[i >> 1][(i & 1) * 2 + 1];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const uint32_t h = pack_bf16x2(x, y);
+      p[t][i] = h;
+      x -= __uint_as_float(h << 16);
+      y -= __uint_as_float(h & 0xffff0000u);
+    }
+  }
+}
+
+// A block takes 16 TM tokens by 64 TN rows of W; its waves are two groups of four that share the inner dimension of the block's
+// slice, first half and second half, 32 elements a stage each.  A wave takes all the tokens by 16 TN rows: its rows go from memory
+// to its own registers and into thirds there, no other wave needs them; a group's tokens are split once, on their way into LDS, in
+// the order in which the instruction takes them (every access one contiguous kilobyte of a wave), in two buffers with one barrier a
+// stage.  A lane's eight elements of a stage are 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3 on both sides (whole 64-byte pieces of
+// a row a load).  The second group multiplies by the tokens' negative: the instruction adds by cutting off (towards minus infinity),
+// six times a stage, and that would move every output of every token the same way (a third of the error of a product of 9,216
+// elements was one vector common to all tokens, which no average over keys or layers removes: logits after prompts of 1,852 tokens
+// were off by 2.6e-6 of their norm instead of 1.9e-6); the two groups' shifts cancel.  W is the first operand, so that a lane ends up with four neighbouring outputs of a token.  The groups' sums meet
+// in LDS, on the way the outputs take to leave as 16-byte pieces of a token's row.  With GeGLU the first half of the block's rows are
+// gate rows, the second half the up rows of the same outputs.  blockIdx, split: as in linear_mfma32_kernel.
+//
+// What bounds it: the matrix instruction at the clock it runs at under this load.  512 tokens by 18,432 x 2,304 with GeGLU:
+// 232 us (183 TFLOP/s of 32-bit products; 1.1 PFLOP/s of bfloat16 ones, what large library products reach here), 183 us with neither
+// loads nor LDS nor splitting; 356 on the 32-bit instruction.  Both operands through LDS, 128 x 128 to 256 x 144 a block: 247 to
+// 330 us; products, splitting and loads interleaved by hand with the next stage's tokens read ahead: the same 275 as without for
+// 64 x 128 a block; one group of four waves: 278.
+template <int TM, int TN>
+__global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ Y,
+                                                               int M, int N, int K, int kslice, int mt, int nt, int epi, float param,
+                                                               int full, int wide) {
+  constexpr int NW = 4, KG = 2, THREADS = 64 * NW * KG, BM = 16 * TM, BN = 16 * TN * NW, XJ = (TM + NW - 1) / NW;
+  constexpr int YROW = BN + 4;
+  constexpr int STAGE = 3 * TM * 64;                          // in units of 16 bytes
+  extern __shared__ __align__(16) u32x4 lds[];
+  __shared__ int again;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) % NW, group = __builtin_amdgcn_readfirstlane(tid >> 6) / NW;
+  auto plane = [&](int buf, int t, int tile) { return lds + (group * 2 + buf) * STAGE + (t * TM + tile) * 64; };
+
+  const int total = mt * nt, per = (total + 7) >> 3;
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (tile >= total) return;                                  // the whole block: no barrier is missed
+  const int m0 = (tile % mt) * BM, nb = tile / mt;
+  const bool geglu = epi == ALICE_EPI_GEGLU;
+  const int n0 = nb * (geglu ? BN / 2 : BN);
+  const int s_begin = blockIdx.y * kslice, s_end = min(K, s_begin + kslice);
+  // a group's share of the slice; the groups take equally many stages, the last ones of zeros alone if need be
+  const int span = ((s_end - s_begin + KG - 1) / KG + BK - 1) / BK * BK;
+  const int k_begin = s_begin + group * span, k_stop = k_begin + span, k_end = min(s_end, k_stop);
+
+  // rows and tokens beyond the last are read as the last and not written
+  const float* wsrc[TN];
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    const int r = (wave * TN + i) * 16 + c;
+    int row = min(n0 + r, N - 1);
+    if (geglu) row = (r >= BN / 2) * N + min(n0 + r % (BN / 2), N - 1);
+    wsrc[i] = W + (size_t)row * K;
+  }
+  const float* xsrc[XJ];
+#pragma unroll
+  for (int j = 0; j < XJ; ++j) xsrc[j] = A + (size_t)min(m0 + (wave + NW * j) * 16 + c, M - 1) * K;
+  f32x4 wr[TN][2], xr[XJ][2];                                 // the stage on its way from memory
+  auto load = [&](const float* p, f32x4 (&v)[2], int k0) {
+    v[0] = *reinterpret_cast<const f32x4*>(p + min(k0 + g * 4, s_end - 4));
+    v[1] = *reinterpret_cast<const f32x4*>(p + min(k0 + 16 + g * 4, s_end - 4));
+  };
+  auto clear_beyond = [&](f32x4 (&v)[2], int k0) {            // the last stage of a slice: nothing beyond its end
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool in = k0 + g * 4 + h * 16 < k_end;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[h][e] = in ? v[h][e] : 0.f;
+    }
+  };
+  f32x4 acc[TN][TM];
+  auto clear = [&] {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
+  if (tid == 0) again = 0;
+  const uint32_t flip = group ? 0x80000000u : 0u;
+  auto turn_sign = [&](f32x4 (&v)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[h][e] = __uint_as_float(__float_as_uint(v[h][e]) ^ flip);
+  };
+  auto put = [&](int j, int buf) {
+    u32x4 p[3];
+    turn_sign(xr[j]);
+    thirds(xr[j], p);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) plane(buf, t, wave + NW * j)[lane] = p[t];
+  };
+  auto mine = [&](int j) { return TM % NW == 0 || wave + NW * j < TM; };
+#pragma unroll
+  for (int j = 0; j < XJ; ++j) load(xsrc[j], xr[j], k_begin);
+#pragma unroll
+  for (int i = 0; i < TN; ++i) load(wsrc[i], wr[i], k_begin);
+#pragma unroll
+  for (int j = 0; j < XJ; ++j) {
+    clear_beyond(xr[j], k_begin);
+    if (mine(j)) put(j, 0);
+    load(xsrc[j], xr[j], k_begin + BK);
+  }
+  lds_barrier();
+  int cur = 0;
+  auto stage = [&](int k0, bool last) {
+    u32x4 x[TM][3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) x[j][t] = plane(cur, t, j)[lane];
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      u32x4 w[3];
+      if (k0 + BK > k_end) clear_beyond(wr[i], k0);
+      thirds(wr[i], w);
+      if (!last) load(wsrc[i], wr[i], k0 + BK);
+      // the smallest products first
+      constexpr int WT[6] = {2, 0, 1, 1, 0, 0}, XT[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+      for (int p = 0; p < 6; ++p)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] = mfma(w[WT[p]], x[j][XT[p]], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!last) {
+#pragma unroll
+      for (int j = 0; j < XJ; ++j) {
+        if (k0 + 2 * BK > k_end) clear_beyond(xr[j], k0 + BK);
+        if (mine(j)) put(j, cur ^ 1);
+        load(xsrc[j], xr[j], k0 + 2 * BK);
+      }
+      lds_barrier();
+      cur ^= 1;
+    }
+  };
+  int k0 = k_begin;
+  for (; k0 + BK < k_stop; k0 += BK) stage(k0, false);
+  stage(k0, true);
+  __syncthreads();
+
+  // A number that is not finite, or that rounds to no finite bfloat16, has a remainder that is none, and every sum that it enters
+  // is then none either.  Sums so small that thirds may have fallen below the smallest bfloat16, and those that are no finite
+  // numbers, are taken again by 32-bit products; so is the whole tile around them.
+  bool odd = false;
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = fabsf(acc[i][j][e]);
+        odd = odd | (!(v >= 0x1p-80f) & (v != 0.f)) | !(v < INFINITY);
+      }
+  if (__ballot(odd) != 0 && lane == 0) again = 1;             // any of them: the same value
+  __syncthreads();
+  if (again) {
+    clear();
+#pragma unroll 1
+    for (int k0 = k_begin; k0 < k_stop; k0 += BK) {
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < XJ; ++j) {
+        load(xsrc[j], xr[j], k0);
+        clear_beyond(xr[j], k0);
+        turn_sign(xr[j]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) if (mine(j)) plane(0, h, wave + NW * j)[lane] = __builtin_bit_cast(u32x4, xr[j][h]);
+      }
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        load(wsrc[i], wr[i], k0);
+        clear_beyond(wr[i], k0);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        f32x4 x[TM];
+#pragma unroll
+        for (int j = 0; j < TM; ++j) x[j] = __builtin_bit_cast(f32x4, plane(0, h, j)[lane]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr[i][h][e], x[j][e], acc[i][j], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+
+  // The outputs go through LDS: 16-byte pieces of a token's row, and the epilogue's functions stand in the code for four elements.
+  auto Ys = reinterpret_cast<float (*)[YROW]>(lds);
+  // the second group's negative sums first, which the first group then takes from its own
+#pragma unroll
+  for (int gr = KG - 1; gr >= 0; --gr) {
+    if (gr == group) {
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int i = 0; i < TN; ++i) {
+          f32x4* p = reinterpret_cast<f32x4*>(&Ys[j * 16 + c][(wave * TN + i) * 16 + g * 4]);
+          *p = gr == KG - 1 ? acc[i][j] : acc[i][j] - *p;
+        }
+    }
+    __syncthreads();
+  }
+  float* __restrict__ y = Y + (size_t)blockIdx.y * M * N;
+  const int pieces = geglu ? BN / 8 : BN / 4;                 // of a row
+#pragma unroll 1
+  for (int id = tid; id < BM * pieces; id += THREADS) {
+    const int r = id / pieces, q = (id % pieces) * 4, m = m0 + r, n = n0 + q;
+    if (m >= M || n >= N) continue;
+    f32x4 v;
+    if (geglu) {
+      const float* p = &Ys[r][q];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = gated_act(p[e], p[BN / 2 + e], param, full);
+    } else {
+      v = *reinterpret_cast<const f32x4*>(&Ys[r][q]);
+      if (epi == ALICE_EPI_SOFTCAP) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = unary_act(v[e], param, full);
+      }
+    }
+    float* dst = y + (size_t)m * N + n;
+    if (wide) {                                               // rows of whole, aligned pieces
+      *reinterpret_cast<f32x4*>(dst) = v;
+      continue;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) dst[e] = v[e];
+  }
+}
+
+template <int TM, int TN>
+int launch(const float* x, const float* w, float* y, int M, int N, int K, int epi, float param, int full, int split, hipStream_t stream) {
+  constexpr int BM = 16 * TM, BN = 64 * TN;
+  constexpr int STAGES = 2 * 2 * 3 * TM * 1024, OUT = BM * (BN + 4) * 4, LDS = STAGES > OUT ? STAGES : OUT;
+  const int mt = ceil_div(M, BM), nt = ceil_div(N, epi == ALICE_EPI_GEGLU ? BN / 2 : BN);
+  ALICE_CHECK((long)mt * nt < (1l << 30), "linear: too many tiles for one launch");
+  const int kslice = ceil_div(ceil_div(K, split), BK) * BK;
+  const int wide = N % 4 == 0 && ((uintptr_t)y & 15) == 0;
+  const dim3 grid(8 * ceil_div((long)mt * nt, 8), split);
+  auto kern = linear_thirds_kernel<TM, TN>;
+  if (LDS > 48 * 1024) {
+    static const hipError_t told = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    ALICE_CHECK(told == hipSuccess, "linear: the device does not give a block %d bytes of LDS", LDS);
+  }
+  kern<<<grid, 512, LDS, stream>>>(x, w, y, M, N, K, kslice, mt, nt, epi, param, full, wide);
+  ALICE_LAUNCH_CHECK();
+  return 0;
+}
+
+// Microseconds that a block takes for a stage of each of its groups with the chip full.
+struct Tile {
+  int bm, bn;
+  float stage;
+};
+constexpr Tile TILES[] = {{128, 128, 2.5f}, {64, 192, 2.1f}, {64, 128, 1.5f}, {64, 64, 1.0f}, {32, 128, 1.35f}, {32, 64, 0.95f}};
+
+}  // namespace
+
+// The tile, and between min_split and max_split slices the number of them, by estimated microseconds: a CU's blocks one after the
+// other; slices cost writing and reading their sums.  (Planned and measured: 512 tokens by 18,432 x 2,304 with GeGLU in 64 x 192,
+// three blocks a CU, 233 and 232; 4,096 x 2,304 in 64 x 128 60 and 58; 2,304 x 9,216 in three slices 123 and 126.)
+ThirdsPlan alice_linear_thirds_plan(int M, int N, int K, bool geglu, int min_split, int max_split) {
+  ThirdsPlan best{-1, 1, 1e30f};
+  for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
+    const Tile& t = TILES[i];
+    const int mt = ceil_div(M, t.bm), nt = ceil_div(N, geglu ? t.bn / 2 : t.bn);
+    for (int s = min_split; s <= max_split; ++s) {
+      const int ks = ceil_div(ceil_div(K, s), BK) * BK;
+      if (s > 1 && (ks < 256 || (long)ks * (s - 1) >= K)) continue;          // no slice without elements
+      const float us = 4.f + ceil_div((long)mt * nt * s, 256) * (ceil_div(ks, 2 * BK) * t.stage + 0.7f) + (s > 1 ? 2.f * s * (float)M * N * 4.f / 4.0e6f : 0.f);
+      if (us < best.us) best = ThirdsPlan{i, s, us};
+    }
+  }
+  return best;
+}
+
+int alice_linear_thirds(const float* x, const float* w, float* y, int M, int N, int K, int epi, float param, int full, const ThirdsPlan& p,
+                        hipStream_t stream) {
+  ALICE_CHECK(K % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 && p.split >= 1, "linear: operands for the products in thirds are not aligned");
+#define GO(TM, TN) return launch<TM, TN>(x, w, y, M, N, K, epi, param, full, p.split, stream)
+  switch (p.tile) {
+    case 0: GO(8, 2);
+    case 1: GO(4, 3);
+    case 2: GO(4, 2);
+    case 3: GO(4, 1);
+    case 4: GO(2, 2);
+    case 5: GO(2, 1);
+  }
+#undef GO
+  alice_set_error("linear: no tile %d for the products in thirds", p.tile);
+  return 1;
+}

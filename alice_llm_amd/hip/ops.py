@@ -48,6 +48,7 @@ def _declare(lib) -> None:
         "alice_add_branches": [P, I, P, P, P, P, I, P, P, P, I, I, I, I, P],
         "alice_linear": [P, I, P, I, I, P, I, I, I, I, I, F, I, I, I, I, I, P],
         "alice_linear_split_hint": [I, I, I, I],
+        "alice_linear_thirds_tile": [I, I, I, I, I],
         "alice_to_frag16": [P, P, I, I, P],
         "alice_frag16_supported": [I, I, I],
         "alice_rope_cache_write": [P, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, I, I, P],
@@ -410,6 +411,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, *, n_out: int, k_i
 
 def linear_split_hint(M: int, N: int, K: int, layout: int) -> int:
     return library().alice_linear_split_hint(M, N, K, layout)
+
+
+def linear_thirds_tile(M: int, N: int, K: int, geglu: bool = False, split_k: int = 1) -> int:
+    """The tile of a float32 product that goes in three bfloat16 parts an operand, -1 for the 32-bit instruction."""
+    return library().alice_linear_thirds_tile(M, N, K, int(geglu), split_k)
 
 
 def to_frag16(w: torch.Tensor) -> torch.Tensor:

@@ -1,0 +1,118 @@
+"""Float32 products on the bfloat16 matrix instruction (operands in three parts): every tile at its edges, against 64 bits; precision
+against the 32-bit instruction; numbers that have no three parts."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from alice_llm_amd.hip import ops
+from test_gpu_kernels import rnd
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def product(x, w, split=1, epi=ops.EPI_NONE, param=0.0):
+    M, K = x.shape
+    N = w.shape[0] // (2 if epi == ops.EPI_GEGLU else 1)
+    y = torch.full(((split,) if split > 1 else ()) + (M, N), float("nan"), device=DEV)
+    ops.linear(x, w, y, n_out=N, k_in=K, epilogue=epi, epi_param=param, split_k=split, full_precision=True)
+    return y
+
+
+def bound(x, w):
+    """What any order of the six products' sums may be off: 2^-23 of every product left out, and six roundings for 32 elements and
+    one for each part's sum, of at most 2^-23 (the instruction adds without rounding to nearest) of all products' sizes."""
+    K = x.shape[1]
+    return (x.double().abs() @ w.double().abs().T) * 2.0 ** -23 * (1 + 6 * (K // 32 + 2) + 8)
+
+
+# tokens, rows, inner elements, slices: tiles 0 .. 5; last rows and tokens of a tile missing, an inner dimension that is no multiple
+# of 32 or of 64, groups of unequally many stages, rows that are no multiple of 16 bytes of outputs
+CASES = [(128, 16384, 2304, 1), (500, 9217, 2304, 1), (500, 4096, 2304, 1), (497, 4095, 2308, 1), (500, 2304, 9216, 3), (500, 2302, 9220, 6),
+         (33, 2304, 9216, 4), (19, 2303, 9212, 8), (17, 2304, 2048, 7), (65, 1000, 16384, 8), (300, 20000, 164, 1), (2000, 1152, 1156, 2)]
+
+
+@pytest.mark.parametrize("M,N,K,split", CASES)
+def test_products_in_thirds(M, N, K, split):
+    assert ops.linear_thirds_tile(M, N, K, False, split) >= 0
+    x, w = rnd(M, K, seed=M), rnd(N, K, seed=N, scale=0.1)
+    got, ref = product(x, w, split), x.double() @ w.double().T
+    got = got.double().sum(0) if split > 1 else got.double()
+    assert torch.isfinite(got).all() and ((got - ref).abs() <= bound(x, w)).all()
+    if split == 1:
+        cap = product(x, w, 1, ops.EPI_SOFTCAP, 2.0)
+        assert ((cap.double() - 2 * torch.tanh(ref / 2)).abs() <= bound(x, w) + 1e-6).all()
+
+
+def test_every_tile_is_among_the_cases():
+    assert {ops.linear_thirds_tile(M, N, K, False, s) for M, N, K, s in CASES} == {0, 1, 2, 3, 4, 5}
+
+
+@pytest.mark.parametrize("M,N,K", [(500, 9216, 2304), (497, 9212, 2308), (500, 4610, 2304), (128, 9218, 2304), (64, 9218, 2304), (2048, 1025, 2304)])
+def test_gated_products_in_thirds(M, N, K):
+    assert ops.linear_thirds_tile(M, N, K, True) >= 0
+    x, w = rnd(M, K, seed=M), rnd(2 * N, K, seed=N, scale=0.02)
+    got, off = product(x, w, epi=ops.EPI_GEGLU).double(), bound(x, w)
+    ref = x.double() @ w.double().T
+    g, u = ref[:, :N], ref[:, N:]
+    # the gate's slope is at most 1.13; 1e-6 for the 32-bit function itself
+    assert ((got - F.gelu(g, approximate="tanh") * u).abs() <= 1.13 * off[:, :N] * u.abs() + off[:, N:] * g.abs() + 1e-6 * (1 + g.abs() * u.abs())).all()
+
+
+@pytest.mark.parametrize("M,N,K,split", [(500, 4096, 2304, 1), (500, 2304, 9216, 3), (500, 20000, 164, 1), (128, 2304, 16384, 8)])
+@pytest.mark.parametrize("spread", [0.0, 3.0])
+def test_no_less_precise_than_the_32_bit_instruction(M, N, K, split, spread):
+    """Normal numbers, and numbers whose sizes are spread over some orders of magnitude.  The same product over rows of one more element
+    that is zero takes the 32-bit instruction (rows that are no multiple of four elements)."""
+    assert ops.linear_thirds_tile(M, N, K, False, split) >= 0
+    x, w = (rnd(n, K, seed=i) * torch.exp(spread * rnd(n, K, seed=i + 2)) for i, n in enumerate((M, N)))
+    ref = x.double() @ w.double().T
+    err = [float((y.double().sum(0) if split > 1 else y.double()).sub(ref).norm() / ref.norm())
+           for y in (product(x, w, split), product(*(F.pad(a, (0, 1)).contiguous() for a in (x, w)), split))]
+    assert err[0] <= err[1], err
+    # and not in one direction: the mean over the tokens is no larger than that of errors of either sign (five standard deviations)
+    e = (product(x, w, split).double().sum(0) if split > 1 else product(x, w, split).double()) - ref
+    assert float(e.mean(0).norm()) <= 1.5 * float(e.norm()) / M, (float(e.mean(0).norm()), float(e.norm()) / M)
+
+
+def test_what_has_no_three_parts():
+    """Infinities, no numbers, numbers that round to no finite bfloat16, and sums of numbers so small that their last part is below
+    the smallest bfloat16: what 32-bit products give."""
+    M, N, K = 500, 4096, 2304
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=0.02)
+    x[3, 7], x[200, 2300], x[201, 5] = float("inf"), float("-inf"), float("nan")
+    w[17, 9], w[4000, 0] = float("inf"), float("nan")
+    x[77] = 0.0
+    x[90, 100] = 3.4e38
+    w[:, 100] *= 1e-3
+    got, ref = product(x, w), x.double() @ w.double().T
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+    ok = torch.isfinite(ref)
+    assert torch.equal(got[~ok & ~torch.isnan(ref)].double(), ref[~ok & ~torch.isnan(ref)])
+    x2, w2 = (torch.where(torch.isfinite(a), a, 0.0) for a in (x, w))
+    assert ((got.double() - ref).abs()[ok] <= (bound(x2, w2) * 16)[ok]).all()      # (32 roundings for 32 elements instead of 6)
+    tiny = rnd(M, K, seed=3) * 1e-34
+    got, ref = product(tiny, w[:, :].nan_to_num(0.0, 0.0, 0.0)), tiny.double() @ w.nan_to_num(0.0, 0.0, 0.0).double().T
+    assert ((got.double() - ref).norm() <= 1e-5 * ref.norm())
+    assert (product(torch.zeros(M, K, device=DEV), w2) == 0).all()
+
+
+def test_a_token_depends_on_no_other_and_captured_steps_add_as_eager_ones():
+    M, N, K = 129, 9216, 2304
+    x, w = rnd(192, K, seed=1), rnd(N, K, seed=2)
+    all_rows = product(x, w)
+    for n in (M, 144, 191):                                       # one multiple of 64: one tile, one order
+        assert torch.equal(product(x[:n].contiguous(), w), all_rows[:n])
+    y = torch.empty(192, N, device=DEV)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        ops.linear(x, w, y, n_out=N, k_in=K, full_precision=True)
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            ops.linear(x, w, y, n_out=N, k_in=K, full_precision=True)
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, all_rows)
