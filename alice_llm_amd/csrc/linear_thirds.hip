@@ -25,17 +25,20 @@ __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// Eight elements of a row as three times eight bfloat16 numbers.
-__device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3]) {
+// Eight elements of a row, times `sign` (1 or -1, with SIGNED), as three times eight bfloat16 numbers.
+template <bool SIGNED>
+__device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3], float sign = 1.f) {
+  const uint32_t flip = (__float_as_uint(sign) >> 31) * 0x80008000u;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float x = v[i >> 1][(i & 1) * 2], y = v[i >> 1][(i & 1) * 2 + 1];
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
-      const uint32_t h = pack_bf16x2(x, y);
+      const uint32_t h = SIGNED && t == 0 ? pack_bf16x2(x, y) ^ flip : pack_bf16x2(x, y);
       p[t][i] = h;
-      x -= __uint_as_float(h << 16);
-      y -= __uint_as_float(h & 0xffff0000u);
+      const float hx = __uint_as_float(h << 16), hy = __uint_as_float(h & 0xffff0000u);
+      x = SIGNED && t == 0 ? fmaf(x, sign, -hx) : x - hx;
+      y = SIGNED && t == 0 ? fmaf(y, sign, -hy) : y - hy;
     }
   }
 }
@@ -50,7 +53,7 @@ __device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3]) {
 // elements was one vector common to all tokens, which no average over keys or layers removes: logits after prompts of 1,852 tokens
 // were off by 2.6e-6 of their norm instead of 1.9e-6); the two groups' shifts cancel.  W is the first operand, so that a lane ends up with four neighbouring outputs of a token.  The groups' sums meet
 // in LDS, on the way the outputs take to leave as 16-byte pieces of a token's row.  With GeGLU the first half of the block's rows are
-// gate rows, the second half the up rows of the same outputs.  blockIdx, split: as in linear_mfma32_kernel.
+// gate rows, the second half the up rows of the same outputs.  split: slices of the inner dimension, slice z to Y + z M N.
 //
 // What bounds it: the matrix instruction at the clock it runs at under this load.  512 tokens by 18,432 x 2,304 with GeGLU:
 // 232 us (183 TFLOP/s of 32-bit products; 1.1 PFLOP/s of bfloat16 ones, what large library products reach here), 183 us with neither
@@ -59,7 +62,7 @@ __device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3]) {
 // 64 x 128 a block; one group of four waves: 278.
 template <int TM, int TN>
 __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ Y,
-                                                               int M, int N, int K, int kslice, int mt, int nt, int epi, float param,
+                                                               int M, int N, int K, int kslice, int split, int mt, int nt, int epi, float param,
                                                                int full, int wide) {
   constexpr int NW = 4, KG = 2, THREADS = 64 * NW * KG, BM = 16 * TM, BN = 16 * TN * NW, XJ = (TM + NW - 1) / NW;
   constexpr int YROW = BN + 4;
@@ -70,13 +73,14 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) % NW, group = __builtin_amdgcn_readfirstlane(tid >> 6) / NW;
   auto plane = [&](int buf, int t, int tile) { return lds + (group * 2 + buf) * STAGE + (t * TM + tile) * 64; };
 
-  const int total = mt * nt, per = (total + 7) >> 3;
-  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if (tile >= total) return;                                  // the whole block: no barrier is missed
+  // tile and slice of this block: neighbours in m first, then in n, a run an XCD (blocks go to the 8 XCDs in turn)
+  const int per = (mt * nt * split + 7) >> 3, item = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (item >= mt * nt * split) return;                        // the whole block: no barrier is missed
+  const int slice = item / (mt * nt), tile = item % (mt * nt);
   const int m0 = (tile % mt) * BM, nb = tile / mt;
   const bool geglu = epi == ALICE_EPI_GEGLU;
   const int n0 = nb * (geglu ? BN / 2 : BN);
-  const int s_begin = blockIdx.y * kslice, s_end = min(K, s_begin + kslice);
+  const int s_begin = slice * kslice, s_end = min(K, s_begin + kslice);
   // a group's share of the slice; the groups take equally many stages, the last ones of zeros alone if need be
   const int span = ((s_end - s_begin + KG - 1) / KG + BK - 1) / BK * BK;
   const int k_begin = s_begin + group * span, k_stop = k_begin + span, k_end = min(s_end, k_stop);
@@ -115,17 +119,10 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   };
   clear();
   if (tid == 0) again = 0;
-  const uint32_t flip = group ? 0x80000000u : 0u;
-  auto turn_sign = [&](f32x4 (&v)[2]) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[h][e] = __uint_as_float(__float_as_uint(v[h][e]) ^ flip);
-  };
+  const float sign = group ? -1.f : 1.f;
   auto put = [&](int j, int buf) {
     u32x4 p[3];
-    turn_sign(xr[j]);
-    thirds(xr[j], p);
+    thirds<true>(xr[j], p, sign);
 #pragma unroll
     for (int t = 0; t < 3; ++t) plane(buf, t, wave + NW * j)[lane] = p[t];
   };
@@ -152,7 +149,7 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
     for (int i = 0; i < TN; ++i) {
       u32x4 w[3];
       if (k0 + BK > k_end) clear_beyond(wr[i], k0);
-      thirds(wr[i], w);
+      thirds<false>(wr[i], w);
       if (!last) load(wsrc[i], wr[i], k0 + BK);
       // the smallest products first
       constexpr int WT[6] = {2, 0, 1, 1, 0, 0}, XT[6] = {0, 2, 1, 0, 1, 0};
@@ -202,9 +199,8 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
       for (int j = 0; j < XJ; ++j) {
         load(xsrc[j], xr[j], k0);
         clear_beyond(xr[j], k0);
-        turn_sign(xr[j]);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) if (mine(j)) plane(0, h, wave + NW * j)[lane] = __builtin_bit_cast(u32x4, xr[j][h]);
+        for (int h = 0; h < 2; ++h) if (mine(j)) plane(0, h, wave + NW * j)[lane] = __builtin_bit_cast(u32x4, xr[j][h] * sign);
       }
 #pragma unroll
       for (int i = 0; i < TN; ++i) {
@@ -244,7 +240,7 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
     }
     __syncthreads();
   }
-  float* __restrict__ y = Y + (size_t)blockIdx.y * M * N;
+  float* __restrict__ y = Y + (size_t)slice * M * N;
   const int pieces = geglu ? BN / 8 : BN / 4;                 // of a row
 #pragma unroll 1
   for (int id = tid; id < BM * pieces; id += THREADS) {
@@ -278,16 +274,16 @@ int launch(const float* x, const float* w, float* y, int M, int N, int K, int ep
   constexpr int BM = 16 * TM, BN = 64 * TN;
   constexpr int STAGES = 2 * 2 * 3 * TM * 1024, OUT = BM * (BN + 4) * 4, LDS = STAGES > OUT ? STAGES : OUT;
   const int mt = ceil_div(M, BM), nt = ceil_div(N, epi == ALICE_EPI_GEGLU ? BN / 2 : BN);
-  ALICE_CHECK((long)mt * nt < (1l << 30), "linear: too many tiles for one launch");
+  ALICE_CHECK((long)mt * nt * split < (1l << 30), "linear: too many tiles for one launch");
   const int kslice = ceil_div(ceil_div(K, split), BK) * BK;
   const int wide = N % 4 == 0 && ((uintptr_t)y & 15) == 0;
-  const dim3 grid(8 * ceil_div((long)mt * nt, 8), split);
+  const int grid = 8 * ceil_div((long)mt * nt * split, 8);
   auto kern = linear_thirds_kernel<TM, TN>;
   if (LDS > 48 * 1024) {
     static const hipError_t told = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     ALICE_CHECK(told == hipSuccess, "linear: the device does not give a block %d bytes of LDS", LDS);
   }
-  kern<<<grid, 512, LDS, stream>>>(x, w, y, M, N, K, kslice, mt, nt, epi, param, full, wide);
+  kern<<<grid, 512, LDS, stream>>>(x, w, y, M, N, K, kslice, split, mt, nt, epi, param, full, wide);
   ALICE_LAUNCH_CHECK();
   return 0;
 }
@@ -312,7 +308,7 @@ ThirdsPlan alice_linear_thirds_plan(int M, int N, int K, bool geglu, int min_spl
     for (int s = min_split; s <= max_split; ++s) {
       const int ks = ceil_div(ceil_div(K, s), BK) * BK;
       if (s > 1 && (ks < 256 || (long)ks * (s - 1) >= K)) continue;          // no slice without elements
-      const float us = 4.f + ceil_div((long)mt * nt * s, 256) * (ceil_div(ks, 2 * BK) * t.stage + 0.7f) + (s > 1 ? 2.f * s * (float)M * N * 4.f / 4.0e6f : 0.f);
+      const float us = 4.f + ceil_div(ceil_div((long)mt * nt * s, 8), 32) * (ceil_div(ks, 2 * BK) * t.stage + 0.7f) + (s > 1 ? 2.f * s * (float)M * N * 4.f / 4.0e6f : 0.f);
       if (us < best.us) best = ThirdsPlan{i, s, us};
     }
   }
