@@ -713,9 +713,9 @@ struct Walk {
 // [sequence][head][split][4 + D] = (max, sum, two unused, unnormalised output).  With one split the output is final.
 template <int DT, bool SOFTCAP>
 __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
-    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
-    bf16_t* __restrict__ out, float* __restrict__ parts, const int* __restrict__ context_lens,
-    const int* __restrict__ block_table, int bt_stride, int nH, int nKV, float scale, float cap, int window, int splits,
+    const int* __restrict__ context_lens, const int* __restrict__ block_table, int bt_stride, int window, int splits,
+    uint32_t splits_reciprocal, int nKV, int group, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ q,
+    const bf16_t* __restrict__ v_pool, bf16_t* __restrict__ out, float* __restrict__ parts, float scale, float cap,
     int out_layout, const float* __restrict__ sink) {
   constexpr int D = DT * 32, NW = 4;
   __shared__ float sm[NW][16], sl[NW][16];
@@ -724,13 +724,13 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
   const int b = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
-  const int group = nH / nKV;
+  const int nH = nKV * group;
   const int pos = context_lens[b] - 1;
   const int first_key = window > 0 ? max(0, pos + 1 - window) : 0;
   const int kb_first = first_key >> 5, kb_last = pos >> 5;
   const int n_blocks = kb_last - kb_first + 1;
-  const int run0 = split * n_blocks / splits, run = (split + 1) * n_blocks / splits - run0;
-  const int my_first = kb_first + run0 + wave * run / NW, my_last = kb_first + run0 + (wave + 1) * run / NW - 1;
+  const int run0 = quotient(split * n_blocks, splits_reciprocal), run = (int)quotient((split + 1) * n_blocks, splits_reciprocal) - run0;
+  const int my_first = kb_first + run0 + (unsigned)(wave * run) / NW, my_last = kb_first + run0 + (unsigned)((wave + 1) * run) / NW - 1;
   const int* bt = block_table + (size_t)b * bt_stride;
   const size_t page_elems = (size_t)64 * D;
 
@@ -998,8 +998,9 @@ extern "C" int alice_attention_decode(const void* q, const void* k_pool, const v
         told = true;                                                                                                        \
       }                                                                                                                     \
     }                                                                                                                       \
-    kern<<<grid, 256, lds, stream>>>((const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool, (bf16_t*)out, parts,   \
-                                     context_lens, block_table, bt_stride, nH, nKV, scale, softcap, window, splits, out_layout, sink); \
+    kern<<<grid, 256, lds, stream>>>(context_lens, block_table, bt_stride, window, splits, reciprocal_of(splits), nKV, nH / nKV,  \
+                                     (const bf16_t*)k_pool, (const bf16_t*)q, (const bf16_t*)v_pool, (bf16_t*)out, parts, scale, \
+                                     softcap, out_layout, sink);                                                           \
   } while (0)
 #define GO(DT)                          \
   do {                                  \

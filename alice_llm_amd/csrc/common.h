@@ -164,6 +164,11 @@ __device__ __forceinline__ size_t out_index(int layout, int r, int i, int H) {
   return ((size_t)((size_t)(r >> 4) * (H >> 5) + (i >> 5)) * 64 + ((i & 31) >> 3) * 16 + (r & 15)) * 8 + (i & 7);
 }
 
+// Whole quotients by a divisor that the host knows: a kernel that waits for nothing else yet spends 25 dependent instructions
+// on a division by a run-time number.  Exact while a * divisor < 2^31 (the host's number is 2^31 / divisor, rounded up).
+__device__ __forceinline__ uint32_t quotient(uint32_t a, uint32_t reciprocal) { return (uint32_t)(((uint64_t)a * reciprocal) >> 31); }
+static inline uint32_t reciprocal_of(uint32_t divisor) { return (uint32_t)(((1ull << 31) + divisor - 1) / divisor); }
+
 // ---- host side -------------------------------------------------------------------------
 void alice_set_error(const char* fmt, ...);
 

@@ -62,10 +62,9 @@ extern "C" int alice_embed(const int* tokens, const void* table, int table_dtype
 //   out = (x - mean(x)) * rsqrt(mean((x - mean(x))^2) + eps_pre) * (off_pre + w_pre) + b_pre
 // All sums are 32-bit; FULL selects 1/sqrtf over the fast reciprocal square root.
 template <typename TW, typename TO, bool FULL, bool LN>
-__global__ void add_norm_kernel(float* __restrict__ resid, const float* __restrict__ branch,
-                                int n_partials, size_t partial_stride,
-                                const TW* __restrict__ w_post, const TW* __restrict__ w_pre, const TW* __restrict__ b_pre,
-                                TO* __restrict__ out, const int* __restrict__ rows, int H,
+__global__ void add_norm_kernel(const int* __restrict__ rows, int H, int n_partials, float* __restrict__ resid,
+                                const float* __restrict__ branch, size_t partial_stride, const TW* __restrict__ w_post,
+                                const TW* __restrict__ w_pre, const TW* __restrict__ b_pre, TO* __restrict__ out,
                                 float eps_post, float eps_pre, float off_post, float off_pre, int out_layout) {
   __shared__ float red[16];
   const int r = blockIdx.x;
@@ -147,11 +146,10 @@ __device__ __forceinline__ void load_partials(float (&t)[EPT][CMAX], const float
 }
 
 template <typename TW, typename TO, bool FULL, bool LN, int EPT>
-__global__ void add_norm_regs_kernel(float* __restrict__ resid, const float* __restrict__ branch,
-                                     int n_partials, size_t partial_stride,
-                                     const TW* __restrict__ w_post, const TW* __restrict__ w_pre, const TW* __restrict__ b_pre,
-                                     TO* __restrict__ out, const int* __restrict__ rows, int H,
-                                     float eps_post, float eps_pre, float off_post, float off_pre, int out_layout) {
+__global__ void add_norm_regs_kernel(const int* __restrict__ rows, int H, int n_partials, float* __restrict__ resid,
+                                const float* __restrict__ branch, size_t partial_stride, const TW* __restrict__ w_post,
+                                const TW* __restrict__ w_pre, const TW* __restrict__ b_pre, TO* __restrict__ out,
+                                float eps_post, float eps_pre, float off_post, float off_pre, int out_layout) {
   typedef typename raw_of<TW>::type RW;
   __shared__ float red[16];
   const int r = blockIdx.x;
@@ -276,11 +274,10 @@ __device__ __forceinline__ float4 raw4_to_f32(const uint2& v) {
 }
 
 template <typename TW, typename TO, bool FULL, bool LN, int E4>
-__global__ __launch_bounds__(1024) void add_norm_row_kernel(float* __restrict__ resid, const float* __restrict__ branch, int n_partials,
-                                                            size_t partial_stride, const TW* __restrict__ w_post,
-                                                            const TW* __restrict__ w_pre, const TW* __restrict__ b_pre,
-                                                            TO* __restrict__ out, const int* __restrict__ rows, int H, float eps_post,
-                                                            float eps_pre, float off_post, float off_pre, int out_layout) {
+__global__ __launch_bounds__(1024) void add_norm_row_kernel(const int* __restrict__ rows, int H, int n_partials, float* __restrict__ resid,
+                                const float* __restrict__ branch, size_t partial_stride, const TW* __restrict__ w_post,
+                                const TW* __restrict__ w_pre, const TW* __restrict__ b_pre, TO* __restrict__ out,
+                                float eps_post, float eps_pre, float off_post, float off_pre, int out_layout) {
   typedef typename raw4_of<TW>::type RW;
   constexpr int CMAX = E4 == 1 ? 8 : 4;                      // partial sums in flight per element (registers)
   __shared__ float red[3][16];
@@ -545,7 +542,8 @@ extern "C" int alice_add_norm(float* resid, const float* branch, int n_partials,
     ept = H <= 256 ? 1 : (H <= 512 ? 2 : (H <= 4096 ? 4 : 8));
     threads = ceil_div(ceil_div(H, ept), 64) * 64;
   }
-#define ARGS resid, branch, n_partials, (size_t)partial_stride, (const TW*)w_post, (const TW*)w_pre, (const TW*)b_pre, (TO*)out, rows, H, \
+// (what a kernel's first loads need comes first: these arguments arrive in registers, see build.py)
+#define ARGS rows, H, n_partials, resid, branch, (size_t)partial_stride, (const TW*)w_post, (const TW*)w_pre, (const TW*)b_pre, (TO*)out, \
              eps_post, eps_pre, off_post, off_pre, out_layout
   // Many rows, no gather: a wave per row (two from 4,097 elements on).  From 320 rows: below, a block per row
   // fills more of the chip (measured at 2,304 and 3,584 elements: up to 256 rows the block-per-row kernel is 0.5

@@ -35,6 +35,7 @@ struct RopeArgs {
   const int* seq_of_token;
   const int* block_table;
   int bt_stride, nH, nKV, d, page_size, n_pages, layout;
+  uint32_t d_reciprocal;                  // of the head size, see quotient()
 };
 
 namespace {
@@ -129,14 +130,29 @@ struct RopeToken {
   bool page_ok;
   size_t page_base;
 };
-__device__ __forceinline__ RopeToken rope_token(const RopeArgs& ra, int m) {
+// In three steps, so that a kernel can have the two lookups behind it when its sums are done (two round trips to memory, which
+// a kernel of 6 us otherwise adds at its end): a token's position and sequence, then its page's number, then the place.
+struct RopeLookup { int pos, seq, page; };
+__device__ __forceinline__ void rope_look_up(const int* __restrict__ positions, const int* __restrict__ seq_of_token, int m, RopeLookup& l) {
+  l.pos = positions[m];
+  l.seq = seq_of_token[m];
+}
+__device__ __forceinline__ void rope_look_up_page(const RopeArgs& ra, RopeLookup& l) {
+  l.page = ra.block_table[(size_t)l.seq * ra.bt_stride + l.pos / ra.page_size];
+}
+__device__ __forceinline__ RopeToken rope_token(const RopeArgs& ra, const RopeLookup& l) {
   RopeToken t;
-  t.pos = ra.positions[m];
+  t.pos = l.pos;
   t.tp = t.pos % ra.page_size;
-  const int page = ra.block_table[(size_t)ra.seq_of_token[m] * ra.bt_stride + t.pos / ra.page_size];
-  t.page_ok = page >= 0 && page < ra.n_pages;
-  t.page_base = (size_t)(t.page_ok ? page : 0) * ra.nKV * ra.page_size * ra.d;
+  t.page_ok = l.page >= 0 && l.page < ra.n_pages;
+  t.page_base = (size_t)(t.page_ok ? l.page : 0) * ra.nKV * ra.page_size * ra.d;
   return t;
+}
+__device__ __forceinline__ RopeToken rope_token(const RopeArgs& ra, int m) {
+  RopeLookup l;
+  rope_look_up(ra.positions, ra.seq_of_token, m, l);
+  rope_look_up_page(ra, l);
+  return rope_token(ra, l);
 }
 // The rotation epilogue for four consecutive output features n .. n+3 (in W's row order) of token m.  The
 // rows of W are all q heads, all k heads, all v heads, the rows of every q and k head in pair order: the four
@@ -146,18 +162,22 @@ __device__ __forceinline__ RopeToken rope_token(const RopeArgs& ra, int m) {
 // Which head features n .. n+3 belong to and where in it they lie: the same for every token of a tile, so the
 // divisions by the head size are done once per tile, not per token.
 struct RopeCol { int head, w; };
-__device__ __forceinline__ RopeCol rope_col(const RopeArgs& ra, int n) { return RopeCol{n / ra.d, n % ra.d}; }
+__device__ __forceinline__ RopeCol rope_col(const RopeArgs& ra, int n) {
+  const int head = quotient(n, ra.d_reciprocal);
+  return RopeCol{head, n - head * ra.d};
+}
 
 // The cosines and sines of the two pairs that the four features make (nothing for a value head).
 struct RopeTrig { float2 c, s; };
-__device__ __forceinline__ RopeTrig rope_trig(const RopeArgs& ra, const RopeToken& t, const RopeCol& col) {
+__device__ __forceinline__ RopeTrig rope_trig(const RopeArgs& ra, int pos, const RopeCol& col) {
   RopeTrig g{float2{1.f, 1.f}, float2{0.f, 0.f}};
   if (col.head < ra.nH + ra.nKV) {
-    g.c = *reinterpret_cast<const float2*>(ra.cos_t + (size_t)t.pos * (ra.d >> 1) + (col.w >> 1));
-    g.s = *reinterpret_cast<const float2*>(ra.sin_t + (size_t)t.pos * (ra.d >> 1) + (col.w >> 1));
+    g.c = *reinterpret_cast<const float2*>(ra.cos_t + (size_t)pos * (ra.d >> 1) + (col.w >> 1));
+    g.s = *reinterpret_cast<const float2*>(ra.sin_t + (size_t)pos * (ra.d >> 1) + (col.w >> 1));
   }
   return g;
 }
+__device__ __forceinline__ RopeTrig rope_trig(const RopeArgs& ra, const RopeToken& t, const RopeCol& col) { return rope_trig(ra, t.pos, col); }
 __device__ __forceinline__ void rope_store4(const RopeArgs& ra, int m, const RopeToken& t, const RopeCol& col, f32x4 acc,
                                             const RopeTrig& tr) {
   const int d = ra.d, half = d >> 1;
@@ -185,10 +205,6 @@ __device__ __forceinline__ void rope_store4(const RopeArgs& ra, int m, const Rop
 #pragma unroll
     for (int e = 0; e < 4; ++e) dst[v_offset(ra.layout, t.tp, w + e, d)] = f32_to_bf16(x[e]);
   }
-}
-__device__ __forceinline__ void rope_store4(const RopeArgs& ra, int m, const RopeToken& t, int n, f32x4 acc) {
-  const RopeCol col = rope_col(ra, n);
-  rope_store4(ra, m, t, col, acc, rope_trig(ra, t, col));
 }
 
 }  // namespace

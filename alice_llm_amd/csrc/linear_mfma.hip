@@ -121,7 +121,7 @@ extern "C" int alice_linear_rope_cache(const void* x, int x_layout, const void* 
   if (M == 0) return 0;
   const int N = (nH + 2 * nKV) * d;
   RopeArgs ra{(bf16_t*)q_out, (bf16_t*)k_pool, (bf16_t*)v_pool, cos_t, sin_t, positions, seq_of_token, block_table,
-              bt_stride, nH, nKV, d, page_size, n_pages, kv_layout};
+              bt_stride, nH, nKV, d, page_size, n_pages, kv_layout, reciprocal_of(d)};
   const int x_frag = x_layout == ALICE_LAYOUT_FRAG16;
   if (M > 64 || alice_mfma_tiled_plan(M, N, K, ALICE_EPI_ROPE, DT_BF16, 1, x_frag).wn != 0)
     return alice_mfma_tiled_rope(x, w, M, N, K, x_frag, stream, ra);

@@ -20,23 +20,26 @@ namespace {
 // oldest alone (s_waitcnt vmcnt(n)); a load under a branch makes it wait for all of them.
 template <int RT, int MT, int NW, int EPI, typename TO, bool FULL, bool XF, bool STREAM = false, int WINDOW = 0>
 __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wf,
-                                                            TO* __restrict__ y, int M, int N, int K, int KT, int NT,
-                                                            int kt_per_slice, float epi, int y_frag, RopeArgs ra) {
+                                                            void* __restrict__ y_or_positions, const int* __restrict__ seq_of_token,
+                                                            int M, int KT, int NT, int kt_per_slice, uint32_t turn, uint32_t last_turn,
+                                                            int N, int K, float epi, int y_frag, RopeArgs ra) {
+  // (the arguments up to last_turn come in registers: what the first loads need, with the rotation epilogue its lookups too)
   extern __shared__ __align__(16) float red[];            // [NW - 1][RT*MT][64][4]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // (the wave's number as a scalar: all that follows from it, the addresses of its tiles above all, is scalar arithmetic too)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int kb = blockIdx.y * kt_per_slice, ke = min(KT, kb + kt_per_slice);
 
   int tile[RT];
 #pragma unroll
   for (int i = 0; i < RT; ++i) {
-    if (EPI == ALICE_EPI_GEGLU) tile[i] = (i & 1) ? (N / 16 + blockIdx.x * (RT / 2) + (i >> 1)) : (blockIdx.x * (RT / 2) + (i >> 1));
+    if (EPI == ALICE_EPI_GEGLU) tile[i] = (i & 1 ? NT / 2 : 0) + blockIdx.x * (RT / 2) + (i >> 1);
     else tile[i] = blockIdx.x * RT + i;
   }
-  // where this lane reads its weight fragments (rows beyond the matrix: the last tile's, results unused)
+  // where the wave reads its weight fragments (rows beyond the matrix: the last tile's, results unused)
   const bf16_t* wrow[RT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i) wrow[i] = wf + (size_t)min(tile[i], NT - 1) * KT * 512 + lane * 8;
+  for (int i = 0; i < RT; ++i) wrow[i] = wf + (size_t)min(tile[i], NT - 1) * KT * 512;
   f32x4 acc[RT][MT];
 #pragma unroll
   for (int i = 0; i < RT; ++i)
@@ -45,12 +48,12 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __
 
   bool row_ok[MT];
   int row[MT];
-  const bf16_t* xrow[MT];        // this lane's place in the activations at k-tile 0
+  const bf16_t* xrow[MT];        // the wave's (rows: this lane's) place in the activations at k-tile 0
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
     row[j] = j * 16 + r;
     row_ok[j] = row[j] < M;
-    if constexpr (XF) xrow[j] = x + ((size_t)min(j, (M - 1) >> 4) * KT * 64 + lane) * 8;
+    if constexpr (XF) xrow[j] = x + (size_t)min(j, (M - 1) >> 4) * KT * 512;
     else xrow[j] = x + (size_t)min(row[j], M - 1) * K;
   }
 
@@ -64,7 +67,7 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __
   // against 25.0 us).  Six and eight were slower everywhere.
   constexpr int U = WINDOW > 0 ? WINDOW : ((RT * MT >= 8) ? 3 : 4);
   u32x4 a[U][RT], b[U][MT];
-  const bf16_t* zero = reinterpret_cast<const bf16_t*>(g_zero_tile) + lane * 8;
+  const bf16_t* zero = reinterpret_cast<const bf16_t*>(g_zero_tile);
   auto fetch = [&](int kt, u32x4 (&aa)[RT], u32x4 (&bb)[MT]) {
     const bool kok = kt < ke;
     const int ktc = kok ? kt : 0;                           // past the slice: zero weights, any activations
@@ -73,14 +76,14 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __
     // projection (42 MB) 8 % and changed the others by 2 % either way.
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
-      const u32x4* src = reinterpret_cast<const u32x4*>(kok ? wrow[i] + (size_t)ktc * 512 : zero);
+      const u32x4* src = reinterpret_cast<const u32x4*>(kok ? wrow[i] + (size_t)ktc * 512 : zero) + (unsigned)lane;
       if constexpr (STREAM) aa[i] = __builtin_nontemporal_load(src);
       else aa[i] = *src;
     }
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
       if constexpr (XF) {
-        bb[j] = *reinterpret_cast<const u32x4*>(xrow[j] + (size_t)ktc * 512);
+        bb[j] = reinterpret_cast<const u32x4*>(xrow[j] + (size_t)ktc * 512)[(unsigned)lane];
       } else {
         // a row's last, partial k-tile: the weights are zero there, so any finite values do
         bb[j] = *reinterpret_cast<const u32x4*>(xrow[j] + min(ktc * 32 + g * 8, K - 8));
@@ -90,16 +93,39 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __
   // Blocks start at different places of their k range and wrap around: all blocks read the same
   // activations, and in lockstep they would all ask the same L2 channel for the same line at once.
   const int J = (ke - kb + NW - 1) / NW;                    // k-tiles per wave (the last ones may be past the end)
-  const int rot = J > 0 ? (int)(blockIdx.x % (unsigned)J) : 0;
+  const int rot = (int)(blockIdx.x - quotient(blockIdx.x, ke < KT ? turn : last_turn) * (unsigned)J);      // blockIdx.x % J
   auto tile_at = [&](int t) {                               // t-th tile of this wave's rotated sequence
     int j = t + rot;
     if (j >= J) j -= J;
     return t < J ? kb + wave + j * NW : ke;                 // past the sequence: nothing to load
   };
+  // The rotation epilogue's lookups: positions and sequences ahead of the weights, what follows from them behind the first
+  // window of weights, so that waiting for the former is no wait for the latter.
+  RopeLookup look[MT];
+  if constexpr (EPI == ALICE_EPI_ROPE) {
+#pragma unroll
+    for (int j = 0; j < MT; ++j) rope_look_up((const int*)y_or_positions, seq_of_token, min(row[j], M - 1), look[j]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     fetch(tile_at(u), a[u], b[u]);
     __builtin_amdgcn_sched_barrier(0);       // slot by slot, oldest first: the loop waits for the oldest only
+  }
+  constexpr bool TRIG_AHEAD = EPI == ALICE_EPI_ROPE && RT * MT <= 4;      // (registers)
+  RopeTrig trig[TRIG_AHEAD ? RT : 1][TRIG_AHEAD ? MT : 1];
+  if constexpr (EPI == ALICE_EPI_ROPE) {
+#pragma unroll
+    for (int j = 0; j < MT; ++j) rope_look_up_page(ra, look[j]);
+    if constexpr (TRIG_AHEAD) {
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const RopeCol col = rope_col(ra, min(tile[i], NT - 1) * 16 + g * 4);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) trig[i][j] = rope_trig(ra, look[j].pos, col);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
   for (int t0 = 0; t0 + U < J; t0 += U) {
 #pragma unroll
@@ -162,14 +188,17 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
       if (!row_ok[j]) continue;
-      const RopeToken t = rope_token(ra, row[j]);
+      const RopeToken t = rope_token(ra, look[j]);
 #pragma unroll
       for (int i = 0; i < RT; ++i)
-        if (wave == owner_of(i, j) && tile[i] < NT) rope_store4(ra, row[j], t, tile[i] * 16 + g * 4, acc[i][j]);
+        if (wave == owner_of(i, j) && tile[i] < NT) {
+          const RopeCol col = rope_col(ra, tile[i] * 16 + g * 4);
+          rope_store4(ra, row[j], t, col, acc[i][j], TRIG_AHEAD ? trig[TRIG_AHEAD ? i : 0][TRIG_AHEAD ? j : 0] : rope_trig(ra, t, col));
+        }
     }
     return;
   }
-  TO* yo = y + (size_t)blockIdx.y * M * N;                // the slice's partial sum
+  TO* yo = (TO*)y_or_positions + (size_t)blockIdx.y * M * N;          // the slice's partial sum
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
     if (!row_ok[j]) continue;
@@ -230,7 +259,9 @@ int launch_skinny(const void* x, const void* w, void* y, int M, int N, int K, in
         told = true;                                                                                                           \
       }                                                                                                                        \
     }                                                                                                                          \
-    kern<<<grid, THREADS, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, (TO*)y, M, N, K, KT, NT, per, epi, y_frag, ra);       \
+    kern<<<grid, THREADS, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, EPI == ALICE_EPI_ROPE ? (void*)ra.positions : y, ra.seq_of_token, \
+                                    M, KT, NT, per, reciprocal_of(ceil_div(per, NWV)),                                         \
+                                    reciprocal_of(max(1, ceil_div(KT - per * (split - 1), NWV))), N, K, epi, y_frag, ra);      \
   } while (0)
 #define BY_INPUT(NWV, THREADS)                                                        \
   do {                                                                                \

@@ -27,8 +27,8 @@ constexpr int WM = 8;   // a wave's tile: up to 8 x 4 MFMA tiles = 128 tokens x 
 // row-major path a third of its speed).
 template <int EPI, typename TO, bool FULL, int TM, bool XF, int WN, int KC>
 __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wf,
-                                                               TO* __restrict__ y, int M, int N, int K, int KT, int NT,
-                                                               float epi, int gx, int gy, int kt_per_slice, int y_frag,
+                                                               int M, int KT, int NT, int gx, int gy, int kt_per_slice,
+                                                               int K, int N, TO* __restrict__ y, float epi, int y_frag,
                                                                RopeArgs ra) {
   constexpr int XJ = TM / 4;                               // token tiles each wave stages
   // The rotation epilogue stages 64 tokens x 256 features in the same memory afterwards (ROPE_PITCH elements a token).
@@ -36,7 +36,7 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
   constexpr int LDS_WORDS = (EPI == ALICE_EPI_ROPE && WN == 4 && XS_WORDS < 64 * ROPE_PITCH / 2) ? 64 * ROPE_PITCH / 2 : XS_WORDS;
   __shared__ __align__(16) uint32_t xs_raw[LDS_WORDS];
   u32x4* xs = reinterpret_cast<u32x4*>(xs_raw);            // [2][KC][TM][64]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   // Blocks go to the XCDs round robin by index; XCD x works through the x-th eighth of the tiles in
   // column-major order, so that tiles with the same weight columns meet in one L2.
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
   const int per = (gx * gy + 7) >> 3;
   const int item = xcd * per + local;
   if (local >= per || item >= gx * gy) return;
-  const int bx = item / gy, by = item % gy;
+  const int bx = gy == 1 ? item : item / gy, by = gy == 1 ? 0 : item % gy;
   const int m0 = by * (16 * TM);
   int tile[WN];
 #pragma unroll
@@ -59,15 +59,15 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
   }
   // Loads are unconditional (see the streaming kernel): rows and tiles beyond the matrix are clamped, and
   // k-tiles beyond the slice bring zero weights.
-  const bf16_t* xsrc[XJ];        // this lane's place in the activations at k-tile 0, for the token tiles it stages
+  const bf16_t* xsrc[XJ];        // the wave's (rows: this lane's) place in the activations at k-tile 0, for the token tiles it stages
 #pragma unroll
   for (int j = 0; j < XJ; ++j) {
-    if constexpr (XF) xsrc[j] = x + ((size_t)min((m0 >> 4) + XJ * wave + j, (M - 1) >> 4) * KT * 64 + lane) * 8;
+    if constexpr (XF) xsrc[j] = x + (size_t)min((m0 >> 4) + XJ * wave + j, (M - 1) >> 4) * KT * 512;
     else xsrc[j] = x + (size_t)min(m0 + (XJ * wave + j) * 16 + r, M - 1) * K;
   }
   const bf16_t* wsrc[WN];
 #pragma unroll
-  for (int i = 0; i < WN; ++i) wsrc[i] = wf + (size_t)min(tile[i], NT - 1) * KT * 512 + lane * 8;
+  for (int i = 0; i < WN; ++i) wsrc[i] = wf + (size_t)min(tile[i], NT - 1) * KT * 512;
 
   f32x4 acc[WN][TM];
 #pragma unroll
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
 #pragma unroll
       for (int j = 0; j < XJ; ++j) {
         const int kt = max(0, min(kt_base + s * KC + kc, kt_end - 1));      // past the slice: the weights are zeros
-        if constexpr (XF) xr[kc][j] = *reinterpret_cast<const u32x4*>(xsrc[j] + (size_t)kt * 512);
+        if constexpr (XF) xr[kc][j] = reinterpret_cast<const u32x4*>(xsrc[j] + (size_t)kt * 512)[(unsigned)lane];
         else xr[kc][j] = *reinterpret_cast<const u32x4*>(xsrc[j] + min(kt * 32 + g * 8, K - 8));
       }
   };
@@ -93,22 +93,35 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
 #pragma unroll
       for (int j = 0; j < XJ; ++j) xs[((buf * KC + kc) * TM + XJ * wave + j) * 64 + lane] = xr[kc][j];
   };
-  const bf16_t* zero = reinterpret_cast<const bf16_t*>(g_zero_tile) + lane * 8;
+  const bf16_t* zero = reinterpret_cast<const bf16_t*>(g_zero_tile);
   auto w_load = [&](int rel, u32x4 (&w)[WN]) {                // rel: k-tile relative to the slice
     const int kt = kt_base + rel;
     const bool kok = kt < kt_end;
 #pragma unroll
-    for (int i = 0; i < WN; ++i) w[i] = *reinterpret_cast<const u32x4*>(kok ? wsrc[i] + (size_t)kt * 512 : zero);
+    for (int i = 0; i < WN; ++i) w[i] = reinterpret_cast<const u32x4*>(kok ? wsrc[i] + (size_t)kt * 512 : zero)[(unsigned)lane];
   };
   // blockIdx.y: the slice of the inner dimension this block sums (its own partial result y[slice][M][N])
   const int kt_lo = blockIdx.y * kt_per_slice, kt_hi = min(KT, kt_lo + kt_per_slice);
   const int S = (kt_hi - kt_lo + KC - 1) / KC;
   y += (size_t)blockIdx.y * M * N;
+  // Narrow tiles with the rotation epilogue: its lookups ahead of the products (see the streaming kernel).
+  constexpr bool LOOK_AHEAD = EPI == ALICE_EPI_ROPE && WN != 4;
+  RopeLookup look[LOOK_AHEAD ? TM : 1];
+  if constexpr (LOOK_AHEAD) {
+#pragma unroll
+    for (int j = 0; j < TM; ++j) rope_look_up(ra.positions, ra.seq_of_token, min(m0 + j * 16 + r, M - 1), look[j]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   stage_load(0);
   stage_store(0);
 #pragma unroll
   for (int kc = 0; kc < KC; ++kc) {
     w_load(kc, wk[kc]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if constexpr (LOOK_AHEAD) {
+#pragma unroll
+    for (int j = 0; j < TM; ++j) rope_look_up_page(ra, look[j]);
     __builtin_amdgcn_sched_barrier(0);
   }
   // Loads run one stage ahead and are unconditional (a k-tile beyond the slice in the last, partial stage
@@ -134,7 +147,7 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
           // this weight tile's registers are free again: fetch the same tile of the next stage now, so that the
           // loads of a stage are spread over its products instead of arriving at the memory system in a burst
           __builtin_amdgcn_sched_barrier(0);
-          wk[kc][i] = *reinterpret_cast<const u32x4*>(kok ? wsrc[i] + (size_t)kt_next * 512 : zero);
+          wk[kc][i] = reinterpret_cast<const u32x4*>(kok ? wsrc[i] + (size_t)kt_next * 512 : zero)[(unsigned)lane];
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -157,14 +170,24 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
     RopeCol col[WN];
 #pragma unroll
     for (int i = 0; i < WN; ++i) col[i] = rope_col(ra, min(tile[i], NT - 1) * 16 + g * 4);
+    // the cosines and sines of four token tiles at a time: their loads are in flight together and ahead of the stores
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      const int m = m0 + j * 16 + r;
-      if (m >= M) continue;
-      const RopeToken t = rope_token(ra, m);
+    for (int j0 = 0; j0 < TM; j0 += 4) {
+      RopeTrig tr[4][WN];
 #pragma unroll
-      for (int i = 0; i < WN; ++i)
-        if (tile[i] < NT) rope_store4(ra, m, t, col[i], acc[i][j], rope_trig(ra, t, col[i]));
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < WN; ++i) tr[j][i] = rope_trig(ra, look[j0 + j].pos, col[i]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int m = m0 + (j0 + j) * 16 + r;
+        if (m >= M) continue;
+        const RopeToken t = rope_token(ra, look[j0 + j]);
+#pragma unroll
+        for (int i = 0; i < WN; ++i)
+          if (tile[i] < NT) rope_store4(ra, m, t, col[i], acc[i][j0 + j], tr[j][i]);
+      }
     }
     return;
   } else if constexpr (EPI == ALICE_EPI_ROPE) {
@@ -348,8 +371,8 @@ int launch_tiled_as(const void* x, const void* w, void* y, int M, int N, int K, 
   const int gx = EPI == ALICE_EPI_GEGLU ? ceil_div(N / 16, 4 * WN / 2) : ceil_div(NT, 4 * WN);
   const int gy = ceil_div(M, 16 * TM);
   dim3 grid(8 * ceil_div(gx * gy, 8), split);
-  linear_tiled_lds_kernel<EPI, TO, false, TM, XF, WN, KC><<<grid, 256, 0, s>>>((const bf16_t*)x, (const bf16_t*)w, (TO*)y, M, N, K, KT, NT,
-                                                                             epi, gx, gy, per, y_frag, ra);
+  linear_tiled_lds_kernel<EPI, TO, false, TM, XF, WN, KC><<<grid, 256, 0, s>>>((const bf16_t*)x, (const bf16_t*)w, M, KT, NT, gx, gy, per, K, N,
+                                                                             (TO*)y, epi, y_frag, ra);
   ALICE_LAUNCH_CHECK();
   return 0;
 }

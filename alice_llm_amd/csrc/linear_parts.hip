@@ -20,10 +20,10 @@ __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2
 
 template <int WN, int SR>
 __global__ __launch_bounds__(256) void linear_parts_kernel(const float* __restrict__ parts, const bf16_t* __restrict__ wf,
-                                                         float* __restrict__ y, int M, int N, int KT, int NT, int per,
-                                                         int S, int D, int nH) {
+                                                         float* __restrict__ y, int KT, int NT, int per, int M, int S,
+                                                         uint32_t chunks_reciprocal, int D, uint32_t D_reciprocal, int nH, int N) {
   __shared__ __align__(16) u32x4 xs[PARTS_MAX_TILES * 64];             // the slice's activations, one token tile
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int kt0 = blockIdx.y * per;                                    // the slice's first k-tile
   const int k0 = kt0 * 32;
@@ -32,35 +32,35 @@ __global__ __launch_bounds__(256) void linear_parts_kernel(const float* __restri
 #pragma unroll
   for (int i = 0; i < WN; ++i) {
     tile[i] = (blockIdx.x * 4 + wave) * WN + i;
-    wsrc[i] = wf + ((size_t)min(tile[i], NT - 1) * KT + kt0) * 512 + lane * 8;
+    wsrc[i] = wf + ((size_t)min(tile[i], NT - 1) * KT + kt0) * 512;
   }
   // the first weight tiles: they come from memory, everything below from the L2
   u32x4 wk[PARTS_U][WN];
 #pragma unroll
   for (int u = 0; u < PARTS_U; ++u)
 #pragma unroll
-    for (int i = 0; i < WN; ++i) wk[u][i] = *reinterpret_cast<const u32x4*>(wsrc[i] + (size_t)min(u, per - 1) * 512);
+    for (int i = 0; i < WN; ++i) wk[u][i] = reinterpret_cast<const u32x4*>(wsrc[i] + (size_t)min(u, per - 1) * 512)[(unsigned)lane];
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- the combined output of the slice: an item is eight consecutive features of one token.  A thread works
   // out the weights of its token's splits itself (the 32 threads of a token and head read the same maxima and sums),
   // so nothing but the loads stands between the kernel's start and the product; they are all in flight at once
   // (at most SR splits: with more, which single sequences at long contexts have, the combine stays a kernel).
-  const size_t pstride = (size_t)(D + ALICE_ATTN_PARTS_HEAD);
+  const unsigned pstride = D + ALICE_ATTN_PARTS_HEAD;
   const int chunks = per * 4;
   for (int it = threadIdx.x; it < 16 * chunks; it += 256) {
-    const int m = it / chunks, c = it % chunks;
+    const int m = quotient(it, chunks_reciprocal), c = it - m * chunks;
     u32x4 packed = {0u, 0u, 0u, 0u};
     if (m < M) {
-      const int k = k0 + c * 8, e0 = k % D;
-      const float* pr = parts + ((size_t)m * nH + k / D) * S * pstride;
+      const int k = k0 + c * 8, head = quotient(k, D_reciprocal), e0 = k - head * D;
+      const unsigned pr = (unsigned)(m * nH + head) * S * pstride;       // elements: the launcher keeps them within 32 bits
       float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       float ll = 0.f;
       float2 ml[SR];
       float4 v[SR][2];
 #pragma unroll
       for (int q = 0; q < SR; ++q) {
-        const float* src = pr + (size_t)min(q, S - 1) * pstride;
+        const float* src = parts + (pr + (unsigned)min(q, S - 1) * pstride);
         ml[q] = *reinterpret_cast<const float2*>(src);
 #pragma unroll
         for (int j = 0; j < 2; ++j) v[q][j] = *reinterpret_cast<const float4*>(src + ALICE_ATTN_PARTS_HEAD + e0 + 4 * j);
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void linear_parts_kernel(const float* __restri
         for (int i = 0; i < WN; ++i) acc[i] = mfma16(wk[u][i], b, acc[i]);
         if (t + PARTS_U < per) {
 #pragma unroll
-          for (int i = 0; i < WN; ++i) wk[u][i] = *reinterpret_cast<const u32x4*>(wsrc[i] + (size_t)(t + PARTS_U) * 512);
+          for (int i = 0; i < WN; ++i) wk[u][i] = reinterpret_cast<const u32x4*>(wsrc[i] + (size_t)(t + PARTS_U) * 512)[(unsigned)lane];
         }
       }
     }
@@ -155,14 +155,15 @@ extern "C" int alice_linear_parts(const float* parts, int splits, int nH, int d,
                                   hipStream_t stream) {
   ALICE_CHECK(parts && w && y, "linear (attention parts): a pointer is missing");
   const PartsPlan p = parts_plan(M, N, nH, d, splits);
+  static_assert(16l * 16384 / 32 * 16 * (32 + ALICE_ATTN_PARTS_HEAD) < (1l << 29), "offsets of parts and of their bytes are 32-bit");
   ALICE_CHECK(p.split > 0, "linear (attention parts): %d tokens, %d heads of %d, %d splits and %d output features are not covered", M, nH, d, splits, N);
   ALICE_CHECK(((uintptr_t)parts & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)y & 15) == 0, "linear (attention parts): operands are not aligned");
   const int KT = nH * d / 32, NT = ceil_div(N, 16), per = KT / p.split;
   dim3 grid(ceil_div(NT, 4 * p.wn), p.split);
 #define GO(WNV)                                                                                                       \
   do {                                                                                                                \
-    if (splits <= 8) linear_parts_kernel<WNV, 8><<<grid, 256, 0, stream>>>(parts, (const bf16_t*)w, y, M, N, KT, NT, per, splits, d, nH); \
-    else linear_parts_kernel<WNV, 16><<<grid, 256, 0, stream>>>(parts, (const bf16_t*)w, y, M, N, KT, NT, per, splits, d, nH); \
+    if (splits <= 8) linear_parts_kernel<WNV, 8><<<grid, 256, 0, stream>>>(parts, (const bf16_t*)w, y, KT, NT, per, M, splits, reciprocal_of(4 * per), d, reciprocal_of(d), nH, N); \
+    else linear_parts_kernel<WNV, 16><<<grid, 256, 0, stream>>>(parts, (const bf16_t*)w, y, KT, NT, per, M, splits, reciprocal_of(4 * per), d, reciprocal_of(d), nH, N); \
   } while (0)
   if (p.wn == 4) GO(4); else if (p.wn == 2) GO(2); else GO(1);
 #undef GO
