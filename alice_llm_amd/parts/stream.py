@@ -130,16 +130,18 @@ class ResidualStream:
             self._add_pointwise(norm, out, ops.LAYOUT_FRAG16 if frag else ops.LAYOUT_ROW)
             return out
         pre = _fused_pre(norm)
-        if fragments and pre is not None and out_dtype == torch.bfloat16 and FragmentActs.possible(self.precision, T, H):
+        # (without a norm the stream itself, rounded, is what the consumer reads)
+        if fragments and (pre is not None or norm is None) and out_dtype == torch.bfloat16 and FragmentActs.possible(self.precision, T, H):
             post = self._post
             pf = post.fused() if post is not None and hasattr(post, "fused") else None
-            if self._branch is not None and not ((post is None or pf is not None) and (pf is None or pf[0].dtype == pre[0].dtype)):
+            if self._branch is not None and not ((post is None or pf is not None) and (pf is None or pre is None or pf[0].dtype == pre[0].dtype)):
                 self.flush()
             n, b = self._partials() if self._branch is not None else (1, None)
             w_post, eps_post, off_post = pf if (pf is not None and b is not None) else (None, 0.0, 0.0)
+            w_pre, eps_pre, off_pre, b_pre = pre if pre is not None else (None, 0.0, 0.0, None)
             out = FragmentActs.empty(T, H, self.x.device)
-            ops.add_norm(self.x, b, w_post, pre[0], out.data, eps_post=eps_post, eps_pre=pre[1], off_post=off_post,
-                         off_pre=pre[2], b_pre=pre[3], n_partials=n, full_precision=self.precision.full, out_layout=ops.LAYOUT_FRAG16)
+            ops.add_norm(self.x, b, w_post, w_pre, out.data, eps_post=eps_post, eps_pre=eps_pre, off_post=off_post,
+                         off_pre=off_pre, b_pre=b_pre, n_partials=n, full_precision=self.precision.full, out_layout=ops.LAYOUT_FRAG16)
             self._branch = None
             self._post = None
             return out

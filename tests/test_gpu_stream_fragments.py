@@ -1,0 +1,31 @@
+"""The stream itself, without a norm, in the matrix products' fragment order: the same numbers as in rows."""
+import pytest
+import torch
+
+from alice_llm_amd.parts.base import FragmentActs, Precision
+from alice_llm_amd.parts.norm import RMSNorm
+from alice_llm_amd.parts.stream import ResidualStream
+from test_gpu_kernels import acts_from_fragments, rnd
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("T,H", [(1, 64), (15, 2304), (17, 96), (64, 2048), (319, 160), (320, 256), (333, 2048), (700, 4128)])
+@pytest.mark.parametrize("slices,post", [(0, False), (1, False), (1, True), (3, True)])
+def test_the_stream_without_a_norm_in_fragment_order(T, H, slices, post):
+    precision = Precision.of("bfloat16")
+    norm = None
+    if post:
+        norm = RMSNorm(precision, dim=H, eps=1e-6, weight_offset=1.0)
+        norm.assign("weight", rnd(H, seed=3, scale=0.1, dtype=torch.bfloat16))
+    outs, streams = [], []
+    for fragments in (False, True):
+        s = ResidualStream(rnd(T, H, seed=1), precision)
+        if slices:
+            s.push(rnd(*((slices,) if slices > 1 else ()), T, H, seed=2), norm)
+        outs.append(s.normed(None, fragments=fragments))
+        streams.append(s)
+    assert isinstance(outs[1], FragmentActs) and outs[1].shape == (T, H)
+    assert torch.equal(acts_from_fragments(outs[1].data, T, H), outs[0].cpu())
+    assert torch.equal(streams[0].x, streams[1].x) and streams[1]._branch is None
