@@ -100,11 +100,12 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __
     return t < J ? kb + wave + j * NW : ke;                 // past the sequence: nothing to load
   };
   // The rotation epilogue's lookups: positions and sequences ahead of the weights, what follows from them behind the first
-  // window of weights, so that waiting for the former is no wait for the latter.
-  RopeLookup look[MT];
+  // window of weights, so that waiting for the former is no wait for the latter.  (The output tiles that a wave owns below are
+  // all of one token tile, wave % MT: its tokens' places are all that the wave looks up.)
+  static_assert(NW % MT == 0, "a wave owns output tiles of one token tile");
+  RopeLookup look;
   if constexpr (EPI == ALICE_EPI_ROPE) {
-#pragma unroll
-    for (int j = 0; j < MT; ++j) rope_look_up((const int*)y_or_positions, seq_of_token, min(row[j], M - 1), look[j]);
+    rope_look_up((const int*)y_or_positions, seq_of_token, min(wave % MT * 16 + r, M - 1), look);
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
@@ -112,19 +113,11 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __
     fetch(tile_at(u), a[u], b[u]);
     __builtin_amdgcn_sched_barrier(0);       // slot by slot, oldest first: the loop waits for the oldest only
   }
-  constexpr bool TRIG_AHEAD = EPI == ALICE_EPI_ROPE && RT * MT <= 4;      // (registers)
-  RopeTrig trig[TRIG_AHEAD ? RT : 1][TRIG_AHEAD ? MT : 1];
+  RopeTrig trig[RT];
   if constexpr (EPI == ALICE_EPI_ROPE) {
+    rope_look_up_page(ra, look);
 #pragma unroll
-    for (int j = 0; j < MT; ++j) rope_look_up_page(ra, look[j]);
-    if constexpr (TRIG_AHEAD) {
-#pragma unroll
-      for (int i = 0; i < RT; ++i) {
-        const RopeCol col = rope_col(ra, min(tile[i], NT - 1) * 16 + g * 4);
-#pragma unroll
-        for (int j = 0; j < MT; ++j) trig[i][j] = rope_trig(ra, look[j].pos, col);
-      }
-    }
+    for (int i = 0; i < RT; ++i) trig[i] = rope_trig(ra, look.pos, rope_col(ra, min(tile[i], NT - 1) * 16 + g * 4));
     __builtin_amdgcn_sched_barrier(0);
   }
   for (int t0 = 0; t0 + U < J; t0 += U) {
@@ -185,16 +178,13 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __
     }
 
   if constexpr (EPI == ALICE_EPI_ROPE) {
+    const RopeToken t = rope_token(ra, look);
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
       if (!row_ok[j]) continue;
-      const RopeToken t = rope_token(ra, look[j]);
 #pragma unroll
       for (int i = 0; i < RT; ++i)
-        if (wave == owner_of(i, j) && tile[i] < NT) {
-          const RopeCol col = rope_col(ra, tile[i] * 16 + g * 4);
-          rope_store4(ra, row[j], t, col, acc[i][j], TRIG_AHEAD ? trig[TRIG_AHEAD ? i : 0][TRIG_AHEAD ? j : 0] : rope_trig(ra, t, col));
-        }
+        if (wave == owner_of(i, j) && tile[i] < NT) rope_store4(ra, row[j], t, rope_col(ra, tile[i] * 16 + g * 4), acc[i][j], trig[i]);
     }
     return;
   }
