@@ -27,8 +27,8 @@ constexpr int WM = 8;   // a wave's tile: up to 8 x 4 MFMA tiles = 128 tokens x 
 // row-major path a third of its speed).
 template <int EPI, typename TO, bool FULL, int TM, bool XF, int WN, int KC>
 __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wf,
-                                                               int M, int KT, int NT, int gx, int gy, int kt_per_slice,
-                                                               int K, int N, TO* __restrict__ y, float epi, int y_frag,
+                                                               int M, int KT, int NT, int items, int tiles, int gy, uint32_t gy_reciprocal,
+                                                               int kt_per_slice, TO* __restrict__ y, int N, int K, float epi, int y_frag,
                                                                RopeArgs ra) {
   constexpr int XJ = TM / 4;                               // token tiles each wave stages
   // The rotation epilogue stages 64 tokens x 256 features in the same memory afterwards (ROPE_PITCH elements a token).
@@ -38,21 +38,38 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
   u32x4* xs = reinterpret_cast<u32x4*>(xs_raw);            // [2][KC][TM][64]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  // Blocks go to the XCDs round robin by index; XCD x works through the x-th eighth of the tiles in
-  // column-major order, so that tiles with the same weight columns meet in one L2.
+  // Blocks go to the XCDs round robin by index; XCD x works through the x-th eighth of the items.  An item is a tile of a
+  // slice of the inner dimension: the slices one after the other, so that an XCD reads the activations of its slices alone; a slice's
+  // tiles in bands of 1,024 tokens, a band column by column, so that the 64 blocks that run on an XCD at a time are 8 by 8 tiles,
+  // which read 3,072 rows of both operands between them; the whole height of 8,192 tokens by one column is 8,448.  What the blocks
+  // of an XCD read in common comes from its L2; what each XCD reads for itself comes through the fabric, and that is what bounds
+  // this kernel beside the matrix cores.  (Every XCD through all slices of its tiles, whole columns, before: 9B shape, down product
+  // at 300 / 700 tokens 66 and 106 us, 41 and 74 so; a layer's four products at 2,048 / 4,096 / 8,192 tokens 700, 1,397 and 2,747, and
+  // 671, 1,281 and 2,538 so; 2B at 117 / 2,048 / 8,192 61, 317 and 1,147, and 59, 305 and 1,075.  Bands of 512 and 768 tokens are within
+  // 1 % of that, 2,048 and more lose most of it.  Each output's sums are the same in the same order.)
   const int id = blockIdx.x, xcd = id & 7, local = id >> 3;
-  const int per = (gx * gy + 7) >> 3;
+  const int per = (items + 7) >> 3;
   const int item = xcd * per + local;
-  if (local >= per || item >= gx * gy) return;
-  const int bx = gy == 1 ? item : item / gy, by = gy == 1 ? 0 : item % gy;
+  if (local >= per || item >= items) return;
+  const int slice = items == tiles ? 0 : (unsigned)item / (unsigned)tiles, t = item - slice * tiles;
+  constexpr int BAND = 1024 / (16 * TM);                   // tiles
+  int bx, by;
+  if (gy <= BAND) {
+    bx = quotient(t, gy_reciprocal);
+    by = t - bx * gy;
+  } else {
+    const unsigned gx = tiles / (unsigned)gy, band = t / (BAND * gx), in = t - band * BAND * gx, high = min(BAND, gy - (int)band * BAND);
+    bx = in / high;
+    by = band * BAND + in - bx * high;
+  }
   const int m0 = by * (16 * TM);
   int tile[WN];
 #pragma unroll
   for (int i = 0; i < WN; ++i) {
     if (EPI == ALICE_EPI_GEGLU) {
       const int pair = (bx * 4 + wave) * (WN / 2) + (i >> 1);
-      tile[i] = (i & 1) ? N / 16 + pair : pair;
-      if (pair >= N / 16) tile[i] = NT;
+      tile[i] = (i & 1) ? NT / 2 + pair : pair;
+      if (pair >= NT / 2) tile[i] = NT;
     } else {
       tile[i] = (bx * 4 + wave) * WN + i;
     }
@@ -76,7 +93,7 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
     for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   u32x4 xr[KC][XJ], wk[KC][WN];
-  const int kt_base = blockIdx.y * kt_per_slice, kt_end = min(KT, kt_base + kt_per_slice);
+  const int kt_base = slice * kt_per_slice, kt_end = min(KT, kt_base + kt_per_slice);
   auto stage_load = [&](int s) {
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc)
@@ -100,10 +117,8 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
 #pragma unroll
     for (int i = 0; i < WN; ++i) w[i] = reinterpret_cast<const u32x4*>(kok ? wsrc[i] + (size_t)kt * 512 : zero)[(unsigned)lane];
   };
-  // blockIdx.y: the slice of the inner dimension this block sums (its own partial result y[slice][M][N])
-  const int kt_lo = blockIdx.y * kt_per_slice, kt_hi = min(KT, kt_lo + kt_per_slice);
-  const int S = (kt_hi - kt_lo + KC - 1) / KC;
-  y += (size_t)blockIdx.y * M * N;
+  const int S = (kt_end - kt_base + KC - 1) / KC;
+  y += (size_t)slice * M * N;                               // the slice's own partial result
   // Narrow tiles with the rotation epilogue: its lookups ahead of the products (see the streaming kernel).
   constexpr bool LOOK_AHEAD = EPI == ALICE_EPI_ROPE && WN != 4;
   RopeLookup look[LOOK_AHEAD ? TM : 1];
@@ -370,9 +385,10 @@ int launch_tiled_as(const void* x, const void* w, void* y, int M, int N, int K, 
   const int per = ceil_div(KT, split);
   const int gx = EPI == ALICE_EPI_GEGLU ? ceil_div(N / 16, 4 * WN / 2) : ceil_div(NT, 4 * WN);
   const int gy = ceil_div(M, 16 * TM);
-  dim3 grid(8 * ceil_div(gx * gy, 8), split);
-  linear_tiled_lds_kernel<EPI, TO, false, TM, XF, WN, KC><<<grid, 256, 0, s>>>((const bf16_t*)x, (const bf16_t*)w, M, KT, NT, gx, gy, per, K, N,
-                                                                             (TO*)y, epi, y_frag, ra);
+  ALICE_CHECK((long)gx * gy * split < (1l << 30), "linear: too many tiles for one launch");
+  const int tiles = gx * gy, items = tiles * split, grid = 8 * ceil_div(items, 8);
+  linear_tiled_lds_kernel<EPI, TO, false, TM, XF, WN, KC><<<grid, 256, 0, s>>>((const bf16_t*)x, (const bf16_t*)w, M, KT, NT, items, tiles, gy, reciprocal_of(gy),
+                                                                             per, (TO*)y, N, K, epi, y_frag, ra);
   ALICE_LAUNCH_CHECK();
   return 0;
 }
