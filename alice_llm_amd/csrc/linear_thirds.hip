@@ -17,6 +17,7 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int BK = THIRDS_BK;                                 // inner elements a stage: one product's
@@ -26,8 +27,9 @@ __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x
 }
 
 // Eight elements of a row, times `sign` (1 or -1, with SIGNED), as three times eight bfloat16 numbers.
+// top: the largest sizes met so far, as bfloat16 bits.
 template <bool SIGNED>
-__device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3], float sign = 1.f) {
+__device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3], u16x2& top, float sign = 1.f) {
   const uint32_t flip = (__float_as_uint(sign) >> 31) * 0x80008000u;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -36,6 +38,7 @@ __device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3], float
     for (int t = 0; t < 3; ++t) {
       const uint32_t h = SIGNED && t == 0 ? pack_bf16x2(x, y) ^ flip : pack_bf16x2(x, y);
       p[t][i] = h;
+      if (t == 0) top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, h & 0x7fff7fffu));
       const float hx = __uint_as_float(h << 16), hy = __uint_as_float(h & 0xffff0000u);
       x = SIGNED && t == 0 ? fmaf(x, sign, -hx) : x - hx;
       y = SIGNED && t == 0 ? fmaf(y, sign, -hy) : y - hy;
@@ -120,9 +123,10 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   clear();
   if (tid == 0) again = 0;
   const float sign = group ? -1.f : 1.f;
+  u16x2 top = {0, 0};                                         // the largest sizes among the numbers that this lane splits
   auto put = [&](int j, int buf) {
     u32x4 p[3];
-    thirds<true>(xr[j], p, sign);
+    thirds<true>(xr[j], p, top, sign);
 #pragma unroll
     for (int t = 0; t < 3; ++t) plane(buf, t, wave + NW * j)[lane] = p[t];
   };
@@ -149,7 +153,7 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
     for (int i = 0; i < TN; ++i) {
       u32x4 w[3];
       if (k0 + BK > k_end) clear_beyond(wr[i], k0);
-      thirds<false>(wr[i], w);
+      thirds<false>(wr[i], w, top);
       if (!last) load(wsrc[i], wr[i], k0 + BK);
       // the smallest products first
       constexpr int WT[6] = {2, 0, 1, 1, 0, 0}, XT[6] = {0, 2, 1, 0, 1, 0};
@@ -176,9 +180,10 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   __syncthreads();
 
   // A number that is not finite, or that rounds to no finite bfloat16, has a remainder that is none, and every sum that it enters
-  // is then none either.  Sums so small that thirds may have fallen below the smallest bfloat16, and those that are no finite
-  // numbers, are taken again by 32-bit products; so is the whole tile around them.
-  bool odd = false;
+  // is then none either.  What of a number is below the smallest normal bfloat16, 2^-126, may be lost: with 16,384 others of at most
+  // 2^20 that is 2^-92 of a sum, less than its own rounding from 2^-64 on.  Smaller sums, those that are no finite numbers, and all
+  // where a number is larger than 2^20, are taken again by 32-bit products; so is the whole tile around them.
+  bool odd = max(top.x, top.y) > 0x4980;                      // 2^20; infinities and no numbers are larger
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float v = fabsf(acc[i][j][e]);
-        odd = odd | (!(v >= 0x1p-80f) & (v != 0.f)) | !(v < INFINITY);
+        odd = odd | (!(v >= 0x1p-64f) & (v != 0.f)) | !(v < INFINITY);
       }
   if (__ballot(odd) != 0 && lane == 0) again = 1;             // any of them: the same value
   __syncthreads();

@@ -97,6 +97,16 @@ def test_what_has_no_three_parts():
     assert (product(torch.zeros(M, K, device=DEV), w2) == 0).all()
 
 
+@pytest.mark.parametrize("ex,ew", [(-112, 60), (60, -112), (-120, 21), (-110, 100)])
+def test_small_numbers_times_large_ones(ex, ew):
+    """The last parts of the small factor are below the smallest normal bfloat16 while the sums are ordinary numbers."""
+    M, N, K = 500, 4096, 2304
+    x, w = torch.ldexp(rnd(M, K, seed=4), torch.tensor(ex, device=DEV)), torch.ldexp(rnd(N, K, seed=5), torch.tensor(ew, device=DEV))
+    got, ref = product(x, w).double(), x.double() @ w.double().T
+    assert ((got - ref).abs() <= 16 * bound(x, w)).all()          # (32 roundings for 32 elements instead of 6)
+    assert float((got - ref).norm() / ref.norm()) <= 1e-5
+
+
 def test_a_token_depends_on_no_other_and_captured_steps_add_as_eager_ones():
     M, N, K = 129, 9216, 2304
     x, w = rnd(192, K, seed=1), rnd(N, K, seed=2)
