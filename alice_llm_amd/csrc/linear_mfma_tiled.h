@@ -11,7 +11,7 @@ namespace {
 constexpr int WM = 8;   // a wave's tile: up to 8 x 4 MFMA tiles = 128 tokens x 64 output features
 
 // ---------------------------------------------------------------- tiled, many tokens
-// Block: 4 waves side by side along N; every wave computes 16 TM (128 or 64) tokens x 16 WN (64, 32 or 16)
+// Block: 4 waves side by side along N; every wave computes 16 TM (128, 64 or 32) tokens x 16 WN (64, 32 or 16)
 // output features (at most 8 x 4 MFMA tiles, 128 accumulator registers per lane) and streams its own weight
 // tiles straight from memory.  The block's tokens x 64 inner elements of activations are staged once in LDS (in
 // fragment order, so LDS reads and writes are linear) and read by all four waves.  Two stages are kept: while one is used for the
@@ -30,7 +30,8 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
                                                                int M, int KT, int NT, int items, int tiles, int gy, uint32_t gy_reciprocal,
                                                                int kt_per_slice, TO* __restrict__ y, int N, int K, float epi, int y_frag,
                                                                RopeArgs ra) {
-  constexpr int XJ = TM / 4;                               // token tiles each wave stages
+  constexpr int XJ = TM >= 4 ? TM / 4 : 1;                 // token tiles each wave stages
+  constexpr int XW = TM >= 4 ? 1 : 4 / TM, XK = KC / XW;   // waves that share a token tile; k-tiles of a stage that each of them takes
   // The rotation epilogue stages 64 tokens x 256 features in the same memory afterwards (ROPE_PITCH elements a token).
   constexpr int XS_WORDS = 2 * KC * TM * 64 * 4;
   constexpr int LDS_WORDS = (EPI == ALICE_EPI_ROPE && WN == 4 && XS_WORDS < 64 * ROPE_PITCH / 2) ? 64 * ROPE_PITCH / 2 : XS_WORDS;
@@ -76,11 +77,12 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
   }
   // Loads are unconditional (see the streaming kernel): rows and tiles beyond the matrix are clamped, and
   // k-tiles beyond the slice bring zero weights.
+  const int xtile = TM >= 4 ? XJ * wave : wave % TM, xkt = TM >= 4 ? 0 : wave / TM;      // the wave's first token tile, its first k-tile of a stage
   const bf16_t* xsrc[XJ];        // the wave's (rows: this lane's) place in the activations at k-tile 0, for the token tiles it stages
 #pragma unroll
   for (int j = 0; j < XJ; ++j) {
-    if constexpr (XF) xsrc[j] = x + (size_t)min((m0 >> 4) + XJ * wave + j, (M - 1) >> 4) * KT * 512;
-    else xsrc[j] = x + (size_t)min(m0 + (XJ * wave + j) * 16 + r, M - 1) * K;
+    if constexpr (XF) xsrc[j] = x + (size_t)min((m0 >> 4) + xtile + j, (M - 1) >> 4) * KT * 512;
+    else xsrc[j] = x + (size_t)min(m0 + (xtile + j) * 16 + r, M - 1) * K;
   }
   const bf16_t* wsrc[WN];
 #pragma unroll
@@ -92,23 +94,23 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
 #pragma unroll
     for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  u32x4 xr[KC][XJ], wk[KC][WN];
+  u32x4 xr[XK][XJ], wk[KC][WN];
   const int kt_base = slice * kt_per_slice, kt_end = min(KT, kt_base + kt_per_slice);
   auto stage_load = [&](int s) {
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc)
+    for (int kc = 0; kc < XK; ++kc)
 #pragma unroll
       for (int j = 0; j < XJ; ++j) {
-        const int kt = max(0, min(kt_base + s * KC + kc, kt_end - 1));      // past the slice: the weights are zeros
+        const int kt = max(0, min(kt_base + s * KC + kc * XW + xkt, kt_end - 1));      // past the slice: the weights are zeros
         if constexpr (XF) xr[kc][j] = reinterpret_cast<const u32x4*>(xsrc[j] + (size_t)kt * 512)[(unsigned)lane];
         else xr[kc][j] = *reinterpret_cast<const u32x4*>(xsrc[j] + min(kt * 32 + g * 8, K - 8));
       }
   };
   auto stage_store = [&](int buf) {
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc)
+    for (int kc = 0; kc < XK; ++kc)
 #pragma unroll
-      for (int j = 0; j < XJ; ++j) xs[((buf * KC + kc) * TM + XJ * wave + j) * 64 + lane] = xr[kc][j];
+      for (int j = 0; j < XJ; ++j) xs[((buf * KC + kc * XW + xkt) * TM + xtile + j) * 64 + lane] = xr[kc][j];
   };
   const bf16_t* zero = reinterpret_cast<const bf16_t*>(g_zero_tile);
   auto w_load = [&](int rel, u32x4 (&w)[WN]) {                // rel: k-tile relative to the slice
@@ -182,20 +184,21 @@ __global__ __launch_bounds__(256, 2) void linear_tiled_lds_kernel(const bf16_t* 
 
   if constexpr (EPI == ALICE_EPI_ROPE && WN != 4) {
     // narrow tiles (a few hundred tokens): every lane stores its own pairs, as the streaming kernel does
+    constexpr int JB = TM < 4 ? TM : 4;
     RopeCol col[WN];
 #pragma unroll
     for (int i = 0; i < WN; ++i) col[i] = rope_col(ra, min(tile[i], NT - 1) * 16 + g * 4);
     // the cosines and sines of four token tiles at a time: their loads are in flight together and ahead of the stores
 #pragma unroll
-    for (int j0 = 0; j0 < TM; j0 += 4) {
-      RopeTrig tr[4][WN];
+    for (int j0 = 0; j0 < TM; j0 += JB) {
+      RopeTrig tr[JB][WN];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < JB; ++j)
 #pragma unroll
         for (int i = 0; i < WN; ++i) tr[j][i] = rope_trig(ra, look[j0 + j].pos, col[i]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < JB; ++j) {
         const int m = m0 + (j0 + j) * 16 + r;
         if (m >= M) continue;
         const RopeToken t = rope_token(ra, look[j0 + j]);

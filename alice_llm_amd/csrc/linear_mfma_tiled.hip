@@ -56,6 +56,14 @@ bool narrow_built(int epi, int y_dtype) {
   return (epi == ALICE_EPI_NONE && y_dtype == DT_F32) || (epi == ALICE_EPI_GEGLU && y_dtype == DT_BF16) || epi == ALICE_EPI_ROPE;
 }
 
+// With the rotation epilogue the inner dimension cannot be cut into slices, and up to 128 tokens blocks of 64 tokens leave half of the
+// chip without one: blocks of 32 tokens x 64 features, where all of them fit on the chip at a time.  A block's time is that of its
+// own loads (a CU gets 40 to 54 GB/s), and these are three quarters of the larger block's.  The 2B shape at 65 / 96 / 128 tokens 12.0,
+// 12.2 and 12.9 us, and 9.9, 10.2 and 10.1 so; 9B at 33 / 48 / 64 tokens 18.1, 18.4 and 19.4, and 15.1, 15.1 and 16.0; 2,560 x 2,048 at 150
+// 10.8 and 8.3; with more than 256 blocks (2B at 150 tokens 12.2 and 15.0, 9B at 65 17.7 and 23.5) the larger ones stay.  (Stages of
+// sixteen k-tiles: 10.3 and 10.8 us at 80 and 117 tokens of 2B where stages of eight take 9.9 and 10.2.)  The same sums in the same order.
+bool low_blocks(int M, int NT, int epi) { return epi == ALICE_EPI_ROPE && (long)ceil_div(M, 32) * ceil_div(NT, 4) <= 256; }
+
 }  // namespace
 
 TiledPlan alice_mfma_tiled_plan(int M, int N, int K, int epi, int y_dtype, int split, int x_frag) {
@@ -83,7 +91,7 @@ TiledPlan alice_mfma_tiled_plan(int M, int N, int K, int epi, int y_dtype, int s
         if (b <= 256 && (b > best_b || (b == best_b && sp < best_sp))) { best_b = b; best_wn = wn; best_sp = sp; }
       }
     }
-    if (best_b >= 190 || (M > 32 && epi != ALICE_EPI_GEGLU && best_b >= 96)) return TiledPlan{best_wn, 4, 8, best_sp};
+    if (best_b >= 190 || (M > 32 && epi != ALICE_EPI_GEGLU && best_b >= 96)) return TiledPlan{best_wn, best_wn == 1 && low_blocks(M, NT, epi) ? 2 : 4, 8, best_sp};
     return none;
   }
   const int sp0 = split > 0 ? split : (may_split ? tiled_split_wide(M, N, K) : 1);
@@ -95,6 +103,7 @@ TiledPlan alice_mfma_tiled_plan(int M, int N, int K, int epi, int y_dtype, int s
   // Between 65 and 1,024 tokens (what the cost rule was fitted on) another tile is taken where the rule says it is
   // 8 % cheaper; the narrow tiles exist for activations in fragment order and for the layers' own products.
   if (!(x_frag && M <= 1024 && narrow_built(epi, y_dtype))) return wide;
+  if (low_blocks(M, NT, epi)) return TiledPlan{1, 2, 8, 1};
   TiledPlan best = wide;
   float best_cost = tiled_cost(M, N, K, epi, wide.wn, wide.tm, wide.kc, wide.split) * 0.92f;
   static const int slices[] = {1, 2, 3, 4, 6, 8};
