@@ -1,6 +1,7 @@
 // Matrix product y[M, N] = x[M, K] . W[N, K]^T for every combination of 32-bit and bfloat16
 // operands, with 32-bit products and 32-bit accumulation: the kernels of the true 32-bit path, and
-// the fallback of the bfloat16 path for matrices that stay in 32-bit.
+// the fallback of the bfloat16 path for matrices that stay in 32-bit.  (Of more than 16 tokens most products of 32-bit
+// operands go to linear_thirds.hip, see in_thirds().)
 //
 // Weight layout and orientation as in the reference: row-major [out, in], y[r] = sum_c W[r,c] x[c]
 // (gguf.rs:4063-4074, f32_matvec).  Epilogues: none; GeGLU gelu_tanh(gate) * up with W = [gate; up]
@@ -32,8 +33,9 @@ __device__ __forceinline__ f32x4 load_row4(const T* __restrict__ row, int k, int
   return f32x4{load_f32(row, min(k, end - 1)), load_f32(row, min(k + 1, end - 1)), load_f32(row, min(k + 2, end - 1)), load_f32(row, min(k + 3, end - 1))};
 }
 
-// More than 16 tokens: the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: 32-bit products and sums, the rate of the
-// vector unit's FMA at a quarter of its register reads).  A block of 2 x 2 waves takes 32 TM tokens by 32 TN rows of W, a
+// More than 16 tokens of what linear_thirds.hip does not take (an operand in bfloat16, unaligned rows, or no time to gain there):
+// the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: 32-bit products and sums, the rate of the vector unit's FMA at a quarter
+// of its register reads).  A block of 2 x 2 waves takes 32 TM tokens by 32 TN rows of W, a
 // wave 16 TM by 16 TN; both operands go through LDS 32 inner elements at a time in two buffers (one barrier a stage), the
 // stage after the next on its way from memory meanwhile.  Every LDS and memory instruction stands behind a product of the
 // same wave: with all of them ahead of a stage's products the waves of a SIMD fell into step and left the matrix unit idle

@@ -20,8 +20,8 @@ class Precision:
 
     bfloat16: matrix operands, activations between kernels and the cache are bfloat16; sums,
     softmax, norms, rotation and the residual stream are 32-bit.
-    float32: everything is 32-bit, with full-precision tanh/exp/sqrt; of the matrix instructions only the one with
-    32-bit operands.
+    float32: everything is 32-bit, with full-precision tanh/exp/sqrt; products of up to 16 tokens on 32-bit arithmetic,
+    those of more also on the bfloat16 matrix instruction with every operand in three parts, whose error is smaller.
 
     keep_stored: on the bfloat16 path a matrix that its file stores in 32-bit is rounded to bfloat16 once, at
     load, so that it runs on the matrix cores like any other (the reference converts its stored formats once at
