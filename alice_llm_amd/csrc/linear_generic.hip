@@ -238,7 +238,7 @@ int planned_tokens(int M) { return M <= 32 ? 32 : ceil_div(M, 64) * 64; }
 static_assert(THIRDS_BK == BK, "both ways cut the inner dimension into the same slices");
 // Whether a product goes in thirds on the bfloat16 instruction: where that is estimated to be faster.  Both estimates are within a tenth of
 // what measures, and where they are that close either way will do.  (2B shape, the 32-bit instruction and thirds: 500 tokens gate and up 356
-// and 232 us, down 177 and 117, q, k, v 84 and 58, output 40 and 34; 128 tokens 105 and 75, 87 and 42, 32 and 38 (stays), 16 and 15; 32 tokens
+// and 244 us, down 177 and 121, q, k, v 84 and 61, output 40 and 34; 128 tokens 105 and 75, 87 and 42, 32 and 38 (stays), 16 and 15; 32 tokens
 // 48 and 46, 28 and 23, 31 and 30, 8 and 8.)
 bool in_thirds(const ThirdsPlan& t, const Plan& p) { return t.us < p.us; }
 

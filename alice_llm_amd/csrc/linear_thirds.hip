@@ -58,9 +58,9 @@ __device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3], u16x2
 // in LDS, on the way the outputs take to leave as 16-byte pieces of a token's row.  With GeGLU the first half of the block's rows are
 // gate rows, the second half the up rows of the same outputs.  split: slices of the inner dimension, slice z to Y + z M N.
 //
-// What bounds it: the matrix instruction at the clock it runs at under this load.  512 tokens by 18,432 x 2,304 with GeGLU:
-// 232 us (183 TFLOP/s of 32-bit products; 1.1 PFLOP/s of bfloat16 ones, what large library products reach here), 183 us with neither
-// loads nor LDS nor splitting; 356 on the 32-bit instruction.  Both operands through LDS, 128 x 128 to 256 x 144 a block: 247 to
+// What bounds it: the matrix instruction at the clock it runs at under this load.  500 tokens by 18,432 x 2,304 with GeGLU:
+// 244 us (174 TFLOP/s of 32-bit products; 1.04 PFLOP/s of bfloat16 ones, where large library products reach 1.07 to 1.14), 232 without
+// the largest size kept beside the splitting, 183 with neither loads nor LDS nor splitting; 356 on the 32-bit instruction.  Both operands through LDS, 128 x 128 to 256 x 144 a block: 247 to
 // 330 us; products, splitting and loads interleaved by hand with the next stage's tokens read ahead: the same 275 as without for
 // 64 x 128 a block; one group of four waves: 278.
 template <int TM, int TN>
