@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-@pytest.mark.parametrize("T,H", [(1, 64), (15, 2304), (17, 96), (64, 2048), (319, 160), (320, 256), (333, 2048), (700, 4128)])
+@pytest.mark.parametrize("T,H", [(1, 64), (15, 2304), (17, 96), (32, 2048), (65, 2048), (319, 160), (320, 256), (333, 2048), (700, 4128)])
 @pytest.mark.parametrize("slices,post", [(0, False), (1, False), (1, True), (3, True)])
 def test_the_stream_without_a_norm_in_fragment_order(T, H, slices, post):
     precision = Precision.of("bfloat16")
@@ -29,3 +29,11 @@ def test_the_stream_without_a_norm_in_fragment_order(T, H, slices, post):
     assert isinstance(outs[1], FragmentActs) and outs[1].shape == (T, H)
     assert torch.equal(acts_from_fragments(outs[1].data, T, H), outs[0].cpu())
     assert torch.equal(streams[0].x, streams[1].x) and streams[1]._branch is None
+
+
+@pytest.mark.parametrize("T", [33, 64])
+def test_rows_where_the_order_of_the_sums_would_change(T):
+    s = ResidualStream(rnd(T, 256, seed=1), Precision.of("bfloat16"))
+    s.push(rnd(T, 256, seed=2))
+    out = s.normed(None, fragments=True)
+    assert torch.equal(out, s.x.to(torch.bfloat16))
