@@ -21,9 +21,9 @@ namespace {
 template <int RT, int MT, int NW, int EPI, typename TO, bool FULL, bool XF, bool STREAM = false, int WINDOW = 0>
 __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wf,
                                                             void* __restrict__ y_or_positions, const int* __restrict__ seq_of_token,
-                                                            int M, int KT, int NT, int kt_per_slice, uint32_t turn, uint32_t last_turn,
+                                                            int M, int KT, int NT, int kt_per_slice, uint32_t turn, uint32_t rest_turn,
                                                             int N, int K, float epi, int y_frag, RopeArgs ra) {
-  // (the arguments up to last_turn come in registers: what the first loads need, with the rotation epilogue its lookups too)
+  // (the arguments up to rest_turn come in registers: what the first loads need, with the rotation epilogue its lookups too)
   extern __shared__ __align__(16) float red[];            // [NW - 1][RT*MT][64][4]
   // (the wave's number as a scalar: all that follows from it, the addresses of its tiles above all, is scalar arithmetic too)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -93,7 +93,9 @@ __global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(const bf16_t* __
   // Blocks start at different places of their k range and wrap around: all blocks read the same
   // activations, and in lockstep they would all ask the same L2 channel for the same line at once.
   const int J = (ke - kb + NW - 1) / NW;                    // k-tiles per wave (the last ones may be past the end)
-  const int rot = (int)(blockIdx.x - quotient(blockIdx.x, ke < KT ? turn : last_turn) * (unsigned)J);      // blockIdx.x % J
+  // blockIdx.x % J.  A slice is whole, or the one with the rest (the last one that has elements: slices behind it, which rounding
+  // up the others can leave, have none and read nothing).
+  const int rot = J > 0 ? (int)(blockIdx.x - quotient(blockIdx.x, kb + kt_per_slice <= KT ? turn : rest_turn) * (unsigned)J) : 0;
   auto tile_at = [&](int t) {                               // t-th tile of this wave's rotated sequence
     int j = t + rot;
     if (j >= J) j -= J;
@@ -251,7 +253,7 @@ int launch_skinny(const void* x, const void* w, void* y, int M, int N, int K, in
     }                                                                                                                          \
     kern<<<grid, THREADS, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, EPI == ALICE_EPI_ROPE ? (void*)ra.positions : y, ra.seq_of_token, \
                                     M, KT, NT, per, reciprocal_of(ceil_div(per, NWV)),                                         \
-                                    reciprocal_of(max(1, ceil_div(KT - per * (split - 1), NWV))), N, K, epi, y_frag, ra);      \
+                                    reciprocal_of(max(1, ceil_div(KT % per, NWV))), N, K, epi, y_frag, ra);      \
   } while (0)
 #define BY_INPUT(NWV, THREADS)                                                        \
   do {                                                                                \
