@@ -79,6 +79,9 @@ int alice_linear(const void* x, int x_dtype, const void* w, int w_dtype, int w_l
                  int full_precision, int x_layout, int y_layout, hipStream_t stream);
 // How many partial sums AUTO would like for this shape (1 = none).
 int alice_linear_split_hint(int M, int N, int K, int w_layout);
+// Whether products of M tokens by every fragment-layout matrix of K inner elements add in one order for activations in rows and in
+// fragment order.
+int alice_linear_one_order(int M, int K);
 // Which tile a float32 product of more than 16 tokens takes on the bfloat16 instruction (operands in three parts), -1: the 32-bit one.
 int alice_linear_thirds_tile(int M, int N, int K, int geglu, int split_k);
 

@@ -64,7 +64,15 @@ bool narrow_built(int epi, int y_dtype) {
 // sixteen k-tiles: 10.3 and 10.8 us at 80 and 117 tokens of 2B where stages of eight take 9.9 and 10.2.)  The same sums in the same order.
 bool low_blocks(int M, int NT, int epi) { return epi == ALICE_EPI_ROPE && (long)ceil_div(M, 32) * ceil_div(NT, 4) <= 256; }
 
+// Whether products of M <= 64 tokens by some matrix of K inner elements take these tiles when the activations come in fragment
+// order (see the plan): rows always take the streaming kernel, whose waves share the inner dimension.
+bool low_tiles(int M, int K) { return M > 32 || K >= 4096; }
+
 }  // namespace
+
+// Whether products of M tokens add in one order by every matrix of K inner elements, activations in rows or in fragment order.
+// (From 65 tokens on a wave of the tiled kernel goes through a slice from its first element to its last, whatever the tile.)
+extern "C" int alice_linear_one_order(int M, int K) { return M > 64 || !low_tiles(M, K); }
 
 TiledPlan alice_mfma_tiled_plan(int M, int N, int K, int epi, int y_dtype, int split, int x_frag) {
   const int KT = ceil_div(K, 32), NT = ceil_div(N * (epi == ALICE_EPI_GEGLU ? 2 : 1), 16);
@@ -79,8 +87,8 @@ TiledPlan alice_mfma_tiled_plan(int M, int N, int K, int epi, int y_dtype, int s
     // in slices (output and down projections: 2 to 17 % for the tiled kernel on eight shapes of 16 to 134 MB; a
     // matrix of 340 MB, which the streaming kernel reads with the streaming hint, is 4 to 10 % slower tiled).
     TiledPlan none{0, 4, 8, split > 0 ? split : 1};
-    if (!(x_frag && narrow_built(epi, y_dtype))) return none;
-    if (M <= 32 && !(may_split && K >= 4096 && (size_t)N * K < ((size_t)128 << 20))) return none;
+    if (!(x_frag && narrow_built(epi, y_dtype) && low_tiles(M, K))) return none;
+    if (M <= 32 && !(may_split && (size_t)N * K < ((size_t)128 << 20))) return none;
     static const int slices[] = {1, 2, 3, 4, 6, 8, 12, 16};
     int best_b = 0, best_wn = 0, best_sp = 0;
     for (int wn = 2; wn >= 1; --wn) {

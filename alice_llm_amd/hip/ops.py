@@ -48,6 +48,7 @@ def _declare(lib) -> None:
         "alice_add_branches": [P, I, P, P, P, P, I, P, P, P, I, I, I, I, P],
         "alice_linear": [P, I, P, I, I, P, I, I, I, I, I, F, I, I, I, I, I, P],
         "alice_linear_split_hint": [I, I, I, I],
+        "alice_linear_one_order": [I, I],
         "alice_linear_thirds_tile": [I, I, I, I, I],
         "alice_to_frag16": [P, P, I, I, P],
         "alice_frag16_supported": [I, I, I],
@@ -411,6 +412,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, *, n_out: int, k_i
 
 def linear_split_hint(M: int, N: int, K: int, layout: int) -> int:
     return library().alice_linear_split_hint(M, N, K, layout)
+
+
+def linear_one_order(M: int, K: int) -> bool:
+    """Whether M tokens' products of K inner elements add in one order for activations in rows and in fragment order."""
+    return bool(library().alice_linear_one_order(M, K))
 
 
 def linear_thirds_tile(M: int, N: int, K: int, geglu: bool = False, split_k: int = 1) -> int:

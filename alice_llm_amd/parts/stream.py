@@ -130,9 +130,10 @@ class ResidualStream:
             self._add_pointwise(norm, out, ops.LAYOUT_FRAG16 if frag else ops.LAYOUT_ROW)
             return out
         pre = _fused_pre(norm)
-        # Without a norm the stream itself, rounded, is what the consumer reads.  At 33 to 64 tokens it stays in rows: the products
-        # choose between two kernels by the order of the activations there, and these add up in different orders.
-        if fragments and (pre is not None or norm is None and not 32 < T <= 64) and out_dtype == torch.bfloat16 and FragmentActs.possible(self.precision, T, H):
+        # Without a norm the stream itself, rounded, is what the consumer reads.  It stays in rows where products choose between two
+        # kernels by the order of the activations, which add up in different orders (33 to 64 tokens; rows of 4,096 elements from one on).
+        if fragments and (pre is not None or norm is None and ops.linear_one_order(T, H)) and out_dtype == torch.bfloat16 \
+                and FragmentActs.possible(self.precision, T, H):
             post = self._post
             pf = post.fused() if post is not None and hasattr(post, "fused") else None
             if self._branch is not None and not ((post is None or pf is not None) and (pf is None or pre is None or pf[0].dtype == pre[0].dtype)):

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from alice_llm_amd.parts.base import FragmentActs, Precision
+from alice_llm_amd.parts.linear import Linear
 from alice_llm_amd.parts.norm import RMSNorm
 from alice_llm_amd.parts.stream import ResidualStream
 from test_gpu_kernels import acts_from_fragments, rnd
@@ -37,3 +38,21 @@ def test_rows_where_the_order_of_the_sums_would_change(T):
     s.push(rnd(T, 256, seed=2))
     out = s.normed(None, fragments=True)
     assert torch.equal(out, s.x.to(torch.bfloat16))
+
+
+# outputs and widths of a delta layer's projection (tiled from one token on if it were given fragment order), and streaming ones; GeGLU
+@pytest.mark.parametrize("T", [1, 8, 16, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("N,H", [(12576, 4096), (12224, 4096), (2304, 4128), (12576, 2048), (2560, 1024)])
+def test_the_product_behind_the_stream_without_a_norm(T, N, H):
+    """The same bits whether the consumer says that it reads fragment order or not."""
+    precision = Precision.of("bfloat16")
+    part = Linear(H, N, precision)
+    part.load(rnd(N, H, seed=5, scale=0.1, dtype=torch.bfloat16))
+    x, branch = rnd(T, H, seed=1), rnd(T, H, seed=2)
+    outs = []
+    for fragments in (False, True):
+        s = ResidualStream(x.clone(), precision)
+        s.push(branch)
+        acts = s.normed(None, fragments=fragments)
+        outs.append([part(acts, torch.float32, allow_partials=True), part(acts, torch.float32), part(acts, torch.bfloat16)])
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
