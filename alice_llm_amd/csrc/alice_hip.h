@@ -79,6 +79,8 @@ int alice_linear(const void* x, int x_dtype, const void* w, int w_dtype, int w_l
                  int full_precision, int x_layout, int y_layout, hipStream_t stream);
 // How many partial sums AUTO would like for this shape (1 = none).
 int alice_linear_split_hint(int M, int N, int K, int w_layout);
+// The same for row-major weights by what the operands are: their dtypes, and whether both start on 16 bytes (above: float32, aligned).
+int alice_linear_split_hint_for(int M, int N, int K, int w_layout, int x_dtype, int w_dtype, int aligned);
 // Whether products of M tokens by every fragment-layout matrix of K inner elements add in one order for activations in rows and in
 // fragment order.
 int alice_linear_one_order(int M, int K);

@@ -945,12 +945,19 @@ static int single_split(int N, int K) {
 
 // Into how many slices of the inner dimension a product without an epilogue is best cut (for 2 to 16 tokens one
 // number, whatever captured steps round theirs to).
-int alice_linear_split_hint_generic(int M, int N, int K) {
+// floats: both operands are float32.  Where one is bfloat16 or starts on no 16 bytes the product stays with the 32-bit instruction, and
+// with the slices of its own plan, except that the plan's cost is too low for blocks that are alone on a CU: up to 128 tokens, and where
+// it would take one slice, the thirds' number is the better one.  (Product and the norm that reads the slices, thirds' against own number,
+// float32 tokens by bfloat16 weights, 18 shapes of 2,048 x 2,048 to 3,584 x 14,336 at 17 to 2,000 tokens: 17 tokens by 3,584 x 14,336 62 and
+// 94 us, 128 by 4,096 x 2,304 40 and 70, 256 by 4,096 x 2,304 in 4 and 1 slices 68 and 93, on the whole 1.24 times, at worst 6 % slower;
+// the others 140 and 103 at 256 by 4,608 x 4,096, 224 and 210 at 500 by 2,304 x 9,216.  Bfloat16 tokens by float32 weights: 1.22 times.)
+int alice_linear_split_hint_generic(int M, int N, int K, bool floats, bool aligned) {
   if (M == 1) return few_by_length(K, 1) ? single_split(N, K) : 1;
   if (M <= 16) return rows_split(N, K);
   const Plan p = plan_mfma32(planned_tokens(M), N, K, false, 1, MAX_SPLIT);
+  if (!aligned || K % 4 != 0 || (!floats && planned_tokens(M) > 128 && p.split > 1)) return p.split;
   const ThirdsPlan t = alice_linear_thirds_plan(planned_tokens(M), N, K, false, 1, MAX_SPLIT);
-  return K % 4 == 0 && in_thirds(t, p) ? t.split : p.split;
+  return in_thirds(t, p) ? t.split : p.split;
 }
 
 // The tile of a product of more than 16 tokens that goes in thirds, -1 if it goes on the 32-bit instruction (float32 and aligned operands).

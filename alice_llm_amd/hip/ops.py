@@ -48,6 +48,7 @@ def _declare(lib) -> None:
         "alice_add_branches": [P, I, P, P, P, P, I, P, P, P, I, I, I, I, P],
         "alice_linear": [P, I, P, I, I, P, I, I, I, I, I, F, I, I, I, I, I, P],
         "alice_linear_split_hint": [I, I, I, I],
+        "alice_linear_split_hint_for": [I, I, I, I, I, I, I],
         "alice_linear_one_order": [I, I],
         "alice_linear_thirds_tile": [I, I, I, I, I],
         "alice_to_frag16": [P, P, I, I, P],
@@ -410,8 +411,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, *, n_out: int, k_i
           int(full_precision), int(x_layout), int(y_layout), _stream())
 
 
-def linear_split_hint(M: int, N: int, K: int, layout: int) -> int:
-    return library().alice_linear_split_hint(M, N, K, layout)
+def linear_split_hint(M: int, N: int, K: int, layout: int, x: Optional[torch.Tensor] = None, w: Optional[torch.Tensor] = None) -> int:
+    """The slices of the inner dimension that a product would like.  x, w: its operands, whose dtypes and alignment choose the kernel of
+    row-major weights (float32 and aligned if not given)."""
+    if layout == LAYOUT_FRAG16 or x is None or w is None:
+        return library().alice_linear_split_hint(M, N, K, layout)
+    return library().alice_linear_split_hint_for(M, N, K, layout, dtype_code(x.dtype), dtype_code(w.dtype),
+                                                 int((x.data_ptr() | w.data_ptr()) % 16 == 0))
 
 
 def linear_one_order(M: int, K: int) -> bool:

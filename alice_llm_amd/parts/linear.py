@@ -87,7 +87,7 @@ class Linear:
             raise ValueError("this projection cannot read activations in fragment order")
         split = 1
         if allow_partials and self.epilogue == ops.EPI_NONE and out_dtype == torch.float32:
-            split = ops.linear_split_hint(M, self.n, self.k, self.layout)
+            split = ops.linear_split_hint(M, self.n, self.k, self.layout, x, self.weight)
         if out_fragments:
             if not self.can_write_fragments(M) or out_dtype != torch.bfloat16:
                 raise ValueError("this projection cannot write activations in fragment order here")
