@@ -72,6 +72,7 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   constexpr int STAGE = 3 * TM * 64;                          // in units of 16 bytes
   extern __shared__ __align__(16) u32x4 lds[];
   __shared__ int again;
+  __shared__ uint32_t xmask[KG][TM];                          // a token tile's tokens with a number above 2^20, a bit each
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) % NW, group = __builtin_amdgcn_readfirstlane(tid >> 6) / NW;
   auto plane = [&](int buf, int t, int tile) { return lds + (group * 2 + buf) * STAGE + (t * TM + tile) * 64; };
@@ -114,19 +115,16 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
     }
   };
   f32x4 acc[TN][TM];
-  auto clear = [&] {
 #pragma unroll
-    for (int i = 0; i < TN; ++i)
+  for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  };
-  clear();
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (tid == 0) again = 0;
   const float sign = group ? -1.f : 1.f;
-  u16x2 top = {0, 0};                                         // the largest sizes among the numbers that this lane splits
+  u16x2 xtop[XJ] = {}, wtop[TN] = {};                         // the largest sizes among the numbers of a row that this lane splits
   auto put = [&](int j, int buf) {
     u32x4 p[3];
-    thirds<true>(xr[j], p, top, sign);
+    thirds<true>(xr[j], p, xtop[j], sign);
 #pragma unroll
     for (int t = 0; t < 3; ++t) plane(buf, t, wave + NW * j)[lane] = p[t];
   };
@@ -153,7 +151,7 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
     for (int i = 0; i < TN; ++i) {
       u32x4 w[3];
       if (k0 + BK > k_end) clear_beyond(wr[i], k0);
-      thirds<false>(wr[i], w, top);
+      thirds<false>(wr[i], w, wtop[i]);
       if (!last) load(wsrc[i], wr[i], k0 + BK);
       // the smallest products first
       constexpr int WT[6] = {2, 0, 1, 1, 0, 0}, XT[6] = {0, 2, 1, 0, 1, 0};
@@ -177,26 +175,43 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   int k0 = k_begin;
   for (; k0 + BK < k_stop; k0 += BK) stage(k0, false);
   stage(k0, true);
-  __syncthreads();
 
   // A number that is not finite, or that rounds to no finite bfloat16, has a remainder that is none, and every sum that it enters
   // is then none either.  What of a number is below the smallest normal bfloat16, 2^-126, may be lost: with 16,384 others of at most
   // 2^20 that is 2^-92 of a sum, less than its own rounding from 2^-64 on.  Smaller sums, those that are no finite numbers, and all
-  // where a number is larger than 2^20, are taken again by 32-bit products; so is the whole tile around them.
-  bool odd = max(top.x, top.y) > 0x4980;                      // 2^20; infinities and no numbers are larger
+  // of a token or a row of W with a number larger than 2^20, are taken again by 32-bit products, and no others: what a token gets
+  // hangs on its own numbers and W's, not on the tokens beside it.
+  auto rows_of = [](uint64_t lanes) { return (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu; };     // lanes c + 16 g hold row c
+  auto above = [](const u16x2& top) { return max(top.x, top.y) > 0x4980; };          // 2^20; infinities and no numbers are larger
+  auto odd = [](float sum) {
+    const float v = fabsf(sum);
+    return (!(v >= 0x1p-64f) & (v != 0.f)) | !(v < INFINITY);
+  };
+  bool any = false;
 #pragma unroll
-  for (int i = 0; i < TN; ++i)
+  for (int j = 0; j < XJ; ++j) {
+    any = any | above(xtop[j]);
+    const uint32_t mask = rows_of(__ballot(above(xtop[j])));
+    if (mine(j) && lane == 0) xmask[group][wave + NW * j] = mask;
+  }
+  uint32_t wmask[TN];
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    any = any | above(wtop[i]);
+    wmask[i] = rows_of(__ballot(above(wtop[i])));
 #pragma unroll
     for (int j = 0; j < TM; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float v = fabsf(acc[i][j][e]);
-        odd = odd | (!(v >= 0x1p-64f) & (v != 0.f)) | !(v < INFINITY);
-      }
-  if (__ballot(odd) != 0 && lane == 0) again = 1;             // any of them: the same value
+      for (int e = 0; e < 4; ++e) any = any | odd(acc[i][j][e]);
+  }
+  if (__ballot(any) != 0 && lane == 0) again = 1;             // any of them: the same value
   __syncthreads();
   if (again) {
-    clear();
+    f32x4 sum[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int k0 = k_begin; k0 < k_stop; k0 += BK) {
       __syncthreads();
@@ -214,18 +229,23 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
       }
       __syncthreads();
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        f32x4 x[TM];
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < TM; ++j) x[j] = __builtin_bit_cast(f32x4, plane(0, h, j)[lane]);
+        for (int j = 0; j < TM; ++j) {
+          const f32x4 x = __builtin_bit_cast(f32x4, plane(0, h, j)[lane]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+          for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int i = 0; i < TN; ++i)
-#pragma unroll
-            for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr[i][h][e], x[j][e], acc[i][j], 0, 0, 0);
-      }
+            for (int i = 0; i < TN; ++i) sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr[i][h][e], x[e], sum[i][j], 0, 0, 0);
+        }
     }
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)                           // output 4 g + e of row tile i, token c of token tile j
+          if (((wmask[i] >> (g * 4 + e) | xmask[group][j] >> c) & 1) || odd(acc[i][j][e])) acc[i][j][e] = sum[i][j][e];
     __syncthreads();
   }
 

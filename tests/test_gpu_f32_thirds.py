@@ -126,3 +126,26 @@ def test_a_token_depends_on_no_other_and_captured_steps_add_as_eager_ones():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, all_rows)
+
+
+@pytest.mark.parametrize("M,N,K,split", [c for c in CASES if c[0] >= 17])
+@pytest.mark.parametrize("odd", [float("nan"), float("-inf"), 2.0 ** 21, 2.0 ** -80])
+def test_tokens_beside_one_that_has_no_three_parts(M, N, K, split, odd):
+    """A token with a number that sends its sums to the 32-bit instruction (a token of tiny numbers: tiny sums) changes no other token's
+    bits, a row of W with one no other output's."""
+    x, w = rnd(M, K, seed=M), rnd(N, K, seed=N, scale=0.1)
+    plain = product(x, w, split)
+    x2, w2, token, row = x.clone(), w.clone(), M // 2, N // 3
+    if odd < 1 and odd > 0:
+        x2[token] *= odd
+        w2[row] *= odd
+    else:
+        x2[token, K // 3] = w2[row, K - 1] = odd
+    got = product(x2, w, split)
+    keep = [t for t in range(M) if t != token]
+    assert torch.equal(got[..., keep, :], plain[..., keep, :]) and not torch.equal(got[..., token, :], plain[..., token, :])
+    # and what the token gets does not hang on who its neighbours are
+    assert torch.equal(product(x2.flip(0).contiguous(), w, split)[..., M - 1 - token, :].nan_to_num(7.0), got[..., token, :].nan_to_num(7.0))
+    got = product(x, w2, split)
+    keep = [n for n in range(N) if n != row]
+    assert torch.equal(got[..., keep], plain[..., keep]) and not torch.equal(got[..., row], plain[..., row])
