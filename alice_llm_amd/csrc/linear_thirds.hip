@@ -17,7 +17,6 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int BK = THIRDS_BK;                                 // inner elements a stage: one product's
@@ -27,18 +26,18 @@ __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x
 }
 
 // Eight elements of a row, times `sign` (1 or -1, with SIGNED), as three times eight bfloat16 numbers.
-// top: the largest sizes met so far, as bfloat16 bits.
+// top: the largest size met so far (of numbers: what is none leaves it, and every sum that it enters tells).
 template <bool SIGNED>
-__device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3], u16x2& top, float sign = 1.f) {
+__device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3], float& top, float sign = 1.f) {
   const uint32_t flip = (__float_as_uint(sign) >> 31) * 0x80008000u;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float x = v[i >> 1][(i & 1) * 2], y = v[i >> 1][(i & 1) * 2 + 1];
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(top) : "v"(x), "v"(y));      // (fmaxf quiets every operand first: three times the instructions)
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
       const uint32_t h = SIGNED && t == 0 ? pack_bf16x2(x, y) ^ flip : pack_bf16x2(x, y);
       p[t][i] = h;
-      if (t == 0) top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, h & 0x7fff7fffu));
       const float hx = __uint_as_float(h << 16), hy = __uint_as_float(h & 0xffff0000u);
       x = SIGNED && t == 0 ? fmaf(x, sign, -hx) : x - hx;
       y = SIGNED && t == 0 ? fmaf(y, sign, -hy) : y - hy;
@@ -72,7 +71,7 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   constexpr int STAGE = 3 * TM * 64;                          // in units of 16 bytes
   extern __shared__ __align__(16) u32x4 lds[];
   __shared__ int again;
-  __shared__ uint32_t xmask[KG][TM];                          // a token tile's tokens with a number above 2^20, a bit each
+  __shared__ uint32_t xmask[KG][TM];                          // a token tile's tokens that marks() marks, a bit each
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) % NW, group = __builtin_amdgcn_readfirstlane(tid >> 6) / NW;
   auto plane = [&](int buf, int t, int tile) { return lds + (group * 2 + buf) * STAGE + (t * TM + tile) * 64; };
@@ -121,7 +120,7 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
     for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (tid == 0) again = 0;
   const float sign = group ? -1.f : 1.f;
-  u16x2 xtop[XJ] = {}, wtop[TN] = {};                         // the largest sizes among the numbers of a row that this lane splits
+  float xtop[XJ] = {}, wtop[TN] = {};                         // the largest sizes among the numbers of a row that this lane splits
   auto put = [&](int j, int buf) {
     u32x4 p[3];
     thirds<true>(xr[j], p, xtop[j], sign);
@@ -180,9 +179,15 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   // is then none either.  What of a number is below the smallest normal bfloat16, 2^-126, may be lost: with 16,384 others of at most
   // 2^20 that is 2^-92 of a sum, less than its own rounding from 2^-64 on.  Smaller sums, those that are no finite numbers, and all
   // of a token or a row of W with a number larger than 2^20, are taken again by 32-bit products, and no others: what a token gets
-  // hangs on its own numbers and W's, not on the tokens beside it.
-  auto rows_of = [](uint64_t lanes) { return (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu; };     // lanes c + 16 g hold row c
-  auto above = [](const u16x2& top) { return max(top.x, top.y) > 0x4980; };          // 2^20; infinities and no numbers are larger
+  // hangs on its own numbers and W's, not on the tokens beside it.  Below 2^-134 all of a number is lost, and a sum of exactly zero
+  // tells nothing (they come by chance too, one of some millions): tokens and rows of which all numbers are below 2^-102, but not all
+  // zero, are taken again as well.  What stays is a zero instead of a sum below 2^-100, where a token's larger numbers meet nothing but
+  // zeros of the row and what is left of it is all below 2^-134.
+  // Marks of 16 rows, a bit each; lanes c + 16 g hold row c.
+  auto marks = [](float top) {
+    auto rows = [](uint64_t lanes) { return (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu; };
+    return rows(__ballot(top > 0x1p20f)) | (rows(__ballot(top != 0.f)) & ~rows(__ballot(top >= 0x1p-102f)));
+  };
   auto odd = [](float sum) {
     const float v = fabsf(sum);
     return (!(v >= 0x1p-64f) & (v != 0.f)) | !(v < INFINITY);
@@ -190,15 +195,15 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   bool any = false;
 #pragma unroll
   for (int j = 0; j < XJ; ++j) {
-    any = any | above(xtop[j]);
-    const uint32_t mask = rows_of(__ballot(above(xtop[j])));
+    const uint32_t mask = marks(xtop[j]);
+    any = any | (mask != 0);
     if (mine(j) && lane == 0) xmask[group][wave + NW * j] = mask;
   }
   uint32_t wmask[TN];
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
-    any = any | above(wtop[i]);
-    wmask[i] = rows_of(__ballot(above(wtop[i])));
+    wmask[i] = marks(wtop[i]);
+    any = any | (wmask[i] != 0);
 #pragma unroll
     for (int j = 0; j < TM; ++j)
 #pragma unroll

@@ -149,3 +149,29 @@ def test_tokens_beside_one_that_has_no_three_parts(M, N, K, split, odd):
     got = product(x, w2, split)
     keep = [n for n in range(N) if n != row]
     assert torch.equal(got[..., keep], plain[..., keep]) and not torch.equal(got[..., row], plain[..., row])
+
+
+@pytest.mark.parametrize("M,N,K,split", [(500, 4096, 2304, 1), (500, 2304, 9216, 3), (17, 2304, 2048, 7), (128, 16384, 2304, 1)])
+def test_sums_of_zero(M, N, K, split):
+    """Factors of which no part is left give zeros that are none; tokens and rows of zeros, and pairs that cancel, give zeros."""
+    assert ops.linear_thirds_tile(M, N, K, False, split) >= 0
+    x, w = rnd(M, K, seed=M, scale=2.0 ** 17).clamp(-2.0 ** 20, 2.0 ** 20), rnd(N, K, seed=N)
+    few = torch.zeros_like(x)
+    few[3, :] = torch.ldexp(rnd(K, seed=3), torch.tensor(-138, device=DEV))      # subnormal, less than any bfloat16
+    few[5, ::16] = x[5, ::16]
+    few[9, 1] = x[9, 1]
+    few[11, 0], few[11, 1] = 3.0 * 2.0 ** -116 * (1 + 2.0 ** -22), -3.0 * 2.0 ** -116      # what is left of the sum is a lost part
+    w[:, 1] = w[:, 0]
+    w[4], w[7] = 0.0, torch.ldexp(rnd(K, seed=7), torch.tensor(-139, device=DEV))
+    big = w * 2.0 ** 17
+    for a, b in ((few, big.clamp(-2.0 ** 20, 2.0 ** 20)), (x, w)):
+        got, ref = product(a, b, split), a.double() @ b.double().T
+        got = got.double().sum(0) if split > 1 else got.double()
+        assert ((got - ref).abs() <= 16 * bound(a, b) + 2.0 ** -140).all()
+        assert torch.equal(got == 0, ref.abs() < 2.0 ** -150)      # (a token and a row of such numbers: less than any float32)
+    # the token of what is left is the only difference
+    other = few.clone()
+    other[3] = other[11] = 0.0
+    b = big.clamp(-2.0 ** 20, 2.0 ** 20)
+    keep = [t for t in range(M) if t not in (3, 11)]
+    assert torch.equal(product(other, b, split)[..., keep, :], product(few, b, split)[..., keep, :])
