@@ -1,14 +1,17 @@
 // 32-bit products of more than 16 tokens on the bfloat16 matrix instruction: y[M, N] = x[M, K] . W[N, K]^T, all float32
-// (gguf.rs:4063-4074; GeGLU llama3.rs:14519-14534, softcap llama3.rs:14606-14611), with 32-bit sums and no less precision than
-// 32-bit products have.
+// (gguf.rs:4063-4074; GeGLU llama3.rs:14519-14534, softcap llama3.rs:14606-14611), with 32-bit sums and the precision of 32-bit
+// products.
 //
 // A float32 is the sum of three bfloat16 numbers: each takes the next eight bits of the mantissa, rounded to nearest, and what it
 // leaves is exact.  Of the nine products of two such sums the six largest are taken, every one of them exact in 32 bits; the three
-// left out are at most 2^-23 of the whole product and of either sign.  The six go into one float32 accumulator, the smallest first.
-// An accumulator is rounded six times for 32 inner elements instead of 32 times, and that outweighs what is left out: against
-// 64 bits the error is 0.3 to 0.6 of the 32-bit instruction's (normal numbers, K 64 / 2,304 / 9,216 / 16,384: 0.46, 5.1, 6.0 (three
-// slices) and 13.8e-7 of the result's norm; 1.44, 8.6, 9.9 and 22.9), that of the 2B shape's logits after a prompt of 500 tokens 1.6e-6
-// instead of 2.8e-6.
+// left out are at most 2^-24 of the whole product and of either sign.  The largest of the six goes into one float32 accumulator, the
+// other five, 2^-6.5 of it at most, into a second one, and the two are added at the end: the largest product has 16 bits, which an
+// accumulator of 24 takes without rounding until it is some hundred times the product, and what the second accumulator rounds is
+// that much less.  Against 64 bits the error is 0.23 to 0.33 of the 32-bit instruction's (normal numbers, K 64 / 2,304 / 9,216 in three
+// slices / 16,384: 0.48, 2.0, 2.3 and 5.7e-7 of the result's norm; 1.44, 8.6, 9.9 and 22.9), that of the 2B shape's logits after a
+// prompt of 500 tokens 0.76e-6 instead of 2.8e-6.  With all six in one accumulator (in the same time) it was 0.46, 5.1, 6.0, 13.8 and
+// 1.6e-6, and tokens of few elements, up to some 500 of 2,304, were up to 1.5 times as far off as on the 32-bit instruction, which
+// rounds nothing where a product is zero: they have 1.03 of its error now with one to three elements, 0.54 with 16, 0.28 with 256.
 #include "common.h"
 #include "alice_hip.h"
 #include "linear_thirds.h"
@@ -51,17 +54,18 @@ __device__ __forceinline__ void thirds(const f32x4 (&v)[2], u32x4 (&p)[3], float
 // the order in which the instruction takes them (every access one contiguous kilobyte of a wave), in two buffers with one barrier a
 // stage.  A lane's eight elements of a stage are 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3 on both sides (whole 64-byte pieces of
 // a row a load).  The second group multiplies by the tokens' negative: the instruction adds by cutting off (towards minus infinity),
-// six times a stage, and that would move every output of every token the same way (a third of the error of a product of 9,216
+// and that would move every output of every token the same way (with one accumulator a third of the error of a product of 9,216
 // elements was one vector common to all tokens, which no average over keys or layers removes: logits after prompts of 1,852 tokens
-// were off by 2.6e-6 of their norm instead of 1.9e-6); the two groups' shifts cancel.  W is the first operand, so that a lane ends up with four neighbouring outputs of a token.  The groups' sums meet
-// in LDS, on the way the outputs take to leave as 16-byte pieces of a token's row.  With GeGLU the first half of the block's rows are
+// were off by 2.6e-6 of their norm instead of 1.9e-6); the two groups' shifts cancel.  W is the first operand, so that a lane ends
+// up with four neighbouring outputs of a token.  The groups' sums meet in LDS, on the way the outputs take to leave as 16-byte
+// pieces of a token's row.  With GeGLU the first half of the block's rows are
 // gate rows, the second half the up rows of the same outputs.  split: slices of the inner dimension, slice z to Y + z M N.
 //
 // What bounds it: the matrix instruction at the clock it runs at under this load.  500 tokens by 18,432 x 2,304 with GeGLU:
-// 244 us (174 TFLOP/s of 32-bit products; 1.04 PFLOP/s of bfloat16 ones, where large library products reach 1.07 to 1.14), 232 without
-// the largest size kept beside the splitting, 183 with neither loads nor LDS nor splitting; 356 on the 32-bit instruction.  Both operands through LDS, 128 x 128 to 256 x 144 a block: 247 to
-// 330 us; products, splitting and loads interleaved by hand with the next stage's tokens read ahead: the same 275 as without for
-// 64 x 128 a block; one group of four waves: 278.
+// 246 us (173 TFLOP/s of 32-bit products; 1.03 PFLOP/s of bfloat16 ones, where large library products reach 1.07 to 1.14), 183 with
+// neither loads nor LDS nor splitting (with one accumulator); 356 on the 32-bit instruction.  Both operands through LDS, 128 x 128 to
+// 256 x 144 a block: 247 to 330 us; products, splitting and loads interleaved by hand with the next stage's tokens read ahead: the
+// same 275 as without for 64 x 128 a block; one group of four waves: 278.
 template <int TM, int TN>
 __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ Y,
                                                                int M, int N, int K, int kslice, int split, int mt, int nt, int epi, float param,
@@ -113,11 +117,11 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
       for (int e = 0; e < 4; ++e) v[h][e] = in ? v[h][e] : 0.f;
     }
   };
-  f32x4 acc[TN][TM];
+  f32x4 acc[TN][TM], rest[TN][TM];                            // the sums of the largest of the six products, and of the other five
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < TM; ++j) acc[i][j] = rest[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (tid == 0) again = 0;
   const float sign = group ? -1.f : 1.f;
   float xtop[XJ] = {}, wtop[TN] = {};                         // the largest sizes among the numbers of a row that this lane splits
@@ -141,24 +145,49 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   lds_barrier();
   int cur = 0;
   auto stage = [&](int k0, bool last) {
-    u32x4 x[TM][3];
-#pragma unroll
-    for (int t = 0; t < 3; ++t)
-#pragma unroll
-      for (int j = 0; j < TM; ++j) x[j][t] = plane(cur, t, j)[lane];
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
-      u32x4 w[3];
+    u32x4 w[TN][3];
+    auto split = [&](int i) {
       if (k0 + BK > k_end) clear_beyond(wr[i], k0);
-      thirds<false>(wr[i], w, wtop[i]);
+      thirds<false>(wr[i], w[i], wtop[i]);
       if (!last) load(wsrc[i], wr[i], k0 + BK);
-      // the smallest products first
-      constexpr int WT[6] = {2, 0, 1, 1, 0, 0}, XT[6] = {0, 2, 1, 0, 1, 0};
+    };
+    auto products = [&](int i, int wt, const u32x4 (&x)[TM], f32x4 (&sum)[TM]) {
 #pragma unroll
-      for (int p = 0; p < 6; ++p)
+      for (int j = 0; j < TM; ++j) sum[j] = mfma(w[i][wt], x[j], sum[j]);
+    };
+    u32x4 x[3][TM];
+    auto fetch = [&](int t) {
 #pragma unroll
-        for (int j = 0; j < TM; ++j) acc[i][j] = mfma(w[WT[p]], x[j][XT[p]], acc[i][j]);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < TM; ++j) x[t][j] = plane(cur, t, j)[lane];
+    };
+    // Blocks of 128 tokens take a part of the tokens at a time, or two accumulators do not fit beside them (245 registers, no time lost
+    // at two row tiles a wave); the others all three, a row tile after the other (64 x 192 by parts: 246 to 262 us).
+    if constexpr (TM < 8) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t) fetch(t);
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        split(i);
+        products(i, 2, x[0], rest[i]);
+        products(i, 0, x[2], rest[i]);
+        products(i, 1, x[1], rest[i]);
+        products(i, 1, x[0], rest[i]);
+        products(i, 0, x[1], rest[i]);
+        products(i, 0, x[0], acc[i]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int t = 2; t >= 0; --t) {
+        fetch(t);
+#pragma unroll
+        for (int i = 0; i < TN; ++i) {
+          if (t == 2) split(i);
+#pragma unroll
+          for (int wt = 2 - t; wt >= 0; --wt) products(i, wt, x[t], t + wt == 0 ? acc[i] : rest[i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     if (!last) {
 #pragma unroll
@@ -174,6 +203,10 @@ __global__ __launch_bounds__(512, 2) void linear_thirds_kernel(const float* __re
   int k0 = k_begin;
   for (; k0 + BK < k_stop; k0 += BK) stage(k0, false);
   stage(k0, true);
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] += rest[i][j];
 
   // A number that is not finite, or that rounds to no finite bfloat16, has a remainder that is none, and every sum that it enters
   // is then none either.  What of a number is below the smallest normal bfloat16, 2^-126, may be lost: with 16,384 others of at most
@@ -328,8 +361,10 @@ constexpr Tile TILES[] = {{128, 128, 2.5f}, {64, 192, 2.1f}, {64, 128, 1.5f}, {6
 }  // namespace
 
 // The tile, and between min_split and max_split slices the number of them, by estimated microseconds: a CU's blocks one after the
-// other; slices cost writing and reading their sums.  (Planned and measured: 512 tokens by 18,432 x 2,304 with GeGLU in 64 x 192,
-// three blocks a CU, 233 and 232; 4,096 x 2,304 in 64 x 128 60 and 58; 2,304 x 9,216 in three slices 123 and 126.)
+// other; slices cost writing and reading their sums.  (Planned and measured, by weights that no cache holds: 512 tokens by 18,432 x
+// 2,304 with GeGLU in 64 x 192, three blocks a CU, 233 and 246; 4,096 x 2,304 in two slices of 128 x 128 58 and 54; 2,304 x 9,216 in seven 127
+// and 123, 2,304 x 2,048 in three 39 and 34; 128 tokens 80 and 78, 22 and 21, 40 and 41 in 64 x 192 and 64 x 128; 33 tokens by 2,304 x 9,216
+// in 64 x 64 28 and 27; 17 by 28,672 x 2,304 with GeGLU in 32 x 128 53 and 54.)
 ThirdsPlan alice_linear_thirds_plan(int M, int N, int K, bool geglu, int min_split, int max_split) {
   ThirdsPlan best{-1, 1, 1e30f};
   for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {

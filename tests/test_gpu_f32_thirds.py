@@ -48,7 +48,11 @@ def test_every_tile_is_among_the_cases():
     assert {ops.linear_thirds_tile(M, N, K, False, s) for M, N, K, s in CASES} == {0, 1, 2, 3, 4, 5}
 
 
-@pytest.mark.parametrize("M,N,K", [(500, 9216, 2304), (497, 9212, 2308), (500, 4610, 2304), (128, 9218, 2304), (64, 9218, 2304), (2048, 1025, 2304)])
+GATED = [(500, 9216, 2304), (497, 9212, 2308), (500, 4610, 2304), (128, 9218, 2304), (64, 9218, 2304), (2048, 1025, 2304),
+         (300, 5000, 2308), (65, 2305, 2308), (19, 14336, 2304)]
+
+
+@pytest.mark.parametrize("M,N,K", GATED)
 def test_gated_products_in_thirds(M, N, K):
     assert ops.linear_thirds_tile(M, N, K, True) >= 0
     x, w = rnd(M, K, seed=M), rnd(2 * N, K, seed=N, scale=0.02)
@@ -57,6 +61,81 @@ def test_gated_products_in_thirds(M, N, K):
     g, u = ref[:, :N], ref[:, N:]
     # the gate's slope is at most 1.13; 1e-6 for the 32-bit function itself
     assert ((got - F.gelu(g, approximate="tanh") * u).abs() <= 1.13 * off[:, :N] * u.abs() + off[:, N:] * g.abs() + 1e-6 * (1 + g.abs() * u.abs())).all()
+
+
+def single(M, K, seed):
+    """Tokens of one element each, the others zeros, in places all over the inner dimension."""
+    gen = torch.Generator().manual_seed(seed)
+    x = torch.zeros(M, K)
+    x[torch.arange(M), (torch.arange(M) * K // M + torch.randint(0, max(1, K // M), (M,), generator=gen)).clamp(max=K - 1)] = torch.randn(M, generator=gen)
+    x[0] = x[M - 1] = 0.0
+    x[0, 0], x[M - 1, K - 1] = 1.7, -1.3
+    return x.to(DEV)
+
+
+# One product alone: three parts' products left out, 2^-24 of it at most, and the sum of the largest one and the others rounded to nearest,
+# 2^-24; the others are 2^-6.5 of it at most and are cut off five times, at 2^-23 of themselves.  Without x0 w2 or x2 w0 it would be off by
+# up to 2^-17, without x1 w1 by up to 2^-16.
+ALONE = 2.0 ** -23 * 1.06
+
+
+@pytest.mark.parametrize("M,N,K,split", CASES)
+def test_single_products(M, N, K, split):
+    """All six products are there, at every tile and wherever in the inner dimension."""
+    assert ops.linear_thirds_tile(M, N, K, False, split) >= 0
+    x, w = single(M, K, M), rnd(N, K, seed=N)
+    got, ref = product(x, w, split), x.double() @ w.double().T
+    got = got.double().sum(0) if split > 1 else got.double()
+    assert ((got - ref).abs() <= ALONE * ref.abs()).all()
+
+
+@pytest.mark.parametrize("M,N,K", GATED)
+def test_single_gated_products(M, N, K):
+    assert ops.linear_thirds_tile(M, N, K, True) >= 0
+    x, w = single(M, K, M), rnd(2 * N, K, seed=N)
+    got, ref = product(x, w, epi=ops.EPI_GEGLU).double(), x.double() @ w.double().T
+    g, u = ref[:, :N], ref[:, N:]
+    assert ((got - F.gelu(g, approximate="tanh") * u).abs() <= 2.13 * ALONE * (g * u).abs() + 1e-6 * (1 + (g * u).abs())).all()
+
+
+def on_the_32_bit_instruction(x, w, split=1, epi=ops.EPI_NONE):
+    """The same product over rows of one more element that is zero: rows that are no multiple of four elements take that instruction."""
+    return product(*(F.pad(a, (0, 1)).contiguous() for a in (x, w)), split, epi)
+
+
+@pytest.mark.parametrize("M,N,K,split", CASES)
+@pytest.mark.parametrize("spread", [0.0, 3.0])
+def test_every_tile_is_no_less_precise_than_the_32_bit_instruction(M, N, K, split, spread):
+    x, w = (rnd(n, K, seed=i) * torch.exp(spread * rnd(n, K, seed=i + 2)) for i, n in enumerate((M, N)))
+    ref = x.double() @ w.double().T
+    err = [float((y.double().sum(0) if split > 1 else y.double()).sub(ref).norm() / ref.norm())
+           for y in (product(x, w, split), on_the_32_bit_instruction(x, w, split))]
+    assert err[0] <= err[1], err
+
+
+@pytest.mark.parametrize("M,N,K,split", [(500, 4096, 2304, 1), (500, 9217, 2304, 1), (500, 2304, 9216, 3), (65, 1000, 16384, 8)])
+@pytest.mark.parametrize("elements", [1, 2, 4, 16, 64, 256])
+def test_tokens_of_few_elements(M, N, K, split, elements):
+    """Sums of few products, which leave nothing to average, against the 32-bit instruction, which rounds once a product.  A product of two
+    normal numbers is rounded by 2.5e-8 of it in the mean, the products left out are 2^-25 sqrt(2) / 3 of it for mantissas of 1, 0.6e-8
+    in the mean: 3 % more where the sums themselves round next to nothing (a slice has one to three of them), less from then on."""
+    assert ops.linear_thirds_tile(M, N, K, False, split) >= 0
+    gen = torch.Generator().manual_seed(elements)
+    at = torch.rand(M, K, generator=gen).argsort(1)[:, :elements]
+    x, w = torch.zeros(M, K).scatter_(1, at, torch.randn(M, elements, generator=gen)).to(DEV), rnd(N, K, seed=N)
+    ref = x.double() @ w.double().T
+    err = [float((y.double().sum(0) if split > 1 else y.double()).sub(ref).norm() / ref.norm())
+           for y in (product(x, w, split), on_the_32_bit_instruction(x, w, split))]
+    assert err[0] <= (1.05 if elements <= 3 * split else 1.0) * err[1], err
+
+
+@pytest.mark.parametrize("M,N,K", GATED)
+def test_gated_products_are_no_less_precise_than_the_32_bit_instruction(M, N, K):
+    x, w = rnd(M, K, seed=M), rnd(2 * N, K, seed=N, scale=0.1)
+    g, u = (x.double() @ w.double().T).chunk(2, 1)
+    ref = F.gelu(g, approximate="tanh") * u
+    err = [float((y.double() - ref).norm() / ref.norm()) for y in (product(x, w, epi=ops.EPI_GEGLU), on_the_32_bit_instruction(x, w, epi=ops.EPI_GEGLU))]
+    assert err[0] <= err[1], err
 
 
 @pytest.mark.parametrize("M,N,K,split", [(500, 4096, 2304, 1), (500, 2304, 9216, 3), (500, 20000, 164, 1), (128, 2304, 16384, 8)])
