@@ -85,6 +85,7 @@ int alice_linear_split_hint_for(int M, int N, int K, int w_layout, int x_dtype, 
 // fragment order.
 int alice_linear_one_order(int M, int K);
 // Which tile a float32 product of more than 16 tokens takes on the bfloat16 instruction (operands in three parts), -1: the 32-bit one.
+// (No caller needs it to take a product: tests ask, so that their sizes reach every tile.)
 int alice_linear_thirds_tile(int M, int N, int K, int geglu, int split_k);
 
 // Rearranges a row-major bfloat16 [N, K] matrix into the fragment layout ([Np/16][Kp/32][64][8],
