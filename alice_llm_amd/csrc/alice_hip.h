@@ -33,6 +33,9 @@
 #define ALICE_LINEAR_MFMA 3
 #define ALICE_LINEAR_TILED_W16 4   // the tiled kernel with a wave tile of 16 output features (activations in fragment order)
 #define ALICE_LINEAR_TILED_W32 5   // the same with 32
+#define ALICE_LINEAR_LARGE_256 6   // the kernel with tiles of 256 tokens by 256 output features (activations in fragment order)
+#define ALICE_LINEAR_LARGE_192 7   // the same by 192
+#define ALICE_LINEAR_LARGE_128 8   // the same by 128
 
 #ifdef __cplusplus
 extern "C" {
@@ -77,9 +80,10 @@ int alice_softcap(float* x, long n, float cap, int full_precision, hipStream_t s
 int alice_linear(const void* x, int x_dtype, const void* w, int w_dtype, int w_layout, void* y, int y_dtype,
                  int M, int N, int K, int epilogue, float epi_param, int split_k, int variant,
                  int full_precision, int x_layout, int y_layout, hipStream_t stream);
-// How many partial sums AUTO would like for this shape (1 = none).
+// How many partial sums AUTO would like for this shape (1 = none); of weights in fragment order with the activations in it too.
 int alice_linear_split_hint(int M, int N, int K, int w_layout);
-// The same for row-major weights by what the operands are: their dtypes, and whether both start on 16 bytes (above: float32, aligned).
+// The same by what the operands are: for row-major weights their dtypes, and whether both start on 16 bytes (above: float32, aligned);
+// for weights in fragment order with the activations in rows.
 int alice_linear_split_hint_for(int M, int N, int K, int w_layout, int x_dtype, int w_dtype, int aligned);
 // Whether products of M tokens by every fragment-layout matrix of K inner elements add in one order for activations in rows and in
 // fragment order.

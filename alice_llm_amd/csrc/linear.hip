@@ -2,18 +2,19 @@
 #include "common.h"
 #include "alice_hip.h"
 
-int alice_linear_split_hint_frag(int M, int N, int K);
+int alice_linear_split_hint_frag(int M, int N, int K, int x_frag);
 int alice_linear_split_hint_generic(int M, int N, int K, bool floats, bool aligned);
 int alice_linear_frag(const void* x, int x_dtype, const void* w, void* y, int y_dtype, int M, int N, int K,
                       int epi, float epi_param, int split_k, int variant, int x_layout, int y_layout,
                       hipStream_t stream);
 
 extern "C" int alice_linear_split_hint_for(int M, int N, int K, int w_layout, int x_dtype, int w_dtype, int aligned) {
-  if (w_layout == ALICE_LAYOUT_FRAG16) return alice_linear_split_hint_frag(M, N, K);
+  if (w_layout == ALICE_LAYOUT_FRAG16) return alice_linear_split_hint_frag(M, N, K, 0);
   return alice_linear_split_hint_generic(M, N, K, x_dtype == DT_F32 && w_dtype == DT_F32, aligned != 0);
 }
 
 extern "C" int alice_linear_split_hint(int M, int N, int K, int w_layout) {
+  if (w_layout == ALICE_LAYOUT_FRAG16) return alice_linear_split_hint_frag(M, N, K, 1);
   return alice_linear_split_hint_for(M, N, K, w_layout, DT_F32, DT_F32, 1);
 }
 

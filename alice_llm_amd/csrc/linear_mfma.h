@@ -11,14 +11,14 @@
 // activations the second (columns = tokens m).  Lane l then holds D[n = 4*(l/16) + i][m = l%16],
 // i = 0..3: four consecutive output features of one token, stored with one vector store.
 //
-// Two kernels share this: a weight-streaming kernel for up to 64 tokens (decode), whose four waves
-// split the inner dimension and add their parts in a fixed order, and a tiled kernel for many
-// tokens (prompts).  The math is the reference's y[r] = sum_c W[r,c] x[c] (gguf.rs:4063-4074) with the
+// Three kernels share this: a weight-streaming kernel for up to 64 tokens (decode), whose four waves
+// split the inner dimension and add their parts in a fixed order, a tiled kernel for many
+// tokens (prompts), and one with larger tiles for prompts of several hundred tokens and more.  The math is the reference's y[r] = sum_c W[r,c] x[c] (gguf.rs:4063-4074) with the
 // GeGLU (llama3.rs:14519-14534) and softcap (llama3.rs:14606-14611) epilogues.
 //
 // This header holds what the kernels' source files share: the operand types, the stores, and the rotation epilogue's
-// helpers.  linear_mfma_stream.hip has the streaming kernel, linear_mfma_tiled.hip the tiled one, linear_mfma.hip the
-// entry points; each is compiled on its own, which halves the time of a build.
+// helpers.  linear_mfma_stream.hip has the streaming kernel, linear_mfma_tiled.hip the tiled one, linear_mfma_large.hip the one
+// with larger tiles, linear_mfma.hip the entry points; each is compiled on its own, which halves the time of a build.
 #pragma once
 #include "common.h"
 #include "alice_hip.h"
@@ -227,6 +227,13 @@ struct TiledPlan { int wn, tm, kc, split; };
 TiledPlan alice_mfma_tiled_plan(int M, int N, int K, int epi, int y_dtype, int split, int x_frag);
 int alice_mfma_tiled_narrow(const void* x, const void* w, void* y, int y_dtype, int M, int N, int K, int epi, float epi_param,
                             const TiledPlan& p, int y_frag, hipStream_t s, const RopeArgs& ra);
+// The kernel of tiles of 256 tokens by 16 ft features, and its tile for a product that the tiled kernel would take as `tiled` says (ft 0:
+// that one stays; split 0: the slices are chosen too).  Activations in fragment order.
+struct LargePlan { int ft, split; };
+LargePlan alice_mfma_large_plan(int M, int N, int K, int epi, float epi_param, int y_dtype, int split, const TiledPlan& tiled);
+bool alice_mfma_large_takes(int M, int N, int K, int epi, float epi_param, int y_dtype, int split);
+int alice_mfma_large(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int split, int ft, int y_frag,
+                     hipStream_t s);
 // The streaming kernel's choice of row tiles a block and what the launcher's cost rule says of a choice.
 int alice_mfma_stream_row_tiles(int M, int N, int epi, int split, int K);
 int alice_mfma_stream_row_tiles_base(int M, int N, int epi, int split, int K);

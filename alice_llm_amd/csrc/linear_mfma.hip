@@ -55,9 +55,12 @@ static int skinny_split_with_six(int M, int N, int K, int split0) {
   return best;
 }
 
-int alice_linear_split_hint_frag(int M, int N, int K) {
-  // more than 64 tokens: the tiled kernel's own rule (activations in fragment order, as prompts bring them)
-  if (M > 64) return alice_mfma_tiled_plan(M, N, K, ALICE_EPI_NONE, DT_F32, 0, 1).split;
+int alice_linear_split_hint_frag(int M, int N, int K, int x_frag) {
+  // more than 64 tokens: the tiled kernel's own rule, or that of the kernel with larger tiles, which reads fragment order only
+  if (M > 64) {
+    const TiledPlan tiled = alice_mfma_tiled_plan(M, N, K, ALICE_EPI_NONE, DT_F32, 0, 1);
+    return x_frag ? alice_mfma_large_plan(M, N, K, ALICE_EPI_NONE, 0.f, DT_F32, 0, tiled).split : tiled.split;
+  }
   const int KT = (K + 31) / 32;
   const TiledPlan p = alice_mfma_tiled_plan(M, N, K, ALICE_EPI_NONE, DT_F32, 0, 1);
   if (p.wn != 0) return p.split;                             // the tiled kernel's narrow tiles are the better ones here
@@ -97,6 +100,15 @@ int alice_linear_frag(const void* x, int x_dtype, const void* w, void* y, int y_
               "linear: output in fragment order needs bfloat16, N %% 32 == 0, no softcap and no partial sums");
   const int x_frag = x_layout == ALICE_LAYOUT_FRAG16, y_frag = y_layout == ALICE_LAYOUT_FRAG16;
   if (skinny) return alice_mfma_stream(x, w, y, y_dtype, M, N, K, epi, epi_param, split_k, x_frag, y_frag, stream);
+  if (variant >= ALICE_LINEAR_LARGE_256) {
+    ALICE_CHECK(variant <= ALICE_LINEAR_LARGE_128 && x_frag && alice_mfma_large_takes(M, N, K, epi, epi_param, y_dtype, split_k),
+                "linear: no kernel with tiles of 256 tokens for M=%d N=%d K=%d in %d slices with this epilogue, output type and activation layout", M, N, K, split_k);
+    return alice_mfma_large(x, w, y, M, N, K, epi, epi_param, split_k, 16 - 4 * (variant - ALICE_LINEAR_LARGE_256), y_frag, stream);
+  }
+  if (variant == ALICE_LINEAR_AUTO && x_frag) {
+    const LargePlan large = alice_mfma_large_plan(M, N, K, epi, epi_param, y_dtype, split_k, alice_mfma_tiled_plan(M, N, K, epi, y_dtype, split_k, 1));
+    if (large.ft) return alice_mfma_large(x, w, y, M, N, K, epi, epi_param, split_k, large.ft, y_frag, stream);
+  }
   const int force_wn = variant == ALICE_LINEAR_TILED_W16 ? 1 : variant == ALICE_LINEAR_TILED_W32 ? 2 : 0;
   return alice_mfma_tiled(x, w, y, y_dtype, M, N, K, epi, epi_param, split_k, x_frag, y_frag, force_wn, stream);
 }

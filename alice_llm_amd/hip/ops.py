@@ -20,6 +20,7 @@ EPI_NONE, EPI_GEGLU, EPI_SOFTCAP = 0, 1, 2
 LAYOUT_ROW, LAYOUT_FRAG16 = 0, 1
 KV_ROW, KV_FRAGMENT = 0, 1
 LINEAR_AUTO, LINEAR_GENERIC, LINEAR_SKINNY, LINEAR_MFMA, LINEAR_TILED_W16, LINEAR_TILED_W32 = 0, 1, 2, 3, 4, 5
+LINEAR_LARGE_256, LINEAR_LARGE_192, LINEAR_LARGE_128 = 6, 7, 8
 ABI_VERSION = 16
 GATED_SILU = -1.0        # epi_param of EPI_GEGLU that picks silu(gate) * up
 UNARY_RELU2 = -1.0       # epi_param of EPI_SOFTCAP that picks the square of max(y, 0) instead of the capped form
@@ -413,8 +414,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, *, n_out: int, k_i
 
 def linear_split_hint(M: int, N: int, K: int, layout: int, x: Optional[torch.Tensor] = None, w: Optional[torch.Tensor] = None) -> int:
     """The slices of the inner dimension that a product would like.  x, w: its operands, whose dtypes and alignment choose the kernel of
-    row-major weights (float32 and aligned if not given)."""
-    if layout == LAYOUT_FRAG16 or x is None or w is None:
+    row-major weights (float32 and aligned if not given); activations in fragment order (anything but a tensor) have a kernel more."""
+    if x is None or w is None or (layout == LAYOUT_FRAG16 and not isinstance(x, torch.Tensor)):
         return library().alice_linear_split_hint(M, N, K, layout)
     return library().alice_linear_split_hint_for(M, N, K, layout, dtype_code(x.dtype), dtype_code(w.dtype),
                                                  int((x.data_ptr() | w.data_ptr()) % 16 == 0))
