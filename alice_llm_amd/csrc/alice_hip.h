@@ -132,7 +132,10 @@ int alice_attention_prefill(const void* q, const void* k_pool, const void* v_poo
                             const int* cu_seqlens, const int* context_lens, const int* block_table,
                             int bt_stride, int B, int max_new, int nH, int nKV, int d, int page_size,
                             float scale, float softcap, int window, int variant, int out_layout, const float* sink,
-                            hipStream_t stream);
+                            int max_context, int cut, float* parts, int* arrivals, int n_arrivals, hipStream_t stream);
+int alice_attention_prefill_cut(int B, int max_new, int max_context, int nH, int nKV, int d, int window);
+long alice_attention_prefill_counts(int B, int max_new, int max_context, int nH, int nKV, int d, int window, int cut);
+long alice_attention_prefill_workspace(long counts);
 // out[t, h, :] *= sigmoid(gate[t * gate_stride + h]) in place on a bfloat16 attention output in either layout.
 // alice_attention_generic with further parameters of the mask and the softmax (0 / null: off): gate: float32 rows,
 // gate_mode 1: a number a head, 2: a number an output element ([T, nH dv]); out_scale: a constant factor of the

@@ -15,6 +15,8 @@
 // S[key 4(l/16) + i][query l%16]; two such tiles, rounded to bfloat16, are exactly the second operand
 // of the value product in the key order that the value layout above stores, so the probabilities
 // never move between lanes.  Each lane keeps the running maximum and sum of its query column.
+#include <algorithm>
+#include <functional>
 #include <type_traits>
 #include "common.h"
 #include "alice_hip.h"
@@ -442,12 +444,38 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
 // the next block is on its way from memory into registers while this one is computed, and one barrier a
 // step suffices.  Against whole tiles per wave, memory traffic falls by the number of waves.
 // grid: (tiles of 16 NW / HB tokens, from the end backwards; sequences; kv heads x passes over the group).
-template <int DT, bool SOFTCAP, int NW, int KS>
+//
+// PARTS: where a block a CU or little more is all there is, the tiles that see the most keys set the time while half of the chip is idle.
+// The keys of each tile are then cut into 1 to MAX_PARTS even parts (prefill_parts() says how many) that blocks of their own walk, those
+// of the last tiles first, kv heads fastest so that an XCD meets few of them.  The waves of a tile's blocks that hold the same columns
+// leave their parts in memory, and the one that comes last adds all of them up in their order and writes the output: the bits
+// are the same whichever it is.  What they hand over goes past the L2, which another XCD does not see, by stores and loads of
+// agent scope, and nothing else needs to be seen: a wave's stores have arrived (s_waitcnt) before its count goes up, and only the wave
+// that finds all the others' counts reads.  Nobody waits for anybody.  arrivals: a count a (tile, wave), zero before the launch and after.
+__device__ __forceinline__ void store_far(float* p, float a, float b) {
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), __builtin_bit_cast(unsigned long long, float2{a, b}), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 load_far(const float* p) {
+  return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+// Floats of a wave's part: its output registers, and the maximum and sum of each lane's column.
+constexpr int part_floats(int D) { return 64 * (D / 4 + 2); }
+constexpr int MAX_PARTS = 8, MAX_ENTRIES = 512;
+template <bool PARTS>
+struct PartPlan {};
+template <>
+struct PartPlan<true> {
+  uint32_t entry[MAX_ENTRIES];                               // a block of a sequence's kv head: tile | part << 16 | the tile's parts << 24
+};
+
+template <int DT, bool SOFTCAP, int NW, int KS, bool PARTS>
 __global__ __launch_bounds__(64 * NW * KS, NW * KS == 4 ? 2 : 1) void attn_prefill_shared_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
     bf16_t* __restrict__ out, const int* __restrict__ cu_seqlens, const int* __restrict__ context_lens,
     const int* __restrict__ block_table, int bt_stride, int nH, int nKV, float scale, float cap, int window, int HB,
-    int out_layout, int xcd_map, const float* __restrict__ sink) {
+    int out_layout, int xcd_map, const float* __restrict__ sink, PartPlan<PARTS> plan, int n_seqs,
+    float* __restrict__ parts, int* __restrict__ arrivals) {
   // KS = 2: two sets of NW waves, the second takes the later half of the block's keys (its own buffers in LDS);
   // at the end the first set adds the second's part to its own, each scaled to the common maximum.  Halves the
   // longest block's run when there are too few blocks to fill the chip.
@@ -467,7 +495,7 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 4 ? 2 : 1) void attn_prefi
   // Z, the Z / 8 values from x Z / 8 on.  (Measured on the 2B, 9B and 27B head shapes at 1,024 to 6,000 tokens: 25
   // to 65 % faster wherever there are more blocks than CUs, 2 to 6 % slower where all blocks run at once.)
   int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
-  if (xcd_map) {
+  if (!PARTS && xcd_map) {
     const int X = gridDim.x, Y = gridDim.y, Z = gridDim.z;
     const long lin = bx + (long)X * (by + (long)Y * bz);
     const int xcd = (int)(lin & 7);
@@ -478,10 +506,20 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 4 ? 2 : 1) void attn_prefi
     bx = (int)(r % X);
     by = (int)(r / X);
   }
+  int tile = (int)gridDim.x - 1 - bx, part = 0, n_parts = 1;
+  if constexpr (PARTS) {
+    const int Z = nKV * passes, i = __builtin_amdgcn_readfirstlane((int)blockIdx.x / (Z * n_seqs));
+    const uint32_t e = plan.entry[i];
+    bx = i;
+    by = __builtin_amdgcn_readfirstlane((int)blockIdx.x / Z % n_seqs);
+    bz = __builtin_amdgcn_readfirstlane((int)blockIdx.x % Z);
+    tile = e & 0xffff;
+    part = (e >> 16) & 0xff;
+    n_parts = e >> 24;
+  }
   const int b = by, kvh = bz / passes, hh = (bz % passes) * HB + wave % HB;
   const int tokens = 16 * NW / HB;
   const int t_begin = cu_seqlens[b], n_new = cu_seqlens[b + 1] - t_begin;
-  const int tile = (int)gridDim.x - 1 - bx;
   const int block_first = tile * tokens;                     // first token of the block among the sequence's new ones
   if (block_first >= n_new) return;                          // the whole block
   const int start_len = context_lens[b] - n_new;
@@ -495,7 +533,13 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 4 ? 2 : 1) void attn_prefi
   const ScoreConsts sc(scale, cap);
   // the block's run of key blocks, this set's part of it, and this wave's own within that
   const int block_last_pos = start_len + min(block_first + tokens, n_new) - 1;
-  const int run_begin = (window > 0 ? max(0, start_len + block_first + 1 - window) : 0) >> 5, run_end = block_last_pos >> 5;
+  int run_begin = (window > 0 ? max(0, start_len + block_first + 1 - window) : 0) >> 5, run_end = block_last_pos >> 5;
+  const int last_block = run_end;
+  if constexpr (PARTS) {                                     // (of fewer blocks of keys than parts, some have none)
+    const int n = run_end - run_begin + 1, begin = run_begin + n * part / n_parts;
+    run_end = run_begin + n * (part + 1) / n_parts - 1;
+    run_begin = begin;
+  }
   const int steps = (run_end - run_begin + KS) / KS;         // of the first set: ceil(blocks / KS)
   const int kb_begin = run_begin + set * steps, kb_end = min(run_end, kb_begin + steps - 1);
   const int my_begin = max(kb_begin, (window > 0 ? max(0, start_len + first + 1 - window) : 0) >> 5);
@@ -503,7 +547,7 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 4 ? 2 : 1) void attn_prefi
 
   Core<DT, 1> c;
   c.init();
-  if (sink && set == 0 && hh < group) c.start_at_sink(0, sink[kvh * group + hh], lane);
+  if (sink && set == 0 && part == 0 && hh < group) c.start_at_sink(0, sink[kvh * group + hh], lane);
   {
     const bf16_t* qrow = q + ((size_t)(t_begin + (tok_ok ? my_tok : 0)) * nH + kvh * group + (hh < group ? hh : 0)) * D;
 #pragma unroll
@@ -517,7 +561,7 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 4 ? 2 : 1) void attn_prefi
   // end is the last piece.
   u32x4 st[CH];
   auto fetch = [&](int kb32) {
-    kb32 = min(min(kb32, max(kb_end, kb_begin)), run_end);
+    kb32 = min(min(kb32, max(kb_end, kb_begin)), last_block);
     const int page = bt[kb32 >> 1];
     const u32x4* kp = reinterpret_cast<const u32x4*>(k_pool + ((size_t)page * nKV + kvh) * page_elems) + (size_t)(kb32 & 1) * 2 * DT * 64;
     const u32x4* vp = reinterpret_cast<const u32x4*>(v_pool + ((size_t)page * nKV + kvh) * page_elems) + (size_t)(kb32 & 1) * 2 * DT * 64;
@@ -560,19 +604,66 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 4 ? 2 : 1) void attn_prefi
         *reinterpret_cast<f32x4*>(&so[((size_t)wave * 16 + col) * (D + 4) + t * 16 + g * 4]) = c.o[0][t];
     }
     __syncthreads();
-    if (set == 1 || !tok_ok) return;
+    if (set == 1 || !wave_ok) return;
     const float m1 = sm[wave * 16 + col], l1 = sl[wave * 16 + col];
     const float mm = fmaxf(c.m[0], m1);
     const float f0 = (c.m[0] == -INFINITY) ? 0.f : exp2_fast(c.m[0] - mm), f1 = (m1 == -INFINITY) ? 0.f : exp2_fast(m1 - mm);
-    const float inv = 1.f / (c.l[0] * f0 + l1 * f1);
 #pragma unroll
-    for (int t = 0; t < 2 * DT; ++t) {
-      f32x4 v = c.o[0][t] * f0 + *reinterpret_cast<const f32x4*>(&so[((size_t)wave * 16 + col) * (D + 4) + t * 16 + g * 4]) * f1;
-      v *= inv;
-      uint2 pk = {pack2(v[0], v[1]), pack2(v[2], v[3])};
-      *reinterpret_cast<uint2*>(out + decode_out_index(out_layout, t_begin + my_tok, (kvh * group + hh) * D + t * 16 + g * 4, nH * D)) = pk;
+    for (int t = 0; t < 2 * DT; ++t)
+      c.o[0][t] = c.o[0][t] * f0 + *reinterpret_cast<const f32x4*>(&so[((size_t)wave * 16 + col) * (D + 4) + t * 16 + g * 4]) * f1;
+    c.l[0] = c.l[0] * f0 + l1 * f1;
+    c.m[0] = mm;
+  }
+  if constexpr (PARTS) {
+    if (n_parts > 1 && wave_ok) {
+      // a part: pairs of output registers, then the maximum and the sum, each [64 lanes] of float2
+      const size_t stride = (size_t)n_seqs * nKV * passes * NW, slot = ((size_t)by * nKV * passes + bz) * NW + wave;   // of a plan's entry
+      const unsigned at = lane * 2;
+      float* mine = parts + (bx * stride + slot) * part_floats(D);
+#pragma unroll
+      for (int t = 0; t < 2 * DT; ++t) {
+        store_far(mine + 256 * t + at, c.o[0][t][0], c.o[0][t][1]);
+        store_far(mine + 256 * t + 128 + at, c.o[0][t][2], c.o[0][t][3]);
+      }
+      store_far(mine + 512 * DT + at, c.m[0], c.l[0]);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // the part is where every XCD sees it
+      int* count = arrivals + (bx - part) * stride + slot;
+      int before = 0;
+      if (lane == 0) before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__builtin_amdgcn_readfirstlane(before) != n_parts - 1) return;
+      if (lane == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const float* first = parts + ((bx - part) * stride + slot) * part_floats(D);
+      const size_t next = stride * part_floats(D);
+      float2 ml[MAX_PARTS];                                  // (a part that there is not: the last again)
+      float mm = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < MAX_PARTS; ++j) ml[j] = load_far(first + min(j, n_parts - 1) * next + 512 * DT + at);
+#pragma unroll
+      for (int j = 0; j < MAX_PARTS; ++j) mm = fmaxf(mm, ml[j].x);
+      c.l[0] = 0.f;
+      f32x4 sum[2 * DT];
+#pragma unroll
+      for (int t = 0; t < 2 * DT; ++t) sum[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < MAX_PARTS; ++j) {
+        if (j >= n_parts) break;
+        const float f = ml[j].x == -INFINITY ? 0.f : exp2_fast(ml[j].x - mm);
+        c.l[0] += ml[j].y * f;
+        if (j == part) {
+#pragma unroll
+          for (int t = 0; t < 2 * DT; ++t) sum[t] += c.o[0][t] * f;
+        } else {
+          const float* theirs = first + j * next;
+#pragma unroll
+          for (int t = 0; t < 2 * DT; ++t) {
+            const float2 v = load_far(theirs + 256 * t + at), w = load_far(theirs + 256 * t + 128 + at);
+            sum[t] += f32x4{v.x, v.y, w.x, w.y} * f;
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 2 * DT; ++t) c.o[0][t] = sum[t];
     }
-    return;
   }
   if (!tok_ok) return;
   const float inv = 1.f / c.l[0];
@@ -865,11 +956,119 @@ extern "C" int alice_head_gate(void* out, int out_layout, const void* gate, int 
   return 0;
 }
 
+static int heads_a_block(int group) { return group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1); }
+
+// The form for heads of 128 and 256 (AUTO: none of those whose waves share keys).
+static int prefill_variant(int B, int max_new, int nH, int nKV, int d) {
+  if (d < 128) return ALICE_PREFILL_AUTO;
+  const int group = nH / nKV, hb = heads_a_block(group);
+  const long per_tile = (long)B * nKV * ceil_div(group, hb);
+  if (per_tile * ceil_div(max_new, 64 / hb) >= 2048) return ALICE_PREFILL_SHARED4;
+  if (per_tile * ceil_div(max_new, 128 / hb) >= 192) return ALICE_PREFILL_SHARED8;
+  if (per_tile * ceil_div(max_new, 64 / hb) >= 192 && max_new >= 1024) return ALICE_PREFILL_SHARED4X2;
+  return ALICE_PREFILL_AUTO;
+}
+
+// Into how many parts the keys of the longest tiles are cut for eight waves that share them, 1: not at all; the shorter tiles
+// in proportion.  From times of what either takes, in microseconds (heads of 256, one to eight prompts of 257 to 8,000 tokens, with
+// and without 500 to 4,000 tokens before them, windows of 1,024 and 4,096): a block of 32 keys 1.35 and a tile's start and end as
+// much as four of them, a launch of cut tiles 4.6 and 2 a part (the parts, 135 KB a block, to memory and back), one of
+// uncut ones 0; two sets of four waves 7.6 and 1.35 for two blocks of keys; a tile's keys over the waves of a block 6 and 0.42
+// a block of keys and wave of a CU.  Before and cut: 2B, 2,048 tokens 58 and 46, 3,072 130 and 83, 4,096 171 and 128, 640 after 2,000 53 and
+// 41; 9B, 768 after 2,000 109 and 72, 2,048 91 and 76.  With more blocks than two rounds cutting gains little.
+// Heads of 128 lose everywhere (66 -> 75 at 512 tokens after 2,000: the merge's registers leave room for one block a CU, not two).
+struct TileBlocks {                                          // blocks of 32 keys that a tile of a sequence of max_context keys sees
+  int start, max_new, tokens, window;
+  int operator()(int tile) const {
+    const int last = start + min((tile + 1) * tokens, max_new) - 1;
+    return (last >> 5) - ((window > 0 ? max(0, start + tile * tokens + 1 - window) : 0) >> 5) + 1;
+  }
+};
+
+static int prefill_cut(int B, int max_new, int max_context, int nH, int nKV, int d, int window) {
+  // (steps of up to 256 tokens may be captured for other lengths, and give the bits of uncaptured ones)
+  if (d != 256 || B < 1 || max_new <= 256 || max_context < max_new) return 1;
+  const int group = nH / nKV, hb = heads_a_block(group), tokens = 128 / hb, tiles = ceil_div(max_new, tokens);
+  const long columns = (long)B * nKV * ceil_div(group, hb);
+  if (tiles > MAX_ENTRIES || columns * tiles > 512) return 1;
+  const TileBlocks blocks_of{max_context - max_new, max_new, tokens, window};
+  int longest = 0;
+  long work = 0;
+  for (int t = 0; t < tiles; ++t) { longest = max(longest, blocks_of(t)); work += blocks_of(t); }
+  const int slots = max(1, (int)(256 / columns));            // blocks of a sequence's kv head that the chip holds at once
+  int length[MAX_ENTRIES];
+  // the chip's time in blocks of keys (1e30: more than two rounds; of two the second's longest meets the first's shortest)
+  auto rounds = [&](int n) {
+    if (n > 2 * slots) return 1e30f;
+    std::sort(length, length + n, std::greater<int>());
+    int most = length[0] + 4;
+    for (int i = slots; i < n; ++i) most = max(most, length[i] + length[2 * slots - 1 - i] + 8);
+    return (float)most;
+  };
+  const int variant = prefill_variant(B, max_new, nH, nKV, d);
+  float least;
+  if (variant == ALICE_PREFILL_SHARED8) {
+    for (int t = 0; t < tiles; ++t) length[t] = blocks_of(t);
+    least = 1.35f * rounds(tiles);
+  } else if (variant == ALICE_PREFILL_SHARED4X2) {
+    const TileBlocks half{blocks_of.start, max_new, tokens / 2, window};
+    const int n = ceil_div(max_new, tokens / 2);
+    if (n > MAX_ENTRIES) return 1;
+    for (int t = 0; t < n; ++t) length[t] = ceil_div(half(t), 2);
+    least = 7.6f + 1.35f * rounds(n);
+  } else if (variant == ALICE_PREFILL_AUTO) {
+    least = 6.f + 0.42f * work * (8 / hb) * nH * B / 256;
+  } else {
+    return 1;
+  }
+  int best = 1;
+  least *= 0.92f;                                            // (the times above are met within 8 %)
+  for (int cut = 2; cut <= MAX_PARTS; ++cut) {
+    const int size = ceil_div(longest, cut);
+    int n = 0;
+    for (int t = 0; t < tiles; ++t) {
+      const int count = ceil_div(blocks_of(t), size);
+      for (int j = 0; j < count; ++j, ++n)
+        if (n < MAX_ENTRIES) length[n] = ceil_div(blocks_of(t), count);
+    }
+    if (n > 2 * slots || n > MAX_ENTRIES) break;             // (more parts make more blocks)
+    const float cost = 4.6f + 2.f * cut + 1.35f * rounds(n);
+    if (cost < least) { least = cost; best = cut; }
+  }
+  return best;
+}
+
+static int prefill_parts(int B, int max_new, int max_context, int nH, int nKV, int d, int window, int cut, PartPlan<true>* plan) {
+  const int group = nH / nKV, hb = heads_a_block(group), tokens = 128 / hb, tiles = ceil_div(max_new, tokens);
+  const TileBlocks blocks_of{max_context - max_new, max_new, tokens, window};
+  int longest = 0, n = 0;
+  for (int t = 0; t < tiles; ++t) longest = max(longest, blocks_of(t));
+  const int size = ceil_div(longest, cut);
+  for (int t = tiles - 1; t >= 0; --t) {
+    const int count = ceil_div(blocks_of(t), size);
+    if (n + count > MAX_ENTRIES) return -1;
+    for (int j = 0; j < count; ++j) plan->entry[n++] = (uint32_t)t | (uint32_t)j << 16 | (uint32_t)count << 24;
+  }
+  return n;
+}
+
+// Cut (see prefill_cut), and for a cut of more than 1 the counts (int32 zeros) and workspace (float32) that a call with it takes.
+extern "C" int alice_attention_prefill_cut(int B, int max_new, int max_context, int nH, int nKV, int d, int window) {
+  return nKV < 1 || nH < 1 || nH % nKV ? 1 : prefill_cut(B, max_new, max_context, nH, nKV, d, window);
+}
+extern "C" long alice_attention_prefill_counts(int B, int max_new, int max_context, int nH, int nKV, int d, int window, int cut) {
+  if (d != 256 || nKV < 1 || nH < 1 || nH % nKV || B < 1 || max_new < 1 || max_context < max_new || cut < 1 || cut > MAX_PARTS) return 0;
+  PartPlan<true> plan;
+  return (long)max(0, prefill_parts(B, max_new, max_context, nH, nKV, d, window, cut, &plan)) * 8 * B * nKV *
+         ceil_div(nH / nKV, heads_a_block(nH / nKV));
+}
+extern "C" long alice_attention_prefill_workspace(long counts) { return counts * part_floats(256); }
+
 extern "C" int alice_attention_prefill(const void* q, const void* k_pool, const void* v_pool, void* out,
                                        const int* cu_seqlens, const int* context_lens, const int* block_table,
                                        int bt_stride, int B, int max_new, int nH, int nKV, int d, int page_size,
                                        float scale, float softcap, int window, int variant, int out_layout, const float* sink,
-                                       hipStream_t stream) {
+                                       int max_context, int cut, float* parts, int* arrivals, int n_arrivals, hipStream_t stream) {
   ALICE_CHECK(alice_attention_mfma_supported(d), "attention (matrix cores): head_dim %d is not covered (64, 128 or 256)", d);
   ALICE_CHECK(out_layout == 0 || (out_layout == 1 && (nH * d) % 32 == 0), "attention: unknown output layout %d", out_layout);
   ALICE_CHECK(nKV >= 1 && nH % nKV == 0, "attention: bad head counts nH=%d nKV=%d", nH, nKV);
@@ -906,41 +1105,53 @@ extern "C" int alice_attention_prefill(const void* q, const void* k_pool, const 
   } while (0)
   // Few waves (one prompt of a few thousand tokens): split every tile's keys over four waves.  Many: whole
   // tiles per wave, two heads a wave where the group is even.
-#define GOL(DT, NW, KS)                                                                                                     \
+#define GOL_AS(DT, NW, KS, PARTS, GRID, PLAN)                                                                               \
   do {                                                                                                                      \
-    const int hb = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);                                                           \
-    ALICE_CHECK((long)nKV * ceil_div(group, hb) <= 65535, "attention: too many heads for one launch");                      \
-    dim3 lgrid(ceil_div(max_new, 16 * NW / hb), B, nKV * ceil_div(group, hb));                                              \
-    const long blocks = (long)lgrid.x * lgrid.y * lgrid.z;                                                                  \
-    const int xcd_map = blocks > 256 && blocks % 8 == 0 && (8 % lgrid.z == 0 || lgrid.z % 8 == 0);                          \
     const size_t lds = (size_t)KS * 2 * 4 * DT * 1024;                                                                      \
     static bool prepared = false;                                                                                           \
     if (lds > 65536 && !prepared) {                                                                                         \
-      ALICE_CHECK(hipFuncSetAttribute((const void*)attn_prefill_shared_kernel<DT, true, NW, KS>,                            \
+      ALICE_CHECK(hipFuncSetAttribute((const void*)attn_prefill_shared_kernel<DT, true, NW, KS, PARTS>,                     \
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&                \
-                  hipFuncSetAttribute((const void*)attn_prefill_shared_kernel<DT, false, NW, KS>,                           \
+                  hipFuncSetAttribute((const void*)attn_prefill_shared_kernel<DT, false, NW, KS, PARTS>,                    \
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess,                  \
                   "attention: the device does not give a block %d bytes of LDS", (int)lds);                                 \
       prepared = true;                                                                                                      \
     }                                                                                                                       \
     if (softcap > 0.f)                                                                                                      \
-      attn_prefill_shared_kernel<DT, true, NW, KS><<<lgrid, 64 * NW * KS, lds, stream>>>((const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool, \
-          (bf16_t*)out, cu_seqlens, context_lens, block_table, bt_stride, nH, nKV, scale, softcap, window, hb, out_layout, xcd_map, sink); \
+      attn_prefill_shared_kernel<DT, true, NW, KS, PARTS><<<GRID, 64 * NW * KS, lds, stream>>>((const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool, \
+          (bf16_t*)out, cu_seqlens, context_lens, block_table, bt_stride, nH, nKV, scale, softcap, window, hb, out_layout, xcd_map, sink, PLAN, B, parts, arrivals); \
     else                                                                                                                    \
-      attn_prefill_shared_kernel<DT, false, NW, KS><<<lgrid, 64 * NW * KS, lds, stream>>>((const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool, \
-          (bf16_t*)out, cu_seqlens, context_lens, block_table, bt_stride, nH, nKV, scale, softcap, window, hb, out_layout, xcd_map, sink); \
+      attn_prefill_shared_kernel<DT, false, NW, KS, PARTS><<<GRID, 64 * NW * KS, lds, stream>>>((const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool, \
+          (bf16_t*)out, cu_seqlens, context_lens, block_table, bt_stride, nH, nKV, scale, softcap, window, hb, out_layout, xcd_map, sink, PLAN, B, parts, arrivals); \
+  } while (0)
+#define GOL(DT, NW, KS)                                                                                                     \
+  do {                                                                                                                      \
+    const int hb = heads_a_block(group);                                                                                    \
+    ALICE_CHECK((long)nKV * ceil_div(group, hb) <= 65535, "attention: too many heads for one launch");                      \
+    dim3 lgrid(ceil_div(max_new, 16 * NW / hb), B, nKV * ceil_div(group, hb));                                              \
+    const long blocks = (long)lgrid.x * lgrid.y * lgrid.z;                                                                  \
+    const int xcd_map = blocks > 256 && blocks % 8 == 0 && (8 % lgrid.z == 0 || lgrid.z % 8 == 0);                          \
+    GOL_AS(DT, NW, KS, false, lgrid, PartPlan<false>{});                                                                    \
   } while (0)
   // Which form (measured on Gemma 2 shapes): with many blocks, four waves sharing their keys; with fewer, eight
   // (half as many blocks, half the key traffic); with too few blocks to fill the chip, the keys of a block split
   // over two sets of four waves, or one tile's keys split over a block's waves.  Small heads spend their time in
   // the softmax arithmetic and gain nothing from sharing.
-  if (variant == ALICE_PREFILL_AUTO && d >= 128) {
-    const int hb = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
-    const long per_tile = (long)B * nKV * ceil_div(group, hb);
-    if (per_tile * ceil_div(max_new, 64 / hb) >= 2048) variant = ALICE_PREFILL_SHARED4;
-    else if (per_tile * ceil_div(max_new, 128 / hb) >= 192) variant = ALICE_PREFILL_SHARED8;
-    else if (per_tile * ceil_div(max_new, 64 / hb) >= 192 && max_new >= 1024) variant = ALICE_PREFILL_SHARED4X2;
+  if (cut > 1) {
+    ALICE_CHECK(variant == ALICE_PREFILL_AUTO && d == 256 && cut <= MAX_PARTS && parts && arrivals && max_context >= max_new,
+                "attention: keys cannot be cut in %d parts here", cut);
+    const int hb = heads_a_block(group), xcd_map = 0;
+    const long columns = (long)B * nKV * ceil_div(group, hb);
+    PartPlan<true> plan;
+    const int entries = prefill_parts(B, max_new, max_context, nH, nKV, d, window, cut, &plan);
+    ALICE_CHECK(entries > 0 && entries * columns < (1 << 28), "attention: too many tiles for keys in %d parts", cut);
+    ALICE_CHECK(entries * columns * 8 <= n_arrivals, "attention: %ld arrival counts are needed, found %d", entries * columns * 8, n_arrivals);
+    const dim3 pgrid((unsigned)(entries * columns));
+    GOL_AS(8, 8, 1, true, pgrid, plan);
+    ALICE_LAUNCH_CHECK();
+    return 0;
   }
+  if (variant == ALICE_PREFILL_AUTO) variant = prefill_variant(B, max_new, nH, nKV, d);
   if (variant == ALICE_PREFILL_SHARED4 || variant == ALICE_PREFILL_SHARED8 || variant == ALICE_PREFILL_SHARED4X2) {
     if (variant == ALICE_PREFILL_SHARED4) { if (d == 64) GOL(2, 4, 1); else if (d == 128) GOL(4, 4, 1); else GOL(8, 4, 1); }
     else if (variant == ALICE_PREFILL_SHARED8) { if (d == 64) GOL(2, 8, 1); else if (d == 128) GOL(4, 8, 1); else GOL(8, 8, 1); }
@@ -958,6 +1169,7 @@ extern "C" int alice_attention_prefill(const void* q, const void* k_pool, const 
     else { if (gh == 2) GO(8, 2); else GO(8, 1); }
   }
 #undef GOL
+#undef GOL_AS
 #undef GOS
 #undef GO
   ALICE_LAUNCH_CHECK();

@@ -53,6 +53,8 @@ class StepContext:
     # that both kinds of step add in the same order and give the same bits
     rounded_seqs: int = 0
     rounded_context: int = 0
+    # zeros that the step's attention kernels count arrivals in and leave as zeros, one layer after the other
+    arrivals: Optional[torch.Tensor] = None
 
 
 Want = Union[str, Sequence[Sequence[int]]]

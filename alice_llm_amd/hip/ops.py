@@ -62,7 +62,8 @@ def _declare(lib) -> None:
         "alice_gelu_mul_rows": [P, I, P, I, I, I, P, P, I, I, I, I, I, P],
         "alice_linear_rope_cache": [P, I, P, I, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P],
         "alice_attention_mfma_supported": [I],
-        "alice_attention_prefill": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, F, I, I, I, P, P],
+        "alice_attention_prefill": [P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, F, I, I, I, P, I, I, P, P, I, P],
+        "alice_attention_prefill_cut": [I, I, I, I, I, I, I],
         "alice_attention_decode": [P, P, P, P, P, P, P, I, I, I, I, I, I, F, F, I, I, I, P, I, P, P],
         "alice_attention_generic": [P, I, P, P, P, P, P, P, I, I, I, I, I, I, F, F, I, P, I, I, P, I, P],
         "alice_attention_f32_supported": [I, I, I, I],
@@ -121,6 +122,10 @@ def _declare(lib) -> None:
         fn.restype = I
     lib.alice_attention_decode_workspace.argtypes = [I, I, I, I]
     lib.alice_attention_decode_workspace.restype = L
+    lib.alice_attention_prefill_counts.argtypes = [I, I, I, I, I, I, I, I]
+    lib.alice_attention_prefill_counts.restype = L
+    lib.alice_attention_prefill_workspace.argtypes = [L]
+    lib.alice_attention_prefill_workspace.restype = L
     lib.alice_attention_split_workspace.argtypes = [I, I, I, I, I, I]
     lib.alice_attention_split_workspace.restype = L
     lib.alice_mlstm_chunks_workspace.argtypes = [I, I, I, I, I, I]
@@ -1548,14 +1553,30 @@ def decode_splits(n_seqs: int, num_kv_heads: int, max_context: int, head_dim: in
 PREFILL_AUTO, PREFILL_TILES, PREFILL_SPLIT, PREFILL_SHARED4, PREFILL_SHARED8, PREFILL_SHARED4X2 = 0, 1, 2, 3, 4, 5
 
 
+def prefill_cut(n_seqs: int, max_new: int, max_context: int, num_heads: int, num_kv_heads: int, head_dim: int,
+                window: Optional[int]) -> int:
+    """Into how many parts attention_prefill() had best cut the keys of a step's longest tiles; 1: not at all."""
+    return library().alice_attention_prefill_cut(n_seqs, max_new, max_context, num_heads, num_kv_heads, head_dim, int(window or 0))
+
+
+def prefill_counts(n_seqs: int, max_new: int, max_context: int, num_heads: int, num_kv_heads: int, head_dim: int,
+                   window: Optional[int], cut: int) -> int:
+    """Arrival counts that attention_prefill() takes for keys in `cut` parts."""
+    return library().alice_attention_prefill_counts(n_seqs, max_new, max_context, num_heads, num_kv_heads, head_dim, int(window or 0), cut)
+
+
 def attention_prefill(q, k_pool, v_pool, out, cu_seqlens, context_lens, block_table, *, num_heads: int, n_seqs: int,
                       max_new: int, max_context: int, scale: float, softcap: Optional[float], window: Optional[int],
-                      variant: int = PREFILL_AUTO, out_layout: int = LAYOUT_ROW, sink: Optional[torch.Tensor] = None) -> None:
+                      variant: int = PREFILL_AUTO, out_layout: int = LAYOUT_ROW, sink: Optional[torch.Tensor] = None,
+                      cut: int = 1, arrivals: Optional[torch.Tensor] = None) -> None:
     """Prompt attention on the matrix cores.  variant: whole query tiles per wave; one tile's keys split over a
     block's four waves (what fills the chip when there are few tiles); or the four or eight waves of a block
     sharing each block of keys and values through LDS.  AUTO picks by the grid's size.
     out_layout FRAG16: `out` is a flat buffer of ceil16(T) * num_heads * d elements in fragment order.
-    sink: float32 [num_heads], exp(sink) joins the softmax's denominator."""
+    sink: float32 [num_heads], exp(sink) joins the softmax's denominator.
+    cut: prefill_cut(); more than 1 spreads the keys of the longest tiles over that many blocks (AUTO, heads of 256).
+    arrivals, then: int32 zeros, prefill_counts() of them or more, which the call leaves as zeros.  Calls that share them follow
+    one another on a stream."""
     n_pages, nKV, page_size, d = k_pool.shape
     T = q.shape[0]
     _dev(q, "q", torch.bfloat16, (T, num_heads * d))
@@ -1570,10 +1591,16 @@ def attention_prefill(q, k_pool, v_pool, out, cu_seqlens, context_lens, block_ta
     _dev(block_table, "block_table", torch.int32)
     if block_table.dim() != 2 or block_table.shape[0] < n_seqs or (max_context - 1) // page_size >= block_table.shape[1]:
         raise HipLibraryError(f"{max_context} keys are beyond the block table {tuple(block_table.shape)}")
+    if cut > 1:
+        _dev(arrivals, "arrivals", torch.int32)
+        counts = prefill_counts(n_seqs, max_new, max_context, num_heads, nKV, d, window, cut)
+        parts = torch.empty(library().alice_attention_prefill_workspace(counts), dtype=torch.float32, device=q.device)
     _call("alice_attention_prefill", q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), out.data_ptr(),
           cu_seqlens.data_ptr(), context_lens.data_ptr(), block_table.data_ptr(), block_table.shape[1], n_seqs,
           max_new, num_heads, nKV, d, page_size, float(scale), float(softcap or 0.0), int(window or 0), int(variant),
-          int(out_layout), _opt(sink, "sink", torch.float32, (num_heads,)), _stream())
+          int(out_layout), _opt(sink, "sink", torch.float32, (num_heads,)), int(max_context),
+          int(cut), None if cut <= 1 else parts.data_ptr(), None if cut <= 1 else arrivals.data_ptr(),
+          0 if cut <= 1 else arrivals.numel(), _stream())
 
 
 def attention_decode(q, k_pool, v_pool, out, context_lens, block_table, *, num_heads: int, max_context: int,
@@ -1674,10 +1701,15 @@ def attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, out: 
             if gate is not None and res[2]:
                 return                                         # gated where the key splits were combined
         else:
+            sizes = (ctx.n_seqs, ctx.max_new, ctx.max_context, num_heads, nKV, k_pool.shape[3], window)
+            cut = prefill_cut(*sizes)
+            arrivals = getattr(ctx, "arrivals", None)
+            if cut > 1 and (arrivals is None or arrivals.numel() < prefill_counts(*sizes, cut)):
+                arrivals = ctx.arrivals = torch.zeros(prefill_counts(*sizes, cut), dtype=torch.int32, device=q.device)
             attention_prefill(q, k_pool, v_pool, out, ctx.cu_seqlens, ctx.context_lens, block_table,
                               num_heads=num_heads, n_seqs=ctx.n_seqs, max_new=ctx.max_new,
                               max_context=ctx.max_context, scale=scale, softcap=softcap, window=window,
-                              out_layout=out_layout, sink=sink)
+                              out_layout=out_layout, sink=sink, cut=cut, arrivals=arrivals)
         if gate is not None:
             head_gate(out, out_layout, gate, q.shape[0], num_heads, k_pool.shape[3])
         return
