@@ -395,10 +395,14 @@ __global__ __launch_bounds__(1024) void add_norm_row_kernel(const int* __restric
   }
 }
 
-// The same operation for many rows (prompts): one wave per row, four rows a block, four consecutive
-// elements a lane at a time (H a multiple of 4, at most 256 * K4); or, for rows too wide for one wave's
-// registers, two waves per row (WPR = 2, at most 512 * K4 elements: the first wave takes the first 256 * K4),
-// whose sums meet in LDS.  Reduction orders differ from the block-per-row kernels by rounding only.
+// The same operation for many rows (prompts): WPR waves a row and RB rows a block, four consecutive elements a lane at a time
+// (H a multiple of 4, at most 256 * K4 * WPR; the first wave of two takes the first 256 * K4), whose sums meet in LDS.
+// Reduction orders differ from the block-per-row kernels by rounding only.  Memory bounds it (a row is read twice and written one
+// and a half times), and how many loads are in flight: two waves with 7 float4 a lane each have 128 registers, so that 16 waves fit a CU;
+// one with 14 had 286, and 4 fit.  Output in fragment order goes through LDS: from the registers a wave writes 32 pieces of
+// 16 bytes, from LDS 64 consecutive bytes of RB = 4 rows, and the blocks of a tile of 16 rows are one XCD's, whose L2 puts
+// the lines together.  14,494 rows of 3,584, in fragment order 197 -> 167 us, in rows 189 -> 143 (a copy's rate: 138);
+// 2,048 of 3,584 27.2 -> 19.7; 2,048 of 2,304 13.3 -> 12.2; 8,192 of 4,608 in fragment order 147 -> 128.
 template <typename TW> __device__ __forceinline__ float4 load4_f32(const TW* p, int e);
 template <> __device__ __forceinline__ float4 load4_f32<float>(const float* p, int e) { return *reinterpret_cast<const float4*>(p + e); }
 template <> __device__ __forceinline__ float4 load4_f32<bf16_t>(const bf16_t* p, int e) {
@@ -406,19 +410,24 @@ template <> __device__ __forceinline__ float4 load4_f32<bf16_t>(const bf16_t* p,
   return float4{bf16_bits_to_f32(v.x & 0xffffu), bf16_bits_to_f32(v.x >> 16), bf16_bits_to_f32(v.y & 0xffffu), bf16_bits_to_f32(v.y >> 16)};
 }
 
-template <typename TW, typename TO, bool FULL, bool LN, int K4, int WPR>
-__global__ __launch_bounds__(256) void add_norm_rows_kernel(float* __restrict__ resid, const float* __restrict__ branch,
+template <typename TW, typename TO, bool FULL, bool LN, int K4, int WPR, int RB>
+__global__ __launch_bounds__(64 * WPR * RB, K4 <= 7 ? 4 : 1) void add_norm_rows_kernel(float* __restrict__ resid, const float* __restrict__ branch,
                                                             int n_partials, size_t partial_stride,
                                                             const TW* __restrict__ w_post, const TW* __restrict__ w_pre,
                                                             const TW* __restrict__ b_pre,
                                                             TO* __restrict__ out, int T, int H,
                                                             float eps_post, float eps_pre, float off_post, float off_pre,
                                                             int out_layout) {
-  __shared__ float red[LN ? 3 : 2][4];
+  __shared__ float red[LN ? 3 : 2][RB * WPR];
+  extern __shared__ __align__(16) char staged[];             // [RB rows][2 H + 64 bytes], with out_layout FRAG16
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, part = wave % WPR;
-  const int r_own = blockIdx.x * (4 / WPR) + wave / WPR;
-  if (WPR == 1 && r_own >= T) return;
-  const bool row_ok = r_own < T;                              // two waves a row: every wave reaches the barriers
+  int block = blockIdx.x;
+  if (out_layout == 1) {
+    constexpr int G = 16 / RB;                               // blocks of a tile of 16 rows
+    block = ((block >> 3) / G * 8 + (block & 7)) * G + (block >> 3) % G;
+  }
+  const int r_own = block * RB + wave / WPR;
+  const bool row_ok = r_own < T;                              // (every wave reaches the barriers)
   const int r = row_ok ? r_own : T - 1;
   const size_t src = (size_t)r * H;
   int e[K4];
@@ -512,11 +521,21 @@ __global__ __launch_bounds__(256) void add_norm_rows_kernel(float* __restrict__ 
         o = float4{o.x + b.x, o.y + b.y, o.z + b.z, o.w + b.w};
       }
     }
-    const size_t at = out_index(out_layout, r, e[k], H);     // four consecutive elements are neighbours in both layouts
     if constexpr (sizeof(TO) == 4) {
-      *reinterpret_cast<float4*>((float*)out + at) = o;
+      *reinterpret_cast<float4*>((float*)out + src + e[k]) = o;
     } else {
-      *reinterpret_cast<uint2*>((bf16_t*)out + at) = uint2{pack_bf16x2(o.x, o.y), pack_bf16x2(o.z, o.w)};
+      const uint2 pair = {pack_bf16x2(o.x, o.y), pack_bf16x2(o.z, o.w)};
+      if (out_layout == 1) *reinterpret_cast<uint2*>(staged + (size_t)(wave / WPR) * (2 * H + 64) + 2 * e[k]) = pair;
+      else *reinterpret_cast<uint2*>((bf16_t*)out + src + e[k]) = pair;
+    }
+  }
+  if (sizeof(TO) == 2 && out_layout == 1) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < H / 8 * RB; i += 64 * WPR * RB) {   // a piece of eight elements: row i % RB, elements 8 (i / RB) on
+      const int row = block * RB + i % RB;
+      if (row < T)
+        *reinterpret_cast<uint4*>((bf16_t*)out + out_index(1, row, i / RB * 8, H)) =
+            *reinterpret_cast<const uint4*>(staged + (size_t)(i % RB) * (2 * H + 64) + i / RB * 16);
     }
   }
 }
@@ -545,12 +564,13 @@ extern "C" int alice_add_norm(float* resid, const float* branch, int n_partials,
 // (what a kernel's first loads need comes first: these arguments arrive in registers, see build.py)
 #define ARGS rows, H, n_partials, resid, branch, (size_t)partial_stride, (const TW*)w_post, (const TW*)w_pre, (const TW*)b_pre, (TO*)out, \
              eps_post, eps_pre, off_post, off_pre, out_layout
-  // Many rows, no gather: a wave per row (two from 4,097 elements on).  From 320 rows: below, a block per row
-  // fills more of the chip (measured at 2,304 and 3,584 elements: up to 256 rows the block-per-row kernel is 0.5
-  // to 6 us faster, from 384 rows on the wave-per-row kernel is, by half at 2,048 rows).
+  // Many rows, no gather: a wave per row (two from 1,025 elements on: at 2,048 rows of 2,048 12.5 and 11.3 us).  From 320 rows:
+  // below, a block per row fills more of the chip (measured at 2,304 and 3,584 elements: up to 256 rows the block-per-row kernel is
+  // 0.5 to 6 us faster, from 384 rows on this one is, by half at 2,048 rows).
   const bool aligned = (((uintptr_t)resid | (uintptr_t)branch | (uintptr_t)out | (uintptr_t)w_post | (uintptr_t)w_pre | (uintptr_t)b_pre) & 15) == 0;
   const int k4 = (!rows && aligned && T >= 320 && H % 4 == 0 && H >= 256 && H <= 8192 && (partial_stride % 4 == 0 || !branch)) ? ceil_div(H, 256) : 0;
-#define ROWS(TW, TO, FULL, LN, K4, WPR) add_norm_rows_kernel<TW, TO, FULL, LN, K4, WPR><<<ceil_div(T, 4 / WPR), 256, 0, stream>>>( \
+#define ROWS(TW, TO, FULL, LN, K4, WPR, RB) add_norm_rows_kernel<TW, TO, FULL, LN, K4, WPR, RB>                                  \
+    <<<out_layout == 1 ? ceil_div(T, 128) * (128 / RB) : ceil_div(T, RB), 64 * WPR * RB, out_layout == 1 ? RB * (2 * H + 64) : 0, stream>>>( \
     resid, branch, n_partials, (size_t)partial_stride, (const TW*)w_post, (const TW*)w_pre, (const TW*)b_pre, (TO*)out, T, H,   \
     eps_post, eps_pre, off_post, off_pre, out_layout)
   // Fewer rows, or a gather: four elements a thread where width and addresses allow it.
@@ -558,11 +578,12 @@ extern "C" int alice_add_norm(float* resid, const float* branch, int n_partials,
   const int threads4 = ceil_div(ceil_div(H, H <= 4096 ? 4 : 8), 64) * 64;
 #define LAUNCH(TW, TO, FULL, LN)                                                                     \
   do {                                                                                               \
-    if (k4 > 0 && k4 <= 4) ROWS(TW, TO, FULL, LN, 4, 1);                                             \
-    else if (k4 > 4 && k4 <= 9) ROWS(TW, TO, FULL, LN, 9, 1);                                        \
-    else if (k4 > 9 && k4 <= 16) ROWS(TW, TO, FULL, LN, 16, 1);                                      \
-    else if (k4 > 16 && k4 <= 18) ROWS(TW, TO, FULL, LN, 9, 2);                                      \
-    else if (k4 > 18) ROWS(TW, TO, FULL, LN, 16, 2);                                                 \
+    if (k4 > 0 && k4 <= 4) ROWS(TW, TO, FULL, LN, 4, 1, 4);                                          \
+    else if (k4 > 4 && k4 <= 8) ROWS(TW, TO, FULL, LN, 4, 2, 4);                                     \
+    else if (k4 > 8 && k4 <= 10) ROWS(TW, TO, FULL, LN, 5, 2, 4);                                    \
+    else if (k4 > 10 && k4 <= 14) ROWS(TW, TO, FULL, LN, 7, 2, 4);                                   \
+    else if (k4 > 14 && k4 <= 18) ROWS(TW, TO, FULL, LN, 9, 2, 2);                                   \
+    else if (k4 > 18) ROWS(TW, TO, FULL, LN, 16, 2, 2);                                              \
     else if (by_four && H <= 4096) add_norm_row_kernel<TW, TO, FULL, LN, 1><<<T, threads4, 0, stream>>>(ARGS); \
     else if (by_four) add_norm_row_kernel<TW, TO, FULL, LN, 2><<<T, threads4, 0, stream>>>(ARGS);    \
     else if (ept == 1) add_norm_regs_kernel<TW, TO, FULL, LN, 1><<<T, threads, 0, stream>>>(ARGS);   \
