@@ -4,7 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define ALICE_ABI_VERSION 16
+#define ALICE_ABI_VERSION 17
 
 #define ALICE_EPI_NONE 0
 #define ALICE_EPI_GEGLU 1     // W = [gate; up] stacked; epi_param 0: y = gelu_tanh(gate x) * (up x); epi_param = limit > 0:
@@ -127,6 +127,8 @@ int alice_attention_generic(const void* q, int dtype, const void* k_pool, const 
 // bfloat16 attention on the matrix cores over a cache in the fragment layout (kv_layout 1 of
 // alice_rope_cache_write): prompts, and single tokens with the keys split over `splits` blocks.  sink (float32 [nH] or null):
 // exp(sink[h]) joins the softmax's denominator of head h.
+// A prompt's cut (alice_attention_prefill_cut; 1: none) spreads the keys of its longest tiles over that many blocks; it takes that many
+// counts (int32 zeros, left as zeros) and the workspace of so many counts, for one call at a time.
 int alice_attention_mfma_supported(int d);
 int alice_attention_prefill(const void* q, const void* k_pool, const void* v_pool, void* out,
                             const int* cu_seqlens, const int* context_lens, const int* block_table,

@@ -401,7 +401,8 @@ __global__ __launch_bounds__(1024) void add_norm_row_kernel(const int* __restric
 // and a half times), and how many loads are in flight: two waves with 7 float4 a lane each have 128 registers, so that 16 waves fit a CU;
 // one with 14 had 286, and 4 fit.  Output in fragment order goes through LDS: from the registers a wave writes 32 pieces of
 // 16 bytes, from LDS 64 consecutive bytes of RB = 4 rows, and the blocks of a tile of 16 rows are one XCD's, whose L2 puts
-// the lines together.  14,494 rows of 3,584, in fragment order 197 -> 167 us, in rows 189 -> 143 (a copy's rate: 138);
+// the lines together.  14,494 rows of 3,584, in fragment order 197 -> 167 us over buffers in turn and 200 -> 137 in a prompt, in rows 189
+// -> 143 (a copy's rate: 138);
 // 2,048 of 3,584 27.2 -> 19.7; 2,048 of 2,304 13.3 -> 12.2; 8,192 of 4,608 in fragment order 147 -> 128.
 template <typename TW> __device__ __forceinline__ float4 load4_f32(const TW* p, int e);
 template <> __device__ __forceinline__ float4 load4_f32<float>(const float* p, int e) { return *reinterpret_cast<const float4*>(p + e); }

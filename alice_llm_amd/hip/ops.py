@@ -21,7 +21,7 @@ LAYOUT_ROW, LAYOUT_FRAG16 = 0, 1
 KV_ROW, KV_FRAGMENT = 0, 1
 LINEAR_AUTO, LINEAR_GENERIC, LINEAR_SKINNY, LINEAR_MFMA, LINEAR_TILED_W16, LINEAR_TILED_W32 = 0, 1, 2, 3, 4, 5
 LINEAR_LARGE_256, LINEAR_LARGE_192, LINEAR_LARGE_128 = 6, 7, 8
-ABI_VERSION = 16
+ABI_VERSION = 17
 GATED_SILU = -1.0        # epi_param of EPI_GEGLU that picks silu(gate) * up
 UNARY_RELU2 = -1.0       # epi_param of EPI_SOFTCAP that picks the square of max(y, 0) instead of the capped form
 UNARY_SILU = -2.0        # likewise y * sigmoid(y)
