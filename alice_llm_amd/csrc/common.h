@@ -133,10 +133,9 @@ __device__ __forceinline__ float gelu_tanh_f(float z, bool full) {
   return z * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(q));
 }
 
-__device__ __forceinline__ float silu_f(float z, bool full) {
-  if (full) return z / (1.f + expf(-z));
-  return z * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
-}
+// z / (1 + e^-z) by one division, rounded once, here and in unary_act() below.  (By the hardware's reciprocal and a product the l2
+// error over [-9, 9] goes from 4.3e-8 to 4.6e-8, for 0.7 % of a prompt whose feed-forwards are SiLU gates.)
+__device__ __forceinline__ float silu_f(float z, bool full) { return z / (1.f + (full ? expf(-z) : __expf(-z))); }
 
 // The gated product of two stacked matrices' outputs (gate g, up u), the epilogue ALICE_EPI_GEGLU.  Its
 // parameter picks the form: 0 gives gelu_tanh(g) * u; a positive `limit` gives the limited form
@@ -155,7 +154,7 @@ __device__ __forceinline__ float gated_act(float g, float u, float limit, bool f
 // The function of one output element, the epilogue ALICE_EPI_SOFTCAP.  Its parameter picks the form: a positive cap
 // gives cap * tanh(v / cap); ALICE_UNARY_RELU2 (-1) the square of max(v, 0); ALICE_UNARY_SILU (-2) v * sigmoid(v).
 __device__ __forceinline__ float unary_act(float v, float p, bool full) {
-  if (p < -1.5f) return v / (1.f + (full ? expf(-v) : __expf(-v)));
+  if (p < -1.5f) return silu_f(v, full);
   if (p < 0.f) {
     const float r = fmaxf(v, 0.f);
     return r * r;
