@@ -85,8 +85,9 @@ int alice_linear_split_hint(int M, int N, int K, int w_layout);
 // The same by what the operands are: for row-major weights their dtypes, and whether both start on 16 bytes (above: float32, aligned);
 // for weights in fragment order with the activations in rows.
 int alice_linear_split_hint_for(int M, int N, int K, int w_layout, int x_dtype, int w_dtype, int aligned);
-// Whether products of M tokens by every fragment-layout matrix of K inner elements add in one order for activations in rows and in
-// fragment order.
+// Whether products of M tokens by every fragment-layout matrix of K inner elements, taken whole or in one number of slices, add in one
+// order for activations in rows and in fragment order.  (How many slices either order would like is another matter: from 448 tokens on
+// fragment order has a kernel more, and the two numbers above differ.)
 int alice_linear_one_order(int M, int K);
 // Which tile a float32 product of more than 16 tokens takes on the bfloat16 instruction (operands in three parts), -1: the 32-bit one.
 // (No caller needs it to take a product: tests ask, so that their sizes reach every tile.)

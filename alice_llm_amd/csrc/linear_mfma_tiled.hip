@@ -70,8 +70,9 @@ bool low_tiles(int M, int K) { return M > 32 || K >= 4096; }
 
 }  // namespace
 
-// Whether products of M tokens add in one order by every matrix of K inner elements, activations in rows or in fragment order.
-// (From 65 tokens on a wave of the tiled kernel goes through a slice from its first element to its last, whatever the tile.)
+// Whether products of M tokens add in one order by every matrix of K inner elements, activations in rows or in fragment order, the
+// number of slices being the same.  (From 65 tokens on a wave of the tiled kernel, and of the one with larger tiles, goes through a slice
+// from its first element to its last, whatever the tile.)
 extern "C" int alice_linear_one_order(int M, int K) { return M > 64 || !low_tiles(M, K); }
 
 TiledPlan alice_mfma_tiled_plan(int M, int N, int K, int epi, int y_dtype, int split, int x_frag) {

@@ -417,9 +417,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, *, n_out: int, k_i
           int(full_precision), int(x_layout), int(y_layout), _stream())
 
 
-def linear_split_hint(M: int, N: int, K: int, layout: int, x: Optional[torch.Tensor] = None, w: Optional[torch.Tensor] = None) -> int:
+def linear_split_hint(M: int, N: int, K: int, layout: int, x=None, w: Optional[torch.Tensor] = None) -> int:
     """The slices of the inner dimension that a product would like.  x, w: its operands, whose dtypes and alignment choose the kernel of
-    row-major weights (float32 and aligned if not given); activations in fragment order (anything but a tensor) have a kernel more."""
+    row-major weights (float32 and aligned if not given); activations in fragment order (FragmentActs) have a kernel more, unless
+    they are to be added up as rows are."""
+    if x is not None and not isinstance(x, torch.Tensor) and x.as_rows:
+        x = x.data
     if x is None or w is None or (layout == LAYOUT_FRAG16 and not isinstance(x, torch.Tensor)):
         return library().alice_linear_split_hint(M, N, K, layout)
     return library().alice_linear_split_hint_for(M, N, K, layout, dtype_code(x.dtype), dtype_code(w.dtype),
@@ -427,7 +430,8 @@ def linear_split_hint(M: int, N: int, K: int, layout: int, x: Optional[torch.Ten
 
 
 def linear_one_order(M: int, K: int) -> bool:
-    """Whether M tokens' products of K inner elements add in one order for activations in rows and in fragment order."""
+    """Whether M tokens' products of K inner elements, whole or in one number of slices, add in one order for activations in rows and in
+    fragment order."""
     return bool(library().alice_linear_one_order(M, K))
 
 

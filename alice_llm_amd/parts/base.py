@@ -59,10 +59,12 @@ class FragmentActs:
     """bfloat16 activations [rows, cols] stored in the order in which the matrix-core kernels read them
     ([rows/16][cols/32][64 lanes][8], rows padded to 16): a wave fetches a whole operand tile with one
     contiguous 1 KB read instead of sixteen pieces of 64 bytes.  Only parts that declare
-    `accepts_fragment_activations` are ever handed one; everything else sees plain tensors."""
+    `accepts_fragment_activations` are ever handed one; everything else sees plain tensors.
+    as_rows: a consumer that adds up slices of the inner dimension takes as many as for the same numbers in rows, so that
+    both orders give the same bits."""
 
-    def __init__(self, data: torch.Tensor, rows: int, cols: int):
-        self.data, self.rows, self.cols = data, rows, cols
+    def __init__(self, data: torch.Tensor, rows: int, cols: int, as_rows: bool = False):
+        self.data, self.rows, self.cols, self.as_rows = data, rows, cols, as_rows
 
     @property
     def shape(self):
@@ -77,9 +79,9 @@ class FragmentActs:
         return precision.act == torch.bfloat16 and rows >= 1 and cols % 32 == 0
 
     @staticmethod
-    def empty(rows: int, cols: int, device) -> "FragmentActs":
+    def empty(rows: int, cols: int, device, as_rows: bool = False) -> "FragmentActs":
         padded = -(-rows // 16) * 16
-        return FragmentActs(torch.empty(padded * cols, dtype=torch.bfloat16, device=device), rows, cols)
+        return FragmentActs(torch.empty(padded * cols, dtype=torch.bfloat16, device=device), rows, cols, as_rows)
 
 
 # --------------------------------------------------------------------------- parameters

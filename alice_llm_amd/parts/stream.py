@@ -131,7 +131,8 @@ class ResidualStream:
             return out
         pre = _fused_pre(norm)
         # Without a norm the stream itself, rounded, is what the consumer reads.  It stays in rows where products choose between two
-        # kernels by the order of the activations, which add up in different orders (33 to 64 tokens; rows of 4,096 elements from one on).
+        # kernels by the order of the activations, which add up in different orders (33 to 64 tokens; rows of 4,096 elements from one on);
+        # elsewhere the slices are those of rows too.
         if fragments and (pre is not None or norm is None and ops.linear_one_order(T, H)) and out_dtype == torch.bfloat16 \
                 and FragmentActs.possible(self.precision, T, H):
             post = self._post
@@ -141,7 +142,7 @@ class ResidualStream:
             n, b = self._partials() if self._branch is not None else (1, None)
             w_post, eps_post, off_post = pf if (pf is not None and b is not None) else (None, 0.0, 0.0)
             w_pre, eps_pre, off_pre, b_pre = pre if pre is not None else (None, 0.0, 0.0, None)
-            out = FragmentActs.empty(T, H, self.x.device)
+            out = FragmentActs.empty(T, H, self.x.device, as_rows=norm is None)
             ops.add_norm(self.x, b, w_post, w_pre, out.data, eps_post=eps_post, eps_pre=eps_pre, off_post=off_post,
                          off_pre=off_pre, b_pre=b_pre, n_partials=n, full_precision=self.precision.full, out_layout=ops.LAYOUT_FRAG16)
             self._branch = None

@@ -41,8 +41,9 @@ def test_rows_where_the_order_of_the_sums_would_change(T):
 
 
 # outputs and widths of a delta layer's projection (tiled from one token on if it were given fragment order), and streaming ones; GeGLU
-@pytest.mark.parametrize("T", [1, 8, 16, 32, 33, 64, 65, 130])
-@pytest.mark.parametrize("N,H", [(12576, 4096), (12224, 4096), (2304, 4128), (12576, 2048), (2560, 1024)])
+# (from 448 tokens on fragment order has a kernel more, which would like other slices)
+@pytest.mark.parametrize("T", [1, 8, 16, 32, 33, 64, 65, 130, 447, 448, 700, 2048])
+@pytest.mark.parametrize("N,H", [(12576, 4096), (12224, 4096), (2304, 4128), (12576, 2048), (2560, 1024), (2304, 2304)])
 def test_the_product_behind_the_stream_without_a_norm(T, N, H):
     """The same bits whether the consumer says that it reads fragment order or not."""
     precision = Precision.of("bfloat16")
