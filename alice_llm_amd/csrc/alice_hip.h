@@ -4,7 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#define ALICE_ABI_VERSION 17
+#define ALICE_ABI_VERSION 18
 
 #define ALICE_EPI_NONE 0
 #define ALICE_EPI_GEGLU 1     // W = [gate; up] stacked; epi_param 0: y = gelu_tanh(gate x) * (up x); epi_param = limit > 0:
@@ -89,6 +89,9 @@ int alice_linear_split_hint_for(int M, int N, int K, int w_layout, int x_dtype, 
 // order for activations in rows and in fragment order.  (How many slices either order would like is another matter: from 448 tokens on
 // fragment order has a kernel more, and the two numbers above differ.)
 int alice_linear_one_order(int M, int K);
+// The features of the 256-token tile that AUTO takes for a product with weights and activations in fragment order, 0: the kernels of smaller
+// tiles; split_k 0: behind the number of slices that alice_linear_split_hint proposes.  (No caller needs it to take a product: tests ask.)
+int alice_linear_large_tile(int M, int N, int K, int epilogue, float epi_param, int y_dtype, int split_k);
 // Which tile a float32 product of more than 16 tokens takes on the bfloat16 instruction (operands in three parts), -1: the 32-bit one.
 // (No caller needs it to take a product: tests ask, so that their sizes reach every tile.)
 int alice_linear_thirds_tile(int M, int N, int K, int geglu, int split_k);

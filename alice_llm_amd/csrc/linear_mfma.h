@@ -231,6 +231,8 @@ int alice_mfma_tiled_narrow(const void* x, const void* w, void* y, int y_dtype, 
 // that one stays; split 0: the slices are chosen too).  Activations in fragment order.
 struct LargePlan { int ft, split; };
 LargePlan alice_mfma_large_plan(int M, int N, int K, int epi, float epi_param, int y_dtype, int split, const TiledPlan& tiled);
+// What a call with `split` slices takes: the tile behind the proposed number of slices if that is what it was given, else the plan for it.
+LargePlan alice_mfma_large_choice(int M, int N, int K, int epi, float epi_param, int y_dtype, int split);
 bool alice_mfma_large_takes(int M, int N, int K, int epi, float epi_param, int y_dtype, int split);
 int alice_mfma_large(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int split, int ft, int y_frag,
                      hipStream_t s);

@@ -106,7 +106,7 @@ int alice_linear_frag(const void* x, int x_dtype, const void* w, void* y, int y_
     return alice_mfma_large(x, w, y, M, N, K, epi, epi_param, split_k, 16 - 4 * (variant - ALICE_LINEAR_LARGE_256), y_frag, stream);
   }
   if (variant == ALICE_LINEAR_AUTO && x_frag) {
-    const LargePlan large = alice_mfma_large_plan(M, N, K, epi, epi_param, y_dtype, split_k, alice_mfma_tiled_plan(M, N, K, epi, y_dtype, split_k, 1));
+    const LargePlan large = alice_mfma_large_choice(M, N, K, epi, epi_param, y_dtype, split_k);
     if (large.ft) return alice_mfma_large(x, w, y, M, N, K, epi, epi_param, split_k, large.ft, y_frag, stream);
   }
   const int force_wn = variant == ALICE_LINEAR_TILED_W16 ? 1 : variant == ALICE_LINEAR_TILED_W32 ? 2 : 0;

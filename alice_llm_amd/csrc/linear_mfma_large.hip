@@ -281,6 +281,19 @@ LargePlan alice_mfma_large_plan(int M, int N, int K, int epi, float epi_param, i
   return best;
 }
 
+// (A plan weighs both kernels at their own numbers of slices.  Weighed again at the number that was chosen, the other kernel may win: 2 slices
+// of 1,100 tokens by 2,304 x 2,048 are proposed for this one, where the tiled kernel would like 3 and take 2 a little faster.)
+LargePlan alice_mfma_large_choice(int M, int N, int K, int epi, float epi_param, int y_dtype, int split) {
+  if (epi == ALICE_EPI_NONE && y_dtype == DT_F32) {
+    const LargePlan proposed = alice_mfma_large_plan(M, N, K, epi, epi_param, y_dtype, 0, alice_mfma_tiled_plan(M, N, K, epi, y_dtype, 0, 1));
+    if (proposed.split == split) return proposed;
+  }
+  return alice_mfma_large_plan(M, N, K, epi, epi_param, y_dtype, split, alice_mfma_tiled_plan(M, N, K, epi, y_dtype, split, 1));
+}
+extern "C" int alice_linear_large_tile(int M, int N, int K, int epilogue, float epi_param, int y_dtype, int split_k) {
+  return M > 64 ? 16 * alice_mfma_large_choice(M, N, K, epilogue, epi_param, y_dtype, split_k).ft : 0;
+}
+
 int alice_mfma_large(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int split, int ft, int y_frag,
                      hipStream_t s) {
   const int NT = N / 16 * (epi == ALICE_EPI_GEGLU ? 2 : 1), gx = ceil_div(NT, ft), gy = ceil_div(M, 16 * LARGE_XT);

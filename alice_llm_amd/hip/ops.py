@@ -21,7 +21,7 @@ LAYOUT_ROW, LAYOUT_FRAG16 = 0, 1
 KV_ROW, KV_FRAGMENT = 0, 1
 LINEAR_AUTO, LINEAR_GENERIC, LINEAR_SKINNY, LINEAR_MFMA, LINEAR_TILED_W16, LINEAR_TILED_W32 = 0, 1, 2, 3, 4, 5
 LINEAR_LARGE_256, LINEAR_LARGE_192, LINEAR_LARGE_128 = 6, 7, 8
-ABI_VERSION = 17
+ABI_VERSION = 18
 GATED_SILU = -1.0        # epi_param of EPI_GEGLU that picks silu(gate) * up
 UNARY_RELU2 = -1.0       # epi_param of EPI_SOFTCAP that picks the square of max(y, 0) instead of the capped form
 UNARY_SILU = -2.0        # likewise y * sigmoid(y)
@@ -51,6 +51,7 @@ def _declare(lib) -> None:
         "alice_linear_split_hint": [I, I, I, I],
         "alice_linear_split_hint_for": [I, I, I, I, I, I, I],
         "alice_linear_one_order": [I, I],
+        "alice_linear_large_tile": [I, I, I, I, F, I, I],
         "alice_linear_thirds_tile": [I, I, I, I, I],
         "alice_to_frag16": [P, P, I, I, P],
         "alice_frag16_supported": [I, I, I],
@@ -433,6 +434,13 @@ def linear_one_order(M: int, K: int) -> bool:
     """Whether M tokens' products of K inner elements, whole or in one number of slices, add in one order for activations in rows and in
     fragment order."""
     return bool(library().alice_linear_one_order(M, K))
+
+
+def linear_large_tile(M: int, N: int, K: int, *, epilogue: int = EPI_NONE, epi_param: float = 0.0, dtype: torch.dtype = torch.float32,
+                      split_k: int = 1) -> int:
+    """The features of the 256-token tile that a product takes with weights and activations in fragment order, 0 for a smaller tile.
+    split_k 0: the tile behind the slices that linear_split_hint() proposes."""
+    return library().alice_linear_large_tile(M, N, K, epilogue, float(epi_param), dtype_code(dtype), split_k)
 
 
 def linear_thirds_tile(M: int, N: int, K: int, geglu: bool = False, split_k: int = 1) -> int:

@@ -18,3 +18,10 @@ def test_activations_that_stand_for_rows_have_the_slices_of_rows(N, K):
             assert ops.linear_split_hint(M, N, K, ops.LAYOUT_FRAG16, FragmentActs(flat, M, K, as_rows=True), w) == row, M
         differ += ops.linear_split_hint(M, N, K, ops.LAYOUT_FRAG16, FragmentActs(flat, M, K), w) != row
     assert differ or (N, K) in [(2560, 1024)]           # (of so few inner elements neither order wants slices at many tokens)
+
+
+@pytest.mark.parametrize("N,K", SIZES)
+def test_a_product_takes_the_kernel_that_its_slices_were_proposed_for(N, K):
+    for M in list(range(384, 1300, 16)) + list(range(433, 8200, 61)):
+        split = ops.linear_split_hint(M, N, K, ops.LAYOUT_FRAG16)
+        assert ops.linear_large_tile(M, N, K, split_k=split) == ops.linear_large_tile(M, N, K, split_k=0), (M, split)
