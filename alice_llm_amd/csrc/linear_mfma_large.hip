@@ -240,17 +240,22 @@ bool alice_mfma_large_takes(int M, int N, int K, int epi, float epi_param, int y
   return per % 2 == 0 && last >= 4 && last <= per;
 }
 
-// Microseconds of a product by this kernel and by the tiled one with its widest tile, fitted to 108 products of the 2B, 9B and 27B
-// widths and of 2,048 at 512 to 8,192 tokens (to 4.6 and 2.3 %; the choices that follow are 0.3 % behind the best measured ones on
-// average).  A block of this kernel takes 0.66, 0.49 or 0.37 us a k-tile and 4 to 10 us a tile beside them; the last round of blocks, with part of the
-// chip idle, runs faster for the power that these leave.  Every slice is a partial result that the add and norm behind it reads.
+// Microseconds of a product by this kernel and by the tiled one with its widest tile.  A block of this kernel takes 0.64, 0.52 or 0.42 us a
+// k-tile and 4 to 11 us a tile beside them; the last round of blocks, with part of the chip idle, runs faster for the power that these
+// leave.  Every slice is a partial result that the add and norm behind it reads.
+// Sums without an epilogue: fitted to 170 products, ten matrices of the 2B, 9B and 27B widths and of 2,048 and 2,560 at 450 to 8,192 tokens,
+// with weights that no cache holds, as a model's layers find them (to 4 % either kernel's; the choices that follow are 1.08 times as fast as
+// the tiled kernel, 1.4 % behind the best measured ones on average, and none is more than 2 % slower than the tiled kernel.  Costs
+// fitted to weights that a cache held took 128 features too cheaply: 39 of the 170 lost 2 to 12 %, 1,024 tokens by 2,304 x 2,048 for one).
+// Gated products: fitted to 34 of them at 512 to 8,192 tokens.
 static float large_cost(int M, int N, int K, int epi, int ft, int split) {
   const bool gated = epi == ALICE_EPI_GEGLU;
-  const float k_tile = ft == 16 ? 0.66f : ft == 12 ? 0.49f : 0.37f;
-  const float tile = gated ? (ft == 16 ? 7.f : ft == 12 ? 5.9f : 3.9f) : (ft == 16 ? 10.4f : ft == 12 ? 7.8f : 5.1f);
+  const float k_tile = gated ? (ft == 16 ? 0.66f : ft == 12 ? 0.49f : 0.37f) : (ft == 16 ? 0.64f : ft == 12 ? 0.516f : 0.42f);
+  const float tile = gated ? (ft == 16 ? 7.f : ft == 12 ? 5.9f : 3.9f) : (ft == 16 ? 10.6f : ft == 12 ? 7.9f : 5.f);
+  const float part = gated ? 0.68f : ft == 16 ? 0.726f : ft == 12 ? 0.759f : 0.825f;     // a round's time with hardly a block in it
   const int items = ceil_div(N / 16 * (gated ? 2 : 1), ft) * ceil_div(M, 16 * LARGE_XT) * split, rounds = ceil_div(items, 256);
-  const float busy = rounds - 1 + 0.68f + 0.32f * (items / 256.f - (rounds - 1));
-  return 3.6f + busy * (ceil_div(K / 32, split) * k_tile + tile) + 0.9e-6f * (split - 1) * M * N;
+  const float busy = rounds - 1 + part + (1.f - part) * (items / 256.f - (rounds - 1));
+  return 3.5f + busy * (ceil_div(K / 32, split) * k_tile + tile) + 0.99e-6f * (split - 1) * M * N;
 }
 static float tiled_wide_cost(int M, int N, int K, int epi, int split) {
   const bool gated = epi == ALICE_EPI_GEGLU;
@@ -262,15 +267,21 @@ static float tiled_wide_cost(int M, int N, int K, int epi, int split) {
 }
 
 // The tile for a product that the tiled kernel would take as `tiled` says, ft 0: that one.  split 0: the slices are chosen too.  From 448
-// tokens on, below which the tiled kernel's narrow tiles, in one round of blocks that wait for memory, are the better ones; where it
-// has a narrow tile for the sums of a few hundred tokens the cost above is its widest tile's and this kernel must promise a quarter
-// less.  1.03 to 1.35 times as fast at the products it takes: 2B gate/up at 2,048 tokens 147 -> 130 us, down 80 -> 73 with two
-// slices instead of three, output 31 -> 28; 9B at 8,192 tokens gate/up 1,249 -> 1,140, down 677 -> 615, output 206 -> 186; whole
-// prompts of 2,048 tokens of 2B 10,711 -> 9,890, of 14,494 of 9B 227.4 -> 216.9 ms.
+// tokens on: below, sums in one round of blocks that wait for memory are better off in the tiled kernel's tiles (this kernel
+// gains at a few gated products of 320 to 447 tokens, 9B at 384 101 -> 83 us, for which the costs are not fitted).  Where the tiled kernel has a
+// narrow tile for the sums of a few hundred tokens the cost above is its widest tile's and this kernel must promise a quarter less; where it has
+// low blocks of long slices, two on some CUs, it takes a fifth longer than the cost says (4,096 inner elements, 342 blocks: 74 us for 57).
+// With weights that no cache holds, 2B down at 2,048 tokens 87 -> 72 us, 9B output at 3,072 92 -> 76, 27B down at 1,024 307 -> 241; gated
+// ones, with weights from a cache, 2B at 2,048 tokens 147 -> 130, 9B at 8,192 1,249 -> 1,140.
 LargePlan alice_mfma_large_plan(int M, int N, int K, int epi, float epi_param, int y_dtype, int split, const TiledPlan& tiled) {
   LargePlan best{0, tiled.split};
   if (M < 448 || !alice_frag16_supported(N * (epi == ALICE_EPI_GEGLU ? 2 : 1), K, epi)) return best;
-  float least = tiled_wide_cost(M, N, K, epi, split > 0 ? split : tiled.split) * (tiled.wn < 4 && epi != ALICE_EPI_GEGLU ? 0.74f : 0.97f);
+  const int slices = split > 0 ? split : tiled.split;
+  float least = tiled_wide_cost(M, N, K, epi, slices);
+  if (epi == ALICE_EPI_GEGLU) least *= 0.97f;
+  else if (tiled.wn < 4) least *= 0.74f;
+  else if (tiled.tm == 4 && (long)ceil_div(N, 256) * ceil_div(M, 64) * slices > 256 && ceil_div(K / 32, slices) >= 64) least *= 1.19f;
+  else least *= 0.99f;
   for (int sp = split > 0 ? split : 1; sp <= (split > 0 ? split : 4); ++sp) {
     if (!alice_mfma_large_takes(M, N, K, epi, epi_param, y_dtype, sp) || (sp > 1 && split == 0 && K / 32 / sp < 16)) continue;
     for (int ft = 16; ft >= 8; ft -= 4) {
