@@ -10,8 +10,8 @@ loops over prompts and requests (llama3.rs:17783-17835).
 """
 from __future__ import annotations
 
-from dataclasses import dataclass
-from typing import List, Optional, Sequence, Union
+from dataclasses import dataclass, field
+from typing import Dict, List, Optional, Sequence, Tuple, Union
 
 import numpy as np
 import torch
@@ -53,8 +53,10 @@ class StepContext:
     # that both kinds of step add in the same order and give the same bits
     rounded_seqs: int = 0
     rounded_context: int = 0
-    # zeros that the step's attention kernels count arrivals in and leave as zeros, one layer after the other
-    arrivals: Optional[torch.Tensor] = None
+    # prompt attention with the keys of the longest tiles cut over several blocks: how many parts and counts layers of some sizes
+    # take (worked out once a step), and, a stream each, the zeros that kernels count arrivals in and leave as zeros, one after the other
+    cuts: Dict[tuple, Tuple[int, int]] = field(default_factory=dict)
+    arrivals: Dict[int, torch.Tensor] = field(default_factory=dict)
 
 
 Want = Union[str, Sequence[Sequence[int]]]

@@ -1577,6 +1577,25 @@ def prefill_counts(n_seqs: int, max_new: int, max_context: int, num_heads: int, 
     return library().alice_attention_prefill_counts(n_seqs, max_new, max_context, num_heads, num_kv_heads, head_dim, int(window or 0), cut)
 
 
+def _cut_of(ctx, num_heads: int, num_kv_heads: int, head_dim: int, window: Optional[int], device):
+    """The cut of a step's prompt attention and the counts that it takes.  The step keeps what is worked out from its sizes, and the
+    counts for its later layers (a stream each: calls on two streams must not count in the same ones).  A context without places for
+    them gets both anew."""
+    cuts, kept = getattr(ctx, "cuts", {}), getattr(ctx, "arrivals", {})
+    sizes = (ctx.n_seqs, ctx.max_new, ctx.max_context, num_heads, num_kv_heads, head_dim, window)
+    plan = cuts.get(sizes)
+    if plan is None:
+        cut = prefill_cut(*sizes)
+        plan = cuts[sizes] = (cut, prefill_counts(*sizes, cut) if cut > 1 else 0)
+    cut, counts = plan
+    if cut == 1:
+        return 1, None
+    arrivals = kept.get(_stream())
+    if arrivals is None or arrivals.numel() < counts:
+        arrivals = kept[_stream()] = torch.zeros(counts, dtype=torch.int32, device=device)
+    return cut, arrivals
+
+
 def attention_prefill(q, k_pool, v_pool, out, cu_seqlens, context_lens, block_table, *, num_heads: int, n_seqs: int,
                       max_new: int, max_context: int, scale: float, softcap: Optional[float], window: Optional[int],
                       variant: int = PREFILL_AUTO, out_layout: int = LAYOUT_ROW, sink: Optional[torch.Tensor] = None,
@@ -1713,11 +1732,7 @@ def attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, out: 
             if gate is not None and res[2]:
                 return                                         # gated where the key splits were combined
         else:
-            sizes = (ctx.n_seqs, ctx.max_new, ctx.max_context, num_heads, nKV, k_pool.shape[3], window)
-            cut = prefill_cut(*sizes)
-            arrivals = getattr(ctx, "arrivals", None)
-            if cut > 1 and (arrivals is None or arrivals.numel() < prefill_counts(*sizes, cut)):
-                arrivals = ctx.arrivals = torch.zeros(prefill_counts(*sizes, cut), dtype=torch.int32, device=q.device)
+            cut, arrivals = _cut_of(ctx, num_heads, nKV, k_pool.shape[3], window, q.device)
             attention_prefill(q, k_pool, v_pool, out, ctx.cu_seqlens, ctx.context_lens, block_table,
                               num_heads=num_heads, n_seqs=ctx.n_seqs, max_new=ctx.max_new,
                               max_context=ctx.max_context, scale=scale, softcap=softcap, window=window,

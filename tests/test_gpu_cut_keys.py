@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from alice_llm_amd.engine.step import StepContext
 from alice_llm_amd.hip import ops
 from test_gpu_kernels import DEV, acts_from_fragments, close, frag_case
 
@@ -54,3 +55,31 @@ def test_what_is_cut():
     with pytest.raises(ops.HipLibraryError):
         ops.attention_prefill(q, kp, vp, torch.empty_like(q), cu, ctx, bt, arrivals=torch.zeros(n, dtype=torch.int32, device=DEV),
                               variant=ops.PREFILL_SHARED8, **kw)
+
+
+# a whole prompt, tokens after a prefix, and two sequences of unlike lengths; a window that asks for other counts than none does
+@pytest.mark.parametrize("lens,new,windows", [((2048,), (2048,), (None, 1900)), ((2640,), (640,), (None,)), ((1500, 900), (1000, 450), (None, 800))])
+def test_layers_of_a_step(lens, new, windows):
+    """The path of a model's layers: the step picks the cut and keeps the counts, which a layer with more of them replaces."""
+    nH, nKV, d = 8, 4, 256
+    sizes = (len(lens), max(new), max(lens), nH, nKV, d)
+    counts = {w: ops.prefill_counts(*sizes, w, ops.prefill_cut(*sizes, w)) for w in windows if ops.prefill_cut(*sizes, w) > 1}
+    assert len(set(counts.values())) == len(windows)         # all are cut, with unlike numbers of counts
+    none = torch.empty(0, dtype=torch.int32, device=DEV)
+    ctx = None
+    for w in sorted(counts, key=counts.get) * 2:             # the fewest first: the second layer's counts are new ones
+        q, kp, vp, bt, cu, ctxl, ref, scale = frag_case(nH, nKV, d, lens, new, 50.0, w, seed=5, dense=True)
+        if ctx is None:
+            ctx = StepContext(tokens=none, positions=none, seq_of_token=none, slots=none, want_rows=None, cu_seqlens=cu, context_lens=ctxl,
+                              n_tokens=sum(new), n_seqs=len(lens), is_decode=False, max_new=max(new), max_context=max(lens),
+                              max_position=max(lens) - 1)
+        whole, out = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+        ops.attention_prefill(q, kp, vp, whole, cu, ctxl, bt, variant=ops.PREFILL_SHARED8, num_heads=nH, n_seqs=len(lens), max_new=max(new),
+                              max_context=max(lens), scale=scale, softcap=50.0, window=w)
+        ops.attention(q, kp, vp, out, ctx, bt, num_heads=nH, scale=scale, softcap=50.0, window=w, full_precision=False, kv_layout=ops.KV_FRAGMENT)
+        close(out, whole.double(), 4.5 * 2 ** -8, 2 ** -7)   # (the bound of the test above)
+        close(out, ref, 2e-2)
+        assert not torch.equal(out, whole)                   # it is the cut form that ran
+        (kept,) = ctx.arrivals.values()
+        assert kept.numel() >= counts[w] and not kept.any()
+    assert kept.numel() == max(counts.values()) and len(ctx.cuts) == len(windows)
