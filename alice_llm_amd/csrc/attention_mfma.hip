@@ -974,7 +974,9 @@ static int prefill_variant(int B, int max_new, int nH, int nKV, int d) {
 // and without 500 to 4,000 tokens before them, windows of 1,024 and 4,096): a block of 32 keys 1.35 and a tile's start and end as
 // much as four of them, a launch of cut tiles 4.6 and 2 a part (the parts, 135 KB a block, to memory and back), one of
 // uncut ones 0; two sets of four waves 7.6 and 1.35 for two blocks of keys; a tile's keys over the waves of a block 6 and 0.42
-// a block of keys and wave of a CU.  Before and cut: 2B, 2,048 tokens 58 and 46, 3,072 130 and 83, 4,096 171 and 128, 640 after 2,000 53 and
+// a block of keys and wave of a CU.  These are met within 8 % for most sizes, not for all: a tile's keys over the waves of a block take up to
+// 1.7 times as long as this says where every head has its own keys (1,024 tokens after 500: 55 us where a cut takes 33), four prompts of 500 1.5
+// times, and beyond two rounds, where nothing is cut, a cut could gain as well (2B, 8,000 tokens: 526 and 423).  Before and cut: 2B, 2,048 tokens 58 and 46, 3,072 130 and 83, 4,096 171 and 128, 640 after 2,000 53 and
 // 41; 9B, 768 after 2,000 109 and 72, 2,048 91 and 76.  With more blocks than two rounds cutting gains little.
 // Heads of 128 lose everywhere (66 -> 75 at 512 tokens after 2,000: the merge's registers leave room for one block a CU, not two).
 struct TileBlocks {                                          // blocks of 32 keys that a tile of a sequence of max_context keys sees
@@ -1022,7 +1024,10 @@ static int prefill_cut(int B, int max_new, int max_context, int nH, int nKV, int
     return 1;
   }
   int best = 1;
-  least *= 0.92f;                                            // (the times above are met within 8 %)
+  // What a cut must promise: of 405 sizes measured either way none is then more than 1.5 % slower than uncut and 138 are cut, 1.15 times
+  // as fast on average.  With 8 % for all of them five were 3 to 6 % slower: sequences of unlike lengths, of which the rule knows
+  // the longest alone, and windows that begin late in a prompt (2B, 2,000 and 300 tokens after 500: 107 -> 113 us).
+  least *= B > 1 || window > 0 ? 0.84f : 0.92f;
   for (int cut = 2; cut <= MAX_PARTS; ++cut) {
     const int size = ceil_div(longest, cut);
     int n = 0;
