@@ -451,7 +451,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_split_kernel(
 // leave their parts in memory, and the one that comes last adds all of them up in their order and writes the output: the bits
 // are the same whichever it is.  What they hand over goes past the L2, which another XCD does not see, by stores and loads of
 // agent scope, and nothing else needs to be seen: a wave's stores have arrived (s_waitcnt) before its count goes up, and only the wave
-// that finds all the others' counts reads.  Nobody waits for anybody.  arrivals: a count a (tile, wave), zero before the launch and after.
+// that finds all the others' counts reads, behind the branch on the count's result (which the hardware waits for there; that the
+// compiler moves no load across it is said by an empty statement that touches memory: relaxed accesses alone are in no order).  Nobody waits for anybody.  arrivals: a count a (tile, wave), zero before the launch and after.
 __device__ __forceinline__ void store_far(float* p, float a, float b) {
   __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), __builtin_bit_cast(unsigned long long, float2{a, b}), __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_AGENT);
@@ -631,6 +632,7 @@ __global__ __launch_bounds__(64 * NW * KS, NW * KS == 4 ? 2 : 1) void attn_prefi
       int before = 0;
       if (lane == 0) before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (__builtin_amdgcn_readfirstlane(before) != n_parts - 1) return;
+      asm volatile("" ::: "memory");                         // (no load of a part goes ahead of the count, which has arrived here)
       if (lane == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const float* first = parts + ((bx - part) * stride + slot) * part_floats(D);
       const size_t next = stride * part_floats(D);
