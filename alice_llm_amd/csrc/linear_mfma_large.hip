@@ -11,11 +11,11 @@ constexpr int LARGE_XT = 16;            // token tiles of a block: 256 tokens
 constexpr int LARGE_SLOTS = 5;          // k-tiles that LDS holds: 160, 140 or 120 KB
 
 // One tile of 1 KB from memory into LDS, lane l's 16 bytes to place `lds` + `AT` KB + 16 l of the block's memory.  The instruction
-// has no register for its result; what it counts on (vmcnt) is waited for ahead of the barriers below.
+// has no register for its result; what it counts on (vmcnt) is waited for ahead of the barriers below.  m0, which names the place, is an
+// operand, so that the compiler knows what it holds; after a write of it the instruction needs one wait state.
 template <int AT>
 __device__ __forceinline__ void tile_to_lds(const bf16_t* src, unsigned off, uint32_t lds) {
-  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(src), "s"(lds), "n"(AT * 1024)
-               : "memory", "m0", "scc");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(src), "{m0}"(lds + AT * 1024) : "memory");
 }
 
 enum { GATE_GELU, GATE_SILU };
