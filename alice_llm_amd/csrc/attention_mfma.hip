@@ -1115,15 +1115,11 @@ extern "C" int alice_attention_prefill(const void* q, const void* k_pool, const 
 #define GOL_AS(DT, NW, KS, PARTS, GRID, PLAN)                                                                               \
   do {                                                                                                                      \
     const size_t lds = (size_t)KS * 2 * 4 * DT * 1024;                                                                      \
-    static bool prepared = false;                                                                                           \
-    if (lds > 65536 && !prepared) {                                                                                         \
-      ALICE_CHECK(hipFuncSetAttribute((const void*)attn_prefill_shared_kernel<DT, true, NW, KS, PARTS>,                     \
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&                \
-                  hipFuncSetAttribute((const void*)attn_prefill_shared_kernel<DT, false, NW, KS, PARTS>,                    \
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess,                  \
+    static std::atomic<uint64_t> told[2] = {};                                                                              \
+    if (lds > 65536)                                                                                                        \
+      ALICE_CHECK(lds_granted((const void*)attn_prefill_shared_kernel<DT, true, NW, KS, PARTS>, (int)lds, told[0]) &&       \
+                  lds_granted((const void*)attn_prefill_shared_kernel<DT, false, NW, KS, PARTS>, (int)lds, told[1]),        \
                   "attention: the device does not give a block %d bytes of LDS", (int)lds);                                 \
-      prepared = true;                                                                                                      \
-    }                                                                                                                       \
     if (softcap > 0.f)                                                                                                      \
       attn_prefill_shared_kernel<DT, true, NW, KS, PARTS><<<GRID, 64 * NW * KS, lds, stream>>>((const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool, \
           (bf16_t*)out, cu_seqlens, context_lens, block_table, bt_stride, nH, nKV, scale, softcap, window, hb, out_layout, xcd_map, sink, PLAN, B, parts, arrivals); \
@@ -1210,12 +1206,9 @@ extern "C" int alice_attention_decode(const void* q, const void* k_pool, const v
   do {                                                                                                                      \
     auto kern = attn_decode_kernel<DT, CAP>;                                                                                \
     if (lds > 48 * 1024) {                                                                                                  \
-      static bool told = false;                                                                                             \
-      if (!told) {                                                                                                          \
-        ALICE_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 16 * (DT * 32 + 4) * (int)sizeof(float)) == hipSuccess, \
-                    "attention (decode): the device does not give a block %d bytes of LDS", (int)lds);                      \
-        told = true;                                                                                                        \
-      }                                                                                                                     \
+      static std::atomic<uint64_t> told{0};                                                                                 \
+      ALICE_CHECK(lds_granted((const void*)kern, 4 * 16 * (DT * 32 + 4) * (int)sizeof(float), told),                        \
+                  "attention (decode): the device does not give a block %d bytes of LDS", (int)lds);                        \
     }                                                                                                                       \
     kern<<<grid, 256, lds, stream>>>(context_lens, block_table, bt_stride, window, splits, reciprocal_of(splits), nKV, nH / nKV,  \
                                      (const bf16_t*)k_pool, (const bf16_t*)q, (const bf16_t*)v_pool, (bf16_t*)out, parts, scale, \

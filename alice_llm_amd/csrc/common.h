@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
+#include <atomic>
 
 #define ALICE_WAVE 64
 
@@ -185,6 +186,21 @@ void alice_set_error(const char* fmt, ...);
       return 1;                           \
     }                                     \
   } while (0)
+
+// Blocks of a kernel take more LDS than they may without asking: the device is asked once for each kernel, whichever thread comes first.
+// told: the kernel's own, a bit a device.
+inline bool lds_granted(const void* kernel, int bytes, std::atomic<uint64_t>& told) {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return false;
+  const uint64_t bit = device < 64 ? 1ull << device : 0;
+  if (told.load(std::memory_order_acquire) & bit) return true;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  told.fetch_or(bit, std::memory_order_release);
+  return true;
+}
 
 #define ALICE_LAUNCH_CHECK()                                                   \
   do {                                                                         \

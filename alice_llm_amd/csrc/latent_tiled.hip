@@ -467,12 +467,9 @@ template <int DP, int DVP, bool SINGLE>
 int launch_as(const LatentArgs& a, dim3 grid, hipStream_t stream) {
   constexpr size_t lds = SINGLE ? (size_t)DVP * VPAD * sizeof(bf16_t) + 4 * 2 * 64 * sizeof(f32x4)
                                 : ((size_t)KT * (DP + 8) + (size_t)DVP * VPAD) * sizeof(bf16_t);
-  static bool raised = false;                            // once a process and instance: more LDS than the static limit
-  if (lds > 48 * 1024 && !raised) {
-    ALICE_CHECK(hipFuncSetAttribute((const void*)latent_tiled_kernel<DP, DVP, SINGLE>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds) == hipSuccess, "latent attention: %zu bytes of LDS were refused", lds);
-    raised = true;
-  }
+  static std::atomic<uint64_t> told{0};
+  ALICE_CHECK(lds <= 48 * 1024 || lds_granted((const void*)latent_tiled_kernel<DP, DVP, SINGLE>, (int)lds, told),
+              "latent attention: %zu bytes of LDS were refused", lds);
   latent_tiled_kernel<DP, DVP, SINGLE><<<grid, 256, lds, stream>>>(a);
   return 0;
 }

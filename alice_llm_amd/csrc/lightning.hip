@@ -430,18 +430,15 @@ __global__ __launch_bounds__(NT) void lightning_outputs_kernel(LightningArgs a) 
 }
 
 template <typename K>
-bool raise_lds(K kernel, size_t bytes, bool* raised) {
-  if (bytes <= 48 * 1024 || *raised) return true;
-  if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) return false;
-  *raised = true;                      // once a process and instance
-  return true;
+bool raise_lds(K kernel, size_t bytes, std::atomic<uint64_t>* told) {
+  return bytes <= 48 * 1024 || lds_granted((const void*)kernel, 160 * 1024, *told);
 }
 
 template <typename TX, int TW, bool V4>
 int launch_chunks(const LightningArgs& a, long chunks, hipStream_t stream) {
   constexpr int DP = 64 * TW;
   constexpr size_t lds_s = (size_t)(CHUNK * (DP + 16) + CHUNK * 16) * sizeof(float), lds_o = (size_t)2 * CHUNK * (DP + 18) * sizeof(float);
-  static bool rs = false, r1 = false, r2 = false;
+  static std::atomic<uint64_t> rs{0}, r1{0}, r2{0};
   ALICE_CHECK(raise_lds(lightning_states_kernel<TX, TW, V4>, lds_s, &rs), "lightning: %zu bytes of LDS were refused", lds_s);
   lightning_states_kernel<TX, TW, V4><<<dim3(a.n_seqs, a.H, ceil_div(a.dv, 16)), NT, lds_s, stream>>>(a);
   ALICE_LAUNCH_CHECK();

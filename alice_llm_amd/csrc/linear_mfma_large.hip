@@ -218,12 +218,8 @@ template <int EPI, typename TO, int FT, int GATE>
 int launch_large(const void* x, const void* w, void* y, const LargeShape& sh, int N, int y_frag, hipStream_t s) {
   auto kern = linear_large_kernel<EPI, TO, FT, GATE>;
   constexpr int lds = LARGE_SLOTS * (LARGE_XT + FT) * 1024;
-  static bool told = false;
-  if (!told) {
-    ALICE_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess,
-                "linear: the device does not give a block %d bytes of LDS", lds);
-    told = true;
-  }
+  static std::atomic<uint64_t> told{0};
+  ALICE_CHECK(lds_granted((const void*)kern, lds, told), "linear: the device does not give a block %d bytes of LDS", lds);
   const int blocks = sh.items < 256 ? 8 * ceil_div(sh.items, 8) : 256;
   kern<<<blocks, 256, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, sh, (TO*)y, N, y_frag);
   ALICE_LAUNCH_CHECK();

@@ -244,12 +244,8 @@ int launch_skinny(const void* x, const void* w, void* y, int M, int N, int K, in
   do {                                                                                                                         \
     auto kern = linear_skinny_kernel<RT, MT, NWV, EPI, TO, false, XFV, STREAMV, WINV>;                                        \
     if (lds > 48 * 1024) {                                                                                                     \
-      static bool told = false;                                                                                                \
-      if (!told) {                                                                                                             \
-        ALICE_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess, \
-                    "linear: the device does not give a block %d bytes of LDS", (int)lds);                                     \
-        told = true;                                                                                                           \
-      }                                                                                                                        \
+      static std::atomic<uint64_t> told{0};                                                                                    \
+      ALICE_CHECK(lds_granted((const void*)kern, (int)lds, told), "linear: the device does not give a block %d bytes of LDS", (int)lds); \
     }                                                                                                                          \
     kern<<<grid, THREADS, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, EPI == ALICE_EPI_ROPE ? (void*)ra.positions : y, ra.seq_of_token, \
                                     M, KT, NT, per, reciprocal_of(ceil_div(per, NWV)),                                         \

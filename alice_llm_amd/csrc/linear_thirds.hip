@@ -342,10 +342,8 @@ int launch(const float* x, const float* w, float* y, int M, int N, int K, int ep
   const int wide = N % 4 == 0 && ((uintptr_t)y & 15) == 0;
   const int grid = 8 * ceil_div((long)mt * nt * split, 8);
   auto kern = linear_thirds_kernel<TM, TN>;
-  if (LDS > 48 * 1024) {
-    static const hipError_t told = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-    ALICE_CHECK(told == hipSuccess, "linear: the device does not give a block %d bytes of LDS", LDS);
-  }
+  static std::atomic<uint64_t> told{0};
+  ALICE_CHECK(LDS <= 48 * 1024 || lds_granted((const void*)kern, LDS, told), "linear: the device does not give a block %d bytes of LDS", LDS);
   kern<<<grid, 512, LDS, stream>>>(x, w, y, M, N, K, kslice, split, mt, nt, epi, param, full, wide);
   ALICE_LAUNCH_CHECK();
   return 0;

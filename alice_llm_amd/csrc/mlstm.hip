@@ -798,12 +798,8 @@ extern "C" int alice_mlstm_chunks(const float* proj, int row_w, const float* bia
   const size_t lds = chunk_lds_bytes(C, VS, d);
 #define GO_MODE(CC, VV, MODE, GX)                                                                                    \
   do {                                                                                                               \
-    static bool raised = false; /* blocks of more than 64 KB of shared memory: said once per kernel */              \
-    if (!raised) {                                                                                                   \
-      hipFuncSetAttribute((const void*)mlstm_chunk_kernel<CC, VV, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
-      (void)hipGetLastError();                                                                                       \
-      raised = true;                                                                                                 \
-    }                                                                                                                \
+    static std::atomic<uint64_t> told{0}; /* (blocks of more than 64 KB; refused, the launch says so) */            \
+    (void)lds_granted((const void*)mlstm_chunk_kernel<CC, VV, MODE>, 160 * 1024, told);                              \
     mlstm_chunk_kernel<CC, VV, MODE><<<dim3(GX, H, dv / VS), CTHREADS, lds, stream>>>(proj, row_w, bias_i, bias_f, work, dens, \
         cu_seqlens, slots, S, n, m, H, d, dv, cap, ws);                                                              \
   } while (0)
