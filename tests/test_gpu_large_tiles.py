@@ -78,7 +78,8 @@ def test_what_it_does_not_take():
 
 @pytest.mark.parametrize("M", [447, 448, 1000, 2048])
 @pytest.mark.parametrize("N,K", [(2304, 9216), (2304, 2048), (4096, 2304)])
-def test_the_slices_that_are_proposed_are_taken(M, N, K):
+def test_the_proposed_slices_have_the_tiled_kernels_bits(M, N, K):
+    """(Which kernel takes them does not show in the bits: test_product_slices.py asks the rule.)"""
     x, w = rnd(M, K, seed=9, dtype=torch.bfloat16), rnd(N, K, seed=10, dtype=torch.bfloat16)
     split = ops.linear_split_hint(M, N, K, ops.LAYOUT_FRAG16)
     wf = ops.to_frag16(w)
