@@ -398,8 +398,9 @@ __global__ __launch_bounds__(1024) void add_norm_row_kernel(const int* __restric
 // The same operation for many rows (prompts): WPR waves a row and RB rows a block, four consecutive elements a lane at a time
 // (H a multiple of 4, at most 256 * K4 * WPR; the first wave of two takes the first 256 * K4), whose sums meet in LDS.
 // Reduction orders differ from the block-per-row kernels by rounding only.  Memory bounds it (a row is read twice and written one
-// and a half times), and how many loads are in flight: two waves with 7 float4 a lane each have 128 registers, so that 16 waves fit a CU;
-// one with 14 had 286, and 4 fit.  Output in fragment order goes through LDS: from the registers a wave writes 32 pieces of
+// and a half times), and how many loads are in flight: two waves with 7 float4 a lane each have 128 registers, so that 16 waves fit a CU
+// (the launch bound asks for that; with bfloat16 output two to four registers more, up to 20 bytes a lane, go to scratch); one with 14 had 286,
+// and 4 fit.  Output in fragment order goes through LDS: from the registers a wave writes 32 pieces of
 // 16 bytes, from LDS 64 consecutive bytes of RB = 4 rows, and the blocks of a tile of 16 rows are one XCD's, whose L2 puts
 // the lines together.  14,494 rows of 3,584, in fragment order 197 -> 167 us over buffers in turn and 200 -> 137 in a prompt, in rows 189
 // -> 143 (a copy's rate: 138);

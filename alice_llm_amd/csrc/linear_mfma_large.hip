@@ -40,7 +40,8 @@ struct LargeShape {
 //     until the next barrier.
 // A block goes through its tiles of the output in one run: behind a tile's last k-tiles the next tile's first ones are staged,
 // so that only the epilogue stands between two tiles.  K-tiles come in pairs: a slice has an even number of them, four at least.
-// GATE: which gated form (a choice at run time, made once an output, took the epilogue of GELU from 5 to 8 us a tile).
+// GATE: which gated form (a choice at run time, made once an output, took the epilogue of GELU from 5 to 8 us a tile).  The gated
+// instances of 256 features keep one to three registers in scratch, written and read outside the loops over k-tiles.
 template <int EPI, typename TO, int FT, int GATE>
 __global__ __launch_bounds__(256, 1) void linear_large_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ wf, LargeShape sh,
                                                            TO* __restrict__ y, int N, int y_frag) {
