@@ -230,6 +230,7 @@ int alice_mfma_tiled_narrow(const void* x, const void* w, void* y, int y_dtype, 
 // The kernel of tiles of 256 tokens by 16 ft features, and its tile for a product that the tiled kernel would take as `tiled` says (ft 0:
 // that one stays; split 0: the slices are chosen too).  Activations in fragment order.
 struct LargePlan { int ft, split; };
+constexpr int LARGE_FROM = 448;              // tokens; below, no rule of it need be asked
 LargePlan alice_mfma_large_plan(int M, int N, int K, int epi, float epi_param, int y_dtype, int split, const TiledPlan& tiled);
 // What a call with `split` slices takes: the tile behind the proposed number of slices if that is what it was given, else the plan for it.
 LargePlan alice_mfma_large_choice(int M, int N, int K, int epi, float epi_param, int y_dtype, int split);

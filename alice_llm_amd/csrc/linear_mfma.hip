@@ -105,7 +105,7 @@ int alice_linear_frag(const void* x, int x_dtype, const void* w, void* y, int y_
                 "linear: no kernel with tiles of 256 tokens for M=%d N=%d K=%d in %d slices with this epilogue, output type and activation layout", M, N, K, split_k);
     return alice_mfma_large(x, w, y, M, N, K, epi, epi_param, split_k, 16 - 4 * (variant - ALICE_LINEAR_LARGE_256), y_frag, stream);
   }
-  if (variant == ALICE_LINEAR_AUTO && x_frag) {
+  if (variant == ALICE_LINEAR_AUTO && x_frag && M >= LARGE_FROM) {
     const LargePlan large = alice_mfma_large_choice(M, N, K, epi, epi_param, y_dtype, split_k);
     if (large.ft) return alice_mfma_large(x, w, y, M, N, K, epi, epi_param, split_k, large.ft, y_frag, stream);
   }

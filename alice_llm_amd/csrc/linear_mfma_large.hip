@@ -272,7 +272,7 @@ static float tiled_wide_cost(int M, int N, int K, int epi, int split) {
 // ones, with weights from a cache, 2B at 2,048 tokens 147 -> 130, 9B at 8,192 1,249 -> 1,140.
 LargePlan alice_mfma_large_plan(int M, int N, int K, int epi, float epi_param, int y_dtype, int split, const TiledPlan& tiled) {
   LargePlan best{0, tiled.split};
-  if (M < 448 || !alice_frag16_supported(N * (epi == ALICE_EPI_GEGLU ? 2 : 1), K, epi)) return best;
+  if (M < LARGE_FROM || !alice_frag16_supported(N * (epi == ALICE_EPI_GEGLU ? 2 : 1), K, epi)) return best;
   const int slices = split > 0 ? split : tiled.split;
   float least = tiled_wide_cost(M, N, K, epi, slices);
   if (epi == ALICE_EPI_GEGLU) least *= 0.97f;
@@ -299,7 +299,7 @@ LargePlan alice_mfma_large_choice(int M, int N, int K, int epi, float epi_param,
   return alice_mfma_large_plan(M, N, K, epi, epi_param, y_dtype, split, alice_mfma_tiled_plan(M, N, K, epi, y_dtype, split, 1));
 }
 extern "C" int alice_linear_large_tile(int M, int N, int K, int epilogue, float epi_param, int y_dtype, int split_k) {
-  return M > 64 ? 16 * alice_mfma_large_choice(M, N, K, epilogue, epi_param, y_dtype, split_k).ft : 0;
+  return M >= LARGE_FROM ? 16 * alice_mfma_large_choice(M, N, K, epilogue, epi_param, y_dtype, split_k).ft : 0;
 }
 
 int alice_mfma_large(const void* x, const void* w, void* y, int M, int N, int K, int epi, float epi_param, int split, int ft, int y_frag,
