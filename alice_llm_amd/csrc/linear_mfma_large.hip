@@ -244,7 +244,8 @@ bool alice_mfma_large_takes(int M, int N, int K, int epi, float epi_param, int y
 // with weights that no cache holds, as a model's layers find them (to 4 % either kernel's; the choices that follow are 1.08 times as fast as
 // the tiled kernel, 1.4 % behind the best measured ones on average, and none is more than 2 % slower than the tiled kernel.  Costs
 // fitted to weights that a cache held took 128 features too cheaply: 39 of the 170 lost 2 to 12 %, 1,024 tokens by 2,304 x 2,048 for one).
-// Gated products: fitted to 34 of them at 512 to 8,192 tokens.
+// Gated products: fitted to 34 of them at 512 to 8,192 tokens, of weights that a cache held; of 68 with cold weights one is 1.8 % slower than
+// the tiled kernel (2,048 wide at 505 tokens) and two that could gain an eighth stay with it (2B and 2,048 wide at 600).
 static float large_cost(int M, int N, int K, int epi, int ft, int split) {
   const bool gated = epi == ALICE_EPI_GEGLU;
   const float k_tile = gated ? (ft == 16 ? 0.66f : ft == 12 ? 0.49f : 0.37f) : (ft == 16 ? 0.64f : ft == 12 ? 0.516f : 0.42f);
@@ -268,6 +269,8 @@ static float tiled_wide_cost(int M, int N, int K, int epi, int split) {
 // gains at a few gated products of 320 to 447 tokens, 9B at 384 101 -> 83 us, for which the costs are not fitted).  Where the tiled kernel has a
 // narrow tile for the sums of a few hundred tokens the cost above is its widest tile's and this kernel must promise a quarter less; where it has
 // low blocks of long slices, two on some CUs, it takes a fifth longer than the cost says (4,096 inner elements, 342 blocks: 74 us for 57).
+// Elsewhere sums must promise 2 % and gated products 3: nearer than that (2,048 tokens by 2,048 x 8,192: 60.5 and 61.4 us in one run, 63.1 and
+// 60.3 in another) a model was faster with the tiled kernel.
 // With weights that no cache holds, 2B down at 2,048 tokens 87 -> 72 us, 9B output at 3,072 92 -> 76, 27B down at 1,024 307 -> 241; gated
 // ones, with weights from a cache, 2B at 2,048 tokens 147 -> 130, 9B at 8,192 1,249 -> 1,140.
 LargePlan alice_mfma_large_plan(int M, int N, int K, int epi, float epi_param, int y_dtype, int split, const TiledPlan& tiled) {
@@ -278,7 +281,7 @@ LargePlan alice_mfma_large_plan(int M, int N, int K, int epi, float epi_param, i
   if (epi == ALICE_EPI_GEGLU) least *= 0.97f;
   else if (tiled.wn < 4) least *= 0.74f;
   else if (tiled.tm == 4 && (long)ceil_div(N, 256) * ceil_div(M, 64) * slices > 256 && ceil_div(K / 32, slices) >= 64) least *= 1.19f;
-  else least *= 0.99f;
+  else least *= 0.98f;
   for (int sp = split > 0 ? split : 1; sp <= (split > 0 ? split : 4); ++sp) {
     if (!alice_mfma_large_takes(M, N, K, epi, epi_param, y_dtype, sp) || (sp > 1 && split == 0 && K / 32 / sp < 16)) continue;
     for (int ft = 16; ft >= 8; ft -= 4) {
